@@ -591,6 +591,105 @@ __device__ __forceinline__ void match_stage_pipe(const CU32* arow, int w0, int n
 }
 
 // ---------------------------------------------------------------------------
+// Output of one pair (row gi, column gj) from its match counts: count(k) is
+// the count at k-mer length index k.  Pairs outside the pass (padding, or at
+// and below the diagonal of a self pass) write nothing.
+// ---------------------------------------------------------------------------
+template <typename P>
+__device__ __forceinline__ bool pair_valid(const P& p, int64_t gi, int64_t gj) {
+  if (p.self_mode && !p.full_square) return gi < gj && gj < p.n_cols;
+  return gi < p.n_rows && gj < p.n_cols;
+}
+
+template <typename P, typename Count>
+__device__ __forceinline__ void pair_output(const P& p, int64_t gi, int64_t gj, double bins,
+                                            double rbins, Count count) {
+  int64_t pos;
+  if (p.full_square) {
+    pos = (gi - p.square_row0) * p.out_stride_rows + gj;
+  } else if (p.self_mode) {
+    pos = p.n_cols * gi - ((gi * (gi + 1)) >> 1) + gj - 1 - gi;  // square_to_condensed
+  } else {
+    pos = gi * p.n_cols + gj;  // query-major: q * n_ref + r
+  }
+  pos -= p.out_row_offset;
+  if (p.out_kind == OUT_COUNTS) {
+    uint16_t* o = reinterpret_cast<uint16_t*>(p.out) + pos * p.n_k;
+    for (int k = 0; k < p.n_k; ++k) o[k] = (uint16_t)count(k);
+    return;
+  }
+  if (p.out_kind == OUT_JACCARD) {
+    float* o = reinterpret_cast<float*>(p.out) + pos * p.n_k;
+    for (int k = 0; k < p.n_k; ++k) {
+      o[k] = (float)jaccard_d(count(k), bins, rbins, random_for(p, k, gi, gj));
+    }
+    return;
+  }
+  if (p.out_kind == OUT_ONE_MINUS_J) {
+    // kNN on Jaccards: (float)(1 - J) of the first two k-mer lengths
+    // (src/api.cpp:368-371 narrows 1.0f - double J to float)
+    float v[2] = {INFINITY, INFINITY};
+    for (int k = 0; k < 2 && k < p.n_k; ++k) {
+      v[k] = (float)(1.0 - jaccard_d(count(k), bins, rbins, random_for(p, k, gi, gj)));
+    }
+    reinterpret_cast<float2*>(p.out)[pos] = make_float2(v[0], v[1]);
+    return;
+  }
+  // core/acc: streaming window fit.  Points before the first valid one are
+  // dropped; invalid points after the last valid one are held as pending
+  // sums and committed only if a later valid point arrives.
+  int first = -1, last = -1;
+  double sy = 0.0, sxy = 0.0, py = 0.0, pxy = 0.0;
+  for (int k = 0; k < p.n_k; ++k) {
+    const float jf = (float)jaccard_d(count(k), bins, rbins, random_for(p, k, gi, gj));
+    const bool ok = (double)jf > p.tolerance;
+    if (!ok && first < 0) continue;
+    const double x = (double)p.kvals[k];
+    const double y = log_jaccard(jf, g_log_tab);
+    if (ok) {
+      if (first < 0) {
+        first = k;
+        sy = y;
+        sxy = x * y;
+      } else {
+        sy += py + y;
+        sxy += pxy + x * y;
+      }
+      py = 0.0;
+      pxy = 0.0;
+      last = k;
+    } else {
+      py += y;
+      pxy += x * y;
+    }
+  }
+  float core = 0.0f, accd = 0.0f;
+  if (first < 0 || last - first + 1 < 2) {
+    atomicAdd(p.fail_count, 1ull);
+    atomicMin(p.fail_first, (unsigned long long)(pos + p.out_row_offset));
+    if (p.fail_rows) atomicAdd(&p.fail_rows[gi], 1u);
+  } else {
+    const double n = (double)(last - first + 1);
+    double sx = 0.0, sxx = 0.0;
+    for (int k = first; k <= last; ++k) {
+      const double x = (double)p.kvals[k];
+      sx += x;
+      sxx += x * x;
+    }
+    const double mx = sx / n;
+    const double my = sy / n;
+    // centred sums: Sxx = sum x^2 - n mx^2, Sxy = sum xy - n mx my
+    const double cxx = sxx - n * mx * mx;
+    const double cxy = sxy - n * mx * my;
+    const double slope = cxy / cxx;
+    const double intercept = my - slope * mx;
+    if (slope < 0) core = (float)(1.0 - exp(slope));
+    if (intercept < 0) accd = (float)(1.0 - exp(intercept));
+  }
+  reinterpret_cast<float2*>(p.out)[pos] = make_float2(core, accd);
+}
+
+// ---------------------------------------------------------------------------
 // Fused epilogue of one tile (run by the last of its n_k workgroups):
 // per-k counts -> random-corrected Jaccard -> dense output.  Out of line so
 // that none of its state occupies registers during the matching loop.
@@ -616,97 +715,9 @@ __device__ __noinline__ void tile_epilogue(CParams* pp, const uint16_t* tile_cou
     const int64_t gi = gi0 + q;
     for (int r = 0; r < RR; ++r) {
       const int64_t gj = col0 + lane + 64 * r;
-      bool valid;
-      if (p.self_mode) {
-        valid = p.full_square ? (gi < p.n_rows && gj < p.n_cols) : (gi < gj && gj < p.n_cols);
-      } else {
-        valid = gi < p.n_rows && gj < p.n_cols;
-      }
-      if (!valid) continue;
-      int64_t pos;
-      if (p.full_square) {
-        pos = (gi - p.square_row0) * p.out_stride_rows + gj;
-      } else if (p.self_mode) {
-        pos = p.n_cols * gi - ((gi * (gi + 1)) >> 1) + gj - 1 - gi;  // square_to_condensed
-      } else {
-        pos = gi * p.n_cols + gj;  // query-major: q * n_ref + r
-      }
-      pos -= p.out_row_offset;
+      if (!pair_valid(p, gi, gj)) continue;
       const uint16_t* cp = tbase + q * TC + 64 * r;
-      if (p.out_kind == OUT_COUNTS) {
-        uint16_t* o = reinterpret_cast<uint16_t*>(p.out) + pos * p.n_k;
-        for (int k = 0; k < p.n_k; ++k) o[k] = cp[k * kstride];
-        continue;
-      }
-      if (p.out_kind == OUT_JACCARD) {
-        float* o = reinterpret_cast<float*>(p.out) + pos * p.n_k;
-        for (int k = 0; k < p.n_k; ++k) {
-          o[k] = (float)jaccard_d(cp[k * kstride], bins, rbins, random_for(p, k, gi, gj));
-        }
-        continue;
-      }
-      if (p.out_kind == OUT_ONE_MINUS_J) {
-        // kNN on Jaccards: (float)(1 - J) of the first two k-mer lengths
-        // (src/api.cpp:368-371 narrows 1.0f - double J to float)
-        float v[2] = {INFINITY, INFINITY};
-        for (int k = 0; k < 2 && k < p.n_k; ++k) {
-          v[k] = (float)(1.0 - jaccard_d(cp[k * kstride], bins, rbins, random_for(p, k, gi, gj)));
-        }
-        reinterpret_cast<float2*>(p.out)[pos] = make_float2(v[0], v[1]);
-        continue;
-      }
-      // core/acc: streaming window fit.  Points before the first valid one are
-      // dropped; invalid points after the last valid one are held as pending
-      // sums and committed only if a later valid point arrives.
-      int first = -1, last = -1;
-      double sy = 0.0, sxy = 0.0, py = 0.0, pxy = 0.0;
-      for (int k = 0; k < p.n_k; ++k) {
-        const float jf = (float)jaccard_d(cp[k * kstride], bins, rbins, random_for(p, k, gi, gj));
-        const bool ok = (double)jf > p.tolerance;
-        if (!ok && first < 0) continue;
-        const double x = (double)p.kvals[k];
-        const double y = log_jaccard(jf, g_log_tab);
-        if (ok) {
-          if (first < 0) {
-            first = k;
-            sy = y;
-            sxy = x * y;
-          } else {
-            sy += py + y;
-            sxy += pxy + x * y;
-          }
-          py = 0.0;
-          pxy = 0.0;
-          last = k;
-        } else {
-          py += y;
-          pxy += x * y;
-        }
-      }
-      float core = 0.0f, accd = 0.0f;
-      if (first < 0 || last - first + 1 < 2) {
-        atomicAdd(p.fail_count, 1ull);
-        atomicMin(p.fail_first, (unsigned long long)(pos + p.out_row_offset));
-        if (p.fail_rows) atomicAdd(&p.fail_rows[gi], 1u);
-      } else {
-        const double n = (double)(last - first + 1);
-        double sx = 0.0, sxx = 0.0;
-        for (int k = first; k <= last; ++k) {
-          const double x = (double)p.kvals[k];
-          sx += x;
-          sxx += x * x;
-        }
-        const double mx = sx / n;
-        const double my = sy / n;
-        // centred sums: Sxx = sum x^2 - n mx^2, Sxy = sum xy - n mx my
-        const double cxx = sxx - n * mx * mx;
-        const double cxy = sxy - n * mx * my;
-        const double slope = cxy / cxx;
-        const double intercept = my - slope * mx;
-        if (slope < 0) core = (float)(1.0 - exp(slope));
-        if (intercept < 0) accd = (float)(1.0 - exp(intercept));
-      }
-      reinterpret_cast<float2*>(p.out)[pos] = make_float2(core, accd);
+      pair_output(p, gi, gj, bins, rbins, [&](int k) { return (uint32_t)cp[k * kstride]; });
     }
   }
 }
@@ -1201,6 +1212,129 @@ __global__ __launch_bounds__(WAVES * 64, 4) void dist_batch_mixed(BatchArgs a) {
       batch_tile<8, 4, 2>(pp, tile, scratch, a.ctl, wave, lane);
     }
   }
+}
+
+// ---------------------------------------------------------------------------
+// Split passes: dist_items counts matches, dist_items_out turns the counts
+// into output.
+//
+// A workgroup of dist_items takes one item: a tile, one k-mer length and one
+// run of that sketch's words, and stores its partial match counts as a block
+// of its own.  A pass of few tiles therefore still spreads over every CU: the
+// host cuts the words into as many runs as make the rounds of items fill the
+// 512 resident workgroups (item_runs in the host layer).  One (tile, k) item
+// over 156 words takes 0.68 ms by itself, however small the pass: calls on 48
+// genomes went from 774 to 268 us, one query against 6,000 references from 756
+// to 269 us, 451 queries from 4.63 to 3.26 ms (8 k-mer lengths, 10,000 bins).
+//
+// Tiles are 64, 32 or 16 rows high, so that the rows past the last multiple
+// of 64 are covered without computing whole tiles of padding.
+//
+// Items are numbered k-mer length first, then word run, then tile, and
+// workgroup b takes item (b % 8) * ceil(n / 8) + b / 8: consecutive workgroups
+// go to the 8 XCDs in turn, so each XCD walks one contiguous eighth of the
+// list and keeps the row and column panels its tiles share in its own L2.
+// ---------------------------------------------------------------------------
+template <int RR>
+__device__ __forceinline__ void match_item(CParams* pp, int row0, int ct, int kk, int w0, int nw,
+                                           uint4* sB0, uint4* sB1, uint4* sR, uint16_t* counts,
+                                           int wave, int lane) {
+  constexpr int RQ = 8, PB = 2;
+  using Cfg = TileCfg<RQ, RR>;
+  const int s64 = pp->s64;
+  const int nb_cols = pp->nb_cols;
+  const int64_t word0 = (int64_t)w0 * (HL * BLK);
+  const uint32_t* rbase =
+      pp->row_stripes + ((int64_t)kk * pp->nb_rows + row0 / BLK) * (int64_t)s64 * (HL * BLK) +
+      word0 + row0 % BLK;
+  const CU32* arow = (CU32*)(rbase + (wave / Cfg::CG) * RQ);
+  const int64_t col0 = (int64_t)ct * Cfg::TC;
+  const uint32_t* cbase =
+      pp->col_stripes + ((int64_t)kk * nb_cols + col0 / BLK) * (int64_t)s64 * (HL * BLK) + word0;
+  const ColOffsets<RQ, RR> off = col_offsets<RQ, RR>(col0, nb_cols, s64, wave, lane);
+  const RowOffsets<RQ, RR> roff = row_offsets<RQ, RR>(wave, lane);
+  const uint32_t rdst = lds_addr(sR) + (uint32_t)(wave * 64 * 16);
+  uint32_t cnt[RQ][RR];
+  tile_stages<RQ, RR, PB, RR>(arow, cbase, off, rbase, roff, rdst, pp->row_prefetch != 0, nw, sB0,
+                              sB1, wave, lane, (wave % Cfg::CG) * 64 * RR + lane, cnt);
+  store_counts<RQ, RR>(counts, 0, wave, lane, cnt);
+}
+
+__global__ __launch_bounds__(WAVES * 64, 4) void dist_items(DistParams p, ItemArgs a) {
+  __shared__ uint4 sB0[TileCfg<8, 4>::STAGE_U4];
+  __shared__ uint4 sB1[TileCfg<8, 4>::STAGE_U4];
+  __shared__ uint4 sR[TileCfg<8, 4>::ROW_LDS_U4];
+  __shared__ int s_stop;
+  // both arguments are read with scalar loads from the kernarg segment
+  CParams* pp = (CParams*)__builtin_amdgcn_kernarg_segment_ptr();
+  const int per = (a.n_items + BATCH_QUEUES - 1) / BATCH_QUEUES;
+  const int item = (int)(blockIdx.x % BATCH_QUEUES) * per + (int)(blockIdx.x / BATCH_QUEUES);
+  if ((int)(blockIdx.x / BATCH_QUEUES) >= per || item >= a.n_items) return;
+  if (a.watch) {
+    // a cancelled call skips the matching; one read per workgroup, shared, so
+    // that every wave takes the same branch (the matching has barriers)
+    if (threadIdx.x == 0) s_stop = cancel_seen(p.ctl.cancel) ? 1 : 0;
+    __syncthreads();
+    if (__builtin_amdgcn_readfirstlane(s_stop)) return;
+  }
+  const int kr = item / a.n_tiles;  // k-mer length * runs + run
+  const int t = item - kr * a.n_tiles;
+  const int kk = kr / a.runs;
+  const int run = kr - kk * a.runs;
+  ItemTile tile = a.tiles[t];
+  const int row0 = __builtin_amdgcn_readfirstlane(tile.row0);
+  const int ct = __builtin_amdgcn_readfirstlane(tile.ct);
+  const int rows = __builtin_amdgcn_readfirstlane(tile.rows);
+  const int w0 = run * a.run_words;
+  const int nw = min(a.run_words, p.s64 - w0);
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int lane = threadIdx.x & 63;
+  uint16_t* counts = p.counts + (((int64_t)t * p.n_k + kk) * a.runs + run) * ITEM_COUNTS;
+  if (rows == 64) {
+    match_item<4>(pp, row0, ct, kk, w0, nw, sB0, sB1, sR, counts, wave, lane);
+  } else if (rows == 32) {
+    match_item<2>(pp, row0, ct, kk, w0, nw, sB0, sB1, sR, counts, wave, lane);
+  } else {
+    match_item<1>(pp, row0, ct, kk, w0, nw, sB0, sB1, sR, counts, wave, lane);
+  }
+  if (threadIdx.x == 0) add_progress(p.ctl, 1ull);
+}
+
+// Output of a split pass: one lane per pair, ITEM_OUT_ROWS rows of one tile
+// per workgroup, the 256 columns of a row read and written side by side.
+// Left to the last workgroup of each tile, as dist_tiles does it, the
+// epilogue of a tile runs 32 pairs per lane one after the other on one CU: the
+// 2.1M pairs of 2,050 samples x 13 k-mer lengths of 1,024 bins (Jaccards) took
+// 3.58 ms that way and take 0.74 ms here (whole calls).
+__global__ __launch_bounds__(256) void dist_items_out(DistParams p, ItemArgs a) {
+  CParams* pp = (CParams*)__builtin_amdgcn_kernarg_segment_ptr();
+  CParams& q = *pp;
+  const int t = (int)(blockIdx.x / (64 / ITEM_OUT_ROWS));
+  const int r0 = (int)(blockIdx.x % (64 / ITEM_OUT_ROWS)) * ITEM_OUT_ROWS;
+  const ItemTile tile = a.tiles[t];
+  if (r0 >= tile.rows) return;
+  const int64_t gj = (int64_t)tile.ct * 256 + threadIdx.x;
+  const double bins = 64.0 * (double)q.s64;
+  const double rbins = 1.0 / bins;
+  const int runs = a.runs;
+  for (int r = r0; r < r0 + ITEM_OUT_ROWS; ++r) {
+    const int64_t gi = tile.row0 + r;
+    if (!pair_valid(q, gi, gj)) continue;
+    const uint16_t* cp = q.counts + (int64_t)t * q.n_k * runs * ITEM_COUNTS + r * 256 + threadIdx.x;
+    pair_output(q, gi, gj, bins, rbins, [&](int k) {
+      uint32_t c = 0;
+      for (int x = 0; x < runs; ++x) c += cp[((int64_t)k * runs + x) * ITEM_COUNTS];
+      return c;
+    });
+  }
+}
+
+hipError_t launch_items(const DistParams& p, const ItemArgs& a, hipStream_t stream) {
+  if (a.n_items <= 0) return hipSuccess;
+  const int per = (a.n_items + BATCH_QUEUES - 1) / BATCH_QUEUES;
+  dist_items<<<(unsigned)(per * BATCH_QUEUES), WAVES * 64, 0, stream>>>(p, a);
+  dist_items_out<<<(unsigned)(a.n_tiles * (64 / ITEM_OUT_ROWS)), 256, 0, stream>>>(p, a);
+  return hipGetLastError();
 }
 
 __global__ void batch_reset_kernel(uint32_t* queue_next, unsigned long long* fail, int n_jobs,

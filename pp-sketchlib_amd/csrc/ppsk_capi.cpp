@@ -278,6 +278,32 @@ int64_t out_row_start(bool self, int64_t r, int64_t n_rows, int64_t n_cols) {
   return n * r - ((r * (r + 1)) >> 1);
 }
 
+// Copies the dense output of sample rows [r0, r1) to the host on the copy
+// stream once `done` has been reached on the launch stream.
+int copy_rows(DeviceCtx* c, int64_t r0, int64_t r1, const ppsk::DistParams& p, bool self,
+              size_t elem, void* host_out, hipEvent_t done) {
+  const int64_t o0 = out_row_start(self, r0, p.n_rows, p.n_cols);
+  const int64_t o1 = out_row_start(self, r1, p.n_rows, p.n_cols);
+  if (o1 > o0) {
+    const char* dev = (const char*)p.out;
+    HIP_TRY(hipStreamWaitEvent(c->copy_stream, done, 0));
+    HIP_TRY(hipMemcpyAsync((char*)host_out + o0 * elem, dev + o0 * elem, (o1 - o0) * elem,
+                           hipMemcpyDeviceToHost, c->copy_stream));
+  }
+  return PPSK_OK;
+}
+
+// Sample rows covered by tiles [a, b) of height tr.
+std::pair<int64_t, int64_t> tile_rows(const std::vector<ppsk::Tile>& tiles, size_t a, size_t b,
+                                      int tr) {
+  int32_t bmin = tiles[a].bi, bmax = tiles[a].bi;
+  for (size_t x = a; x < b; ++x) {
+    bmin = std::min(bmin, tiles[x].bi);
+    bmax = std::max(bmax, tiles[x].bi);
+  }
+  return {(int64_t)bmin * tr, (int64_t)(bmax + 1) * tr};
+}
+
 // Runs the tile kernel over the row tiles covering sample rows
 // [row_begin, row_end) (row_begin a multiple of the tile height) against all
 // columns, writing dense output into the device buffer p.out (row offset 0).
@@ -345,20 +371,9 @@ int run_dense_tiles(DeviceCtx* c, ppsk::DistParams p, int variant, bool upper, i
   // Copies are queued after every launch: a copy into pageable memory may
   // block this thread until it completes, which must not hold back launches.
   for (size_t ci = 0; host_out && ci < chunks.size(); ++ci) {
-    const size_t a = chunks[ci].first, b = chunks[ci].second;
-    int32_t bmin = tiles[a].bi, bmax = tiles[a].bi;
-    for (size_t x = a; x < b; ++x) {
-      bmin = std::min(bmin, tiles[x].bi);
-      bmax = std::max(bmax, tiles[x].bi);
-    }
-    const int64_t r0 = (int64_t)bmin * tr;
-    const int64_t r1 = (int64_t)(bmax + 1) * tr;
-    const int64_t o0 = out_row_start(self, r0, p.n_rows, p.n_cols);
-    const int64_t o1 = out_row_start(self, r1, p.n_rows, p.n_cols);
-    if (o1 > o0) {
-      HIP_TRY(hipStreamWaitEvent(c->copy_stream, c->events[2 * ci + 1], 0));
-      HIP_TRY(hipMemcpyAsync((char*)host_out + o0 * elem, dev + o0 * elem, (o1 - o0) * elem,
-                             hipMemcpyDeviceToHost, c->copy_stream));
+    const auto r = tile_rows(tiles, chunks[ci].first, chunks[ci].second, tr);
+    if (int rc = copy_rows(c, r.first, r.second, p, self, elem, host_out, c->events[2 * ci + 1])) {
+      return rc;
     }
   }
   HIP_TRY(hipStreamSynchronize(c->stream));
@@ -367,26 +382,6 @@ int run_dense_tiles(DeviceCtx* c, ppsk::DistParams p, int variant, bool upper, i
     float ms = 0.f;
     HIP_TRY(hipEventElapsedTime(&ms, c->events[2 * ci], c->events[2 * ci + 1]));
     tm->ms += ms;
-  }
-  return PPSK_OK;
-}
-
-// Copies the finished dense rows of tiles [a, b) to the host on the copy
-// stream once `done` has been reached on the launch stream.
-int copy_rows(DeviceCtx* c, const std::vector<ppsk::Tile>& tiles, size_t a, size_t b, int tr,
-              const ppsk::DistParams& p, bool self, size_t elem, void* host_out, hipEvent_t done) {
-  int32_t bmin = tiles[a].bi, bmax = tiles[a].bi;
-  for (size_t x = a; x < b; ++x) {
-    bmin = std::min(bmin, tiles[x].bi);
-    bmax = std::max(bmax, tiles[x].bi);
-  }
-  const int64_t o0 = out_row_start(self, (int64_t)bmin * tr, p.n_rows, p.n_cols);
-  const int64_t o1 = out_row_start(self, (int64_t)(bmax + 1) * tr, p.n_rows, p.n_cols);
-  if (o1 > o0) {
-    const char* dev = (const char*)p.out;
-    HIP_TRY(hipStreamWaitEvent(c->copy_stream, done, 0));
-    HIP_TRY(hipMemcpyAsync((char*)host_out + o0 * elem, dev + o0 * elem, (o1 - o0) * elem,
-                           hipMemcpyDeviceToHost, c->copy_stream));
   }
   return PPSK_OK;
 }
@@ -547,8 +542,8 @@ int run_dense_persistent(DeviceCtx* c, ppsk::DistParams p, int variant, bool upp
     tm->items += (int64_t)(chunks[ci].second - chunks[ci].first) * p.n_k;
   }
   for (size_t ci = 0; host_out && ci < chunks.size(); ++ci) {
-    if (int rc = copy_rows(c, tiles, chunks[ci].first, chunks[ci].second, tr, p, self, elem,
-                           host_out, c->events[2 * ci + 1])) {
+    const auto r = tile_rows(tiles, chunks[ci].first, chunks[ci].second, tr);
+    if (int rc = copy_rows(c, r.first, r.second, p, self, elem, host_out, c->events[2 * ci + 1])) {
       return rc;
     }
   }
@@ -562,29 +557,210 @@ int run_dense_persistent(DeviceCtx* c, ppsk::DistParams p, int variant, bool upp
   return PPSK_OK;
 }
 
-// Dense pass over rows [row_begin, row_end): the persistent kernel for the
-// shapes it is built for when the pass has at least two tiles per resident
-// workgroup (a smaller pass fills the GPU better split per (tile, k-mer
-// length)); PPSK_PERSISTENT=0 / 1 forces the choice.
-int run_dense(DeviceCtx* c, ppsk::DistParams p, int variant, bool upper, int64_t row_begin,
-              int64_t row_end, bool self, size_t elem, void* host_out, Timing* tm) {
+// Tiles of a split pass over rows [row_begin, row_end) (row_begin a multiple
+// of 64): 64-row tiles, the rows past the last multiple of 64 in 32- and
+// 16-row ones, so that 451 rows compute 464 and not 512.  Groups of
+// `group_rows` rows (a multiple of 64), column by column inside a group, as
+// make_tiles.
+std::vector<ppsk::ItemTile> item_tiles(int64_t n_cols, bool upper, int64_t row_begin,
+                                       int64_t row_end, int64_t group_rows,
+                                       std::vector<size_t>* group_start) {
+  std::vector<ppsk::ItemTile> t;
+  const int64_t nct = (n_cols + 255) / 256;
+  group_start->clear();
+  for (int64_t g0 = row_begin; g0 < row_end; g0 += group_rows) {
+    const int64_t g1 = std::min(row_end, g0 + group_rows);
+    std::vector<std::pair<int64_t, int32_t>> segs;  // first row, height
+    for (int64_t r = g0; r < g1;) {
+      const int64_t left = g1 - r;
+      const int32_t h = left > 48 ? 64 : (left > 16 ? 32 : 16);
+      segs.emplace_back(r, h);
+      r += h;
+    }
+    const size_t before = t.size();
+    for (int64_t ct = 0; ct < nct; ++ct) {
+      for (const auto& sg : segs) {
+        if (upper && (ct + 1) * 256 - 1 <= sg.first) continue;
+        t.push_back({(int32_t)sg.first, (int32_t)ct, sg.second});
+      }
+    }
+    if (t.size() > before) group_start->push_back(before);
+  }
+  group_start->push_back(t.size());
+  return t;
+}
+
+// Word runs per (tile, k-mer length) of a split pass of n_tiles tiles holding
+// `rows64` 64-row tile equivalents: the count of least estimated time over
+// the rounds the 512 resident workgroups (2 per CU) need.  Measured on 64-row
+// tiles: 6.4 us per word with two workgroups on a CU, 3.5 us alone; about 4 us
+// to start an item; and each item's counts are written and read once (about
+// 0.016 us of the chip's memory time).  One launch holds at most 32,768
+// items of counts (1 GiB).
+int item_runs(int64_t n_tiles, double rows64, int n_k, int s64) {
+  const double weight = rows64 / (double)n_tiles;
+  const int64_t base = n_tiles * n_k;
+  int best = 1;
+  double best_t = -1.0;
+  for (int words = s64; words >= 1; --words) {
+    const int runs = (s64 + words - 1) / words;
+    const int64_t n = base * runs;
+    if (runs > 1 && n > 32768) break;
+    const int64_t rest = n % 512;
+    const double rounds = (double)(n / 512) + (rest == 0 ? 0.0 : (rest <= 256 ? 0.55 : 1.0));
+    const double t = rounds * (4.0 + 6.4 * weight * words) + 0.016 * (double)n;
+    if (best_t < 0.0 || t < best_t) {
+      best_t = t;
+      best = runs;
+    }
+  }
+  return best;
+}
+
+// The split pass (dist_items): every tile's words cut into runs when there
+// are too few (tile, k-mer length) items to fill the CUs, then one lane per
+// pair for the output.  Launches are cut at group boundaries so that each
+// fits the count scratch; with host_out, each launch's finished rows are
+// copied out while the next ones compute.
+struct ItemPlan {
+  std::vector<ppsk::ItemTile> tiles;
+  std::vector<std::pair<size_t, size_t>> chunks;  // tiles of each launch
+  int runs = 1, run_words = 0;
+  uint64_t items = 0;
+};
+
+ItemPlan plan_items(int64_t n_cols, int n_k, int s64, bool upper, int64_t row_begin,
+                    int64_t row_end, bool host_out) {
+  ItemPlan pl;
+  // count scratch per launch; PPSK_CHUNK_BYTES lowers it (more, smaller
+  // launches: finer-grained streaming of host output)
+  size_t budget = (size_t)1 << 30;
+  if (const char* env = std::getenv("PPSK_CHUNK_BYTES")) {
+    const long long v = std::atoll(env);
+    if (v > 0) budget = (size_t)v;
+  }
+  const size_t per_tile = (size_t)n_k * ppsk::ITEM_COUNTS * sizeof(uint16_t);
+  size_t most = std::max<size_t>(1, budget / per_tile);
+  const int64_t nct = (n_cols + 255) / 256;
+  const int64_t group_tiles = std::max<int64_t>(1, std::min<int64_t>(tile_group(64), (int64_t)most / nct));
+  std::vector<size_t> gs;
+  pl.tiles = item_tiles(n_cols, upper, row_begin, row_end, group_tiles * 64, &gs);
+  if (pl.tiles.empty()) return pl;
+  if (host_out) most = std::min(most, std::max<size_t>(1024, pl.tiles.size() / 8));
+  for (size_t g = 0; g + 1 < gs.size();) {
+    size_t h = g + 1;
+    while (h + 1 < gs.size() && gs[h + 1] - gs[g] <= most) ++h;
+    pl.chunks.emplace_back(gs[g], gs[h]);
+    g = h;
+  }
+  if (pl.chunks.size() == 1) {
+    double rows64 = 0.0;
+    for (const auto& t : pl.tiles) rows64 += t.rows == 64 ? 1.0 : (t.rows == 32 ? 0.57 : 0.37);
+    pl.runs = item_runs((int64_t)pl.tiles.size(), rows64, n_k, s64);
+  }
+  pl.run_words = (s64 + pl.runs - 1) / pl.runs;
+  pl.runs = (s64 + pl.run_words - 1) / pl.run_words;
+  pl.items = (uint64_t)pl.tiles.size() * n_k * pl.runs;
+  return pl;
+}
+
+int run_dense_items(DeviceCtx* c, ppsk::DistParams p, bool upper, int64_t row_begin,
+                    int64_t row_end, bool self, size_t elem, void* host_out, Timing* tm) {
+  const ItemPlan pl =
+      plan_items(p.n_cols, p.n_k, p.s64, upper, row_begin, row_end, host_out != nullptr);
+  if (pl.tiles.empty()) return PPSK_OK;
+  size_t most = 0;
+  for (auto& ch : pl.chunks) most = std::max(most, ch.second - ch.first);
+  const size_t item_bytes = ppsk::ITEM_COUNTS * sizeof(uint16_t);
+  if (int rc = grow(&c->counts, &c->counts_bytes, most * p.n_k * pl.runs * item_bytes)) return rc;
+  if (int rc = grow(&c->pitems, &c->pitems_bytes, pl.tiles.size() * sizeof(ppsk::ItemTile))) return rc;
+  HIP_TRY(hipMemcpyAsync(c->pitems, pl.tiles.data(), pl.tiles.size() * sizeof(ppsk::ItemTile),
+                         hipMemcpyHostToDevice, c->stream));
+  p.counts = (uint16_t*)c->counts;
+  p.out_row_offset = 0;
+  ppsk::ItemArgs a;
+  std::memset(&a, 0, sizeof(a));
+  a.runs = pl.runs;
+  a.run_words = pl.run_words;
+  // a read of the host's cancellation flag costs an item more than a
+  // microsecond: passes of a few rounds (milliseconds) are left to finish, the
+  // call reports the cancellation either way
+  a.watch = pl.items >= 4096 ? 1 : 0;
+  for (size_t ci = 0; ci < pl.chunks.size(); ++ci) {
+    const size_t x = pl.chunks[ci].first, y = pl.chunks[ci].second;
+    hipEvent_t e0 = pool_event(c, 2 * ci), e1 = pool_event(c, 2 * ci + 1);
+    if (!e0 || !e1) return fail(PPSK_ERR_HIP, "event creation failed");
+    a.tiles = (const ppsk::ItemTile*)c->pitems + x;
+    a.n_tiles = (int32_t)(y - x);
+    a.n_items = (int32_t)((y - x) * p.n_k * pl.runs);
+    HIP_TRY(hipEventRecord(e0, c->stream));
+    HIP_TRY(ppsk::launch_items(p, a, c->stream));
+    HIP_TRY(hipEventRecord(e1, c->stream));
+    tm->launches += 1;
+    tm->items += a.n_items;
+  }
+  // Copies are queued after every launch: a copy into pageable memory may
+  // block this thread until it completes, which must not hold back launches.
+  for (size_t ci = 0; host_out && ci < pl.chunks.size(); ++ci) {
+    int64_t r0 = row_end, r1 = row_begin;
+    for (size_t x = pl.chunks[ci].first; x < pl.chunks[ci].second; ++x) {
+      r0 = std::min<int64_t>(r0, pl.tiles[x].row0);
+      r1 = std::max<int64_t>(r1, pl.tiles[x].row0 + pl.tiles[x].rows);
+    }
+    if (int rc = copy_rows(c, r0, r1, p, self, elem, host_out, c->events[2 * ci + 1])) return rc;
+  }
+  HIP_TRY(hipStreamSynchronize(c->stream));
+  HIP_TRY(hipStreamSynchronize(c->copy_stream));
+  for (size_t ci = 0; ci < pl.chunks.size(); ++ci) {
+    float ms = 0.f;
+    HIP_TRY(hipEventElapsedTime(&ms, c->events[2 * ci], c->events[2 * ci + 1]));
+    tm->ms += ms;
+  }
+  return PPSK_OK;
+}
+
+// How a dense pass runs: whole tiles on the persistent kernel when there are
+// at least two per resident workgroup, else as a split pass.
+// PPSK_TILE_VARIANT forces a tile shape and PPSK_PERSISTENT=0 / 1 the
+// per-(tile, k-mer length) or the persistent kernel of that shape.
+enum class Route { persistent, tiles, items };
+
+Route dense_route(int variant, bool upper, int64_t rows, int64_t n_cols) {
   const char* e = std::getenv("PPSK_PERSISTENT");
-  bool persistent = variant == 2 || variant == 4 || variant == 5;
-  if (e) {
-    persistent = persistent && std::atoi(e) != 0;
-  } else if (persistent) {
+  const bool can = variant == 2 || variant == 4 || variant == 5;
+  if (e) return can && std::atoi(e) != 0 ? Route::persistent : Route::tiles;
+  if (can) {
     const int tr = ppsk::variant_tile_rows(variant), tc = ppsk::variant_tile_cols(variant);
-    const int64_t rt = (row_end - row_begin + tr - 1) / tr, ct = (p.n_cols + tc - 1) / tc;
+    const int64_t rt = (rows + tr - 1) / tr, ct = (n_cols + tc - 1) / tc;
     const int64_t tiles = upper ? rt * ct / 2 : rt * ct;
     int grid = 0;
     if (ppsk::batch_grid(variant == 5 ? ppsk::BATCH_MIXED : variant, &grid) != hipSuccess) grid = 0;
-    persistent = tiles >= 2 * (int64_t)grid;
+    if (grid > 0 && tiles >= 2 * (int64_t)grid) return Route::persistent;
   }
-  if (persistent) {
-    return run_dense_persistent(c, p, variant, upper, row_begin, row_end, self, elem, host_out,
-                                tm);
+  return std::getenv("PPSK_TILE_VARIANT") ? Route::tiles : Route::items;
+}
+
+uint64_t dense_items(const ppsk_set* rows, int64_t n_cols, bool upper, int64_t row_begin,
+                     int64_t row_end, bool host_out) {
+  const int v = default_variant();
+  if (dense_route(v, upper, row_end - row_begin, n_cols) == Route::items) {
+    return plan_items(n_cols, rows->n_k, rows->s64, upper, row_begin, row_end, host_out).items;
   }
-  return run_dense_tiles(c, p, variant, upper, row_begin, row_end, self, elem, host_out, tm);
+  return pass_items(row_end - row_begin, n_cols, rows->n_k, v, upper);
+}
+
+// Dense pass over rows [row_begin, row_end).
+int run_dense(DeviceCtx* c, ppsk::DistParams p, int variant, bool upper, int64_t row_begin,
+              int64_t row_end, bool self, size_t elem, void* host_out, Timing* tm) {
+  switch (dense_route(variant, upper, row_end - row_begin, p.n_cols)) {
+    case Route::persistent:
+      return run_dense_persistent(c, p, variant, upper, row_begin, row_end, self, elem, host_out,
+                                  tm);
+    case Route::items:
+      return run_dense_items(c, p, upper, row_begin, row_end, self, elem, host_out, tm);
+    default:
+      return run_dense_tiles(c, p, variant, upper, row_begin, row_end, self, elem, host_out, tm);
+  }
 }
 
 void fill_common(ppsk::DistParams& p, const ppsk_set* rows, const ppsk_set* cols,
@@ -962,7 +1138,7 @@ int ppsk_dense(ppsk_set* ref, ppsk_set* query, int32_t random_mode, int32_t n_cl
   if (int rc = get_ctx(ref->device, &c)) return rc;
   std::lock_guard<std::mutex> lk(c->mu);
   if (int rc = cancel_status(ref->device)) return rc;
-  CallScope scope(c, pass_items(rows->n, cols->n, ref->n_k, default_variant(), self));
+  CallScope scope(c, dense_items(rows, cols->n, self, 0, rows->n, !out_on_device));
 
   const int64_t n_rows_out = self ? ref->n * (ref->n - 1) / 2 : query->n * ref->n;
   const size_t elem = out_kind == PPSK_OUT_CORE_ACC ? 2 * sizeof(float)
@@ -1015,7 +1191,17 @@ int ppsk_knn(ppsk_set* ref, int32_t random_mode, int32_t n_clusters, const float
   int rc = PPSK_OK;
   const size_t tri_bytes = (size_t)n * (n - 1) / 2 * sizeof(float2);
   const bool symmetric = table_symmetric(rnd, ref->n_k) && tri_bytes <= ((size_t)96 << 30);
-  CallScope scope(c, pass_items(n, n, ref->n_k, default_variant(), symmetric));
+  int64_t band = n;
+  if (!symmetric) {
+    // asymmetric Monte Carlo table: full square rows in bands
+    band = std::max<int64_t>(ppsk::BLK, ((int64_t)(2ll << 30) / (n * 8)) / ppsk::BLK * ppsk::BLK);
+    band = std::min<int64_t>(band, (n + ppsk::BLK - 1) / ppsk::BLK * ppsk::BLK);
+  }
+  uint64_t items = 0;
+  for (int64_t r0 = 0; r0 < n; r0 += band) {
+    items += dense_items(ref, n, symmetric, r0, std::min(n, r0 + band), false);
+  }
+  CallScope scope(c, items);
   if (symmetric) {
     // distances are symmetric: compute the upper triangle once and read both
     // (i, j) and (j, i) from it
@@ -1028,10 +1214,7 @@ int ppsk_knn(ppsk_set* ref, int32_t random_mode, int32_t n_clusters, const float
       rc = knn_from_triangle(c, (const float*)c->out, n, dist_col, kNN, i_vec, j_vec, dists);
     }
   } else {
-    // asymmetric Monte Carlo table: full square rows in bands
     const int variant = default_variant();
-    int64_t band = std::max<int64_t>(ppsk::BLK, ((int64_t)(2ll << 30) / (n * 8)) / ppsk::BLK * ppsk::BLK);
-    band = std::min<int64_t>(band, (n + ppsk::BLK - 1) / ppsk::BLK * ppsk::BLK);
     if ((rc = grow(&c->out, &c->out_bytes, (size_t)band * n * 2 * sizeof(float)))) return rc;
     float* dtab = nullptr;
     if ((rc = upload_table(c, ref, rnd, &dtab))) return rc;
@@ -1115,7 +1298,7 @@ int ppsk_threshold(ppsk_set* ref, int32_t random_mode, int32_t n_clusters, const
   std::lock_guard<std::mutex> lk(c->mu);
   if (int rc = cancel_status(ref->device)) return rc;
   const int64_t n = ref->n;
-  CallScope scope(c, pass_items(n, n, ref->n_k, default_variant(), true));
+  CallScope scope(c, dense_items(ref, n, true, 0, n, false));
   const size_t tri_bytes = std::max<size_t>((size_t)n * (n - 1) / 2 * sizeof(float2), 8);
   if (int rc = grow(&c->out, &c->out_bytes, tri_bytes)) return rc;
   Timing tm;
@@ -1162,7 +1345,7 @@ int ppsk_self_pass(ppsk_set* ref, int32_t random_mode, int32_t n_clusters, const
   std::lock_guard<std::mutex> lk(c->mu);
   if (int rc = cancel_status(ref->device)) return rc;
   const int64_t n = ref->n;
-  CallScope scope(c, pass_items(n, n, ref->n_k, default_variant(), true));
+  CallScope scope(c, dense_items(ref, n, true, 0, n, dense_out != nullptr));
   const size_t tri_bytes = std::max<size_t>((size_t)n * (n - 1) / 2 * sizeof(float2), 8);
   if (int rc = grow(&c->out, &c->out_bytes, tri_bytes)) return rc;
   Timing tm;

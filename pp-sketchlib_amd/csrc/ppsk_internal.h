@@ -105,7 +105,29 @@ struct BatchArgs {
   Control ctl;              // progress and cancellation of the launch (null: neither)
 };
 
+// Split passes (dist_items): an item is one tile, one k-mer length and one run
+// of words; tiles are 64, 32 or 16 rows x 256 columns.
+struct ItemTile {
+  int32_t row0;  // first row, a multiple of `rows`
+  int32_t ct;    // columns [ct * 256, +256)
+  int32_t rows;  // 64, 32 or 16
+};
+constexpr int ITEM_COUNTS = 64 * 256;  // counts of one item (u16), whatever its height
+constexpr int ITEM_OUT_ROWS = 4;       // tile rows per output workgroup
+
+struct ItemArgs {
+  const ItemTile* tiles;  // [n_tiles]
+  int32_t n_tiles;
+  int32_t runs;       // word runs per (tile, k-mer length)
+  int32_t run_words;  // words per run (the last may hold fewer)
+  int32_t n_items;    // n_tiles * n_k * runs
+  int32_t watch;      // read the cancellation flag in every item
+};
+
 // Launchers (dist_kernels.hip).  All work goes on `stream`.
+// Matching and output of a split pass; p.counts holds n_items blocks of
+// ITEM_COUNTS counts.
+hipError_t launch_items(const DistParams& p, const ItemArgs& a, hipStream_t stream);
 hipError_t launch_stripe(const uint64_t* raw, int64_t count, int64_t first,
                          int32_t n_k, int32_t s64, int32_t nb, uint32_t* stripes,
                          hipStream_t stream);
