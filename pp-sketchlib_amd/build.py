@@ -55,8 +55,8 @@ def _check_pipelined_spills(remarks):
     them later; if the compiler spilled or copied one of those SGPR tuples in
     between, it would move data that has not arrived yet.  The kernel
     resource remarks list spills per function: every frame that holds the
-    pipelined matching must report none -- the dist_tiles and dist_items
-    kernels (matching inlined) and batch_tile_k (the persistent kernels' out-of-line matching,
+    pipelined matching must report none -- the dist_tiles, dist_items
+    and dist_coded kernels (matching inlined) and batch_tile_k (the persistent kernels' out-of-line matching,
     the same code as the dist_tiles kernel of its shape).  The persistent
     kernels' own frames (dist_batch, dist_batch_mixed) only take work items
     and call out: no asm operand is in flight there, so a spill in them is
@@ -67,7 +67,8 @@ def _check_pipelined_spills(remarks):
             name = line.split("Function Name:")[1].split()[0]
         elif name and ("SGPRs Spill:" in line or "VGPRs Spill:" in line):
             pipelined = (("dist_tiles" in name or "batch_tile_k" in name) and "ELi2EE" in name
-                         or "dist_tiles_diagonal" in name or "dist_itemsE" in name)
+                         or "dist_tiles_diagonal" in name or "dist_itemsE" in name
+                         or "dist_codedE" in name)
             if pipelined and int(line.rsplit(":", 1)[1].split()[0]) != 0:
                 bad.append(name + ": " + line.split("remark:")[-1].strip())
     if bad:

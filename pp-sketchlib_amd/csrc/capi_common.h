@@ -74,6 +74,8 @@ struct DeviceCtx {
   size_t pitems_bytes = 0;
   ppsk::DistParams* pparams = nullptr;  // the call's parameters in device memory
   uint32_t* pqueue = nullptr;         // queue counters
+  void* codes = nullptr;              // codes of a coded pass (at most CODE_BUDGET)
+  size_t codes_bytes = 0;
   hipStream_t tail_stream = nullptr;  // the tail's (tile, k) launch beside the persistent one
   void* noalloc_scratch = nullptr;    // this device's copy of the fixed scratch array
   ppsk::Control ctl{};                // progress / cancellation pointers of the calls

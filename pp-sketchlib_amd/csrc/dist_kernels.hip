@@ -24,8 +24,10 @@
 //    log-Jaccard-vs-k regression, dense output.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cmath>
 #include <cstdint>
+#include <numeric>
 
 #include "bin_fraction.h"
 #include "log_jaccard.h"
@@ -101,6 +103,7 @@ hipError_t launch_stripe(const uint64_t* raw, int64_t count, int64_t first,
 // ---------------------------------------------------------------------------
 typedef const __attribute__((address_space(4))) uint32_t CU32;
 typedef const __attribute__((address_space(4))) DistParams CParams;
+typedef const __attribute__((address_space(4))) CodeGroup CCodeGroup;
 
 __device__ __forceinline__ uint32_t match_and(uint32_t acc, uint32_t a, uint32_t b) {
   // truth table over (acc, a, b) with src0 = 0xF0, src1 = 0xCC, src2 = 0xAA:
@@ -591,19 +594,21 @@ __device__ __forceinline__ void match_stage_pipe(const CU32* arow, int w0, int n
 }
 
 // ---------------------------------------------------------------------------
-// Output of one pair (row gi, column gj) from its match counts: count(k) is
-// the count at k-mer length index k.  Pairs outside the pass (padding, or at
-// and below the diagonal of a self pass) write nothing.
+// Output of one pair (row gi, column gj) from its match counts.  counts(k0, c)
+// reads those of k-mer lengths k0 .. k0 + 3 (as far as there are so many) into
+// c[0..3]: together, so that a pair waits for memory once per 4 lengths.
 // ---------------------------------------------------------------------------
+constexpr int OUT_K = 4;
+
 template <typename P>
 __device__ __forceinline__ bool pair_valid(const P& p, int64_t gi, int64_t gj) {
   if (p.self_mode && !p.full_square) return gi < gj && gj < p.n_cols;
   return gi < p.n_rows && gj < p.n_cols;
 }
 
-template <typename P, typename Count>
+template <typename P, typename Counts>
 __device__ __forceinline__ void pair_output(const P& p, int64_t gi, int64_t gj, double bins,
-                                            double rbins, Count count) {
+                                            double rbins, Counts counts) {
   int64_t pos;
   if (p.full_square) {
     pos = (gi - p.square_row0) * p.out_stride_rows + gj;
@@ -613,15 +618,29 @@ __device__ __forceinline__ void pair_output(const P& p, int64_t gi, int64_t gj, 
     pos = gi * p.n_cols + gj;  // query-major: q * n_ref + r
   }
   pos -= p.out_row_offset;
+  const int n_k = p.n_k;
+  uint32_t c[OUT_K];
   if (p.out_kind == OUT_COUNTS) {
-    uint16_t* o = reinterpret_cast<uint16_t*>(p.out) + pos * p.n_k;
-    for (int k = 0; k < p.n_k; ++k) o[k] = (uint16_t)count(k);
+    uint16_t* o = reinterpret_cast<uint16_t*>(p.out) + pos * n_k;
+    for (int k0 = 0; k0 < n_k; k0 += OUT_K) {
+      counts(k0, c);
+#pragma unroll
+      for (int i = 0; i < OUT_K; ++i) {
+        if (k0 + i < n_k) o[k0 + i] = (uint16_t)c[i];
+      }
+    }
     return;
   }
   if (p.out_kind == OUT_JACCARD) {
-    float* o = reinterpret_cast<float*>(p.out) + pos * p.n_k;
-    for (int k = 0; k < p.n_k; ++k) {
-      o[k] = (float)jaccard_d(count(k), bins, rbins, random_for(p, k, gi, gj));
+    float* o = reinterpret_cast<float*>(p.out) + pos * n_k;
+    for (int k0 = 0; k0 < n_k; k0 += OUT_K) {
+      counts(k0, c);
+#pragma unroll
+      for (int i = 0; i < OUT_K; ++i) {
+        if (k0 + i < n_k) {
+          o[k0 + i] = (float)jaccard_d(c[i], bins, rbins, random_for(p, k0 + i, gi, gj));
+        }
+      }
     }
     return;
   }
@@ -629,8 +648,12 @@ __device__ __forceinline__ void pair_output(const P& p, int64_t gi, int64_t gj, 
     // kNN on Jaccards: (float)(1 - J) of the first two k-mer lengths
     // (src/api.cpp:368-371 narrows 1.0f - double J to float)
     float v[2] = {INFINITY, INFINITY};
-    for (int k = 0; k < 2 && k < p.n_k; ++k) {
-      v[k] = (float)(1.0 - jaccard_d(count(k), bins, rbins, random_for(p, k, gi, gj)));
+    counts(0, c);
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+      if (k < n_k) {
+        v[k] = (float)(1.0 - jaccard_d(c[k], bins, rbins, random_for(p, k, gi, gj)));
+      }
     }
     reinterpret_cast<float2*>(p.out)[pos] = make_float2(v[0], v[1]);
     return;
@@ -640,27 +663,33 @@ __device__ __forceinline__ void pair_output(const P& p, int64_t gi, int64_t gj, 
   // sums and committed only if a later valid point arrives.
   int first = -1, last = -1;
   double sy = 0.0, sxy = 0.0, py = 0.0, pxy = 0.0;
-  for (int k = 0; k < p.n_k; ++k) {
-    const float jf = (float)jaccard_d(count(k), bins, rbins, random_for(p, k, gi, gj));
-    const bool ok = (double)jf > p.tolerance;
-    if (!ok && first < 0) continue;
-    const double x = (double)p.kvals[k];
-    const double y = log_jaccard(jf, g_log_tab);
-    if (ok) {
-      if (first < 0) {
-        first = k;
-        sy = y;
-        sxy = x * y;
+  for (int k0 = 0; k0 < n_k; k0 += OUT_K) {
+    counts(k0, c);
+#pragma unroll
+    for (int i = 0; i < OUT_K; ++i) {
+      const int k = k0 + i;
+      if (k >= n_k) break;
+      const float jf = (float)jaccard_d(c[i], bins, rbins, random_for(p, k, gi, gj));
+      const bool ok = (double)jf > p.tolerance;
+      if (!ok && first < 0) continue;
+      const double x = (double)p.kvals[k];
+      const double y = log_jaccard(jf, g_log_tab);
+      if (ok) {
+        if (first < 0) {
+          first = k;
+          sy = y;
+          sxy = x * y;
+        } else {
+          sy += py + y;
+          sxy += pxy + x * y;
+        }
+        py = 0.0;
+        pxy = 0.0;
+        last = k;
       } else {
-        sy += py + y;
-        sxy += pxy + x * y;
+        py += y;
+        pxy += x * y;
       }
-      py = 0.0;
-      pxy = 0.0;
-      last = k;
-    } else {
-      py += y;
-      pxy += x * y;
     }
   }
   float core = 0.0f, accd = 0.0f;
@@ -717,7 +746,10 @@ __device__ __noinline__ void tile_epilogue(CParams* pp, const uint16_t* tile_cou
       const int64_t gj = col0 + lane + 64 * r;
       if (!pair_valid(p, gi, gj)) continue;
       const uint16_t* cp = tbase + q * TC + 64 * r;
-      pair_output(p, gi, gj, bins, rbins, [&](int k) { return (uint32_t)cp[k * kstride]; });
+      pair_output(p, gi, gj, bins, rbins, [&](int k0, uint32_t (&c)[OUT_K]) {
+#pragma unroll
+        for (int i = 0; i < OUT_K; ++i) c[i] = cp[min(k0 + i, p.n_k - 1) * kstride];
+      });
     }
   }
 }
@@ -1218,23 +1250,69 @@ __global__ __launch_bounds__(WAVES * 64, 4) void dist_batch_mixed(BatchArgs a) {
 // Split passes: dist_items counts matches, dist_items_out turns the counts
 // into output.
 //
-// A workgroup of dist_items takes one item: a tile, one k-mer length and one
-// run of that sketch's words, and stores its partial match counts as a block
-// of its own.  A pass of few tiles therefore still spreads over every CU: the
-// host cuts the words into as many runs as make the rounds of items fill the
-// 512 resident workgroups (item_runs in the host layer).  One (tile, k) item
-// over 156 words takes 0.68 ms by itself, however small the pass: calls on 48
-// genomes went from 774 to 268 us, one query against 6,000 references from 756
-// to 269 us, 451 queries from 4.63 to 3.26 ms (8 k-mer lengths, 10,000 bins).
+// A workgroup of dist_items takes one item: a tile, one k-mer length and all or
+// one run of that sketch's words, and stores its match counts as a block of
+// its own.  (Tile, k-mer length) pairs that fill whole rounds of the 512
+// resident workgroups are one item each; the others, all of them in a small
+// pass, are cut into the runs of words that make their rounds shortest
+// (item_runs in the host layer), so that a pass of few tiles spreads over
+// every CU and a large one has no idle last round.  One item over 156 words
+// takes 0.68 ms by itself, however small the pass: calls on 48 genomes went
+// from 774 to 148 us, one query against 6,000 references from 756 to 255 us
+// (8 k-mer lengths, 10,000 bins).
 //
 // Tiles are 64, 32 or 16 rows high, so that the rows past the last multiple
 // of 64 are covered without computing whole tiles of padding.
 //
-// Items are numbered k-mer length first, then word run, then tile, and
-// workgroup b takes item (b % 8) * ceil(n / 8) + b / 8: consecutive workgroups
-// go to the 8 XCDs in turn, so each XCD walks one contiguous eighth of the
-// list and keeps the row and column panels its tiles share in its own L2.
+// Workgroup b of a part of n items takes item (b % 8) * ceil(n / 8) + b / 8:
+// consecutive workgroups go to the 8 XCDs in turn, so each XCD walks one
+// contiguous eighth of the list and keeps the row and column panels its tiles
+// share in its own L2.
 // ---------------------------------------------------------------------------
+struct ItemAt {
+  int tile, kk;
+  int unit0, units;  // words or halves
+  int64_t block;     // of the counts
+};
+
+// The item of this workgroup; false: none (padding of the last eighth).
+__device__ __forceinline__ bool item_at(const ItemArgs& a, int n_k, int units, ItemAt& it) {
+  int b = (int)blockIdx.x, n = a.whole;
+  const int first = (n + BATCH_QUEUES - 1) / BATCH_QUEUES * BATCH_QUEUES;
+  const bool whole = b < first;
+  if (!whole) {
+    b -= first;
+    n = a.n_items - a.whole;
+  }
+  const int per = (n + BATCH_QUEUES - 1) / BATCH_QUEUES;
+  const int x = b % BATCH_QUEUES * per + b / BATCH_QUEUES;
+  if (b / BATCH_QUEUES >= per || x >= n) return false;
+  int pair = x;
+  it.unit0 = 0;
+  it.units = units;
+  it.block = x;
+  if (!whole) {
+    const int pairs = n / a.runs;
+    const int run = x / pairs;
+    pair = a.whole + (x - run * pairs);
+    it.unit0 = run * a.run_units;
+    it.units = min(a.run_units, units - it.unit0);
+    it.block = a.whole + (int64_t)(x - run * pairs) * a.runs + run;
+  }
+  const int tall = a.n_tall * n_k;
+  const int at = pair < tall ? pair : pair - tall;
+  const int per_k = pair < tall ? a.n_tall : a.n_tiles - a.n_tall;
+  it.kk = at / per_k;
+  it.tile = at - it.kk * per_k + (pair < tall ? 0 : a.n_tall);
+  return true;
+}
+
+// Number of the pair (tile t, k-mer length k).
+__device__ __forceinline__ int item_pair(const ItemArgs& a, int n_k, int t, int k) {
+  return t < a.n_tall ? k * a.n_tall + t
+                      : a.n_tall * n_k + k * (a.n_tiles - a.n_tall) + t - a.n_tall;
+}
+
 template <int RR>
 __device__ __forceinline__ void match_item(CParams* pp, int row0, int ct, int kk, int w0, int nw,
                                            uint4* sB0, uint4* sB1, uint4* sR, uint16_t* counts,
@@ -1267,9 +1345,8 @@ __global__ __launch_bounds__(WAVES * 64, 4) void dist_items(DistParams p, ItemAr
   __shared__ int s_stop;
   // both arguments are read with scalar loads from the kernarg segment
   CParams* pp = (CParams*)__builtin_amdgcn_kernarg_segment_ptr();
-  const int per = (a.n_items + BATCH_QUEUES - 1) / BATCH_QUEUES;
-  const int item = (int)(blockIdx.x % BATCH_QUEUES) * per + (int)(blockIdx.x / BATCH_QUEUES);
-  if ((int)(blockIdx.x / BATCH_QUEUES) >= per || item >= a.n_items) return;
+  ItemAt it;
+  if (!item_at(a, p.n_k, p.s64, it)) return;
   if (a.watch) {
     // a cancelled call skips the matching; one read per workgroup, shared, so
     // that every wave takes the same branch (the matching has barriers)
@@ -1277,19 +1354,14 @@ __global__ __launch_bounds__(WAVES * 64, 4) void dist_items(DistParams p, ItemAr
     __syncthreads();
     if (__builtin_amdgcn_readfirstlane(s_stop)) return;
   }
-  const int kr = item / a.n_tiles;  // k-mer length * runs + run
-  const int t = item - kr * a.n_tiles;
-  const int kk = kr / a.runs;
-  const int run = kr - kk * a.runs;
-  ItemTile tile = a.tiles[t];
+  const ItemTile tile = a.tiles[it.tile];
   const int row0 = __builtin_amdgcn_readfirstlane(tile.row0);
   const int ct = __builtin_amdgcn_readfirstlane(tile.ct);
   const int rows = __builtin_amdgcn_readfirstlane(tile.rows);
-  const int w0 = run * a.run_words;
-  const int nw = min(a.run_words, p.s64 - w0);
+  const int kk = it.kk, w0 = it.unit0, nw = it.units;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lane = threadIdx.x & 63;
-  uint16_t* counts = p.counts + (((int64_t)t * p.n_k + kk) * a.runs + run) * ITEM_COUNTS;
+  uint16_t* counts = p.counts + it.block * ITEM_COUNTS;
   if (rows == 64) {
     match_item<4>(pp, row0, ct, kk, w0, nw, sB0, sB1, sR, counts, wave, lane);
   } else if (rows == 32) {
@@ -1300,40 +1372,642 @@ __global__ __launch_bounds__(WAVES * 64, 4) void dist_items(DistParams p, ItemAr
   if (threadIdx.x == 0) add_progress(p.ctl, 1ull);
 }
 
-// Output of a split pass: one lane per pair, ITEM_OUT_ROWS rows of one tile
-// per workgroup, the 256 columns of a row read and written side by side.
-// Left to the last workgroup of each tile, as dist_tiles does it, the
-// epilogue of a tile runs 32 pairs per lane one after the other on one CU: the
-// 2.1M pairs of 2,050 samples x 13 k-mer lengths of 1,024 bins (Jaccards) took
-// 3.58 ms that way and take 0.74 ms here (whole calls).
+// Output of a split pass: one lane per pair, a.out_rows rows of one tile per
+// workgroup (1 in a small pass, so that no lane has to do four), the 256
+// columns of a row read and written side by side.  Left to the last workgroup
+// of each tile, as dist_tiles does it, the epilogue of a tile runs 32 pairs per
+// lane one after the other on one CU: the 2.1M pairs of 2,050 samples x 13
+// k-mer lengths of 1,024 bins (Jaccards) took 3.58 ms that way and take 0.67 ms
+// here (whole calls).
 __global__ __launch_bounds__(256) void dist_items_out(DistParams p, ItemArgs a) {
   CParams* pp = (CParams*)__builtin_amdgcn_kernarg_segment_ptr();
   CParams& q = *pp;
-  const int t = (int)(blockIdx.x / (64 / ITEM_OUT_ROWS));
-  const int r0 = (int)(blockIdx.x % (64 / ITEM_OUT_ROWS)) * ITEM_OUT_ROWS;
+  const int parts = 64 / a.out_rows;
+  const int t = (int)(blockIdx.x / parts);
+  const int r0 = (int)(blockIdx.x % parts) * a.out_rows;
   const ItemTile tile = a.tiles[t];
   if (r0 >= tile.rows) return;
   const int64_t gj = (int64_t)tile.ct * 256 + threadIdx.x;
   const double bins = 64.0 * (double)q.s64;
   const double rbins = 1.0 / bins;
-  const int runs = a.runs;
-  for (int r = r0; r < r0 + ITEM_OUT_ROWS; ++r) {
+  for (int r = r0; r < r0 + a.out_rows; ++r) {
     const int64_t gi = tile.row0 + r;
     if (!pair_valid(q, gi, gj)) continue;
-    const uint16_t* cp = q.counts + (int64_t)t * q.n_k * runs * ITEM_COUNTS + r * 256 + threadIdx.x;
-    pair_output(q, gi, gj, bins, rbins, [&](int k) {
-      uint32_t c = 0;
-      for (int x = 0; x < runs; ++x) c += cp[((int64_t)k * runs + x) * ITEM_COUNTS];
-      return c;
+    const uint16_t* cp = q.counts + r * 256 + threadIdx.x;
+    pair_output(q, gi, gj, bins, rbins, [&](int k0, uint32_t (&c)[OUT_K]) {
+      const uint16_t* x[OUT_K];
+      int runs[OUT_K], most = 1;
+#pragma unroll
+      for (int i = 0; i < OUT_K; ++i) {
+        const int pair = item_pair(a, q.n_k, t, min(k0 + i, q.n_k - 1));
+        const bool whole = pair < a.whole;
+        x[i] = cp + (whole ? pair : a.whole + (int64_t)(pair - a.whole) * a.runs) * ITEM_COUNTS;
+        runs[i] = whole ? 1 : a.runs;
+        most = max(most, runs[i]);
+        c[i] = 0;
+      }
+      // 4 runs of 4 lengths at a time
+      for (int y = 0; y < most; y += 4) {
+        uint32_t v[4][OUT_K];
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+#pragma unroll
+          for (int i = 0; i < OUT_K; ++i) {
+            v[j][i] = y + j < runs[i] ? x[i][(int64_t)(y + j) * ITEM_COUNTS] : 0u;
+          }
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+#pragma unroll
+          for (int i = 0; i < OUT_K; ++i) c[i] += v[j][i];
+      }
     });
   }
 }
 
+static unsigned item_grid(const ItemArgs& a) {
+  const int per1 = (a.whole + BATCH_QUEUES - 1) / BATCH_QUEUES;
+  const int per2 = (a.n_items - a.whole + BATCH_QUEUES - 1) / BATCH_QUEUES;
+  return (unsigned)((per1 + per2) * BATCH_QUEUES);
+}
+
 hipError_t launch_items(const DistParams& p, const ItemArgs& a, hipStream_t stream) {
   if (a.n_items <= 0) return hipSuccess;
-  const int per = (a.n_items + BATCH_QUEUES - 1) / BATCH_QUEUES;
-  dist_items<<<(unsigned)(per * BATCH_QUEUES), WAVES * 64, 0, stream>>>(p, a);
-  dist_items_out<<<(unsigned)(a.n_tiles * (64 / ITEM_OUT_ROWS)), 256, 0, stream>>>(p, a);
+  dist_items<<<item_grid(a), WAVES * 64, 0, stream>>>(p, a);
+  dist_items_out<<<(unsigned)(a.n_tiles * (64 / a.out_rows)), 256, 0, stream>>>(p, a);
+  return hipGetLastError();
+}
+
+// ---------------------------------------------------------------------------
+// Coded passes: fewer bit planes per pair.
+//
+// A group of at most CODE_ROWS rows holds V distinct values at a bin, V far
+// below the 2^14 a 14-bit value could take (at most 512; 110-170 in 8,192 tree
+// samples), so equality with a row is decided by the value's rank among those
+// V: code 1 .. V for a value some row of the group holds, 0 for any other.
+// Two codes are equal exactly when the values are, as one of them is always a
+// row's; the match counts are the same whole numbers.  A run of 32 bins
+// ("half", one dword of the sketch words) then needs only the planes of its
+// largest code (its width, 3 .. CODE_PLANES) instead of 14: width + 1 VALU
+// operations per pair and half instead of 15.
+//
+// code_kernel, one workgroup per (group, k-mer length, half), builds the
+// ranks in LDS: per bin a bitmap of the 2^14 values (512 dwords, a row's value
+// sets one bit) and beside each dword the number of values set in the dwords
+// before it (8 bytes an entry, 4 KiB a bin, 128 KiB for the half).  A code is
+// one 8-byte read, a shift, a population count and an add.  Samples arrive and
+// leave bit-sliced; a 16 x 16 bit transpose of both dword halves at once turns
+// the 14 planes of a lane's sample into its 32 values and the 32 codes into
+// planes.  Bound by VALU: 465 instructions per sample and half (of 32 bins),
+// 69% of the time issuing, with about 3 bytes per sample and bin beside it;
+// shared by the group's rows that is under one operation per pair and half,
+// against the 6 or 7 it saves.  8,192 samples against themselves: coding 3.1 ms
+// and matching 21.8 ms (90% of the VALU issue rate, 9 operations per pair and
+// half) instead of 34.4 ms; the call 34.9 -> 26.3 ms, kNN of 3,000 5.5 -> 4.6
+// ms, 451 queries x 6,000 3.26 -> 2.45 ms.
+//
+// Codes: [k-mer length][block of 256 samples][half][CODE_PLANES][256] dwords
+// per group, each half using its first `width` planes.
+// ---------------------------------------------------------------------------
+constexpr int CODE_TB = 1024;
+constexpr int CODE_SLOT = CODE_PLANES * 256;  // dwords of one (block, half)
+
+__device__ __forceinline__ uint32_t bit_select(uint32_t m, uint32_t a, uint32_t b) {
+  return (a & m) | (b & ~m);
+}
+
+// One stage of the transpose below: swaps bit blocks of side S.
+template <int N, int S>
+__device__ __forceinline__ void transpose_stage(uint32_t (&x)[16]) {
+  constexpr uint32_t m = S == 4 ? 0x0F0F0F0Fu : (S == 2 ? 0x33333333u : 0x55555555u);
+#pragma unroll
+  for (int i = 0; i < N; ++i) {
+    if ((i & S) == 0) {
+      const uint32_t a = x[i], b = x[i + S];
+      x[i] = bit_select(m, a, b << S);
+      x[i + S] = bit_select(m, a >> S, b);
+    }
+  }
+}
+
+// Transposes the two 16 x 16 bit matrices held in the low and the high 16
+// bits of x[0..15] (bit j of x[i] <-> bit i of x[j]); its own inverse.  N: only
+// x[0..N-1] is needed of the result (N = 8 or 16).
+template <int N>
+__device__ __forceinline__ void transpose16(uint32_t (&x)[16]) {
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    const uint32_t a = x[i], b = x[i + 8];
+    x[i] = __builtin_amdgcn_perm(b, a, 0x06020400u);
+    if (N > 8) x[i + 8] = __builtin_amdgcn_perm(b, a, 0x07030501u);
+  }
+  transpose_stage<N, 4>(x);
+  transpose_stage<N, 2>(x);
+  transpose_stage<N, 1>(x);
+}
+
+// (device-memory pointers of the kernel's tables: without the address space
+// the compiler writes through flat stores, which also wait for LDS)
+typedef __attribute__((address_space(1))) uint32_t GU32;
+
+// The 14 planes of a sample at one half; transposed, its 32 values: bins i
+// (low 16 bits of x[i]) and 16 + i (high 16 bits).
+__device__ __forceinline__ void load_planes(const GU32* planes, uint32_t (&x)[BBITS]) {
+#pragma unroll
+  for (int l = 0; l < BBITS; ++l) x[l] = planes[l * BLK];
+}
+
+__device__ __forceinline__ void to_values(const uint32_t (&pl)[BBITS], uint32_t (&x)[16]) {
+#pragma unroll
+  for (int l = 0; l < BBITS; ++l) x[l] = pl[l];
+  x[14] = x[15] = 0;
+  transpose16<16>(x);
+}
+
+struct CodeSet {  // samples to code: [s0, s1) of a set
+  const GU32* planes;    // (kk, block 0, word, plane 0 of the half)
+  int64_t block_stride;  // dwords between 128-sample blocks
+  GU32* out;             // (kk, block b0, half)
+  int64_t out_stride;    // dwords between 256-sample blocks
+  int b0;
+  int s0, s1;
+};
+
+__device__ __forceinline__ const GU32* code_source(const CodeSet& cs, int s) {
+  return cs.planes + (int64_t)(s / BLK) * cs.block_stride + s % BLK;
+}
+
+// pl: the planes of the lane's first sample, already loaded; the next sample's
+// are loaded while one is looked up.
+template <int N>
+__device__ __forceinline__ void code_samples(const CodeSet& cs, const uint2* tab, int width,
+                                             uint32_t (&pl)[BBITS]) {
+  for (int s = cs.s0 + (int)threadIdx.x; s < cs.s1; s += CODE_TB) {
+    uint32_t x[16];
+    to_values(pl, x);
+    load_planes(code_source(cs, min(s + CODE_TB, cs.s1 - 1)), pl);
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      const uint32_t v0 = x[i] & 0xFFFFu, v1 = x[i] >> 16;
+      const uint2 e0 = tab[i * 512 + (v0 >> 5)];
+      const uint2 e1 = tab[(16 + i) * 512 + (v1 >> 5)];
+      // the bit of value v is bit 31 - v % 32 of its dword: shifted up to
+      // bit 31, the sign says whether it is set and the population count is
+      // its rank in the dword
+      const uint32_t t0 = e0.x << (v0 & 31), t1 = e1.x << (v1 & 31);
+      const uint32_t c0 = (uint32_t)((int32_t)t0 >> 31) & (e0.y + __popc(t0));
+      const uint32_t c1 = (uint32_t)((int32_t)t1 >> 31) & (e1.y + __popc(t1));
+      x[i] = c0 | (c1 << 16);
+    }
+    transpose16<N>(x);
+    GU32* o = cs.out + (s / 256 - cs.b0) * cs.out_stride + s % 256;
+#pragma unroll
+    for (int l = 0; l < (N < CODE_PLANES ? N : CODE_PLANES); ++l) {
+      if (l < width) o[l * 256] = x[l];
+    }
+  }
+}
+
+// Sum of x over the lanes up to and including this one.
+__device__ __forceinline__ uint32_t wave_prefix(uint32_t x) {
+  // row_shr 1, 2, 4, 8 inside the rows of 16 lanes, then the row totals
+  x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x111, 0xf, 0xf, true);
+  x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x112, 0xf, 0xf, true);
+  x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x114, 0xf, 0xf, true);
+  x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x118, 0xf, 0xf, true);
+  x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x142, 0xa, 0xf, false);  // row_bcast15
+  x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x143, 0xc, 0xf, false);  // row_bcast31
+  return x;
+}
+
+// One (group, k-mer length, half) of a coding launch.
+struct CodeItem {
+  int kh;
+  CodeSet rows, cols;
+  GU32* widths;
+  bool apart;  // rows coded apart from the columns
+};
+
+__device__ __forceinline__ CodeItem code_item(const DistParams& p, const CodeGroup* groups,
+                                              int n_groups, int item) {
+  const CodeGroup cg = groups[item % n_groups];
+  CodeItem it;
+  it.kh = item / n_groups;
+  const int halves = 2 * p.s64;
+  const int kk = it.kh / halves;
+  const int half = it.kh - kk * halves;
+  const int64_t rblock = (int64_t)p.s64 * (HL * BLK);
+  const int64_t at = (int64_t)(half >> 1) * (HL * BLK) + (half & 1) * (BBITS * BLK);
+  const int64_t out_stride = (int64_t)halves * CODE_SLOT;
+  it.cols.planes = (const GU32*)p.col_stripes + (int64_t)kk * p.nb_cols * rblock + at;
+  it.cols.block_stride = rblock;
+  it.cols.out = (GU32*)cg.cols + (int64_t)kk * cg.ncb * out_stride + (int64_t)half * CODE_SLOT;
+  it.cols.out_stride = out_stride;
+  it.cols.b0 = cg.cb0;
+  it.cols.s0 = cg.cb0 * 256;
+  it.cols.s1 = min(p.nb_cols * BLK, (cg.cb0 + cg.ncb) * 256);
+  it.rows = it.cols;
+  it.rows.planes = (const GU32*)p.row_stripes + (int64_t)kk * p.nb_rows * rblock + at;
+  it.rows.out = (GU32*)cg.rows + (int64_t)kk * cg.nrb * out_stride + (int64_t)half * CODE_SLOT;
+  it.rows.b0 = cg.rb0;
+  it.rows.s0 = cg.row0;
+  it.rows.s1 = cg.row0 + cg.n_rows;
+  it.widths = (GU32*)cg.widths;
+  it.apart = cg.rows != cg.cols;
+  return it;
+}
+
+// Persistent: one workgroup per CU (its table fills the LDS) takes items
+// blockIdx.x, + gridDim.x, ...: the row planes of the next item and the first
+// columns of this one are loaded while the table is cleared, filled and
+// summed, which as a launch of one workgroup per item left the CU idle for
+// 11 us of every 15 (1,501 samples) to 40 us (8,192).  The groups of one
+// (k-mer length, half) run side by side, as they read the same columns; the
+// grid has no common factor with the number of groups, so that every
+// workgroup meets long and short ones alike.
+__global__ __launch_bounds__(CODE_TB) void code_kernel(DistParams p, const CodeGroup* groups,
+                                                       int n_groups, int n_items) {
+  __shared__ uint2 tab[32 * 512];
+  __shared__ uint32_t s_most;
+  const int lane = threadIdx.x & 63;
+  const int wave = threadIdx.x >> 6;
+  constexpr int HALF_TB = CODE_TB / 2;
+  const int r = (int)(threadIdx.x & (HALF_TB - 1));
+  const bool high = threadIdx.x >= HALF_TB;
+  CodeItem it = code_item(p, groups, n_groups, (int)blockIdx.x);
+  uint32_t rpl[BBITS];
+  load_planes(code_source(it.rows, min(it.rows.s0 + r, it.rows.s1 - 1)), rpl);
+  for (int item = (int)blockIdx.x; item < n_items; item += (int)gridDim.x) {
+    uint32_t cpl[BBITS];
+    load_planes(code_source(it.cols, min(it.cols.s0 + (int)threadIdx.x, it.cols.s1 - 1)), cpl);
+    uint4* clr = reinterpret_cast<uint4*>(tab);
+    for (int x = threadIdx.x; x < 32 * 512 / 2; x += CODE_TB) clr[x] = make_uint4(0, 0, 0, 0);
+    if (threadIdx.x == 0) s_most = 0;
+    __syncthreads();
+    // rows into the bitmaps: lanes 0 .. 511 the low 16 bins of a row, the
+    // others the high 16
+    for (int row = it.rows.s0 + r; row < it.rows.s1; row += HALF_TB) {
+      if (row >= it.rows.s0 + HALF_TB) load_planes(code_source(it.rows, row), rpl);
+      uint32_t x[16];
+      to_values(rpl, x);
+      uint2* t = tab + (high ? 16 * 512 : 0);
+#pragma unroll
+      for (int i = 0; i < 16; ++i) {
+        const uint32_t v = high ? x[i] >> 16 : x[i] & 0xFFFFu;
+        atomicOr(&t[i * 512 + (v >> 5)].x, 0x80000000u >> (v & 31));
+      }
+    }
+    __syncthreads();
+    // ranks: each wave takes two bins, lane l the dwords l, 64 + l, ...; the
+    // order of the dwords does not matter, only that every value's rank differs
+    {
+      uint2* t0 = tab + (wave * 2) * 512 + lane;
+      uint2* t1 = t0 + 512;
+      uint32_t n0[8], n1[8], sum0 = 0, sum1 = 0;
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        n0[i] = sum0;
+        n1[i] = sum1;
+        sum0 += __popc(t0[i * 64].x);
+        sum1 += __popc(t1[i * 64].x);
+      }
+      const uint32_t incl0 = wave_prefix(sum0), incl1 = wave_prefix(sum1);
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        t0[i * 64].y = incl0 - sum0 + n0[i];
+        t1[i * 64].y = incl1 - sum1 + n1[i];
+      }
+      if (lane == 63) atomicMax(&s_most, max(incl0, incl1));
+    }
+    __syncthreads();
+    const int width = max(3, 32 - __clz((int)s_most));
+    if (threadIdx.x == 0) it.widths[it.kh] = (uint32_t)width;
+    const CodeItem now = it;
+    if (item + (int)gridDim.x < n_items) {
+      it = code_item(p, groups, n_groups, item + (int)gridDim.x);
+      load_planes(code_source(it.rows, min(it.rows.s0 + r, it.rows.s1 - 1)), rpl);
+    }
+    if (width <= 8) {
+      code_samples<8>(now.cols, tab, width, cpl);
+    } else {
+      code_samples<16>(now.cols, tab, width, cpl);
+    }
+    if (now.apart) {
+      load_planes(code_source(now.rows, min(now.rows.s0 + (int)threadIdx.x, now.rows.s1 - 1)), cpl);
+      if (width <= 8) {
+        code_samples<8>(now.rows, tab, width, cpl);
+      } else {
+        code_samples<16>(now.rows, tab, width, cpl);
+      }
+    }
+    __syncthreads();  // the table is free
+  }
+}
+
+// ---------------------------------------------------------------------------
+// Matching of coded planes (dist_coded).  The same wave grid, operand pipeline
+// and rules as match_stage_pipe; a half of width P is P planes in an even
+// number of batches of 2 planes, then of 1 (so that the two register sets keep
+// their roles); the first always has 2, so that the last batch of a half can
+// issue the first of the next half whatever its width.  (Batches of 3 would
+// make widths 5, 9 and 10 shorter, but their third row tuple spills SGPRs.)
+// ---------------------------------------------------------------------------
+constexpr int code_batches(int P) { return P <= 4 ? 2 : (P <= 8 ? 4 : 6); }
+constexpr int code_batch(int P, int b) {  // planes of batch b: as many of 2 as leave 1 for the rest
+  return b < P - code_batches(P) ? 2 : 1;
+}
+constexpr int code_first(int P, int b) { return b == 0 ? 0 : code_first(P, b - 1) + code_batch(P, b - 1); }
+static_assert(code_first(3, 2) == 3 && code_first(4, 2) == 4 && code_first(5, 4) == 5 &&
+                  code_first(6, 4) == 6 && code_first(7, 4) == 7 && code_first(8, 4) == 8 &&
+                  code_first(9, 6) == 9 && code_first(10, 6) == 10,
+              "batches cover the planes of every width");
+static_assert(code_batch(3, 0) == 2 && code_batch(5, 0) == 2 && code_batch(9, 0) == 2,
+              "the first batch has 2 planes");
+
+// Operands of up to 2 planes: 8 rows in SGPRs and RR columns per lane each.
+template <int RR>
+struct CodeBatch {
+  ATuple<8>::T a[2];
+  u32x2 b[2][RR == 4 ? 2 : 1];
+};
+
+// Issue NP planes: row plane x at aw + AOFF + 1024 x bytes, column plane x at
+// LDS address bw + (BP + x) KiB.
+template <int RR, int NP, int AOFF, int BP>
+__device__ __forceinline__ void code_issue(const CU32* aw, uint32_t bw, CodeBatch<RR>& x) {
+  a_load<8, AOFF>(aw, x.a[0]);
+  if constexpr (NP > 1) a_load<8, AOFF + 1024>(aw, x.a[1]);
+#pragma unroll
+  for (int i = 0; i < NP; ++i) {
+    if constexpr (RR == 1) {
+      asm volatile("ds_read_b32 %0, %1 offset:%2"
+                   : "=&v"(x.b[i][0].x)
+                   : "v"(bw), "i"((BP + i) * 1024));
+    } else {
+#pragma unroll
+      for (int r = 0; r < RR / 2; ++r) {
+        asm volatile("ds_read2st64_b32 %0, %1 offset0:%2 offset1:%3"
+                     : "=&v"(x.b[i][r])
+                     : "v"(bw), "i"((BP + i) * 4 + 2 * r), "i"((BP + i) * 4 + 2 * r + 1));
+      }
+    }
+  }
+}
+
+// WAIT: the wait for a batch's loads; else only keeps its registers alive and
+// in place at this point (batch_hold).  Two asm blocks, as the compiler takes
+// every output of a block that also has vector outputs for divergent and would
+// move the row operands through VGPRs where paths join.
+template <int RR, int NP, bool WAIT>
+__device__ __forceinline__ void code_pin(CodeBatch<RR>& x) {
+  if constexpr (WAIT && NP == 2) {
+    asm volatile("s_waitcnt lgkmcnt(0)" : "+s"(x.a[0]), "+s"(x.a[1]));
+  } else if constexpr (WAIT) {
+    asm volatile("s_waitcnt lgkmcnt(0)" : "+s"(x.a[0]));
+  } else if constexpr (NP == 2) {
+    asm volatile("" : "+s"(x.a[0]), "+s"(x.a[1]));
+  } else {
+    asm volatile("" : "+s"(x.a[0]));
+  }
+#pragma unroll
+  for (int i = 0; i < NP; ++i) {
+    if constexpr (RR == 4) {
+      asm volatile("" : "+v"(x.b[i][0]), "+v"(x.b[i][1]));
+    } else if constexpr (RR == 2) {
+      asm volatile("" : "+v"(x.b[i][0]));
+    } else {
+      asm volatile("" : "+v"(x.b[i][0].x));
+    }
+  }
+}
+
+// Batches B .. of one half of width P; cur holds batch B (complete).  The
+// last one issues the first batch of the next half: its row planes lie one
+// slot on, its column planes follow in the stage (past the stage's last half
+// the loads read other bytes of the buffers, which nothing uses).
+template <int RR, int P, int B>
+__device__ __forceinline__ void code_match(const CU32* aw, uint32_t bw, CodeBatch<RR>& cur,
+                                           CodeBatch<RR>& nxt, uint32_t (&acc)[8][RR],
+                                           uint32_t (&cnt)[8][RR]) {
+  constexpr int NB = code_batches(P), NP = code_batch(P, B), P0 = code_first(P, B);
+  if constexpr (B + 1 < NB) {
+    code_issue<RR, code_batch(P, B + 1), (P0 + NP) * 1024, P0 + NP>(aw, bw, nxt);
+  } else {
+    code_issue<RR, 2, CODE_SLOT * 4, P>(aw, bw, nxt);
+  }
+  code_pin<RR, NP, false>(cur);
+#pragma unroll
+  for (int i = 0; i < NP; ++i) {
+#pragma unroll
+    for (int q = 0; q < 8; ++q) {
+#pragma unroll
+      for (int r = 0; r < RR; ++r) {
+        const uint32_t a = cur.a[i][q];
+        const uint32_t b = cur.b[i][r / 2][r % 2];
+        acc[q][r] = P0 + i == 0 ? ~(a ^ b) : match_and(acc[q][r], a, b);
+      }
+    }
+  }
+  if constexpr (B + 1 < NB) {
+    code_pin<RR, code_batch(P, B + 1), true>(nxt);
+    code_match<RR, P, B + 1>(aw, bw, nxt, cur, acc, cnt);
+  } else {
+#pragma unroll
+    for (int q = 0; q < 8; ++q)
+#pragma unroll
+      for (int r = 0; r < RR; ++r) {
+        asm("v_bcnt_u32_b32 %0, %1, %0" : "+v"(cnt[q][r]) : "v"(acc[q][r]));
+      }
+    code_pin<RR, 2, true>(nxt);
+  }
+}
+
+// The next halves of the stage as long as they are P planes wide (widths left
+// in ws, 4 bits each).
+template <int RR, int P>
+__device__ __forceinline__ void code_halves(const CU32*& aw, uint32_t& bw, uint32_t& ws,
+                                            CodeBatch<RR>& c, CodeBatch<RR>& n,
+                                            uint32_t (&cnt)[8][RR]) {
+  while ((ws & 15u) == (uint32_t)P) {
+    uint32_t acc[8][RR];
+    code_match<RR, P, 0>(aw, bw, c, n, acc, cnt);
+    aw += CODE_SLOT;
+    bw += P * 1024;
+    ws >>= 4;
+  }
+}
+
+// A stage: as many whole halves as fit CODE_STAGE planes, at most 8; widths
+// packed 4 bits each.
+struct CodeStage {
+  uint32_t widths;
+  int halves, planes;
+};
+
+typedef uint32_t u32x8 __attribute__((ext_vector_type(8)));
+
+__device__ __forceinline__ CodeStage code_stage(const u32x8& w, int left) {
+  CodeStage st{0, 0, 0};
+#pragma unroll
+  for (int i = 0; i < 8; ++i) st.widths |= (w[i] & 15u) << (4 * i);
+  st.widths = __builtin_amdgcn_readfirstlane(st.widths);
+  const int most = left < 8 ? left : 8;
+  while (st.halves < most) {
+    const int planes = st.planes + (int)((st.widths >> (4 * st.halves)) & 15u);
+    if (planes > CODE_STAGE) break;
+    st.planes = planes;
+    st.halves += 1;
+  }
+  if (st.halves < 8) st.widths &= (1u << (4 * st.halves)) - 1u;
+  return st;
+}
+
+// Copies of one stage: column planes (1 KiB each, one wave instruction)
+// packed into the stage buffer, plane l of a half by wave l % 8; row planes, 4 at a time
+// (64 rows each), into a scratch KiB that nothing reads, only so that the
+// scalar loads find them in L2.
+__device__ __forceinline__ void code_copy(const CodeStage& st, const uint32_t* cols,
+                                          const uint32_t* rows, bool rpf, uint32_t dst,
+                                          uint32_t row_dst, int wave, uint32_t coff,
+                                          uint32_t roff) {
+  for (int x = 0; x < st.halves; ++x) {
+    const int w = (int)(st.widths >> (4 * x)) & 15;
+    if (wave < w) dma16<0>(cols + wave * 256, coff, dst + (uint32_t)wave * 1024);
+    if (wave + WAVES < w) {
+      dma16<WAVES * 1024>(cols + (wave + WAVES) * 256, coff, dst + (uint32_t)wave * 1024);
+    }
+    const int quad = (wave - 3 * x) & (WAVES - 1);  // quads 0 .. 2 of the half
+    if (rpf && 4 * quad < w) dma16<0>(rows + quad * 1024, roff, row_dst);
+    cols += CODE_SLOT;
+    rows += CODE_SLOT;
+    dst += (uint32_t)w * 1024;
+  }
+}
+
+template <int RR>
+__device__ __forceinline__ void coded_item(const CU32* widths, const uint32_t* cols,
+                                           const uint32_t* rows, bool rpf, int halves,
+                                           uint32_t buf, uint32_t row_dst, uint16_t* counts,
+                                           int wave, int lane) {
+  constexpr int CG = TileCfg<8, RR>::CG;
+  const uint32_t coff = (uint32_t)lane * 16;
+  const uint32_t roff = (uint32_t)((lane >> 4) * 1024 + (lane & 15) * 16);
+  const uint32_t col = (uint32_t)((wave % CG) * 64 * RR + lane) * 4;
+  const CU32* arow = (CU32*)(rows + (wave / CG) * 8);
+  uint32_t cnt[8][RR];
+#pragma unroll
+  for (int q = 0; q < 8; ++q)
+#pragma unroll
+    for (int r = 0; r < RR; ++r) cnt[q][r] = 0;
+  CodeBatch<RR> c, n;
+  u32x8 w8;
+  asm volatile("s_load_dwordx8 %0, %1, 0\n\ts_waitcnt lgkmcnt(0)" : "=&s"(w8) : "s"(widths));
+  CodeStage cur = code_stage(w8, halves);
+  code_copy(cur, cols, rows, rpf, buf, row_dst, wave, coff, roff);
+  int h = 0;  // first half of the current stage
+  uint32_t at = buf;
+  asm volatile("s_load_dwordx8 %0, %1, 0\n\ts_waitcnt lgkmcnt(0)"
+               : "=&s"(w8)
+               : "s"(widths + cur.halves));
+  CodeStage nxt = code_stage(w8, halves - cur.halves);
+  for (;;) {
+    // one barrier per stage, as in tile_stages
+    wait_vmcnt<0>();
+    stage_barrier();
+    const int h1 = h + cur.halves;
+    const uint32_t other = buf + (at == buf ? (uint32_t)CODE_STAGE * 1024 : 0u);
+    code_copy(nxt, cols + (int64_t)h1 * CODE_SLOT, rows + (int64_t)h1 * CODE_SLOT, rpf, other,
+              row_dst, wave, coff, roff);
+    const CU32* aw = arow + (int64_t)h * CODE_SLOT;
+    uint32_t bw = at + col;
+    code_issue<RR, 2, 0, 0>(aw, bw, c);
+    // the widths of the stage after the next arrive with the first batch
+    asm volatile("s_load_dwordx8 %0, %1, 0\n\ts_waitcnt lgkmcnt(0)"
+                 : "=&s"(w8)
+                 : "s"(widths + h1 + nxt.halves));
+    code_pin<RR, 2, true>(c);
+    const CodeStage after = code_stage(w8, halves - h1 - nxt.halves);
+    // one loop per width, in turn until the stage is done: a value has one
+    // successor at every step, so the counts and operands stay in their
+    // registers (a switch moves all of them at every half: 44 moves beside the
+    // 288 operations of 8 planes)
+    uint32_t ws = cur.widths;
+    while (ws != 0) {
+      code_halves<RR, 8>(aw, bw, ws, c, n, cnt);
+      code_halves<RR, 7>(aw, bw, ws, c, n, cnt);
+      code_halves<RR, 6>(aw, bw, ws, c, n, cnt);
+      code_halves<RR, 9>(aw, bw, ws, c, n, cnt);
+      code_halves<RR, 5>(aw, bw, ws, c, n, cnt);
+      code_halves<RR, 4>(aw, bw, ws, c, n, cnt);
+      code_halves<RR, 3>(aw, bw, ws, c, n, cnt);
+      code_halves<RR, 10>(aw, bw, ws, c, n, cnt);
+    }
+    if (nxt.halves == 0) break;
+    h = h1;
+    cur = nxt;
+    nxt = after;
+    at = other;
+  }
+  store_counts<8, RR>(counts, 0, wave, lane, cnt);
+}
+
+__global__ __launch_bounds__(WAVES * 64, 4) void dist_coded(DistParams p, ItemArgs a,
+                                                            const CodeGroup* groups) {
+  // two stages; the row scratch KiB, and what the last operand batch of a stage
+  // reads past it (2 planes)
+  __shared__ uint4 s_buf[2 * CODE_STAGE * 64 + 3 * 64];
+  __shared__ int s_stop;
+  const int all = 2 * p.s64;  // halves of a sketch
+  ItemAt it;
+  if (!item_at(a, p.n_k, all, it)) return;
+  if (a.watch) {
+    if (threadIdx.x == 0) s_stop = cancel_seen(p.ctl.cancel) ? 1 : 0;
+    __syncthreads();
+    if (__builtin_amdgcn_readfirstlane(s_stop)) return;
+  }
+  const int kk = it.kk;
+  const ItemTile tile = a.tiles[it.tile];
+  const int row0 = __builtin_amdgcn_readfirstlane(tile.row0);
+  const int ct = __builtin_amdgcn_readfirstlane(tile.ct);
+  const int rows = __builtin_amdgcn_readfirstlane(tile.rows);
+  // scalar loads: the table is never written while the kernel runs
+  CCodeGroup& g = ((CCodeGroup*)groups)[__builtin_amdgcn_readfirstlane(tile.group)];
+  const int h0 = it.unit0;
+  const int halves = it.units;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int lane = threadIdx.x & 63;
+  const int64_t block = (int64_t)all * CODE_SLOT;
+  const int64_t at = (int64_t)h0 * CODE_SLOT;
+  const uint32_t* cols = g.cols + ((int64_t)kk * g.ncb + (ct - g.cb0)) * block + at;
+  const uint32_t* rws =
+      g.rows + ((int64_t)kk * g.nrb + (row0 / 256 - g.rb0)) * block + at + row0 % 256;
+  const CU32* widths = (CU32*)(g.widths + kk * all + h0);
+  uint16_t* counts = p.counts + it.block * ITEM_COUNTS;
+  const uint32_t buf = lds_addr(s_buf);
+  const uint32_t row_dst = buf + 2 * CODE_STAGE * 1024;
+  const bool rpf = p.row_prefetch != 0;
+  if (rows == 64) {
+    coded_item<4>(widths, cols, rws, rpf, halves, buf, row_dst, counts, wave, lane);
+  } else if (rows == 32) {
+    coded_item<2>(widths, cols, rws, rpf, halves, buf, row_dst, counts, wave, lane);
+  } else {
+    coded_item<1>(widths, cols, rws, rpf, halves, buf, row_dst, counts, wave, lane);
+  }
+  if (threadIdx.x == 0) add_progress(p.ctl, 1ull);
+}
+
+hipError_t launch_coded(const DistParams& p, const ItemArgs& a, const CodeGroup* groups,
+                        int first_group, int n_groups, hipStream_t stream) {
+  if (a.n_items <= 0 || n_groups <= 0) return hipSuccess;
+  const int n_code = n_groups * p.n_k * 2 * p.s64;
+  int dev = 0, grid = 0;
+  hipError_t e = hipGetDevice(&dev);
+  if (e == hipSuccess) e = hipDeviceGetAttribute(&grid, hipDeviceAttributeMultiprocessorCount, dev);
+  if (e != hipSuccess) return e;
+  while (grid > 1 && std::gcd(grid, n_groups) != 1) --grid;
+  code_kernel<<<(unsigned)std::min(grid, n_code), CODE_TB, 0, stream>>>(p, groups + first_group,
+                                                                        n_groups, n_code);
+  dist_coded<<<item_grid(a), WAVES * 64, 0, stream>>>(p, a, groups);
+  dist_items_out<<<(unsigned)(a.n_tiles * (64 / a.out_rows)), 256, 0, stream>>>(p, a);
   return hipGetLastError();
 }
 

@@ -557,81 +557,91 @@ int run_dense_persistent(DeviceCtx* c, ppsk::DistParams p, int variant, bool upp
   return PPSK_OK;
 }
 
-// Tiles of a split pass over rows [row_begin, row_end) (row_begin a multiple
-// of 64): 64-row tiles, the rows past the last multiple of 64 in 32- and
-// 16-row ones, so that 451 rows compute 464 and not 512.  Groups of
-// `group_rows` rows (a multiple of 64), column by column inside a group, as
-// make_tiles.
-std::vector<ppsk::ItemTile> item_tiles(int64_t n_cols, bool upper, int64_t row_begin,
-                                       int64_t row_end, int64_t group_rows,
-                                       std::vector<size_t>* group_start) {
-  std::vector<ppsk::ItemTile> t;
-  const int64_t nct = (n_cols + 255) / 256;
-  group_start->clear();
-  for (int64_t g0 = row_begin; g0 < row_end; g0 += group_rows) {
-    const int64_t g1 = std::min(row_end, g0 + group_rows);
-    std::vector<std::pair<int64_t, int32_t>> segs;  // first row, height
-    for (int64_t r = g0; r < g1;) {
-      const int64_t left = g1 - r;
-      const int32_t h = left > 48 ? 64 : (left > 16 ? 32 : 16);
-      segs.emplace_back(r, h);
-      r += h;
-    }
-    const size_t before = t.size();
-    for (int64_t ct = 0; ct < nct; ++ct) {
-      for (const auto& sg : segs) {
-        if (upper && (ct + 1) * 256 - 1 <= sg.first) continue;
-        t.push_back({(int32_t)sg.first, (int32_t)ct, sg.second});
-      }
-    }
-    if (t.size() > before) group_start->push_back(before);
-  }
-  group_start->push_back(t.size());
-  return t;
-}
-
-// Word runs per (tile, k-mer length) of a split pass of n_tiles tiles holding
-// `rows64` 64-row tile equivalents: the count of least estimated time over
-// the rounds the 512 resident workgroups (2 per CU) need.  Measured on 64-row
-// tiles: 6.4 us per word with two workgroups on a CU, 3.5 us alone; about 4 us
-// to start an item; and each item's counts are written and read once (about
-// 0.016 us of the chip's memory time).  One launch holds at most 32,768
-// items of counts (1 GiB).
-int item_runs(int64_t n_tiles, double rows64, int n_k, int s64) {
-  const double weight = rows64 / (double)n_tiles;
-  const int64_t base = n_tiles * n_k;
-  int best = 1;
-  double best_t = -1.0;
-  for (int words = s64; words >= 1; --words) {
-    const int runs = (s64 + words - 1) / words;
-    const int64_t n = base * runs;
-    if (runs > 1 && n > 32768) break;
-    const int64_t rest = n % 512;
-    const double rounds = (double)(n / 512) + (rest == 0 ? 0.0 : (rest <= 256 ? 0.55 : 1.0));
-    const double t = rounds * (4.0 + 6.4 * weight * words) + 0.016 * (double)n;
-    if (best_t < 0.0 || t < best_t) {
-      best_t = t;
-      best = runs;
-    }
-  }
-  return best;
-}
-
-// The split pass (dist_items): every tile's words cut into runs when there
-// are too few (tile, k-mer length) items to fill the CUs, then one lane per
-// pair for the output.  Launches are cut at group boundaries so that each
-// fits the count scratch; with host_out, each launch's finished rows are
-// copied out while the next ones compute.
+// A split pass over rows [row_begin, row_end) (row_begin a multiple of 64).
+// Rows are taken in groups, column by column inside a group (as make_tiles),
+// in 64-row tiles; the rows past a group's last multiple of 64 in 32- and
+// 16-row ones, so that 451 rows compute 464 and not 512.  A slab is a group,
+// or, in a coded pass, a group and as many of its column blocks as fit the
+// scratch; a launch (chunk) is a run of whole slabs.
 struct ItemPlan {
+  struct Chunk {
+    size_t tile0, tile1;
+    int slab0, slab1;
+    int64_t copy0, copy1;  // rows whose last column is computed by this launch
+    double work_us;  // estimated time of the matching
+    int n_tall, whole, runs, run_units;  // ItemArgs (units: words, or halves of a coded pass)
+    int64_t items;
+  };
+  bool coded = false;
   std::vector<ppsk::ItemTile> tiles;
-  std::vector<std::pair<size_t, size_t>> chunks;  // tiles of each launch
-  int runs = 1, run_words = 0;
+  std::vector<ppsk::CodeGroup> slabs;  // coded passes; pointers filled in by the run
+  std::vector<char> apart;             // slab whose rows do not lie among its columns
+  std::vector<Chunk> chunks;
+  size_t code_bytes = 0;  // coded scratch of the largest launch
+  size_t count_blocks = 0;  // items of the largest launch
   uint64_t items = 0;
+  double work_us = 0.0;  // estimated time
 };
 
-ItemPlan plan_items(int64_t n_cols, int n_k, int s64, bool upper, int64_t row_begin,
-                    int64_t row_end, bool host_out) {
+// Items of a launch: whole rounds of the 512 resident workgroups (2 per CU) of
+// 64-row tiles as they are; the other pairs, the shorter tiles among them, cut
+// into runs, about 2,400 items in all, of at least 8 words each.  Fewer leave
+// slots idle at the end, more cost their start (a few us) and their counts,
+// written and read once.  Measured, us per call at 1, 4, 8, 16, 24 runs: 333
+// samples (80 pairs) 664, 348, 286, 257, 265; 1,000 (328 pairs) 1103, 852, 807,
+// 846, 1080; 451 queries x 6,000 (512 pairs after two whole rounds, coded) 2582,
+// 2551, 2409, 2482, 2712.
+void item_runs(ItemPlan::Chunk* ch, const std::vector<ppsk::ItemTile>& tiles, int n_k, int s64,
+               bool coded) {
+  const int units = coded ? 2 * s64 : s64;
+  const double unit_us = coded ? 2.2 : 6.4;
+  int64_t n[3] = {0, 0, 0};  // tiles of 64, 32, 16 rows
+  for (size_t x = ch->tile0; x < ch->tile1; ++x) {
+    ++n[tiles[x].rows == 64 ? 0 : (tiles[x].rows == 32 ? 1 : 2)];
+  }
+  const int64_t pairs = (n[0] + n[1] + n[2]) * n_k;
+  ch->n_tall = (int)n[0];
+  ch->whole = (int)(n[0] * n_k / 512 * 512);
+  ch->runs = 1;
+  ch->run_units = units;
+  ch->items = pairs;
+  ch->work_us = ((double)n[0] + 0.57 * n[1] + 0.37 * n[2]) * n_k * unit_us * units / 512.0;
+  const int64_t rest = pairs - ch->whole;
+  if (rest == 0) return;
+  const int shortest = coded ? 16 : 8;
+  const int64_t want = std::max<int64_t>(1, (2400 + rest / 2) / rest);
+  const int runs = (int)std::min<int64_t>(want, std::max(1, units / shortest));
+  ch->run_units = (units + runs - 1) / runs;
+  ch->runs = (units + ch->run_units - 1) / ch->run_units;
+  ch->items = ch->whole + rest * ch->runs;
+}
+
+// Whether a split pass codes its rows' values (code_kernel).  Coding costs a
+// row group about 44 us and 35 us per 1,024 of its columns, matching coded
+// planes saves about 0.4 us per 1,000 pairs (8 k-mer lengths, 10,000 bins; both
+// scale with the sketch).  Measured, planes / coded (us per call): 64 queries x
+// 6,000 587 / 625, 128 x 6,000 971 / 843, 256 x 1,000 391 / 404, 451 x 1,000
+// 641 / 602; self passes of 700 530 / 547, 1,000 853 / 815, 3,000 5218 / 4386,
+// 8,192 34617 / 26371.  PPSK_CODED=0 / 1 forces the choice.
+bool use_coded(int64_t rows, int64_t n_cols, bool upper) {
+  if (const char* e = std::getenv("PPSK_CODED")) return std::atoi(e) != 0;
+  const double groups = std::ceil((double)rows / ppsk::CODE_ROWS);
+  const double half = upper ? 0.5 : 1.0;  // an upper triangle's share of the square
+  const double cols = groups * (double)n_cols * (upper ? 0.5 * (1.0 + 1.0 / groups) : 1.0);
+  return 0.4e-3 * half * (double)rows * (double)n_cols > 44.0 * groups + 35.0 / 1024 * cols + 40.0;
+}
+
+// Bytes of a slab's codes of nb blocks of 256 samples (one region: columns or
+// rows; the operand pipeline may read one slot past the end).
+size_t code_bytes(int n_k, int s64, int64_t nb) {
+  const size_t slot = (size_t)ppsk::CODE_PLANES * ppsk::CODE_BLOCK * sizeof(uint32_t);
+  return ((size_t)n_k * nb * 2 * s64 + 2) * slot;
+}
+
+ItemPlan plan_items(int64_t n_cols, int n_k, int s64, bool upper, bool same_set, int64_t row_begin,
+                    int64_t row_end, bool host_out, bool coded, size_t code_budget) {
   ItemPlan pl;
+  pl.coded = coded;
   // count scratch per launch; PPSK_CHUNK_BYTES lowers it (more, smaller
   // launches: finer-grained streaming of host output)
   size_t budget = (size_t)1 << 30;
@@ -642,59 +652,211 @@ ItemPlan plan_items(int64_t n_cols, int n_k, int s64, bool upper, int64_t row_be
   const size_t per_tile = (size_t)n_k * ppsk::ITEM_COUNTS * sizeof(uint16_t);
   size_t most = std::max<size_t>(1, budget / per_tile);
   const int64_t nct = (n_cols + 255) / 256;
-  const int64_t group_tiles = std::max<int64_t>(1, std::min<int64_t>(tile_group(64), (int64_t)most / nct));
-  std::vector<size_t> gs;
-  pl.tiles = item_tiles(n_cols, upper, row_begin, row_end, group_tiles * 64, &gs);
+  const int64_t rows = row_end - row_begin;
+  int64_t group = 64 * std::max<int64_t>(
+                           1, std::min<int64_t>(tile_group(64), (int64_t)most / std::max<int64_t>(nct, 1)));
+  if (coded) {
+    // equal groups of at most CODE_ROWS rows (768: at 8,192 samples 26.6 ms
+    // against 27.4 ms with 512, whose codes are half a plane shorter but take
+    // 1.5 times the coding, and 28.4 ms with 1,024)
+    const int64_t n = (rows + ppsk::CODE_ROWS - 1) / ppsk::CODE_ROWS;
+    group = ((rows + n - 1) / n + 63) / 64 * 64;
+  }
+  struct Slab {
+    size_t tile0, tile1, bytes;
+    int64_t r0, r1;  // rows it completes (r0 == r1: none)
+  };
+  std::vector<Slab> slabs;
+  for (int64_t g0 = row_begin; g0 < row_end; g0 += group) {
+    const int64_t g1 = std::min(row_end, g0 + group);
+    std::vector<std::pair<int64_t, int32_t>> segs;  // first row, height
+    for (int64_t r = g0; r < g1;) {
+      const int64_t left = g1 - r;
+      const int32_t h = left > 48 ? 64 : (left > 16 ? 32 : 16);
+      segs.emplace_back(r, h);
+      r += h;
+    }
+    const int64_t cb_first = upper ? g0 / 256 : 0;
+    const int64_t rb0 = g0 / 256, nrb = (g1 + 255) / 256 - rb0;
+    const size_t width_bytes = ((size_t)n_k * 2 * s64 + 64) * sizeof(uint32_t);
+    int64_t step = nct;  // column blocks per slab
+    size_t row_bytes = 0;
+    bool apart = false;
+    if (coded) {
+      const size_t block = code_bytes(n_k, s64, 1);
+      const size_t fixed = width_bytes + block + code_bytes(n_k, s64, nrb);
+      step = std::max<int64_t>(1, code_budget > fixed ? (int64_t)((code_budget - fixed) / block) : 1);
+      step = std::min<int64_t>(step, std::max<int64_t>(1, (int64_t)(most / segs.size())));
+      // the rows of a self pass are coded with the columns they lie among,
+      // unless those are cut
+      apart = !same_set || step < nct - cb_first;
+      if (apart) row_bytes = code_bytes(n_k, s64, nrb);
+    }
+    for (int64_t c0 = cb_first; c0 < nct; c0 += step) {
+      const int64_t c1 = std::min(nct, c0 + step);
+      Slab sl;
+      sl.tile0 = pl.tiles.size();
+      for (int64_t ct = c0; ct < c1; ++ct) {
+        for (const auto& sg : segs) {
+          if (upper && (ct + 1) * 256 - 1 <= sg.first) continue;
+          pl.tiles.push_back({(int32_t)sg.first, (int32_t)ct, sg.second, (int32_t)pl.slabs.size()});
+        }
+      }
+      sl.tile1 = pl.tiles.size();
+      if (sl.tile1 == sl.tile0) continue;
+      sl.r0 = g0;
+      sl.r1 = c1 == nct ? g1 : g0;
+      sl.bytes = coded ? code_bytes(n_k, s64, c1 - c0) + row_bytes + width_bytes : 0;
+      slabs.push_back(sl);
+      ppsk::CodeGroup cg;
+      std::memset(&cg, 0, sizeof(cg));
+      cg.row0 = (int32_t)g0;
+      cg.n_rows = (int32_t)(g1 - g0);
+      cg.cb0 = (int32_t)c0;
+      cg.ncb = (int32_t)(c1 - c0);
+      cg.rb0 = (int32_t)(apart ? rb0 : c0);
+      cg.nrb = (int32_t)(apart ? nrb : c1 - c0);
+      pl.slabs.push_back(cg);
+      pl.apart.push_back(apart ? 1 : 0);
+    }
+  }
   if (pl.tiles.empty()) return pl;
   if (host_out) most = std::min(most, std::max<size_t>(1024, pl.tiles.size() / 8));
-  for (size_t g = 0; g + 1 < gs.size();) {
-    size_t h = g + 1;
-    while (h + 1 < gs.size() && gs[h + 1] - gs[g] <= most) ++h;
-    pl.chunks.emplace_back(gs[g], gs[h]);
+  for (size_t g = 0; g < slabs.size();) {
+    size_t h = g + 1, bytes = slabs[g].bytes;
+    while (h < slabs.size() && slabs[h].tile1 - slabs[g].tile0 <= most &&
+           (!coded || bytes + slabs[h].bytes <= code_budget)) {
+      bytes += slabs[h].bytes;
+      ++h;
+    }
+    int64_t r0 = slabs[h - 1].r1, r1 = r0;
+    for (size_t x = g; x < h; ++x) {
+      if (slabs[x].r1 > slabs[x].r0) r0 = std::min(r0, slabs[x].r0);
+      r1 = std::max(r1, slabs[x].r1);
+    }
+    ItemPlan::Chunk ch;
+    std::memset(&ch, 0, sizeof(ch));
+    ch.tile0 = slabs[g].tile0;
+    ch.tile1 = slabs[h - 1].tile1;
+    ch.slab0 = (int)g;
+    ch.slab1 = (int)h;
+    ch.copy0 = std::min(r0, r1);
+    ch.copy1 = r1;
+    std::stable_partition(pl.tiles.begin() + ch.tile0, pl.tiles.begin() + ch.tile1,
+                          [](const ppsk::ItemTile& t) { return t.rows == 64; });
+    item_runs(&ch, pl.tiles, n_k, s64, coded);
+    pl.chunks.push_back(ch);
+    pl.items += (uint64_t)ch.items;
+    pl.work_us += ch.work_us;
+    pl.count_blocks = std::max(pl.count_blocks, (size_t)ch.items);
+    pl.code_bytes = std::max(pl.code_bytes, bytes);
     g = h;
   }
-  if (pl.chunks.size() == 1) {
-    double rows64 = 0.0;
-    for (const auto& t : pl.tiles) rows64 += t.rows == 64 ? 1.0 : (t.rows == 32 ? 0.57 : 0.37);
-    pl.runs = item_runs((int64_t)pl.tiles.size(), rows64, n_k, s64);
-  }
-  pl.run_words = (s64 + pl.runs - 1) / pl.runs;
-  pl.runs = (s64 + pl.run_words - 1) / pl.run_words;
-  pl.items = (uint64_t)pl.tiles.size() * n_k * pl.runs;
   return pl;
 }
 
+// Scratch a coded pass may take per launch: the codes of 8,192 samples against
+// themselves are 6.8 GiB, so that such a pass is one launch.
+constexpr size_t CODE_BUDGET = (size_t)8 << 30;
+
+// The plan a pass runs: coded when that pays, its scratch in place.  Where the
+// device has no room for the budget the slabs shrink, down to 256 MiB; below
+// that the pass runs on the planes as they are.
+int make_item_plan(DeviceCtx* c, const ppsk::DistParams& p, bool upper, int64_t row_begin,
+                   int64_t row_end, bool host_out, ItemPlan* out) {
+  const bool same = upper;  // the upper triangle of one set
+  uint64_t planned = 0;     // what dense_items reported
+  if (use_coded(row_end - row_begin, p.n_cols, upper)) {
+    for (size_t budget = CODE_BUDGET; budget >= ((size_t)256 << 20); budget /= 2) {
+      *out = plan_items(p.n_cols, p.n_k, p.s64, upper, same, row_begin, row_end, host_out, true, budget);
+      if (planned == 0) planned = out->items;
+      call_state(c->device).total += out->items - planned;
+      planned = out->items;
+      if (out->code_bytes <= c->codes_bytes) return PPSK_OK;
+      if (out->code_bytes > budget) break;  // one block of columns exceeds it
+      if (c->codes) HIP_TRY(hipFree(c->codes));
+      c->codes = nullptr;
+      c->codes_bytes = 0;
+      if (hipMalloc(&c->codes, out->code_bytes) == hipSuccess) {
+        c->codes_bytes = out->code_bytes;
+        return PPSK_OK;
+      }
+      (void)hipGetLastError();  // no room: the next smaller budget
+    }
+  }
+  *out = plan_items(p.n_cols, p.n_k, p.s64, upper, same, row_begin, row_end, host_out, false, 0);
+  if (planned) call_state(c->device).total += out->items - planned;
+  return PPSK_OK;
+}
+
+// The split pass: every tile's words cut into runs when there are too few
+// (tile, k-mer length) items to fill the CUs, then one lane per pair for the
+// output.  With host_out, each launch's finished rows are copied out while the
+// next ones compute.
 int run_dense_items(DeviceCtx* c, ppsk::DistParams p, bool upper, int64_t row_begin,
                     int64_t row_end, bool self, size_t elem, void* host_out, Timing* tm) {
-  const ItemPlan pl =
-      plan_items(p.n_cols, p.n_k, p.s64, upper, row_begin, row_end, host_out != nullptr);
+  ItemPlan pl;
+  if (int rc = make_item_plan(c, p, upper, row_begin, row_end, host_out != nullptr, &pl)) return rc;
   if (pl.tiles.empty()) return PPSK_OK;
-  size_t most = 0;
-  for (auto& ch : pl.chunks) most = std::max(most, ch.second - ch.first);
   const size_t item_bytes = ppsk::ITEM_COUNTS * sizeof(uint16_t);
-  if (int rc = grow(&c->counts, &c->counts_bytes, most * p.n_k * pl.runs * item_bytes)) return rc;
-  if (int rc = grow(&c->pitems, &c->pitems_bytes, pl.tiles.size() * sizeof(ppsk::ItemTile))) return rc;
-  HIP_TRY(hipMemcpyAsync(c->pitems, pl.tiles.data(), pl.tiles.size() * sizeof(ppsk::ItemTile),
-                         hipMemcpyHostToDevice, c->stream));
+  if (int rc = grow(&c->counts, &c->counts_bytes, pl.count_blocks * item_bytes)) return rc;
+  // one upload: the slab table, then the tiles
+  const size_t slab_bytes = pl.coded ? pl.slabs.size() * sizeof(ppsk::CodeGroup) : 0;
+  std::vector<char> lists(slab_bytes + pl.tiles.size() * sizeof(ppsk::ItemTile));
+  if (pl.coded) {
+    const size_t width_bytes = ((size_t)p.n_k * 2 * p.s64 + 64) * sizeof(uint32_t);
+    for (const auto& ch : pl.chunks) {
+      char* at = (char*)c->codes;
+      for (int x = ch.slab0; x < ch.slab1; ++x) {
+        ppsk::CodeGroup& g = pl.slabs[x];
+        g.cols = (uint32_t*)at;
+        at += code_bytes(p.n_k, p.s64, g.ncb);
+        g.rows = g.cols;
+        if (pl.apart[x]) {
+          g.rows = (uint32_t*)at;
+          at += code_bytes(p.n_k, p.s64, g.nrb);
+        }
+        g.widths = (uint32_t*)at;
+        at += width_bytes;
+      }
+    }
+    std::memcpy(lists.data(), pl.slabs.data(), slab_bytes);
+  }
+  std::memcpy(lists.data() + slab_bytes, pl.tiles.data(), pl.tiles.size() * sizeof(ppsk::ItemTile));
+  if (int rc = grow(&c->pitems, &c->pitems_bytes, lists.size())) return rc;
+  HIP_TRY(hipMemcpyAsync(c->pitems, lists.data(), lists.size(), hipMemcpyHostToDevice, c->stream));
+  const ppsk::CodeGroup* d_slabs = (const ppsk::CodeGroup*)c->pitems;
+  const ppsk::ItemTile* d_tiles = (const ppsk::ItemTile*)((char*)c->pitems + slab_bytes);
   p.counts = (uint16_t*)c->counts;
   p.out_row_offset = 0;
   ppsk::ItemArgs a;
   std::memset(&a, 0, sizeof(a));
-  a.runs = pl.runs;
-  a.run_words = pl.run_words;
-  // a read of the host's cancellation flag costs an item more than a
-  // microsecond: passes of a few rounds (milliseconds) are left to finish, the
-  // call reports the cancellation either way
-  a.watch = pl.items >= 4096 ? 1 : 0;
+  // The items of a pass of more than about 10 ms read the host's cancellation
+  // flag and mirror their progress to the host.  Both cross one link for all
+  // CUs (about 0.1 us each: 4,400 short items took 863 us instead of 433), so a
+  // shorter pass is left to finish; its call reports the cancellation and the
+  // final count either way.
+  a.watch = pl.work_us >= 10000.0 ? 1 : 0;
+  if (!a.watch) p.ctl.progress_host = nullptr;
   for (size_t ci = 0; ci < pl.chunks.size(); ++ci) {
-    const size_t x = pl.chunks[ci].first, y = pl.chunks[ci].second;
+    const ItemPlan::Chunk& ch = pl.chunks[ci];
     hipEvent_t e0 = pool_event(c, 2 * ci), e1 = pool_event(c, 2 * ci + 1);
     if (!e0 || !e1) return fail(PPSK_ERR_HIP, "event creation failed");
-    a.tiles = (const ppsk::ItemTile*)c->pitems + x;
-    a.n_tiles = (int32_t)(y - x);
-    a.n_items = (int32_t)((y - x) * p.n_k * pl.runs);
+    a.tiles = d_tiles + ch.tile0;
+    a.n_tiles = (int32_t)(ch.tile1 - ch.tile0);
+    // about 8 workgroups per CU before a workgroup takes more rows
+    a.out_rows = a.n_tiles * 64 <= 2048 ? 1 : 4;
+    a.n_tall = ch.n_tall;
+    a.whole = ch.whole;
+    a.runs = ch.runs;
+    a.run_units = ch.run_units;
+    a.n_items = (int32_t)ch.items;
     HIP_TRY(hipEventRecord(e0, c->stream));
-    HIP_TRY(ppsk::launch_items(p, a, c->stream));
+    if (pl.coded) {
+      HIP_TRY(ppsk::launch_coded(p, a, d_slabs, ch.slab0, ch.slab1 - ch.slab0, c->stream));
+    } else {
+      HIP_TRY(ppsk::launch_items(p, a, c->stream));
+    }
     HIP_TRY(hipEventRecord(e1, c->stream));
     tm->launches += 1;
     tm->items += a.n_items;
@@ -702,12 +864,10 @@ int run_dense_items(DeviceCtx* c, ppsk::DistParams p, bool upper, int64_t row_be
   // Copies are queued after every launch: a copy into pageable memory may
   // block this thread until it completes, which must not hold back launches.
   for (size_t ci = 0; host_out && ci < pl.chunks.size(); ++ci) {
-    int64_t r0 = row_end, r1 = row_begin;
-    for (size_t x = pl.chunks[ci].first; x < pl.chunks[ci].second; ++x) {
-      r0 = std::min<int64_t>(r0, pl.tiles[x].row0);
-      r1 = std::max<int64_t>(r1, pl.tiles[x].row0 + pl.tiles[x].rows);
+    if (int rc = copy_rows(c, pl.chunks[ci].copy0, pl.chunks[ci].copy1, p, self, elem, host_out,
+                           c->events[2 * ci + 1])) {
+      return rc;
     }
-    if (int rc = copy_rows(c, r0, r1, p, self, elem, host_out, c->events[2 * ci + 1])) return rc;
   }
   HIP_TRY(hipStreamSynchronize(c->stream));
   HIP_TRY(hipStreamSynchronize(c->copy_stream));
@@ -729,6 +889,8 @@ Route dense_route(int variant, bool upper, int64_t rows, int64_t n_cols) {
   const char* e = std::getenv("PPSK_PERSISTENT");
   const bool can = variant == 2 || variant == 4 || variant == 5;
   if (e) return can && std::atoi(e) != 0 ? Route::persistent : Route::tiles;
+  const bool shape = std::getenv("PPSK_TILE_VARIANT") != nullptr;
+  if (!shape && use_coded(rows, n_cols, upper)) return Route::items;
   if (can) {
     const int tr = ppsk::variant_tile_rows(variant), tc = ppsk::variant_tile_cols(variant);
     const int64_t rt = (rows + tr - 1) / tr, ct = (n_cols + tc - 1) / tc;
@@ -737,16 +899,19 @@ Route dense_route(int variant, bool upper, int64_t rows, int64_t n_cols) {
     if (ppsk::batch_grid(variant == 5 ? ppsk::BATCH_MIXED : variant, &grid) != hipSuccess) grid = 0;
     if (grid > 0 && tiles >= 2 * (int64_t)grid) return Route::persistent;
   }
-  return std::getenv("PPSK_TILE_VARIANT") ? Route::tiles : Route::items;
+  return shape ? Route::tiles : Route::items;
 }
 
-uint64_t dense_items(const ppsk_set* rows, int64_t n_cols, bool upper, int64_t row_begin,
+// Work items a dense pass reports as progress.
+uint64_t dense_items(const ppsk_set* rows, const ppsk_set* cols, bool upper, int64_t row_begin,
                      int64_t row_end, bool host_out) {
   const int v = default_variant();
-  if (dense_route(v, upper, row_end - row_begin, n_cols) == Route::items) {
-    return plan_items(n_cols, rows->n_k, rows->s64, upper, row_begin, row_end, host_out).items;
+  if (dense_route(v, upper, row_end - row_begin, cols->n) == Route::items) {
+    return plan_items(cols->n, rows->n_k, rows->s64, upper, upper, row_begin, row_end, host_out,
+                      use_coded(row_end - row_begin, cols->n, upper), CODE_BUDGET)
+        .items;
   }
-  return pass_items(row_end - row_begin, n_cols, rows->n_k, v, upper);
+  return pass_items(row_end - row_begin, cols->n, rows->n_k, v, upper);
 }
 
 // Dense pass over rows [row_begin, row_end).
@@ -1138,7 +1303,7 @@ int ppsk_dense(ppsk_set* ref, ppsk_set* query, int32_t random_mode, int32_t n_cl
   if (int rc = get_ctx(ref->device, &c)) return rc;
   std::lock_guard<std::mutex> lk(c->mu);
   if (int rc = cancel_status(ref->device)) return rc;
-  CallScope scope(c, dense_items(rows, cols->n, self, 0, rows->n, !out_on_device));
+  CallScope scope(c, dense_items(rows, cols, self, 0, rows->n, !out_on_device));
 
   const int64_t n_rows_out = self ? ref->n * (ref->n - 1) / 2 : query->n * ref->n;
   const size_t elem = out_kind == PPSK_OUT_CORE_ACC ? 2 * sizeof(float)
@@ -1199,7 +1364,7 @@ int ppsk_knn(ppsk_set* ref, int32_t random_mode, int32_t n_clusters, const float
   }
   uint64_t items = 0;
   for (int64_t r0 = 0; r0 < n; r0 += band) {
-    items += dense_items(ref, n, symmetric, r0, std::min(n, r0 + band), false);
+    items += dense_items(ref, ref, symmetric, r0, std::min(n, r0 + band), false);
   }
   CallScope scope(c, items);
   if (symmetric) {
@@ -1298,7 +1463,7 @@ int ppsk_threshold(ppsk_set* ref, int32_t random_mode, int32_t n_clusters, const
   std::lock_guard<std::mutex> lk(c->mu);
   if (int rc = cancel_status(ref->device)) return rc;
   const int64_t n = ref->n;
-  CallScope scope(c, dense_items(ref, n, true, 0, n, false));
+  CallScope scope(c, dense_items(ref, ref, true, 0, n, false));
   const size_t tri_bytes = std::max<size_t>((size_t)n * (n - 1) / 2 * sizeof(float2), 8);
   if (int rc = grow(&c->out, &c->out_bytes, tri_bytes)) return rc;
   Timing tm;
@@ -1345,7 +1510,7 @@ int ppsk_self_pass(ppsk_set* ref, int32_t random_mode, int32_t n_clusters, const
   std::lock_guard<std::mutex> lk(c->mu);
   if (int rc = cancel_status(ref->device)) return rc;
   const int64_t n = ref->n;
-  CallScope scope(c, dense_items(ref, n, true, 0, n, dense_out != nullptr));
+  CallScope scope(c, dense_items(ref, ref, true, 0, n, dense_out != nullptr));
   const size_t tri_bytes = std::max<size_t>((size_t)n * (n - 1) / 2 * sizeof(float2), 8);
   if (int rc = grow(&c->out, &c->out_bytes, tri_bytes)) return rc;
   Timing tm;

@@ -111,20 +111,48 @@ struct ItemTile {
   int32_t row0;  // first row, a multiple of `rows`
   int32_t ct;    // columns [ct * 256, +256)
   int32_t rows;  // 64, 32 or 16
+  int32_t group;  // row group of a coded pass
 };
 constexpr int ITEM_COUNTS = 64 * 256;  // counts of one item (u16), whatever its height
-constexpr int ITEM_OUT_ROWS = 4;       // tile rows per output workgroup
 
+// The (tile, k-mer length) pairs of a launch, k-mer length first, those of the
+// 64-row tiles before those of the shorter ones: the first `whole` are one
+// item each, every other is cut into `runs` items.  An item's counts go to
+// block L (whole) or whole + (L - whole) * runs + run, L its pair's number.
 struct ItemArgs {
-  const ItemTile* tiles;  // [n_tiles]
+  const ItemTile* tiles;  // [n_tiles], 64-row tiles first
   int32_t n_tiles;
-  int32_t runs;       // word runs per (tile, k-mer length)
-  int32_t run_words;  // words per run (the last may hold fewer)
-  int32_t n_items;    // n_tiles * n_k * runs
+  int32_t n_tall;  // 64-row tiles
+  int32_t whole;
+  int32_t runs;
+  int32_t run_units;  // words (coded pass: halves) per run; the last may hold fewer
+  int32_t n_items;    // whole + (n_tiles * n_k - whole) * runs
   int32_t watch;      // read the cancellation flag in every item
+  int32_t out_rows;   // tile rows per output workgroup (divides 16)
+};
+
+// Coded passes (code_kernel, dist_coded): the rows of a group and the columns
+// they meet, as ranks among the values the group's rows hold at each bin.
+constexpr int CODE_ROWS = 768;    // most rows of a group: ranks 0 .. 768
+constexpr int CODE_PLANES = 10;   // planes of the largest rank
+constexpr int CODE_STAGE = 36;    // planes of one LDS stage (1 KiB each)
+constexpr int CODE_BLOCK = 256;   // samples per block of coded planes
+
+struct CodeGroup {
+  uint32_t* cols;    // [n_k][ncb][2 s64][CODE_PLANES][256]; block 0 holds sample 256 cb0
+  uint32_t* rows;    // the same with nrb, rb0; == cols when the rows are among the columns
+  uint32_t* widths;  // [n_k][2 s64] planes used, and 16 more entries that may be read
+  int32_t row0, n_rows;
+  int32_t cb0, ncb;
+  int32_t rb0, nrb;
 };
 
 // Launchers (dist_kernels.hip).  All work goes on `stream`.
+// Coding of groups [first_group, + n_groups) of the device table `groups`,
+// matching and output of their tiles (tile.group indexes the whole table);
+// p.counts as for launch_items, a.run_units in halves.
+hipError_t launch_coded(const DistParams& p, const ItemArgs& a, const CodeGroup* groups,
+                        int first_group, int n_groups, hipStream_t stream);
 // Matching and output of a split pass; p.counts holds n_items blocks of
 // ITEM_COUNTS counts.
 hipError_t launch_items(const DistParams& p, const ItemArgs& a, hipStream_t stream);
