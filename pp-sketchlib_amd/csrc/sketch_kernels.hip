@@ -22,9 +22,8 @@
 // in LDS per workgroup.  A workgroup takes a run of units of one sample for
 // one k-mer length and keeps that sample's bin minima in LDS (ds_min_u64),
 // merged into the global minima with atomicMin at the end.  A second kernel
-// densifies (in the reference's sequential order) and bit-slices each
-// (sample, k) with one wave: layer word w, layer i is the wave ballot of bit
-// i of bins 64 w .. 64 w + 63.
+// densifies (as the reference's sequential order does) and bit-slices each
+// (sample, k).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -568,47 +567,65 @@ hipError_t run_reads_job(const ReadsJob& j, void* ws, size_t ws_bytes, hipStream
   return hipGetLastError();
 }
 
-// Reference densifybin (sketch/sketch.cpp:93-115) and fillusigs (80-91) for
-// one (sample, k) per 64-lane workgroup.
-__global__ __launch_bounds__(64) void sketch_finish_kernel(SketchArgs a) {
-  const int64_t sk = blockIdx.x;  // sample * n_k + kk
+// Reference densifybin (sketch/sketch.cpp:93-115) and fillusigs (80-91).  The
+// reference fills the empty bins in ascending order, each from the first bin of
+// its probe sequence that is not empty by then: one that was never empty, or an
+// empty one before it.  Which bin that is depends on the original bins alone, so
+// every lane finds the source of its own bin by following such steps until it
+// meets a bin that was never empty (the steps go down, so they end).  One lane
+// filling the bins in turn took 1.5 ms on a read set at 3 occurrences, whose
+// probes are a chain of misses to memory.
+//
+// A workgroup bit-slices every FINISH_WAVES * parts-th word of one (sample, k):
+// layer i of word w is the wave ballot of bit i of bins 64 w .. 64 w + 63.  The
+// occupancy of all bins (one bit each, in LDS) is read by every part, so that
+// few samples still fill the CUs.
+constexpr int FINISH_WAVES = 8;
+constexpr int FINISH_WORDS = 1023;  // largest sketch, in words
+
+__device__ __forceinline__ uint32_t densify_source(const uint64_t* filled, uint32_t i,
+                                                   uint32_t nbins) {
+  auto full = [&](uint32_t b) { return ((filled[b >> 6] >> (b & 63)) & 1ULL) != 0; };
+  uint32_t at = i;
+  do {
+    uint32_t j;
+    uint64_t attempts = 0;
+    do {
+      const uint64_t x = 1009ULL * at + (1000ULL * 1000ULL + 3ULL) * attempts;
+      j = (uint32_t)((48271ULL * x + 11ULL) % ((1ULL << 31) - 1ULL)) % nbins;
+      attempts++;
+    } while (!full(j) && j >= at);
+    at = j;
+  } while (!full(at));
+  return at;
+}
+
+__global__ __launch_bounds__(FINISH_WAVES * 64) void sketch_finish_kernel(SketchArgs a, int parts) {
+  __shared__ uint64_t filled[FINISH_WORDS];
+  const int64_t sk = blockIdx.x / parts;  // sample * n_k + kk
+  const int part = (int)(blockIdx.x % parts);
   const int64_t nbins = (int64_t)a.s64 * 64;
-  uint64_t* sg = a.signs + sk * nbins;
-  const int lane = threadIdx.x;
-  uint64_t mn = ~0ULL, mx = 0;
-  for (int64_t b = lane; b < nbins; b += 64) {
-    const uint64_t v = sg[b];
-    mn = v < mn ? v : mn;
-    mx = v > mx ? v : mx;
+  const uint64_t* sg = a.signs + sk * nbins;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  bool empty = false, full = false;
+  for (int w = wave; w < a.s64; w += FINISH_WAVES) {
+    const uint64_t m = __ballot(sg[(int64_t)w * 64 + lane] != ~0ULL);
+    if (lane == 0) filled[w] = m;
+    empty |= m != ~0ULL;
+    full |= m != 0;
   }
-  for (int off = 32; off > 0; off >>= 1) {
-    const uint64_t omn = __shfl_xor(mn, off), omx = __shfl_xor(mx, off);
-    mn = omn < mn ? omn : mn;
-    mx = omx > mx ? omx : mx;
+  empty = __syncthreads_or(empty) != 0;  // (also: every word of `filled` is written)
+  full = __syncthreads_or(full) != 0;
+  const int dens = !empty ? 0 : (full ? 1 : -1);
+  if (part == 0 && threadIdx.x == 0) {
+    a.inv_minhash[sk] = (double)sg[0] / (double)SIGN_MOD;
+    a.densified[sk] = dens;
   }
-  if (lane == 0) a.inv_minhash[sk] = (double)sg[0] / (double)SIGN_MOD;
-  int dens = 0;
-  if (mx == ~0ULL) {
-    dens = mn == ~0ULL ? -1 : 1;
-    if (dens == 1 && lane == 0) {
-      // sequential, in place: a probe may land on a bin filled earlier
-      for (int64_t i = 0; i < nbins; ++i) {
-        int64_t j = i;
-        uint64_t attempts = 0;
-        while (sg[j] == ~0ULL) {
-          const uint64_t x = 1009ULL * (uint64_t)i + (1000ULL * 1000ULL + 3ULL) * attempts;
-          j = (int64_t)(((48271ULL * x + 11ULL) % ((1ULL << 31) - 1ULL)) % (uint64_t)nbins);
-          attempts++;
-        }
-        sg[i] = sg[j];
-      }
-    }
-    __syncthreads();
-  }
-  if (lane == 0) a.densified[sk] = dens;
   uint64_t* out = a.raw + sk * (int64_t)a.s64 * BBITS_SK;
-  for (int w = 0; w < a.s64; ++w) {
-    const uint64_t v = sg[(int64_t)w * 64 + lane];
+  for (int w = part * FINISH_WAVES + wave; w < a.s64; w += parts * FINISH_WAVES) {
+    const uint32_t bin = (uint32_t)w * 64 + lane;
+    uint64_t v = sg[bin];
+    if (dens == 1 && v == ~0ULL) v = sg[densify_source(filled, bin, (uint32_t)nbins)];
     uint64_t word_i = 0;
 #pragma unroll
     for (int i = 0; i < BBITS_SK; ++i) {
@@ -665,8 +682,7 @@ hipError_t launch_sketch(const SketchArgs& a, int64_t n_groups, bool lds_bins, i
     }
     if (e != hipSuccess) return e;
   }
-  sketch_finish_kernel<<<(unsigned)(a.n_samples * a.n_k), 64, 0, stream>>>(a);
-  return hipGetLastError();
+  return launch_sketch_finish(a, stream);
 }
 
 hipError_t launch_sketch_reset(const SketchArgs& a, hipStream_t stream) {
@@ -677,7 +693,11 @@ hipError_t launch_sketch_reset(const SketchArgs& a, hipStream_t stream) {
 }
 
 hipError_t launch_sketch_finish(const SketchArgs& a, hipStream_t stream) {
-  sketch_finish_kernel<<<(unsigned)(a.n_samples * a.n_k), 64, 0, stream>>>(a);
+  // about 1,024 workgroups (4 per CU), at least one word per wave each
+  const int64_t n = a.n_samples * a.n_k;
+  const int64_t most = (a.s64 + FINISH_WAVES - 1) / FINISH_WAVES;
+  const int parts = (int)std::max<int64_t>(1, std::min<int64_t>(most, 1024 / std::max<int64_t>(n, 1)));
+  sketch_finish_kernel<<<(unsigned)(n * parts), FINISH_WAVES * 64, 0, stream>>>(a, parts);
   return hipGetLastError();
 }
 
