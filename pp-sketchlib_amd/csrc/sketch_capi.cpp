@@ -14,8 +14,8 @@ using namespace ppsk::capi;
 
 namespace {
 
-constexpr int64_t UNIT = 1024;          // k-mer start positions per lane
-constexpr int64_t GROUP_UNITS = 1024;   // units per workgroup task
+constexpr int64_t UNIT = 1024;          // most k-mer start positions per lane
+constexpr int64_t GROUP_UNITS = 1024;   // most units per workgroup task
 
 struct DevBuf {
   void* p = nullptr;
@@ -24,22 +24,58 @@ struct DevBuf {
   }
 };
 
-// Units of one sample's contigs for one k: runs of up to UNIT window starts,
+// Units of one sample's contigs for one k: runs of up to `unit` window starts,
 // pad = 1 on the first unit of a contig; wbase = index of the unit's first
 // window among the sample's windows (sequence order).  Returns the window
 // count.
-int64_t sample_units(const int64_t* contig_off, int64_t c0, int64_t c1, int64_t k,
+int64_t sample_units(const int64_t* contig_off, int64_t c0, int64_t c1, int64_t k, int64_t unit,
                      std::vector<ppsk::SketchUnit>& units, std::vector<int64_t>* wbase) {
   int64_t nw = 0;
   for (int64_t ci = c0; ci < c1; ++ci) {
     const int64_t windows = contig_off[ci + 1] - contig_off[ci] - k + 1;
-    for (int64_t w = 0; w < windows; w += UNIT) {
-      units.push_back({contig_off[ci] + w, (int32_t)std::min(UNIT, windows - w), w == 0 ? 1 : 0});
+    for (int64_t w = 0; w < windows; w += unit) {
+      units.push_back({contig_off[ci] + w, (int32_t)std::min(unit, windows - w), w == 0 ? 1 : 0});
       if (wbase) wbase->push_back(nw + w);
     }
     if (windows > 0) nw += windows;
   }
   return nw;
+}
+
+// Window starts per lane of a hashing launch over `slots` workgroups resident
+// at once.  Units of UNIT windows give the least rolling-in (k - 1 steps per
+// unit), but a launch that fits the slots in one round must spread over all of
+// them: the smallest unit of at least 64 windows whose groups (one unit per
+// lane) need no second round.  6 genomes of 2 Mb at 8 k-mer lengths: 96 groups
+// of 1,024-window units on 512 slots took 494 us, 480 groups of 416 take 248.
+int64_t unit_windows(const int64_t* contig_off, const int64_t* sample_contig, int64_t n_samples,
+                     const std::vector<int64_t>& spans, int64_t slots) {
+  auto groups = [&](int64_t unit) {
+    int64_t g = 0;
+    for (int64_t s = 0; s < n_samples; ++s) {
+      for (int64_t span : spans) {
+        int64_t u = 0;
+        for (int64_t c = sample_contig[s]; c < sample_contig[s + 1]; ++c) {
+          const int64_t w = contig_off[c + 1] - contig_off[c] - span + 1;
+          if (w > 0) u += (w + unit - 1) / unit;
+        }
+        g += (u + ppsk::SKETCH_TB - 1) / ppsk::SKETCH_TB;
+      }
+    }
+    return g;
+  };
+  if (groups(UNIT) > slots) return UNIT;
+  int64_t lo = 64, hi = UNIT;  // groups(hi) <= slots
+  while (lo < hi) {
+    const int64_t mid = (lo + hi) / 2 / 16 * 16;
+    if (mid < lo) break;
+    if (groups(mid) <= slots) {
+      hi = mid;
+    } else {
+      lo = mid + 16;
+    }
+  }
+  return hi;
 }
 
 int sketch_impl(int device_id, int64_t n_samples, const char* seq, int64_t seq_bytes,
@@ -99,24 +135,6 @@ int sketch_impl(int device_id, int64_t n_samples, const char* seq, int64_t seq_b
   if (int rc = get_ctx(device_id, &c)) return rc;
   std::lock_guard<std::mutex> lk(c->mu);
 
-  // unfiltered: units (per k, every contig cut into runs of UNIT windows) and
-  // groups (runs of units of one sample and one k) for one hashing launch
-  std::vector<ppsk::SketchUnit> units;
-  std::vector<ppsk::SketchGroup> groups;
-  if (!filtered) {
-    for (int kk = 0; kk < n_k; ++kk) {
-      for (int64_t s = 0; s < n_samples; ++s) {
-        const int64_t u0 = (int64_t)units.size();
-        sample_units(contig_off, sample_contig[s], sample_contig[s + 1], span(klist[kk]), units,
-                     nullptr);
-        const int64_t u1 = (int64_t)units.size();
-        for (int64_t g = u0; g < u1; g += GROUP_UNITS) {
-          groups.push_back({g, std::min(u1, g + GROUP_UNITS), (int32_t)s, kk});
-        }
-      }
-    }
-  }
-
   const int64_t nbins = (int64_t)sketchsize64 * 64;
   const uint64_t sign_mod = (1ULL << 61) - 1ULL;
   ppsk::SketchArgs a;
@@ -129,6 +147,36 @@ int sketch_impl(int device_id, int64_t n_samples, const char* seq, int64_t seq_b
   a.binsize = (sign_mod + (uint64_t)nbins - 1ULL) / (uint64_t)nbins;
   a.bin_recip = ~0ULL / a.binsize;
   if (a.bin_recip >> 32) return fail(PPSK_ERR_ARG, "bin reciprocal out of range");
+
+  // unfiltered: units (per k, every contig cut into runs of windows) and groups
+  // (runs of units of one sample and one k) for one hashing launch; bin minima
+  // in LDS when one sample's bins fit a workgroup's LDS (the step table takes
+  // another 400 bytes)
+  std::vector<ppsk::SketchUnit> units;
+  std::vector<ppsk::SketchGroup> groups;
+  bool lds_bins = false;
+  if (!filtered) {
+    hipDeviceProp_t prop;
+    HIP_TRY(hipGetDeviceProperties(&prop, device_id));
+    lds_bins = (size_t)nbins * sizeof(uint64_t) + 512 <= prop.sharedMemPerBlock;
+    int slots = 0;
+    HIP_TRY(ppsk::sketch_hash_slots(a, lds_bins, &slots));
+    std::vector<int64_t> spans;
+    for (int kk = 0; kk < n_k; ++kk) spans.push_back(span(klist[kk]));
+    const int64_t unit = unit_windows(contig_off, sample_contig, n_samples, spans, slots);
+    const int64_t per_group = unit < UNIT ? ppsk::SKETCH_TB : GROUP_UNITS;
+    for (int kk = 0; kk < n_k; ++kk) {
+      for (int64_t s = 0; s < n_samples; ++s) {
+        const int64_t u0 = (int64_t)units.size();
+        sample_units(contig_off, sample_contig[s], sample_contig[s + 1], spans[kk], unit, units,
+                     nullptr);
+        const int64_t u1 = (int64_t)units.size();
+        for (int64_t g = u0; g < u1; g += per_group) {
+          groups.push_back({g, std::min(u1, g + per_group), (int32_t)s, kk});
+        }
+      }
+    }
+  }
 
   DevBuf d_seq, d_units, d_groups, d_k, d_signs, d_raw, d_mh, d_dens, d_next;
   const size_t raw_words = (size_t)n_samples * n_k * sketchsize64 * ppsk::BBITS_SK;
@@ -172,11 +220,6 @@ int sketch_impl(int device_id, int64_t n_samples, const char* seq, int64_t seq_b
   HIP_TRY(ppsk::launch_sketch_decode(codes, seq_bytes, c->stream));
   int64_t items = (int64_t)units.size();
   if (!filtered) {
-    // bin minima in LDS when one sample's bins fit a workgroup's LDS (the
-    // step table takes another 400 bytes)
-    hipDeviceProp_t prop;
-    HIP_TRY(hipGetDeviceProperties(&prop, device_id));
-    const bool lds_bins = (size_t)nbins * sizeof(uint64_t) + 512 <= prop.sharedMemPerBlock;
     HIP_TRY(ppsk::launch_sketch(a, (int64_t)groups.size(), lds_bins, (int*)d_next.p, c->stream));
   } else {
     // one (sample, k) at a time through the counting pipeline
@@ -185,7 +228,7 @@ int sketch_impl(int device_id, int64_t n_samples, const char* seq, int64_t seq_b
     for (int64_t s = 0; s < n_samples; ++s) {
       std::vector<ppsk::SketchUnit> u;
       const int64_t w = sample_units(contig_off, sample_contig[s], sample_contig[s + 1],
-                                     span(klist[0]), u, nullptr);
+                                     span(klist[0]), UNIT, u, nullptr);
       max_w = std::max(max_w, w);
       max_u = std::max<int64_t>(max_u, (int64_t)u.size());
     }
@@ -205,7 +248,7 @@ int sketch_impl(int device_id, int64_t n_samples, const char* seq, int64_t seq_b
         jw.clear();
         // the smallest k has the most windows: every later job fits max_w / max_u
         const int64_t nw = sample_units(contig_off, sample_contig[s], sample_contig[s + 1],
-                                        span(klist[kk]), ju, &jw);
+                                        span(klist[kk]), UNIT, ju, &jw);
         if (nw == 0) continue;
         HIP_TRY(hipMemcpyAsync(d_ju.p, ju.data(), ju.size() * sizeof(ppsk::SketchUnit),
                                hipMemcpyHostToDevice, c->stream));

@@ -62,6 +62,9 @@ hipError_t launch_sketch_decode(uint8_t* codes, int64_t n, hipStream_t stream);
 hipError_t launch_sketch(const SketchArgs& a, int64_t n_groups, bool lds_bins, int* next_group,
                          hipStream_t stream);
 
+// Workgroups of the hashing launch that fit the device at once.
+hipError_t sketch_hash_slots(const SketchArgs& a, bool lds_bins, int* slots);
+
 // Bin-minima reset and the densify / bit-slice pass of launch_sketch, for
 // callers that fill the minima themselves (run_reads_job).
 hipError_t launch_sketch_reset(const SketchArgs& a, hipStream_t stream);

@@ -644,8 +644,7 @@ hipError_t launch_sketch_decode(uint8_t* codes, int64_t n, hipStream_t stream) {
 }
 
 template <bool LDS_BINS, int STRIDE>
-hipError_t launch_hash(const SketchArgs& a, int64_t n_groups, size_t lds, int* next_group,
-                       hipStream_t stream) {
+hipError_t hash_slots(size_t lds, int* slots) {
   int dev = 0, cus = 0, per_cu = 0;
   hipError_t e = hipGetDevice(&dev);
   if (e == hipSuccess) e = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
@@ -653,12 +652,26 @@ hipError_t launch_hash(const SketchArgs& a, int64_t n_groups, size_t lds, int* n
     e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, sketch_hash_kernel<LDS_BINS, STRIDE>,
                                                      SKETCH_TB, lds);
   }
+  *slots = std::max(per_cu, 1) * std::max(cus, 1);
+  return e;
+}
+
+template <bool LDS_BINS, int STRIDE>
+hipError_t launch_hash(const SketchArgs& a, int64_t n_groups, size_t lds, int* next_group,
+                       hipStream_t stream) {
+  int slots = 0;
+  const hipError_t e = hash_slots<LDS_BINS, STRIDE>(lds, &slots);
   if (e != hipSuccess) return e;
-  const int64_t grid = std::max<int64_t>(
-      1, std::min<int64_t>(n_groups, (int64_t)std::max(per_cu, 1) * std::max(cus, 1)));
+  const int64_t grid = std::max<int64_t>(1, std::min<int64_t>(n_groups, slots));
   sketch_hash_kernel<LDS_BINS, STRIDE><<<(unsigned)grid, SKETCH_TB, lds, stream>>>(a, n_groups,
                                                                                  next_group);
   return hipGetLastError();
+}
+
+hipError_t sketch_hash_slots(const SketchArgs& a, bool lds_bins, int* slots) {
+  const size_t lds = lds_bins ? (size_t)a.s64 * 64 * sizeof(uint64_t) : 0;
+  if (lds_bins) return a.codon ? hash_slots<true, 3>(lds, slots) : hash_slots<true, 1>(lds, slots);
+  return a.codon ? hash_slots<false, 3>(lds, slots) : hash_slots<false, 1>(lds, slots);
 }
 
 hipError_t launch_sketch(const SketchArgs& a, int64_t n_groups, bool lds_bins, int* next_group,
