@@ -286,8 +286,7 @@ int ppsk_batch_run(ppsk_batch *batch, int32_t variant, uint64_t *n_fail,
 /* Autotuner result: chosen plan and per-plan time (index = plan, 0..6;
  * 0 where not timed); row_tiles (may be NULL, 3 x n_jobs entries): for each
  * job, the row tiles of 64, 32 and 16 rows of its plan-6 split (after
- * tuning: the split of least estimated time; plan 6 is not timed when that
- * is one shape for every job). */
+ * tuning: the split of least estimated time). */
 int ppsk_batch_tuning(const ppsk_batch *batch, int32_t *variant,
                       double *ms_per_variant, int32_t *row_tiles);
 

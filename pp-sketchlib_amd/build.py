@@ -68,6 +68,7 @@ def _check_pipelined_spills(remarks):
         elif name and ("SGPRs Spill:" in line or "VGPRs Spill:" in line):
             pipelined = (("dist_tiles" in name or "batch_tile_k" in name) and "ELi2EE" in name
                          or "dist_tiles_diagonal" in name or "dist_itemsE" in name
+                         or "dist_batch_itemsE" in name
                          or "dist_codedE" in name)
             if pipelined and int(line.rsplit(":", 1)[1].split()[0]) != 0:
                 bad.append(name + ": " + line.split("remark:")[-1].strip())

@@ -7,7 +7,11 @@
 //   5     every job in 16 x 256 tiles, on the mixed-shape kernel;
 //   6     each job's rows split over the three tile heights (row tiles laid
 //         from its first row, e.g. 15 x 64 + 32 + 16 rows for 1,000
-//         queries), on the mixed-shape kernel.
+//         queries): as (tile, k-mer length, word run) items of a split pass
+//         while their counts fit 1 GiB (12 uneven jobs, whose last whole
+//         tiles ran alone on their CUs: 2.83 -> 1.88 ms), else on the
+//         mixed-shape persistent kernel (there the end of the pass is a small
+//         part of it).
 // The autotuner times plans 2, 4 and 5 on the batch itself, derives each
 // shape's throughput on padded work from those runs, splits every job's rows
 // for the least estimated time (padded work / throughput), times that plan
@@ -15,6 +19,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <cmath>
 #include <cstdlib>
 #include <cstring>
 #include <mutex>
@@ -46,6 +51,11 @@ struct ppsk_batch {
     int64_t n_items = 0;
     int64_t queue_begin[ppsk::BATCH_QUEUES + 1] = {};
     int grid = 0;
+    bool split = false;                 // plan 6 as items of a split pass
+    ppsk::BatchTile* tiles = nullptr;   // split: its tiles, items and counts
+    ppsk::BatchRun* runs = nullptr;
+    uint16_t* counts = nullptr;
+    uint64_t progress = 0;              // work items reported
     hipGraph_t graph = nullptr;
     hipGraphExec_t exec = nullptr;
   };
@@ -194,20 +204,28 @@ uint64_t batch_signature(const ppsk_batch* b) {
   return h;
 }
 
+void free_plan(ppsk_batch::Plan& pl) {
+  if (pl.exec) hipGraphExecDestroy(pl.exec);
+  if (pl.graph) hipGraphDestroy(pl.graph);
+  if (pl.items) hipFree(pl.items);
+  if (pl.tiles) hipFree(pl.tiles);
+  if (pl.runs) hipFree(pl.runs);
+  if (pl.counts) hipFree(pl.counts);
+  pl = ppsk_batch::Plan();
+}
+
 // Items of a plan.  Every (job, row segment) unit's tiles (grouped order) are
 // cut into BATCH_QUEUES contiguous runs, run q of every unit going to queue
 // q, so each queue (and the XCD that drains it) gets an equal share of every
 // job and walks compact blocks of it.  Units enter the queues most expensive
 // tile first, leaving the cheap tiles for the end of the launch.
-int build_plan(ppsk_batch* b, int plan) {
-  auto& pl = b->plans[plan];
-  if (pl.exec) return PPSK_OK;
-  const int kernel = plan_kernel(plan);
-  struct Unit {
-    int job;
-    Seg seg;
-    int64_t cost;  // matching work of one tile
-  };
+struct Unit {
+  int job;
+  Seg seg;
+  int64_t cost;  // matching work of one tile
+};
+
+std::vector<Unit> plan_units(const ppsk_batch* b, int plan) {
   std::vector<Unit> units;
   for (int j = 0; j < b->n_jobs; ++j) {
     for (const Seg& sg : plan_split(b, plan, j)) {
@@ -217,15 +235,133 @@ int build_plan(ppsk_batch* b, int plan) {
   }
   std::stable_sort(units.begin(), units.end(),
                    [](const Unit& x, const Unit& y) { return x.cost > y.cost; });
-  std::vector<std::vector<ppsk::BatchItem>> q(ppsk::BATCH_QUEUES);
+  return units;
+}
+
+std::vector<ppsk::Tile> unit_tiles(const ppsk_batch* b, const Unit& u) {
+  const ppsk_job& jb = b->jobs[u.job];
+  const int tr = ppsk::variant_tile_rows(u.seg.shape), tc = ppsk::variant_tile_cols(u.seg.shape);
   std::vector<size_t> gs;
+  return make_tiles(jb.query->n, jb.ref->n, tr, tc, jb.query == jb.ref, u.seg.row_begin,
+                    u.seg.row_end, tile_group(tr), &gs);
+}
+
+// Captures the reset and the plan's launches into its graph, replayed by every
+// run; the counters are reset by a kernel (no memset node).
+template <typename Launch>
+int capture_plan(ppsk_batch* b, ppsk_batch::Plan& pl, DeviceCtx* c, Launch launch) {
+  HIP_TRY(hipStreamBeginCapture(c->stream, hipStreamCaptureModeRelaxed));
+  hipError_t e = ppsk::launch_batch_reset(b->d_queue, b->d_fail, b->n_jobs, c->stream);
+  if (e == hipSuccess) e = launch();
+  hipGraph_t g = nullptr;
+  const hipError_t ec = hipStreamEndCapture(c->stream, &g);
+  if (e == hipSuccess) e = ec;
+  if (e == hipSuccess) e = hipGraphInstantiate(&pl.exec, g, nullptr, nullptr, 0);
+  pl.graph = g;
+  if (e != hipSuccess) return fail(PPSK_ERR_HIP, std::string("batch graph: ") + hipGetErrorString(e));
+  return PPSK_OK;
+}
+
+constexpr int64_t SPLIT_BLOCKS = 32768;  // counts of a split plan: 1 GiB
+
+// Plan 6 as a split pass: every unit's (k-mer length, word run, tile) items,
+// cut into 8 runs like the tiles of the other plans, one for each XCD; the
+// workgroups of a launch go to the XCDs in turn.  Words per item: about 2,400
+// items of equal time in all, at least 8 words (item_runs has the measurements
+// of both).  *made: false when the counts would not fit.
+int build_split(ppsk_batch* b, ppsk_batch::Plan& pl, DeviceCtx* c, bool* made) {
+  *made = false;
+  const std::vector<Unit> units = plan_units(b, ppsk::BATCH_MIXED);
+  // time of one word of a tile, in 64-row tiles (item_runs)
+  auto weight = [](int shape) { return shape == 2 ? 1.0 : (shape == 4 ? 0.57 : 0.37); };
+  std::vector<std::vector<ppsk::Tile>> ut;
+  double total = 0.0;
   for (const Unit& u : units) {
-    const ppsk_job& jb = b->jobs[u.job];
-    const bool self = jb.query == jb.ref;
+    ut.push_back(unit_tiles(b, u));
+    const ppsk_set* r = b->jobs[u.job].ref;
+    total += (double)ut.back().size() * r->n_k * r->s64 * weight(u.seg.shape);
+  }
+  std::vector<ppsk::BatchTile> tiles;
+  std::vector<std::vector<ppsk::BatchRun>> q(ppsk::BATCH_QUEUES);
+  int64_t blocks = 0, n_items = 0;
+  for (size_t x = 0; x < units.size(); ++x) {
+    const Unit& u = units[x];
+    const ppsk_set* r = b->jobs[u.job].ref;
+    const int tr = ppsk::variant_tile_rows(u.seg.shape);
+    int words = (int)std::max(8.0, std::ceil(total / 2400.0 / weight(u.seg.shape)));
+    const int runs = std::max(1, (r->s64 + words - 1) / words);
+    words = (r->s64 + runs - 1) / runs;
+    const int t0 = (int)tiles.size();
+    const int64_t n = (int64_t)ut[x].size();
+    for (const ppsk::Tile& t : ut[x]) {
+      if (blocks + (int64_t)r->n_k * runs > SPLIT_BLOCKS) return PPSK_OK;
+      tiles.push_back({u.job, t.bi * tr, t.ct, tr, (int32_t)blocks, runs});
+      blocks += (int64_t)r->n_k * runs;
+    }
+    const int64_t items = n * r->n_k * runs;
+    for (int qi = 0; qi < ppsk::BATCH_QUEUES; ++qi) {
+      for (int64_t i = items * qi / ppsk::BATCH_QUEUES; i < items * (qi + 1) / ppsk::BATCH_QUEUES; ++i) {
+        const int t = t0 + (int)(i % n), ky = (int)(i / n), kk = ky / runs, y = ky % runs;
+        const int w0 = y * words;
+        if (w0 >= r->s64) continue;  // (runs * words may pass the last word by a run)
+        q[qi].push_back({t, kk, w0, std::min(words, r->s64 - w0), tiles[t].block0 + ky});
+        ++n_items;
+      }
+    }
+  }
+  size_t most = 0;
+  for (const auto& x : q) most = std::max(most, x.size());
+  std::vector<ppsk::BatchRun> all(most * ppsk::BATCH_QUEUES, {-1, 0, 0, 0, 0});
+  for (int qi = 0; qi < ppsk::BATCH_QUEUES; ++qi) {
+    for (size_t i = 0; i < q[qi].size(); ++i) all[i * ppsk::BATCH_QUEUES + qi] = q[qi][i];
+  }
+  // no room for the counts: the persistent kernel, which needs none
+  if (hipMalloc(&pl.counts, (size_t)std::max<int64_t>(blocks, 1) * ppsk::ITEM_COUNTS *
+                                sizeof(uint16_t)) != hipSuccess) {
+    (void)hipGetLastError();
+    pl.counts = nullptr;
+    return PPSK_OK;
+  }
+  HIP_TRY(hipMalloc(&pl.tiles, std::max<size_t>(tiles.size(), 1) * sizeof(ppsk::BatchTile)));
+  HIP_TRY(hipMalloc(&pl.runs, std::max<size_t>(all.size(), 1) * sizeof(ppsk::BatchRun)));
+  HIP_TRY(hipMemcpy(pl.tiles, tiles.data(), tiles.size() * sizeof(ppsk::BatchTile), hipMemcpyHostToDevice));
+  HIP_TRY(hipMemcpy(pl.runs, all.data(), all.size() * sizeof(ppsk::BatchRun), hipMemcpyHostToDevice));
+  ppsk::BatchItemArgs a;
+  std::memset(&a, 0, sizeof(a));
+  a.jobs = b->d_params;
+  a.tiles = pl.tiles;
+  a.items = pl.runs;
+  a.counts = pl.counts;
+  a.n_tiles = (int32_t)tiles.size();
+  a.n_items = (int32_t)all.size();
+  a.out_rows = a.n_tiles * 64 <= 2048 ? 1 : 4;
+  a.ctl = c->ctl;
+  // flag reads and progress mirrors as in a dense split pass (run_dense_items)
+  a.watch = total * 6.4 / 512.0 >= 10000.0 ? 1 : 0;
+  if (!a.watch) a.ctl.progress_host = nullptr;
+  pl.split = true;
+  pl.n_items = n_items;
+  pl.progress = (uint64_t)n_items;
+  *made = true;
+  return capture_plan(b, pl, c, [&] { return ppsk::launch_batch_items(a, c->stream); });
+}
+
+int build_plan(ppsk_batch* b, int plan) {
+  auto& pl = b->plans[plan];
+  if (pl.exec) return PPSK_OK;
+  const int kernel = plan_kernel(plan);
+  DeviceCtx* c = nullptr;
+  if (int rc = get_ctx(b->device, &c)) return rc;
+  if (plan == ppsk::BATCH_MIXED) {
+    bool made = false;
+    if (int rc = build_split(b, pl, c, &made)) return rc;
+    if (made) return PPSK_OK;
+  }
+  const std::vector<Unit> units = plan_units(b, plan);
+  std::vector<std::vector<ppsk::BatchItem>> q(ppsk::BATCH_QUEUES);
+  for (const Unit& u : units) {
     const int shape = u.seg.shape;
-    const int tr = ppsk::variant_tile_rows(shape), tc = ppsk::variant_tile_cols(shape);
-    auto tiles = make_tiles(jb.query->n, jb.ref->n, tr, tc, self, u.seg.row_begin,
-                            u.seg.row_end, tile_group(tr), &gs);
+    const auto tiles = unit_tiles(b, u);
     const size_t n = tiles.size();
     for (int qi = 0; qi < ppsk::BATCH_QUEUES; ++qi) {
       const size_t a = n * qi / ppsk::BATCH_QUEUES, e = n * (qi + 1) / ppsk::BATCH_QUEUES;
@@ -239,8 +375,9 @@ int build_plan(ppsk_batch* b, int plan) {
     pl.queue_begin[qi + 1] = (int64_t)all.size();
   }
   pl.n_items = (int64_t)all.size();
-  DeviceCtx* c = nullptr;
-  if (int rc = get_ctx(b->device, &c)) return rc;
+  for (int j = 0; j < b->n_jobs; ++j) {
+    pl.progress += (uint64_t)plan_tiles(b, plan, j) * b->jobs[j].ref->n_k;
+  }
   HIP_TRY(ppsk::batch_grid(kernel, &pl.grid));
   if (!b->scratch) {
     // sized once for every kernel: captured graphs keep this address (the
@@ -267,18 +404,7 @@ int build_plan(ppsk_batch* b, int plan) {
   a.scratch = b->scratch;
   a.max_k = b->max_k;
   a.ctl = c->ctl;
-  // both launches captured once, replayed by every run; the counters are
-  // reset by a kernel (no memset node)
-  HIP_TRY(hipStreamBeginCapture(c->stream, hipStreamCaptureModeRelaxed));
-  hipError_t e = ppsk::launch_batch_reset(b->d_queue, b->d_fail, b->n_jobs, c->stream);
-  if (e == hipSuccess) e = ppsk::launch_batch(a, kernel, pl.grid, c->stream);
-  hipGraph_t g = nullptr;
-  const hipError_t ec = hipStreamEndCapture(c->stream, &g);
-  if (e == hipSuccess) e = ec;
-  if (e == hipSuccess) e = hipGraphInstantiate(&pl.exec, g, nullptr, nullptr, 0);
-  pl.graph = g;
-  if (e != hipSuccess) return fail(PPSK_ERR_HIP, std::string("batch graph: ") + hipGetErrorString(e));
-  return PPSK_OK;
+  return capture_plan(b, pl, c, [&] { return ppsk::launch_batch(a, kernel, pl.grid, c->stream); });
 }
 
 int run_plan(ppsk_batch* b, int plan, double* ms) {
@@ -286,11 +412,7 @@ int run_plan(ppsk_batch* b, int plan, double* ms) {
   if (int rc = get_ctx(b->device, &c)) return rc;
   if (int rc = build_plan(b, plan)) return rc;
   if (int rc = cancel_status(b->device)) return rc;
-  uint64_t items = 0;
-  for (int j = 0; j < b->n_jobs; ++j) {
-    items += (uint64_t)plan_tiles(b, plan, j) * b->jobs[j].ref->n_k;
-  }
-  CallScope scope(c, items);
+  CallScope scope(c, b->plans[plan].progress);
   hipEvent_t e0 = pool_event(c, 0), e1 = pool_event(c, 1);
   if (!e0 || !e1) return fail(PPSK_ERR_HIP, "event creation failed");
   HIP_TRY(hipEventRecord(e0, c->stream));
@@ -439,20 +561,10 @@ int ppsk_batch_run(ppsk_batch* b, int32_t variant, uint64_t* n_fail, int32_t* us
     if (b->plans[ppsk::BATCH_MIXED].exec && splits != b->job_split) {
       // a per-job plan captured with other shapes: rebuilt on its next use
       auto& pl = b->plans[ppsk::BATCH_MIXED];
-      hipGraphExecDestroy(pl.exec);
-      hipGraphDestroy(pl.graph);
-      hipFree(pl.items);
-      pl = ppsk_batch::Plan();
+      free_plan(pl);
     }
     b->job_split = splits;
-    // every job in one segment of one shape: plan 6 is that uniform plan,
-    // already timed
-    const bool uniform = std::all_of(splits.begin(), splits.end(), [&](const Split& x) {
-      return x.size() == 1 && x[0].shape == splits[0][0].shape;
-    });
-    if (!uniform) {
-      if (int rc = time_plan(ppsk::BATCH_MIXED)) return rc;
-    }
+    if (int rc = time_plan(ppsk::BATCH_MIXED)) return rc;
     std::lock_guard<std::mutex> tl(g_tune_mu);
     g_tuned.push_back({b->signature, b->variant, b->job_split});
     v = b->variant;
@@ -502,11 +614,7 @@ int ppsk_batch_tuning(const ppsk_batch* b, int32_t* variant, double* ms_per_vari
 int ppsk_batch_free(ppsk_batch* b) {
   if (!b) return PPSK_OK;
   hipSetDevice(b->device);
-  for (auto& pl : b->plans) {
-    if (pl.exec) hipGraphExecDestroy(pl.exec);
-    if (pl.graph) hipGraphDestroy(pl.graph);
-    if (pl.items) hipFree(pl.items);
-  }
+  for (auto& pl : b->plans) free_plan(pl);
   for (float* t : b->tables) if (t) hipFree(t);
   if (b->d_params) hipFree(b->d_params);
   if (b->d_fail) hipFree(b->d_fail);

@@ -1372,6 +1372,31 @@ __global__ __launch_bounds__(WAVES * 64, 4) void dist_items(DistParams p, ItemAr
   if (threadIdx.x == 0) add_progress(p.ctl, 1ull);
 }
 
+// Counts of OUT_K k-mer lengths from their runs' blocks, x[i] at the pair's
+// count in the first block: 4 runs of all lengths at a time.
+__device__ __forceinline__ void sum_runs(const uint16_t* const (&x)[OUT_K],
+                                         const int (&runs)[OUT_K], uint32_t (&c)[OUT_K]) {
+  int most = 1;
+#pragma unroll
+  for (int i = 0; i < OUT_K; ++i) {
+    most = max(most, runs[i]);
+    c[i] = 0;
+  }
+  for (int y = 0; y < most; y += 4) {
+    uint32_t v[4][OUT_K];
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+#pragma unroll
+      for (int i = 0; i < OUT_K; ++i) {
+        v[j][i] = y + j < runs[i] ? x[i][(int64_t)(y + j) * ITEM_COUNTS] : 0u;
+      }
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+#pragma unroll
+      for (int i = 0; i < OUT_K; ++i) c[i] += v[j][i];
+  }
+}
+
 // Output of a split pass: one lane per pair, a.out_rows rows of one tile per
 // workgroup (1 in a small pass, so that no lane has to do four), the 256
 // columns of a row read and written side by side.  Left to the last workgroup
@@ -1396,30 +1421,15 @@ __global__ __launch_bounds__(256) void dist_items_out(DistParams p, ItemArgs a) 
     const uint16_t* cp = q.counts + r * 256 + threadIdx.x;
     pair_output(q, gi, gj, bins, rbins, [&](int k0, uint32_t (&c)[OUT_K]) {
       const uint16_t* x[OUT_K];
-      int runs[OUT_K], most = 1;
+      int runs[OUT_K];
 #pragma unroll
       for (int i = 0; i < OUT_K; ++i) {
         const int pair = item_pair(a, q.n_k, t, min(k0 + i, q.n_k - 1));
         const bool whole = pair < a.whole;
         x[i] = cp + (whole ? pair : a.whole + (int64_t)(pair - a.whole) * a.runs) * ITEM_COUNTS;
         runs[i] = whole ? 1 : a.runs;
-        most = max(most, runs[i]);
-        c[i] = 0;
       }
-      // 4 runs of 4 lengths at a time
-      for (int y = 0; y < most; y += 4) {
-        uint32_t v[4][OUT_K];
-#pragma unroll
-        for (int j = 0; j < 4; ++j)
-#pragma unroll
-          for (int i = 0; i < OUT_K; ++i) {
-            v[j][i] = y + j < runs[i] ? x[i][(int64_t)(y + j) * ITEM_COUNTS] : 0u;
-          }
-#pragma unroll
-        for (int j = 0; j < 4; ++j)
-#pragma unroll
-          for (int i = 0; i < OUT_K; ++i) c[i] += v[j][i];
-      }
+      sum_runs(x, runs, c);
     });
   }
 }
@@ -1428,6 +1438,80 @@ static unsigned item_grid(const ItemArgs& a) {
   const int per1 = (a.whole + BATCH_QUEUES - 1) / BATCH_QUEUES;
   const int per2 = (a.n_items - a.whole + BATCH_QUEUES - 1) / BATCH_QUEUES;
   return (unsigned)((per1 + per2) * BATCH_QUEUES);
+}
+
+// The items of a batch: the same matching over the tiles of many jobs, each
+// job's parameters from the batch's table.  12 jobs of 1 to 512 queries x
+// 375 to 3,000 references as whole tiles of the persistent kernel (every
+// k-mer length of a tile on one workgroup) took 2.83 ms, its last tiles alone
+// on their CUs; as items and the output kernel (0.17 ms) 1.88 ms.
+__global__ __launch_bounds__(WAVES * 64, 4) void dist_batch_items(BatchItemArgs a) {
+  __shared__ uint4 sB0[TileCfg<8, 4>::STAGE_U4];
+  __shared__ uint4 sB1[TileCfg<8, 4>::STAGE_U4];
+  __shared__ uint4 sR[TileCfg<8, 4>::ROW_LDS_U4];
+  __shared__ int s_stop;
+  const BatchRun it = a.items[blockIdx.x];
+  const int t = __builtin_amdgcn_readfirstlane(it.tile);
+  if (t < 0) return;
+  if (a.watch) {
+    if (threadIdx.x == 0) s_stop = cancel_seen(a.ctl.cancel) ? 1 : 0;
+    __syncthreads();
+    if (__builtin_amdgcn_readfirstlane(s_stop)) return;
+  }
+  const BatchTile tile = a.tiles[t];
+  const int job = __builtin_amdgcn_readfirstlane(tile.job);
+  const int row0 = __builtin_amdgcn_readfirstlane(tile.row0);
+  const int ct = __builtin_amdgcn_readfirstlane(tile.ct);
+  const int rows = __builtin_amdgcn_readfirstlane(tile.rows);
+  const int kk = __builtin_amdgcn_readfirstlane(it.kk);
+  const int w0 = __builtin_amdgcn_readfirstlane(it.word0);
+  const int nw = __builtin_amdgcn_readfirstlane(it.words);
+  const int block = __builtin_amdgcn_readfirstlane(it.block);
+  CParams* pp = (CParams*)(a.jobs + job);
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int lane = threadIdx.x & 63;
+  uint16_t* counts = a.counts + (int64_t)block * ITEM_COUNTS;
+  if (rows == 64) {
+    match_item<4>(pp, row0, ct, kk, w0, nw, sB0, sB1, sR, counts, wave, lane);
+  } else if (rows == 32) {
+    match_item<2>(pp, row0, ct, kk, w0, nw, sB0, sB1, sR, counts, wave, lane);
+  } else {
+    match_item<1>(pp, row0, ct, kk, w0, nw, sB0, sB1, sR, counts, wave, lane);
+  }
+  if (threadIdx.x == 0) add_progress(a.ctl, 1ull);
+}
+
+__global__ __launch_bounds__(256) void dist_batch_items_out(BatchItemArgs a) {
+  const int parts = 64 / a.out_rows;
+  const BatchTile tile = a.tiles[blockIdx.x / parts];
+  const int r0 = (int)(blockIdx.x % parts) * a.out_rows;
+  if (r0 >= tile.rows) return;
+  CParams& q = *(CParams*)(a.jobs + __builtin_amdgcn_readfirstlane(tile.job));
+  const int64_t gj = (int64_t)tile.ct * 256 + threadIdx.x;
+  const double bins = 64.0 * (double)q.s64;
+  const double rbins = 1.0 / bins;
+  for (int r = r0; r < r0 + a.out_rows; ++r) {
+    const int64_t gi = tile.row0 + r;
+    if (!pair_valid(q, gi, gj)) continue;
+    const uint16_t* cp = a.counts + (int64_t)tile.block0 * ITEM_COUNTS + r * 256 + threadIdx.x;
+    pair_output(q, gi, gj, bins, rbins, [&](int k0, uint32_t (&c)[OUT_K]) {
+      const uint16_t* x[OUT_K];
+      int runs[OUT_K];
+#pragma unroll
+      for (int i = 0; i < OUT_K; ++i) {
+        x[i] = cp + (int64_t)min(k0 + i, q.n_k - 1) * tile.runs * ITEM_COUNTS;
+        runs[i] = tile.runs;
+      }
+      sum_runs(x, runs, c);
+    });
+  }
+}
+
+hipError_t launch_batch_items(const BatchItemArgs& a, hipStream_t stream) {
+  if (a.n_items <= 0) return hipSuccess;
+  dist_batch_items<<<(unsigned)a.n_items, WAVES * 64, 0, stream>>>(a);
+  dist_batch_items_out<<<(unsigned)(a.n_tiles * (64 / a.out_rows)), 256, 0, stream>>>(a);
+  return hipGetLastError();
 }
 
 hipError_t launch_items(const DistParams& p, const ItemArgs& a, hipStream_t stream) {

@@ -147,7 +147,31 @@ struct CodeGroup {
   int32_t rb0, nrb;
 };
 
+// Split batches (dist_batch_items): the same items over the tiles of many jobs.
+struct BatchTile {
+  int32_t job, row0, ct, rows;
+  int32_t block0, runs;  // counts of k-mer length k, run y: block0 + k * runs + y
+};
+
+struct BatchRun {  // one item; tile < 0: none
+  int32_t tile, kk;
+  int32_t word0, words;
+  int32_t block;
+};
+
+struct BatchItemArgs {
+  const DistParams* jobs;
+  const BatchTile* tiles;  // [n_tiles]
+  const BatchRun* items;   // [n_items], workgroup b takes item b
+  uint16_t* counts;        // blocks of ITEM_COUNTS
+  int32_t n_tiles, n_items;
+  int32_t watch;     // read the cancellation flag in every item
+  int32_t out_rows;  // tile rows per output workgroup (divides 16)
+  Control ctl;
+};
+
 // Launchers (dist_kernels.hip).  All work goes on `stream`.
+hipError_t launch_batch_items(const BatchItemArgs& a, hipStream_t stream);
 // Coding of groups [first_group, + n_groups) of the device table `groups`,
 // matching and output of their tiles (tile.group indexes the whole table);
 // p.counts as for launch_items, a.run_units in halves.
