@@ -148,6 +148,18 @@ int check_random(const ppsk_set* rows, const ppsk_set* cols, const RandomIn& rnd
 int tile_group(int tile_rows);
 int default_variant();
 
+// How the (tile, k-mer length) pairs of a split launch are cut into items
+// (ItemArgs; units are words, or halves of a coded pass), from its tiles of 64,
+// 32 and 16 rows, and the estimated time of their matching.
+struct ItemCut {
+  int n_tall, whole, runs, run_units;
+  int64_t items;
+  double work_us;
+};
+ItemCut cut_items(int64_t n64, int64_t n32, int64_t n16, int n_k, int s64, bool coded);
+// The launch's tiles and cut in its arguments.
+void set_items(ppsk::ItemArgs* a, const ppsk::ItemTile* tiles, int64_t n_tiles, const ItemCut& cut);
+
 // Timing of the tile-kernel launches of one call: per-chunk events on the
 // launch stream, summed once the call has finished.
 struct Timing {

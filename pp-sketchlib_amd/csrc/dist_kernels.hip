@@ -2106,6 +2106,41 @@ __global__ void batch_reset_kernel(uint32_t* queue_next, unsigned long long* fai
   }
 }
 
+__global__ void band_setup_kernel(ItemTile* tiles, int64_t rows, int64_t n_ct, int64_t step,
+                                  unsigned long long* fail, uint32_t* fail_rows) {
+  const int64_t x = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (x < rows) fail_rows[x] = 0u;
+  if (x == 0) {
+    fail[0] = 0ull;
+    fail[1] = ~0ull;
+  }
+  if (step == 0) return;
+  const BandTiles b = band_tiles(rows);
+  const int64_t per = b.tall + b.shorts;  // tiles of a column block
+  if (x >= per * n_ct) return;
+  const int64_t c0 = x / (per * step) * step;
+  const int64_t nc = n_ct - c0 < step ? n_ct - c0 : step;
+  const int64_t y = x - c0 * per;
+  if (y < nc * b.tall) {
+    tiles[x] = {(int32_t)(y % b.tall * 64), (int32_t)(c0 + y / b.tall), 64, 0};
+  } else {
+    const int64_t z = y - nc * b.tall;
+    const int second = (int)(z % b.shorts);
+    tiles[x] = {(int32_t)(b.tall * 64 + second * b.first), (int32_t)(c0 + z / b.shorts),
+                second ? 16 : b.first, 0};
+  }
+}
+
+hipError_t launch_band_setup(ItemTile* tiles, int64_t rows, int64_t n_ct, int64_t step,
+                             unsigned long long* fail, uint32_t* fail_rows, hipStream_t stream) {
+  const BandTiles b = band_tiles(rows);
+  int64_t n = rows > 0 ? rows : 1;
+  if (step > 0 && (b.tall + b.shorts) * n_ct > n) n = (b.tall + b.shorts) * n_ct;
+  band_setup_kernel<<<(unsigned)((n + 255) / 256), 256, 0, stream>>>(tiles, rows, n_ct, step, fail,
+                                                                     fail_rows);
+  return hipGetLastError();
+}
+
 bool variant_valid(int v) { return v >= 1 && v <= N_VARIANTS; }
 
 int variant_tile_rows(int v) {

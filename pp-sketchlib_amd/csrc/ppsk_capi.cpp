@@ -568,9 +568,7 @@ struct ItemPlan {
     size_t tile0, tile1;
     int slab0, slab1;
     int64_t copy0, copy1;  // rows whose last column is computed by this launch
-    double work_us;  // estimated time of the matching
-    int n_tall, whole, runs, run_units;  // ItemArgs (units: words, or halves of a coded pass)
-    int64_t items;
+    ItemCut cut;
   };
   bool coded = false;
   std::vector<ppsk::ItemTile> tiles;
@@ -591,29 +589,38 @@ struct ItemPlan {
 // samples (80 pairs) 664, 348, 286, 257, 265; 1,000 (328 pairs) 1103, 852, 807,
 // 846, 1080; 451 queries x 6,000 (512 pairs after two whole rounds, coded) 2582,
 // 2551, 2409, 2482, 2712.
-void item_runs(ItemPlan::Chunk* ch, const std::vector<ppsk::ItemTile>& tiles, int n_k, int s64,
-               bool coded) {
+ItemCut cut_items(int64_t n64, int64_t n32, int64_t n16, int n_k, int s64, bool coded) {
   const int units = coded ? 2 * s64 : s64;
   const double unit_us = coded ? 2.2 : 6.4;
-  int64_t n[3] = {0, 0, 0};  // tiles of 64, 32, 16 rows
-  for (size_t x = ch->tile0; x < ch->tile1; ++x) {
-    ++n[tiles[x].rows == 64 ? 0 : (tiles[x].rows == 32 ? 1 : 2)];
-  }
-  const int64_t pairs = (n[0] + n[1] + n[2]) * n_k;
-  ch->n_tall = (int)n[0];
-  ch->whole = (int)(n[0] * n_k / 512 * 512);
-  ch->runs = 1;
-  ch->run_units = units;
-  ch->items = pairs;
-  ch->work_us = ((double)n[0] + 0.57 * n[1] + 0.37 * n[2]) * n_k * unit_us * units / 512.0;
-  const int64_t rest = pairs - ch->whole;
-  if (rest == 0) return;
+  const int64_t pairs = (n64 + n32 + n16) * n_k;
+  ItemCut cut;
+  cut.n_tall = (int)n64;
+  cut.whole = (int)(n64 * n_k / 512 * 512);
+  cut.runs = 1;
+  cut.run_units = units;
+  cut.items = pairs;
+  cut.work_us = ((double)n64 + 0.57 * n32 + 0.37 * n16) * n_k * unit_us * units / 512.0;
+  const int64_t rest = pairs - cut.whole;
+  if (rest == 0) return cut;
   const int shortest = coded ? 16 : 8;
   const int64_t want = std::max<int64_t>(1, (2400 + rest / 2) / rest);
   const int runs = (int)std::min<int64_t>(want, std::max(1, units / shortest));
-  ch->run_units = (units + runs - 1) / runs;
-  ch->runs = (units + ch->run_units - 1) / ch->run_units;
-  ch->items = ch->whole + rest * ch->runs;
+  cut.run_units = (units + runs - 1) / runs;
+  cut.runs = (units + cut.run_units - 1) / cut.run_units;
+  cut.items = cut.whole + rest * cut.runs;
+  return cut;
+}
+
+void set_items(ppsk::ItemArgs* a, const ppsk::ItemTile* tiles, int64_t n_tiles, const ItemCut& cut) {
+  a->tiles = tiles;
+  a->n_tiles = (int32_t)n_tiles;
+  // about 8 workgroups per CU before a workgroup takes more rows
+  a->out_rows = n_tiles * 64 <= 2048 ? 1 : 4;
+  a->n_tall = cut.n_tall;
+  a->whole = cut.whole;
+  a->runs = cut.runs;
+  a->run_units = cut.run_units;
+  a->n_items = (int32_t)cut.items;
 }
 
 // Whether a split pass codes its rows' values (code_kernel).  Coding costs a
@@ -744,11 +751,15 @@ ItemPlan plan_items(int64_t n_cols, int n_k, int s64, bool upper, bool same_set,
     ch.copy1 = r1;
     std::stable_partition(pl.tiles.begin() + ch.tile0, pl.tiles.begin() + ch.tile1,
                           [](const ppsk::ItemTile& t) { return t.rows == 64; });
-    item_runs(&ch, pl.tiles, n_k, s64, coded);
+    int64_t n[3] = {0, 0, 0};  // tiles of 64, 32, 16 rows
+    for (size_t x = ch.tile0; x < ch.tile1; ++x) {
+      ++n[pl.tiles[x].rows == 64 ? 0 : (pl.tiles[x].rows == 32 ? 1 : 2)];
+    }
+    ch.cut = cut_items(n[0], n[1], n[2], n_k, s64, coded);
     pl.chunks.push_back(ch);
-    pl.items += (uint64_t)ch.items;
-    pl.work_us += ch.work_us;
-    pl.count_blocks = std::max(pl.count_blocks, (size_t)ch.items);
+    pl.items += (uint64_t)ch.cut.items;
+    pl.work_us += ch.cut.work_us;
+    pl.count_blocks = std::max(pl.count_blocks, (size_t)ch.cut.items);
     pl.code_bytes = std::max(pl.code_bytes, bytes);
     g = h;
   }
@@ -842,15 +853,7 @@ int run_dense_items(DeviceCtx* c, ppsk::DistParams p, bool upper, int64_t row_be
     const ItemPlan::Chunk& ch = pl.chunks[ci];
     hipEvent_t e0 = pool_event(c, 2 * ci), e1 = pool_event(c, 2 * ci + 1);
     if (!e0 || !e1) return fail(PPSK_ERR_HIP, "event creation failed");
-    a.tiles = d_tiles + ch.tile0;
-    a.n_tiles = (int32_t)(ch.tile1 - ch.tile0);
-    // about 8 workgroups per CU before a workgroup takes more rows
-    a.out_rows = a.n_tiles * 64 <= 2048 ? 1 : 4;
-    a.n_tall = ch.n_tall;
-    a.whole = ch.whole;
-    a.runs = ch.runs;
-    a.run_units = ch.run_units;
-    a.n_items = (int32_t)ch.items;
+    set_items(&a, d_tiles + ch.tile0, (int64_t)(ch.tile1 - ch.tile0), ch.cut);
     HIP_TRY(hipEventRecord(e0, c->stream));
     if (pl.coded) {
       HIP_TRY(ppsk::launch_coded(p, a, d_slabs, ch.slab0, ch.slab1 - ch.slab0, c->stream));

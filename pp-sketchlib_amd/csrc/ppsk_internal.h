@@ -147,6 +147,18 @@ struct CodeGroup {
   int32_t rb0, nrb;
 };
 
+// Rows of a band in tiles: as many 64-row ones as fit (one more for more than
+// 48 rows left), the rest in one of 32 and / or one of 16.
+struct BandTiles {
+  int64_t tall;
+  int shorts, first;  // shorter tiles (0 .. 2) and the height of the first
+};
+__host__ __device__ inline BandTiles band_tiles(int64_t rows) {
+  const int64_t tall = (rows + 15) / 64, left = rows - tall * 64;
+  if (left <= 0) return {tall, 0, 0};
+  return {tall, left > 32 ? 2 : 1, left > 16 ? 32 : 16};
+}
+
 // Split batches (dist_batch_items): the same items over the tiles of many jobs.
 struct BatchTile {
   int32_t job, row0, ct, rows;
@@ -212,6 +224,12 @@ constexpr int BATCH_MIXED = 6;
 // kernel, so that both launches can be captured in a graph.
 hipError_t batch_grid(int variant, int* grid);
 hipError_t launch_batch(const BatchArgs& a, int variant, int grid, hipStream_t stream);
+// Split pass of a query band (dist_items over rows x every column): tiles of
+// column blocks [0, n_ct), `step` of them per launch, a launch's 64-row tiles
+// before its shorter ones; clears the band's fit failures.  No tiles written
+// when step is 0.
+hipError_t launch_band_setup(ItemTile* tiles, int64_t rows, int64_t n_ct, int64_t step,
+                             unsigned long long* fail, uint32_t* fail_rows, hipStream_t stream);
 hipError_t launch_batch_reset(uint32_t* queue_next, unsigned long long* fail, int n_jobs,
                               hipStream_t stream, unsigned long long* progress = nullptr);
 // Zeroes n tile completion counters and sets fail ([2]: count, first row; may

@@ -148,6 +148,8 @@ struct ppsk_server {
   bool force_persistent = false;  // PPSK_PERSISTENT=1: every step of shape 2 / 4
   size_t per_sample = 0;
   size_t scratch_budget = 0;
+  size_t slot_share = 0;  // arena bytes / slots
+  bool split = true;      // no tile shape or kernel forced
   Arena arena;
   void* arena_mem = nullptr;
   std::mutex mu;
@@ -180,20 +182,34 @@ int step_variant(const ppsk_server* s, int64_t rows) {
 // two tiles per resident workgroup runs the persistent tile kernel (whole
 // tiles from work queues, per-workgroup count blocks), its last partial round
 // as (tile, k-mer length) items when that round would leave most workgroup
-// slots idle (tail tiles, per-tile count scratch); a smaller step is split
-// per (tile, k-mer length) over more workgroups (per-tile count scratch,
-// launched in chunks of chunk_tiles).
+// slots idle (tail tiles, per-tile count scratch).  A smaller step is a split
+// pass: items of a tile, a k-mer length and a run of words, its counts in
+// launches of step_ct column blocks (at most 256 MiB of counts).  A step of 61
+// queries x 8,000 references (8 k-mer lengths, 156 words) took 0.96 ms as
+// (64-row tile, k-mer length) workgroups and takes 0.61 ms as items, which all
+// end together; two overlapping steps of 83 and 92 queries 3.1 and 1.9 ms
+// (96 rows computed for each instead of 128).  Where a slot's share of the
+// arena has no room for that (its counts take up to 4 times as much for a few
+// rows), or a tile shape is forced, it is split per (tile, k-mer length) with
+// per-tile count scratch, launched in chunks of chunk_tiles.
 struct StepLayout {
   size_t staging, stripes, jv, clusters, band, tiles, scratch, tile_done, fail, fail_rows, params;
   size_t tail_tiles, tail_counts, tail_done, counts, knn_lists, total;
   int64_t nbq, n_tiles, chunk_tiles, tail;
   int segs;      // column segments per row of the threshold kernels
   int knn_segs;  // column segments per row of the kNN candidate lists
-  bool persistent;
+  bool persistent, items;
   int grid;
+  int64_t step_ct;
 };
 
-StepLayout layout(const ppsk_server* s, int64_t rows) {
+// Items of a split step's launch over n_ct column blocks.
+ItemCut band_cut(const ppsk_set* ref, const ppsk::BandTiles& b, int64_t n_ct) {
+  const int64_t n32 = b.shorts > 0 && b.first == 32 ? 1 : 0;
+  return cut_items(b.tall * n_ct, n32 * n_ct, (b.shorts - n32) * n_ct, ref->n_k, ref->s64, false);
+}
+
+StepLayout layout_route(const ppsk_server* s, int64_t rows, bool items) {
   const ppsk_set* r = s->ref;
   StepLayout L{};
   const int v = step_variant(s, rows);
@@ -205,6 +221,7 @@ StepLayout layout(const ppsk_server* s, int64_t rows) {
   L.grid = v == 2 ? s->grid2 : (v == 4 ? s->grid4 : 0);
   L.persistent = L.grid > 0 && (s->force_persistent || L.n_tiles >= 2 * (int64_t)L.grid);
   L.chunk_tiles = std::max<int64_t>(1, std::min<int64_t>(L.n_tiles, s->scratch_budget / per_tile));
+  L.items = items && !L.persistent;
   size_t off = 0;
   auto take = [&](size_t bytes) {
     const size_t at = off;
@@ -227,6 +244,15 @@ StepLayout layout(const ppsk_server* s, int64_t rows) {
       L.tail_counts = take((size_t)L.tail * per_tile);
       L.tail_done = take((size_t)L.tail * sizeof(uint32_t));
     }
+  } else if (L.items) {
+    const ppsk::BandTiles b = ppsk::band_tiles(rows);
+    const int64_t n_ct = (r->n + 255) / 256, per = b.tall + b.shorts;
+    const int64_t most = (int64_t)(s->scratch_budget / (ppsk::ITEM_COUNTS * sizeof(uint16_t)));
+    L.step_ct = std::max<int64_t>(1, std::min(n_ct, most / (per * r->n_k)));
+    int64_t blocks = band_cut(r, b, L.step_ct).items;
+    if (n_ct % L.step_ct) blocks = std::max(blocks, band_cut(r, b, n_ct % L.step_ct).items);
+    L.tiles = take((size_t)(per * n_ct) * sizeof(ppsk::ItemTile));
+    L.scratch = take((size_t)blocks * ppsk::ITEM_COUNTS * sizeof(uint16_t));
   } else {
     L.tiles = take((size_t)L.n_tiles * sizeof(ppsk::Tile));
     L.scratch = take((size_t)L.chunk_tiles * per_tile);
@@ -244,6 +270,14 @@ StepLayout layout(const ppsk_server* s, int64_t rows) {
   L.knn_lists = take(ppsk::knn_rect_workspace(rows, L.knn_segs, std::max(1, s->kNN)));
   L.total = off;
   return L;
+}
+
+StepLayout layout(const ppsk_server* s, int64_t rows) {
+  if (s->split) {
+    const StepLayout L = layout_route(s, rows, true);
+    if (L.persistent || L.total <= s->slot_share) return L;
+  }
+  return layout_route(s, rows, false);
 }
 
 // Page-locked host buffer that grows on demand.
@@ -327,12 +361,12 @@ int run_step(ppsk_server* s, Worker& w, std::vector<Piece>& batch, int64_t rows,
   STEP_TRY(ppsk::launch_stripe(staging, rows, 0, n_k, ref->s64, (int32_t)L.nbq, stripes, w.st));
   // per-tile completion counters of the per-(tile, k) kernel (the queue
   // counters of a persistent step are reset by launch_batch_reset)
-  if (!L.persistent) {
+  if (!L.persistent && !L.items) {
     STEP_TRY(hipMemsetAsync(tile_done, 0, (size_t)L.chunk_tiles * sizeof(uint32_t), w.st));
   }
-  STEP_TRY(hipMemsetAsync(fail, 0, sizeof(unsigned long long), w.st));
-  STEP_TRY(hipMemsetAsync(fail + 1, 0xFF, sizeof(unsigned long long), w.st));
-  STEP_TRY(hipMemsetAsync(fail_rows, 0, (size_t)rows * sizeof(uint32_t), w.st));
+  const int64_t n_ct = (ref->n + 255) / 256;
+  STEP_TRY(ppsk::launch_band_setup((ppsk::ItemTile*)(mem + L.tiles), rows, n_ct, L.items ? L.step_ct : 0,
+                                   fail, fail_rows, w.st));
 
   // distances: query rows x every reference, dense band in device memory
   ppsk::DistParams p;
@@ -370,7 +404,8 @@ int run_step(ppsk_server* s, Worker& w, std::vector<Piece>& batch, int64_t rows,
   const int tr = ppsk::variant_tile_rows(variant);
   const int tc = ppsk::variant_tile_cols(variant);
   std::vector<size_t> gs;
-  const auto tiles = make_tiles(rows, ref->n, tr, tc, false, 0, rows, tile_group(tr), &gs);
+  std::vector<ppsk::Tile> tiles;
+  if (!L.items) tiles = make_tiles(rows, ref->n, tr, tc, false, 0, rows, tile_group(tr), &gs);
   if (L.persistent) {
     // whole tiles from 8 queues, each a contiguous eighth of the tile list
     // less its tail
@@ -413,6 +448,18 @@ int run_step(ppsk_server* s, Worker& w, std::vector<Piece>& batch, int64_t rows,
       pt.counts = (uint16_t*)(mem + L.tail_counts);
       pt.tile_done = (uint32_t*)(mem + L.tail_done);
       STEP_TRY(ppsk::launch_dists(pt, variant, L.tail * n_k, w.st));
+    }
+    STEP_TRY(hipEventRecord(w.e1, w.st));
+  } else if (L.items) {
+    const ppsk::BandTiles b = ppsk::band_tiles(rows);
+    const int64_t per = b.tall + b.shorts;
+    ppsk::ItemArgs a;
+    std::memset(&a, 0, sizeof(a));
+    STEP_TRY(hipEventRecord(w.e0, w.st));
+    for (int64_t c0 = 0; c0 < n_ct; c0 += L.step_ct) {
+      const int64_t nc = std::min(n_ct - c0, L.step_ct);
+      set_items(&a, (const ppsk::ItemTile*)(mem + L.tiles) + c0 * per, per * nc, band_cut(ref, b, nc));
+      STEP_TRY(ppsk::launch_items(p, a, w.st));
     }
     STEP_TRY(hipEventRecord(w.e1, w.st));
   } else {
@@ -757,6 +804,7 @@ int ppsk_server_create(ppsk_set* ref, int32_t random_mode, int32_t n_clusters,
   s->thr_col = thr_col;
   s->max_rows = max_rows;
   s->variant = std::getenv("PPSK_TILE_VARIANT") ? default_variant() : 0;
+  s->split = !std::getenv("PPSK_TILE_VARIANT") && !std::getenv("PPSK_PERSISTENT");
   s->per_sample = (size_t)ref->n_k * ref->s64 * ppsk::BBITS * sizeof(uint64_t);
   if (ppsk::batch_grid(2, &s->grid2) != hipSuccess) s->grid2 = 0;
   if (ppsk::batch_grid(4, &s->grid4) != hipSuccess) s->grid4 = 0;
@@ -770,6 +818,7 @@ int ppsk_server_create(ppsk_set* ref, int32_t random_mode, int32_t n_clusters,
     if (hipMemGetInfo(&fr, &tot) != hipSuccess) fr = 0;
     arena_bytes = fr > ((size_t)4 << 30) ? fr - ((size_t)4 << 30) : fr / 2;
   }
+  s->slot_share = arena_bytes / (size_t)n_slots;
   const size_t one = layout(s, 1).total;
   if (arena_bytes < one) {
     delete s;
