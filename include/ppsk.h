@@ -423,6 +423,20 @@ int ppsk_sketch_ex(int device_id, int64_t n_samples, const char *seq,
                    uint64_t *raw_out, double *inv_minhash, int32_t *densified);
 
 /*
+ * ppsk_sketch_ex with each contig where it lies: contig c is the
+ * contig_off[c + 1] - contig_off[c] bytes at contigs[c] (contig_off[0] = 0), so
+ * that the caller need not join them.
+ */
+int ppsk_sketch_contigs(int device_id, int64_t n_samples,
+                        const char *const *contigs, const int64_t *contig_off,
+                        int64_t n_contigs, const int64_t *sample_contig,
+                        int32_t n_k, const int32_t *klist,
+                        int32_t sketchsize64, int32_t use_rc,
+                        int32_t codon_phased, int32_t min_count, int32_t exact,
+                        uint64_t *raw_out, double *inv_minhash,
+                        int32_t *densified);
+
+/*
  * Seeded synthetic sketches (no reference counterpart: a generator for tests
  * and benchmarks, writing the reference word layout directly).  Bins evolve
  * down a random binary tree: a child keeps its parent's 14-bit bin value with

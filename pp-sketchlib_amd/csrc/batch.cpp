@@ -574,8 +574,7 @@ int ppsk_batch_run(ppsk_batch* b, int32_t variant, uint64_t* n_fail, int32_t* us
     if (int rc = run_plan(b, v, &ms)) return rc;
   }
   std::vector<unsigned long long> f((size_t)b->n_jobs * 2);
-  HIP_TRY(hipMemcpy(f.data(), b->d_fail, f.size() * sizeof(unsigned long long),
-                    hipMemcpyDeviceToHost));
+  HIP_TRY(copy_to_host(c, f.data(), b->d_fail, f.size() * sizeof(unsigned long long), c->stream));
   uint64_t total = 0;
   for (int j = 0; j < b->n_jobs; ++j) {
     if (n_fail) n_fail[j] = f[2 * j];

@@ -7,8 +7,10 @@
 
 #include <atomic>
 #include <cstdint>
+#include <functional>
 #include <mutex>
 #include <string>
+#include <utility>
 #include <vector>
 
 #include "../../include/ppsk.h"
@@ -23,6 +25,7 @@ struct ppsk_set {
   int32_t bbits;
   int32_t nb;
   uint32_t* stripes = nullptr;  // [n_k][nb][s64][28][128]
+  size_t stripes_bytes = 0;     // of its allocation (set_memory)
   double* jv = nullptr;         // [n][n_k]
   uint16_t* clusters = nullptr; // [n]
   bool has_lengths = false;
@@ -53,6 +56,17 @@ int fail(int code, const std::string& msg);
 
 // Per-device state: a launch stream, a copy stream, cached workspaces grown on
 // demand.
+// Page-locked blocks that host copies go through (host_io.cpp): two for each of
+// up to LANES copying threads of one copy at a time.
+struct HostStage {
+  static constexpr int LANES = 4;
+  static constexpr size_t BLOCK = (size_t)2 << 20;
+  char* block[2 * LANES] = {};
+  hipEvent_t done[2 * LANES] = {};  // the block's last copy
+  std::mutex mu;
+  hipError_t init();
+};
+
 struct DeviceCtx {
   int device = -1;
   hipStream_t stream = nullptr;
@@ -62,7 +76,11 @@ struct DeviceCtx {
   size_t tile_done_n = 0;
   ppsk::Tile* tiles = nullptr;
   size_t tiles_n = 0;
-  unsigned long long* fail = nullptr;  // [0] count, [1] first row
+  // [0] fit failures, [1] first failed row, [2] progress (ctl.progress): one
+  // read at the end of a call
+  unsigned long long* fail = nullptr;
+  unsigned long long* words = nullptr;  // page-locked copy of the three
+  bool words_read = false;              // `words` holds the call's final values
   void* out = nullptr;
   size_t out_bytes = 0;
   hipStream_t copy_stream = nullptr;  // device -> host copies of finished rows
@@ -78,6 +96,21 @@ struct DeviceCtx {
   size_t codes_bytes = 0;
   hipStream_t tail_stream = nullptr;  // the tail's (tile, k) launch beside the persistent one
   void* noalloc_scratch = nullptr;    // this device's copy of the fixed scratch array
+  void* table = nullptr;              // Monte Carlo table of a dense pass
+  size_t table_bytes = 0;
+  void* sel = nullptr;                // lists and counts of the sparse outputs
+  size_t sel_bytes = 0;
+  void* hits = nullptr;               // threshold hits
+  size_t hits_bytes = 0;
+  void* sketch = nullptr;             // buffers of a sketching call
+  size_t sketch_bytes = 0;
+  HostStage host;
+  std::mutex upload_mu;               // raw sketches on their way to the stripes,
+  void* raw = nullptr;                // two halves of raw_bytes / 2
+  size_t raw_bytes = 0;
+  hipEvent_t raw_copied = nullptr, raw_striped[2] = {};
+  std::mutex spare_mu;
+  std::vector<std::pair<void*, size_t>> spare;  // memory of freed sets (set_memory)
   ppsk::Control ctl{};                // progress / cancellation pointers of the calls
   std::mutex mu;
 };
@@ -124,6 +157,31 @@ DeviceCtx* find_ctx(int device);
 int noalloc_init(void** scratch);
 // Device buffer of at least `need` bytes (reallocated, contents lost).
 int grow(void** ptr, size_t* have, size_t need);
+// Frees a buffer that a call left larger than a context keeps (1 GiB).
+void trim(void** ptr, size_t* have);
+// hipMalloc of a sketch set's stripes, and its release.  A context keeps up to
+// 4 blocks of freed sets, together at most 512 MiB, for the next sets of about
+// their size (a set of 333 samples, 47 MB: hipMalloc 0.5 ms and hipFree 0.2 ms
+// of a call of 2.5 ms), and gives them back when an allocation fails.
+hipError_t set_memory(DeviceCtx* c, size_t bytes, void** out, size_t* got);
+void release_set_memory(DeviceCtx* c, void* p, size_t bytes);
+// hipMalloc that gives the spare blocks back and tries again when it fails.
+hipError_t device_malloc(DeviceCtx* c, void** p, size_t bytes);
+// The same, which before a last try frees the workspaces that no call is using
+// (codes, lists, tables, sketching); locked: the caller holds c->mu.
+hipError_t device_malloc_all(DeviceCtx* c, void** p, size_t bytes, bool locked);
+// c->out of at least `need` bytes, at the start of a call.
+int grow_out(DeviceCtx* c, size_t need);
+
+// Host copies on `stream` (host_io.cpp).  copy_to_device returns when src may be
+// changed, the copy being queued; copy_to_host when dst is complete.  Fill writes
+// bytes [at, at + n) of the source to `to`, from any thread.
+using Fill = std::function<void(char* to, size_t at, size_t n)>;
+hipError_t fill_device(DeviceCtx* c, void* dst, size_t bytes, hipStream_t stream, const Fill& fill);
+hipError_t copy_to_device(DeviceCtx* c, void* dst, const void* src, size_t bytes,
+                          hipStream_t stream);
+hipError_t copy_to_host(DeviceCtx* c, void* dst, const void* src, size_t bytes, hipStream_t stream);
+
 // Tile completion counters, zero on return.
 int grow_tile_done(DeviceCtx* c, size_t n);
 

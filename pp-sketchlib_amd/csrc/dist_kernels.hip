@@ -2141,6 +2141,18 @@ hipError_t launch_band_setup(ItemTile* tiles, int64_t rows, int64_t n_ct, int64_
   return hipGetLastError();
 }
 
+__global__ void call_reset_kernel(unsigned long long* fail, unsigned long long* progress) {
+  fail[0] = 0ull;
+  fail[1] = ~0ull;
+  *progress = 0ull;
+}
+
+hipError_t launch_call_reset(unsigned long long* fail, unsigned long long* progress,
+                             hipStream_t stream) {
+  call_reset_kernel<<<1, 1, 0, stream>>>(fail, progress);
+  return hipGetLastError();
+}
+
 bool variant_valid(int v) { return v >= 1 && v <= N_VARIANTS; }
 
 int variant_tile_rows(int v) {

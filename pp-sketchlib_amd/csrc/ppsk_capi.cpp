@@ -51,12 +51,16 @@ int get_ctx(int device, DeviceCtx** out) {
     c->device = device;
     HIP_TRY(hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking));
     HIP_TRY(hipStreamCreateWithFlags(&c->copy_stream, hipStreamNonBlocking));
-    HIP_TRY(hipMalloc(&c->fail, 2 * sizeof(unsigned long long)));
+    HIP_TRY(hipMalloc(&c->fail, 3 * sizeof(unsigned long long)));
+    HIP_TRY(hipHostMalloc((void**)&c->words, 3 * sizeof(unsigned long long), hipHostMallocDefault));
+    HIP_TRY(c->host.init());
+    HIP_TRY(hipEventCreateWithFlags(&c->raw_copied, hipEventDisableTiming));
+    for (auto& ev : c->raw_striped) HIP_TRY(hipEventCreateWithFlags(&ev, hipEventDisableTiming));
     if (int rc = noalloc_init(&c->noalloc_scratch)) return rc;
     HIP_TRY(ppsk::upload_log_table());
     // progress / cancellation words: a device counter and two host-mapped,
     // coherent words (device_id < MAX_DEVICES here)
-    HIP_TRY(hipMalloc(&c->ctl.progress, sizeof(unsigned long long)));
+    c->ctl.progress = c->fail + 2;
     HIP_TRY(hipMemset(c->ctl.progress, 0, sizeof(unsigned long long)));
     void* hw = nullptr;
     HIP_TRY(hipHostMalloc(&hw, 64, hipHostMallocMapped | hipHostMallocCoherent));
@@ -101,21 +105,32 @@ uint64_t read_progress(CallState& cs) {
   return std::max(v, seen);
 }
 
+// Fit failures and progress of the work queued so far, into c->words.
+hipError_t queue_words(DeviceCtx* c) {
+  return hipMemcpyAsync(c->words, c->fail, 3 * sizeof(unsigned long long), hipMemcpyDeviceToHost,
+                        c->stream);
+}
+
+hipError_t read_words(DeviceCtx* c) {
+  hipError_t e = queue_words(c);
+  if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
+  c->words_read = e == hipSuccess;
+  return e;
+}
+
 CallScope::CallScope(DeviceCtx* ctx, uint64_t total) : c(ctx), cs(g_calls[ctx->device]) {
   cs.total.store(total);
   cs.seen.store(0);
   if (volatile unsigned long long* p = cs.progress_host.load()) *p = 0;
   cs.running.store(1);
-  // the device counter starts from zero in stream order
-  hipMemsetAsync(c->ctl.progress, 0, sizeof(unsigned long long), c->stream);
+  // the device counters start from zero in stream order
+  c->words_read = false;
+  (void)ppsk::launch_call_reset(c->fail, c->ctl.progress, c->stream);
 }
 
 CallScope::~CallScope() {
-  unsigned long long v = 0;
-  if (hipMemcpyAsync(&v, c->ctl.progress, sizeof(v), hipMemcpyDeviceToHost, c->stream) ==
-          hipSuccess &&
-      hipStreamSynchronize(c->stream) == hipSuccess) {
-    cs.seen.store(v);
+  if (c->words_read || read_words(c) == hipSuccess) {
+    cs.seen.store(c->words[2]);
   } else {
     read_progress(cs);
   }
@@ -150,9 +165,107 @@ int grow(void** ptr, size_t* have, size_t need) {
   if (*ptr) HIP_TRY(hipFree(*ptr));
   *ptr = nullptr;
   *have = 0;
-  HIP_TRY(hipMalloc(ptr, need));
+  hipError_t e = hipMalloc(ptr, need);
+  if (e == hipErrorOutOfMemory) {
+    int device = 0;
+    DeviceCtx* c = hipGetDevice(&device) == hipSuccess ? find_ctx(device) : nullptr;
+    if (c) e = device_malloc(c, ptr, need);
+  }
+  HIP_TRY(e);
   *have = need;
   return PPSK_OK;
+}
+
+void trim(void** ptr, size_t* have) {
+  if (*have <= ((size_t)1 << 30)) return;
+  hipFree(*ptr);
+  *ptr = nullptr;
+  *have = 0;
+}
+
+hipError_t device_malloc(DeviceCtx* c, void** p, size_t bytes) {
+  hipError_t e = hipMalloc(p, bytes);
+  if (e != hipErrorOutOfMemory) return e;
+  std::vector<std::pair<void*, size_t>> spare;
+  {
+    std::lock_guard<std::mutex> lk(c->spare_mu);
+    spare.swap(c->spare);
+  }
+  if (spare.empty()) return e;
+  (void)hipGetLastError();
+  for (auto& s : spare) hipFree(s.first);
+  return hipMalloc(p, bytes);
+}
+
+hipError_t device_malloc_all(DeviceCtx* c, void** p, size_t bytes, bool locked) {
+  hipError_t e = device_malloc(c, p, bytes);
+  if (e != hipErrorOutOfMemory) return e;
+  (void)hipGetLastError();
+  std::unique_lock<std::mutex> lk(c->mu, std::defer_lock);
+  if (!locked) lk.lock();
+  const std::pair<void**, size_t*> idle[] = {{&c->codes, &c->codes_bytes}, {&c->sel, &c->sel_bytes},
+                                             {&c->hits, &c->hits_bytes}, {&c->table, &c->table_bytes},
+                                             {&c->sketch, &c->sketch_bytes}};
+  for (auto& w : idle) {
+    if (*w.first) hipFree(*w.first);
+    *w.first = nullptr;
+    *w.second = 0;
+  }
+  return hipMalloc(p, bytes);
+}
+
+int grow_out(DeviceCtx* c, size_t need) {
+  if (c->out_bytes >= need && c->out) return PPSK_OK;
+  if (c->out) HIP_TRY(hipFree(c->out));
+  c->out = nullptr;
+  c->out_bytes = 0;
+  HIP_TRY(device_malloc_all(c, &c->out, need, true));
+  c->out_bytes = need;
+  return PPSK_OK;
+}
+
+constexpr size_t SPARE_BLOCKS = 4, SPARE_BYTES = (size_t)512 << 20;
+
+hipError_t set_memory(DeviceCtx* c, size_t bytes, void** out, size_t* got) {
+  {
+    std::lock_guard<std::mutex> lk(c->spare_mu);
+    auto best = c->spare.end();
+    for (auto s = c->spare.begin(); s != c->spare.end(); ++s) {
+      if (s->second >= bytes && s->second <= bytes + bytes / 4 &&
+          (best == c->spare.end() || s->second < best->second)) {
+        best = s;
+      }
+    }
+    if (best != c->spare.end()) {
+      *out = best->first;
+      *got = best->second;
+      c->spare.erase(best);
+      return hipSuccess;
+    }
+  }
+  *got = bytes;
+  return device_malloc_all(c, out, bytes, false);
+}
+
+void release_set_memory(DeviceCtx* c, void* p, size_t bytes) {
+  // like hipFree, returns once nothing on the device uses the block
+  if (bytes > SPARE_BYTES || hipDeviceSynchronize() != hipSuccess) {
+    hipFree(p);
+    return;
+  }
+  std::vector<void*> old;
+  {
+    std::lock_guard<std::mutex> lk(c->spare_mu);
+    size_t held = bytes;
+    for (auto& s : c->spare) held += s.second;
+    while (c->spare.size() >= SPARE_BLOCKS || held > SPARE_BYTES) {
+      held -= c->spare.front().second;
+      old.push_back(c->spare.front().first);
+      c->spare.erase(c->spare.begin());
+    }
+    c->spare.emplace_back(p, bytes);
+  }
+  for (void* x : old) hipFree(x);
 }
 
 int grow_tile_done(DeviceCtx* c, size_t n) {
@@ -279,16 +392,17 @@ int64_t out_row_start(bool self, int64_t r, int64_t n_rows, int64_t n_cols) {
 }
 
 // Copies the dense output of sample rows [r0, r1) to the host on the copy
-// stream once `done` has been reached on the launch stream.
+// stream once `done` has been reached on the launch stream; the wait comes
+// first, so that other copies can use the blocks meanwhile.
 int copy_rows(DeviceCtx* c, int64_t r0, int64_t r1, const ppsk::DistParams& p, bool self,
               size_t elem, void* host_out, hipEvent_t done) {
   const int64_t o0 = out_row_start(self, r0, p.n_rows, p.n_cols);
   const int64_t o1 = out_row_start(self, r1, p.n_rows, p.n_cols);
   if (o1 > o0) {
     const char* dev = (const char*)p.out;
-    HIP_TRY(hipStreamWaitEvent(c->copy_stream, done, 0));
-    HIP_TRY(hipMemcpyAsync((char*)host_out + o0 * elem, dev + o0 * elem, (o1 - o0) * elem,
-                           hipMemcpyDeviceToHost, c->copy_stream));
+    HIP_TRY(hipEventSynchronize(done));
+    HIP_TRY(copy_to_host(c, (char*)host_out + o0 * elem, dev + o0 * elem, (o1 - o0) * elem,
+                         c->copy_stream));
   }
   return PPSK_OK;
 }
@@ -348,8 +462,7 @@ int run_dense_tiles(DeviceCtx* c, ppsk::DistParams p, int variant, bool upper, i
   if (int rc = grow(&tptr, &tbytes, tiles.size() * sizeof(ppsk::Tile))) return rc;
   c->tiles = (ppsk::Tile*)tptr;
   c->tiles_n = tbytes / sizeof(ppsk::Tile);
-  HIP_TRY(hipMemcpyAsync(c->tiles, tiles.data(), tiles.size() * sizeof(ppsk::Tile),
-                         hipMemcpyHostToDevice, c->stream));
+  HIP_TRY(copy_to_device(c, c->tiles, tiles.data(), tiles.size() * sizeof(ppsk::Tile), c->stream));
   p.counts = (uint16_t*)c->counts;
   p.tile_done = c->tile_done;
   p.out_row_offset = 0;
@@ -484,14 +597,14 @@ int run_dense_persistent(DeviceCtx* c, ppsk::DistParams p, int variant, bool upp
     if (int rc = grow(&tptr, &tbytes, tail_tiles.size() * sizeof(ppsk::Tile))) return rc;
     c->tiles = (ppsk::Tile*)tptr;
     c->tiles_n = tbytes / sizeof(ppsk::Tile);
-    HIP_TRY(hipMemcpyAsync(c->tiles, tail_tiles.data(), tail_tiles.size() * sizeof(ppsk::Tile),
-                           hipMemcpyHostToDevice, c->stream));
+    HIP_TRY(copy_to_device(c, c->tiles, tail_tiles.data(), tail_tiles.size() * sizeof(ppsk::Tile),
+                           c->stream));
     p.counts = (uint16_t*)c->counts;
     p.tile_done = c->tile_done;
   }
-  HIP_TRY(hipMemcpyAsync(c->pitems, items.data(), items.size() * sizeof(ppsk::BatchItem),
-                         hipMemcpyHostToDevice, c->stream));
-  HIP_TRY(hipMemcpyAsync(c->pparams, &p, sizeof(p), hipMemcpyHostToDevice, c->stream));
+  HIP_TRY(copy_to_device(c, c->pitems, items.data(), items.size() * sizeof(ppsk::BatchItem),
+                         c->stream));
+  HIP_TRY(copy_to_device(c, c->pparams, &p, sizeof(p), c->stream));
   ppsk::BatchArgs args;
   std::memset(&args, 0, sizeof(args));
   args.jobs = c->pparams;
@@ -788,7 +901,7 @@ int make_item_plan(DeviceCtx* c, const ppsk::DistParams& p, bool upper, int64_t 
       if (c->codes) HIP_TRY(hipFree(c->codes));
       c->codes = nullptr;
       c->codes_bytes = 0;
-      if (hipMalloc(&c->codes, out->code_bytes) == hipSuccess) {
+      if (device_malloc(c, &c->codes, out->code_bytes) == hipSuccess) {
         c->codes_bytes = out->code_bytes;
         return PPSK_OK;
       }
@@ -835,7 +948,7 @@ int run_dense_items(DeviceCtx* c, ppsk::DistParams p, bool upper, int64_t row_be
   }
   std::memcpy(lists.data() + slab_bytes, pl.tiles.data(), pl.tiles.size() * sizeof(ppsk::ItemTile));
   if (int rc = grow(&c->pitems, &c->pitems_bytes, lists.size())) return rc;
-  HIP_TRY(hipMemcpyAsync(c->pitems, lists.data(), lists.size(), hipMemcpyHostToDevice, c->stream));
+  HIP_TRY(copy_to_device(c, c->pitems, lists.data(), lists.size(), c->stream));
   const ppsk::CodeGroup* d_slabs = (const ppsk::CodeGroup*)c->pitems;
   const ppsk::ItemTile* d_tiles = (const ppsk::ItemTile*)((char*)c->pitems + slab_bytes);
   p.counts = (uint16_t*)c->counts;
@@ -864,6 +977,7 @@ int run_dense_items(DeviceCtx* c, ppsk::DistParams p, bool upper, int64_t row_be
     tm->launches += 1;
     tm->items += a.n_items;
   }
+  HIP_TRY(queue_words(c));
   // Copies are queued after every launch: a copy into pageable memory may
   // block this thread until it completes, which must not hold back launches.
   for (size_t ci = 0; host_out && ci < pl.chunks.size(); ++ci) {
@@ -873,7 +987,7 @@ int run_dense_items(DeviceCtx* c, ppsk::DistParams p, bool upper, int64_t row_be
     }
   }
   HIP_TRY(hipStreamSynchronize(c->stream));
-  HIP_TRY(hipStreamSynchronize(c->copy_stream));
+  c->words_read = true;
   for (size_t ci = 0; ci < pl.chunks.size(); ++ci) {
     float ms = 0.f;
     HIP_TRY(hipEventElapsedTime(&ms, c->events[2 * ci], c->events[2 * ci + 1]));
@@ -920,6 +1034,7 @@ uint64_t dense_items(const ppsk_set* rows, const ppsk_set* cols, bool upper, int
 // Dense pass over rows [row_begin, row_end).
 int run_dense(DeviceCtx* c, ppsk::DistParams p, int variant, bool upper, int64_t row_begin,
               int64_t row_end, bool self, size_t elem, void* host_out, Timing* tm) {
+  c->words_read = false;
   switch (dense_route(variant, upper, row_end - row_begin, p.n_cols)) {
     case Route::persistent:
       return run_dense_persistent(c, p, variant, upper, row_begin, row_end, self, elem, host_out,
@@ -971,23 +1086,26 @@ int upload_table(DeviceCtx* c, const ppsk_set* s, const RandomIn& rnd, float** d
   *dtab = nullptr;
   if (rnd.mode != PPSK_RANDOM_MC) return PPSK_OK;
   const size_t bytes = (size_t)s->n_k * rnd.n_clusters * rnd.n_clusters * sizeof(float);
-  HIP_TRY(hipMalloc((void**)dtab, bytes));
-  HIP_TRY(hipMemcpyAsync(*dtab, rnd.table, bytes, hipMemcpyHostToDevice, c->stream));
+  HIP_TRY(device_malloc(c, (void**)dtab, bytes));
+  HIP_TRY(copy_to_device(c, *dtab, rnd.table, bytes, c->stream));
   return PPSK_OK;
 }
 
-int reset_fail(DeviceCtx* c) {
-  unsigned long long init[2] = {0ull, ~0ull};
-  HIP_TRY(hipMemcpyAsync(c->fail, init, sizeof(init), hipMemcpyHostToDevice, c->stream));
+// The table of a call that holds c->mu, in the context's own buffer.
+int call_table(DeviceCtx* c, const ppsk_set* s, const RandomIn& rnd, float** dtab) {
+  *dtab = nullptr;
+  if (rnd.mode != PPSK_RANDOM_MC) return PPSK_OK;
+  const size_t bytes = (size_t)s->n_k * rnd.n_clusters * rnd.n_clusters * sizeof(float);
+  if (int rc = grow(&c->table, &c->table_bytes, bytes)) return rc;
+  *dtab = (float*)c->table;
+  HIP_TRY(copy_to_device(c, *dtab, rnd.table, bytes, c->stream));
   return PPSK_OK;
 }
 
 int read_fail(DeviceCtx* c, unsigned long long* cnt, unsigned long long* first) {
-  unsigned long long v[2];
-  HIP_TRY(hipMemcpyAsync(v, c->fail, sizeof(v), hipMemcpyDeviceToHost, c->stream));
-  HIP_TRY(hipStreamSynchronize(c->stream));
-  *cnt = v[0];
-  *first = v[1];
+  if (!c->words_read) HIP_TRY(read_words(c));
+  *cnt = c->words[0];
+  *first = c->words[1];
   return PPSK_OK;
 }
 
@@ -1012,7 +1130,7 @@ int dense_pass(DeviceCtx* c, const ppsk_set* rows, const ppsk_set* cols, bool se
                const RandomIn& rnd, double tol, int32_t out_kind, void* dout, void* host_out,
                size_t elem, Timing* tm, unsigned long long* nf, unsigned long long* ff) {
   float* dtab = nullptr;
-  if (int rc = upload_table(c, rows, rnd, &dtab)) return rc;
+  if (int rc = call_table(c, rows, rnd, &dtab)) return rc;
   ppsk::DistParams p;
   fill_common(p, rows, cols, rnd, tol);
   p.self_mode = self ? 1 : 0;
@@ -1024,43 +1142,52 @@ int dense_pass(DeviceCtx* c, const ppsk_set* rows, const ppsk_set* cols, bool se
   p.fail_count = c->fail;
   p.fail_first = c->fail + 1;
   p.ctl = c->ctl;
-  int rc = reset_fail(c);
-  if (rc == PPSK_OK) {
-    const int variant = default_variant();
-    rc = run_dense(c, p, variant, self, 0, rows->n, self, elem, host_out, tm);
-  }
-  if (dtab) hipFree(dtab);
+  const int variant = default_variant();
+  int rc = run_dense(c, p, variant, self, 0, rows->n, self, elem, host_out, tm);
+  trim(&c->table, &c->table_bytes);
   if (rc) return rc;
   // the kernels skip their remaining work once a cancellation is seen
   if ((rc = cancel_status(c->device))) return rc;
   return read_fail(c, nf, ff);
 }
 
+// kNN lists of `rows` rows in the context's buffer, and the row heaps above the
+// LDS limit.
+struct KnnLists {
+  int64_t *i, *j;
+  float* d;
+  void* heap;
+};
+
+int knn_lists(DeviceCtx* c, int64_t rows, int kNN, KnnLists* L) {
+  const size_t m = ((size_t)rows * kNN + 31) / 32 * 32;
+  const size_t hw = ppsk::knn_heap_workspace(rows, kNN);
+  if (int rc = grow(&c->sel, &c->sel_bytes, m * (2 * sizeof(int64_t) + sizeof(float)) + hw)) return rc;
+  L->i = (int64_t*)c->sel;
+  L->j = L->i + m;
+  L->d = (float*)(L->j + m);
+  L->heap = hw ? L->d + m : nullptr;
+  return PPSK_OK;
+}
+
+hipError_t copy_knn(DeviceCtx* c, const KnnLists& L, size_t m, int64_t* i_vec, int64_t* j_vec,
+                    float* dists) {
+  hipError_t e = copy_to_host(c, i_vec, L.i, m * sizeof(int64_t), c->stream);
+  if (e == hipSuccess) e = copy_to_host(c, j_vec, L.j, m * sizeof(int64_t), c->stream);
+  if (e == hipSuccess) e = copy_to_host(c, dists, L.d, m * sizeof(float), c->stream);
+  return e;
+}
+
 // kNN selection over all rows of a symmetric self distance held as a
 // condensed triangle on the device; outputs copied to host.
 int knn_from_triangle(DeviceCtx* c, const float* tri, int64_t n, int col, int kNN, int64_t* i_vec,
                       int64_t* j_vec, float* dists) {
-  int64_t *d_i = nullptr, *d_j = nullptr;
-  float* d_d = nullptr;
-  void* heap_ws = nullptr;  // row heaps above the LDS limit
-  const size_t m = (size_t)n * kNN;
-  const size_t hw = ppsk::knn_heap_workspace(n, kNN);
-  hipError_t e = hipMalloc(&d_i, m * sizeof(int64_t));
-  if (e == hipSuccess) e = hipMalloc(&d_j, m * sizeof(int64_t));
-  if (e == hipSuccess) e = hipMalloc(&d_d, m * sizeof(float));
-  if (e == hipSuccess && hw) e = hipMalloc(&heap_ws, hw);
-  if (e == hipSuccess) {
-    e = ppsk::launch_knn_select_triangle(tri, n, col, kNN, d_i, d_j, d_d, c->stream, heap_ws);
-  }
-  if (e == hipSuccess) e = hipMemcpyAsync(i_vec, d_i, m * sizeof(int64_t), hipMemcpyDeviceToHost, c->stream);
-  if (e == hipSuccess) e = hipMemcpyAsync(j_vec, d_j, m * sizeof(int64_t), hipMemcpyDeviceToHost, c->stream);
-  if (e == hipSuccess) e = hipMemcpyAsync(dists, d_d, m * sizeof(float), hipMemcpyDeviceToHost, c->stream);
-  if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
+  KnnLists L;
+  if (int rc = knn_lists(c, n, kNN, &L)) return rc;
+  hipError_t e = ppsk::launch_knn_select_triangle(tri, n, col, kNN, L.i, L.j, L.d, c->stream, L.heap);
+  if (e == hipSuccess) e = copy_knn(c, L, (size_t)n * kNN, i_vec, j_vec, dists);
   if (e != hipSuccess) hipStreamSynchronize(c->stream);  // nothing queued may outlive its buffers
-  if (d_i) hipFree(d_i);
-  if (d_j) hipFree(d_j);
-  if (d_d) hipFree(d_d);
-  if (heap_ws) hipFree(heap_ws);
+  trim(&c->sel, &c->sel_bytes);
   if (e != hipSuccess) return fail(e == hipErrorOutOfMemory ? PPSK_ERR_MEMORY : PPSK_ERR_HIP,
                                    std::string("kNN selection: ") + hipGetErrorString(e));
   return PPSK_OK;
@@ -1069,22 +1196,41 @@ int knn_from_triangle(DeviceCtx* c, const float* tri, int64_t n, int col, int kN
 // Threshold compaction of a device triangle into library-allocated host arrays.
 int threshold_from_triangle(DeviceCtx* c, const float2* tri, int64_t n, int col, float cutoff,
                             int64_t** i_vec, int64_t** j_vec, float** dists, int64_t* n_out) {
+  // per-row counts, their offsets on the device, then the hits in row order
+  const int64_t rows = n > 1 ? n - 1 : 0;
   int64_t total = 0;
-  int64_t *d_i = nullptr, *d_j = nullptr;
-  float* d_d = nullptr;
-  hipError_t e = ppsk::threshold_compact(tri, n, col, cutoff, &total, &d_i, &d_j, &d_d, c->stream);
+  hipError_t e = hipSuccess;
+  if (rows > 0) {
+    if (int rc = grow(&c->sel, &c->sel_bytes, (size_t)(rows + 1) * sizeof(int64_t))) return rc;
+    int64_t* counts = (int64_t*)c->sel;
+    e = ppsk::launch_threshold_count(tri, rows, n, false, col, cutoff, counts, c->stream);
+    if (e == hipSuccess) e = ppsk::launch_offsets_scan(counts, rows, c->stream);
+    if (e == hipSuccess) e = copy_to_host(c, &total, counts + rows, sizeof(total), c->stream);
+  }
   if (e != hipSuccess) return fail(PPSK_ERR_HIP, std::string("threshold: ") + hipGetErrorString(e));
   auto* hi = (int64_t*)std::malloc(std::max<int64_t>(total, 1) * sizeof(int64_t));
   auto* hj = (int64_t*)std::malloc(std::max<int64_t>(total, 1) * sizeof(int64_t));
   auto* hd = (float*)std::malloc(std::max<int64_t>(total, 1) * sizeof(float));
   if (hi && hj && hd && total > 0) {
-    e = hipMemcpy(hi, d_i, total * sizeof(int64_t), hipMemcpyDeviceToHost);
-    if (e == hipSuccess) e = hipMemcpy(hj, d_j, total * sizeof(int64_t), hipMemcpyDeviceToHost);
-    if (e == hipSuccess) e = hipMemcpy(hd, d_d, total * sizeof(float), hipMemcpyDeviceToHost);
+    const size_t m = (size_t)total;
+    if (int rc = grow(&c->hits, &c->hits_bytes, m * (2 * sizeof(int64_t) + sizeof(float)))) {
+      std::free(hi);
+      std::free(hj);
+      std::free(hd);
+      return rc;
+    }
+    int64_t* d_i = (int64_t*)c->hits;
+    int64_t* d_j = d_i + m;
+    float* d_d = (float*)(d_j + m);
+    e = ppsk::launch_threshold_write(tri, rows, n, false, col, cutoff, (int64_t*)c->sel, d_i, d_j,
+                                     d_d, c->stream);
+    if (e == hipSuccess) e = copy_to_host(c, hi, d_i, m * sizeof(int64_t), c->stream);
+    if (e == hipSuccess) e = copy_to_host(c, hj, d_j, m * sizeof(int64_t), c->stream);
+    if (e == hipSuccess) e = copy_to_host(c, hd, d_d, m * sizeof(float), c->stream);
+    if (e != hipSuccess) hipStreamSynchronize(c->stream);
   }
-  if (d_i) hipFree(d_i);
-  if (d_j) hipFree(d_j);
-  if (d_d) hipFree(d_d);
+  trim(&c->sel, &c->sel_bytes);
+  trim(&c->hits, &c->hits_bytes);
   if (!hi || !hj || !hd || e != hipSuccess) {
     std::free(hi);
     std::free(hj);
@@ -1165,7 +1311,7 @@ int ppsk_set_create(int device_id, int64_t n_samples, int32_t n_k, const int32_t
   s->nb = (int32_t)((n_samples + ppsk::BLK - 1) / ppsk::BLK);
   const size_t bytes = ((size_t)n_k * s->nb * sketchsize64 + ppsk::STRIPE_PAD_WORDS) *
                        ppsk::HL * ppsk::BLK * sizeof(uint32_t);
-  hipError_t e = hipMalloc(&s->stripes, bytes);
+  hipError_t e = set_memory(c, bytes, (void**)&s->stripes, &s->stripes_bytes);
   if (e != hipSuccess) {
     delete s;
     return fail(PPSK_ERR_MEMORY, std::string("sketch set allocation: ") + hipGetErrorString(e));
@@ -1192,23 +1338,33 @@ int ppsk_set_upload(ppsk_set* s, int64_t first, int64_t count, const uint64_t* r
   DeviceCtx* c = nullptr;
   if (int rc = get_ctx(s->device, &c)) return rc;
   const size_t per_sample = (size_t)s->n_k * s->s64 * s->bbits * sizeof(uint64_t);
-  const int64_t chunk = std::max<int64_t>(1, (int64_t)((256u << 20) / per_sample));
-  void* staging = nullptr;
-  HIP_TRY(hipMalloc(&staging, (size_t)std::min(chunk, count) * per_sample));
-  int rc = PPSK_OK;
-  for (int64_t c0 = 0; c0 < count && rc == PPSK_OK; c0 += chunk) {
+  // Through two halves of a kept buffer on the copy stream, each chunk's stripes
+  // written while the next one crosses the link.
+  std::lock_guard<std::mutex> lk(c->upload_mu);
+  const int64_t chunk = std::min<int64_t>(count, std::max<int64_t>(1, (int64_t)((32u << 20) / per_sample)));
+  const size_t half = ((size_t)chunk * per_sample + 255) / 256 * 256;
+  if (int rc = grow(&c->raw, &c->raw_bytes, 2 * half)) return rc;
+  hipError_t e = hipSuccess;
+  int turn = 0;
+  for (int64_t c0 = 0; c0 < count && e == hipSuccess; c0 += chunk, turn ^= 1) {
     const int64_t m = std::min(chunk, count - c0);
-    hipError_t e = hipMemcpyAsync(staging, (const char*)raw + (size_t)c0 * per_sample,
-                                  (size_t)m * per_sample, hipMemcpyHostToDevice, c->stream);
+    uint64_t* to = (uint64_t*)((char*)c->raw + turn * half);
+    e = hipStreamWaitEvent(c->copy_stream, c->raw_striped[turn], 0);
     if (e == hipSuccess) {
-      e = ppsk::launch_stripe((const uint64_t*)staging, m, first + c0, s->n_k, s->s64, s->nb,
-                              s->stripes, c->stream);
+      e = copy_to_device(c, to, (const char*)raw + (size_t)c0 * per_sample, (size_t)m * per_sample,
+                         c->copy_stream);
     }
-    if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
-    if (e != hipSuccess) rc = fail(PPSK_ERR_HIP, std::string("upload: ") + hipGetErrorString(e));
+    if (e == hipSuccess) e = hipEventRecord(c->raw_copied, c->copy_stream);
+    if (e == hipSuccess) e = hipStreamWaitEvent(c->stream, c->raw_copied, 0);
+    if (e == hipSuccess) {
+      e = ppsk::launch_stripe(to, m, first + c0, s->n_k, s->s64, s->nb, s->stripes, c->stream);
+    }
+    if (e == hipSuccess) e = hipEventRecord(c->raw_striped[turn], c->stream);
   }
-  hipFree(staging);
-  return rc;
+  if (e == hipSuccess) e = hipStreamSynchronize(c->copy_stream);  // raw may be changed from here
+  if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
+  if (e != hipSuccess) return fail(PPSK_ERR_HIP, std::string("upload: ") + hipGetErrorString(e));
+  return PPSK_OK;
 }
 
 int ppsk_set_meta(ppsk_set* s, const uint64_t* lengths, int32_t use_rc, const uint16_t* clusters) {
@@ -1233,8 +1389,7 @@ int ppsk_set_meta(ppsk_set* s, const uint64_t* lengths, int32_t use_rc, const ui
       }
     }
     if (!s->jv) HIP_TRY(hipMalloc(&s->jv, jv.size() * sizeof(double)));
-    HIP_TRY(hipMemcpyAsync(s->jv, jv.data(), jv.size() * sizeof(double), hipMemcpyHostToDevice,
-                           c->stream));
+    HIP_TRY(copy_to_device(c, s->jv, jv.data(), jv.size() * sizeof(double), c->stream));
     HIP_TRY(hipStreamSynchronize(c->stream));
     s->has_lengths = true;
     s->use_rc = use_rc;
@@ -1243,8 +1398,7 @@ int ppsk_set_meta(ppsk_set* s, const uint64_t* lengths, int32_t use_rc, const ui
     s->max_cluster = 0;
     for (int64_t i = 0; i < s->n; ++i) s->max_cluster = std::max<int32_t>(s->max_cluster, clusters[i]);
     if (!s->clusters) HIP_TRY(hipMalloc(&s->clusters, (size_t)s->n * sizeof(uint16_t)));
-    HIP_TRY(hipMemcpyAsync(s->clusters, clusters, (size_t)s->n * sizeof(uint16_t),
-                           hipMemcpyHostToDevice, c->stream));
+    HIP_TRY(copy_to_device(c, s->clusters, clusters, (size_t)s->n * sizeof(uint16_t), c->stream));
     HIP_TRY(hipStreamSynchronize(c->stream));
   }
   return PPSK_OK;
@@ -1273,7 +1427,14 @@ int ppsk_set_free(ppsk_set* s) {
     return PPSK_OK;
   }
   hipSetDevice(s->device);
-  if (s->stripes) hipFree(s->stripes);
+  if (s->stripes) {
+    DeviceCtx* c = find_ctx(s->device);
+    if (c) {
+      release_set_memory(c, s->stripes, s->stripes_bytes);
+    } else {
+      hipFree(s->stripes);
+    }
+  }
   if (s->jv) hipFree(s->jv);
   if (s->clusters) hipFree(s->clusters);
   delete s;
@@ -1317,7 +1478,7 @@ int ppsk_dense(ppsk_set* ref, ppsk_set* query, int32_t random_mode, int32_t n_cl
   if (n_rows_out == 0) return PPSK_OK;
   void* dout = out;
   if (!out_on_device) {
-    if (int rc = grow(&c->out, &c->out_bytes, (size_t)n_rows_out * elem)) return rc;
+    if (int rc = grow_out(c, (size_t)n_rows_out * elem)) return rc;
     dout = c->out;
   }
   Timing tm;
@@ -1373,7 +1534,7 @@ int ppsk_knn(ppsk_set* ref, int32_t random_mode, int32_t n_clusters, const float
   if (symmetric) {
     // distances are symmetric: compute the upper triangle once and read both
     // (i, j) and (j, i) from it
-    if ((rc = grow(&c->out, &c->out_bytes, std::max<size_t>(tri_bytes, 8)))) return rc;
+    if ((rc = grow_out(c, std::max<size_t>(tri_bytes, 8)))) return rc;
     if (n > 1) {
       rc = dense_pass(c, ref, ref, true, rnd, tolerance, kind, c->out, nullptr, sizeof(float2),
                       &tm, &nf, &ff);
@@ -1383,19 +1544,11 @@ int ppsk_knn(ppsk_set* ref, int32_t random_mode, int32_t n_clusters, const float
     }
   } else {
     const int variant = default_variant();
-    if ((rc = grow(&c->out, &c->out_bytes, (size_t)band * n * 2 * sizeof(float)))) return rc;
+    if ((rc = grow_out(c, (size_t)band * n * 2 * sizeof(float)))) return rc;
     float* dtab = nullptr;
-    if ((rc = upload_table(c, ref, rnd, &dtab))) return rc;
-    int64_t *d_i = nullptr, *d_j = nullptr;
-    float* d_d = nullptr;
-    void* heap_ws = nullptr;  // row heaps above the LDS limit
-    const size_t hw = ppsk::knn_heap_workspace(band, kNN);
-    hipError_t e = hipMalloc(&d_i, (size_t)band * kNN * sizeof(int64_t));
-    if (e == hipSuccess) e = hipMalloc(&d_j, (size_t)band * kNN * sizeof(int64_t));
-    if (e == hipSuccess) e = hipMalloc(&d_d, (size_t)band * kNN * sizeof(float));
-    if (e == hipSuccess && hw) e = hipMalloc(&heap_ws, hw);
-    if (e != hipSuccess) rc = fail(PPSK_ERR_MEMORY, "kNN output buffers");
-    if (rc == PPSK_OK) rc = reset_fail(c);
+    if ((rc = call_table(c, ref, rnd, &dtab))) return rc;
+    KnnLists L;
+    if ((rc = knn_lists(c, band, kNN, &L))) return rc;
     for (int64_t r0 = 0; r0 < n && rc == PPSK_OK; r0 += band) {
       const int64_t r1 = std::min(n, r0 + band);
       ppsk::DistParams p;
@@ -1414,24 +1567,17 @@ int ppsk_knn(ppsk_set* ref, int32_t random_mode, int32_t n_clusters, const float
       rc = run_dense(c, p, variant, false, r0, r1, true, sizeof(float2), nullptr, &tm);
       if (rc == PPSK_OK) rc = cancel_status(c->device);
       if (rc) break;
-      e = ppsk::launch_knn_select((const float*)c->out, r0, r1 - r0, n, dist_col, kNN, d_i, d_j,
-                                  d_d, c->stream, heap_ws);
-      const size_t m = (size_t)(r1 - r0) * kNN;
-      if (e == hipSuccess)
-        e = hipMemcpyAsync(i_vec + r0 * kNN, d_i, m * sizeof(int64_t), hipMemcpyDeviceToHost, c->stream);
-      if (e == hipSuccess)
-        e = hipMemcpyAsync(j_vec + r0 * kNN, d_j, m * sizeof(int64_t), hipMemcpyDeviceToHost, c->stream);
-      if (e == hipSuccess)
-        e = hipMemcpyAsync(dists + r0 * kNN, d_d, m * sizeof(float), hipMemcpyDeviceToHost, c->stream);
-      if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
+      hipError_t e = ppsk::launch_knn_select((const float*)c->out, r0, r1 - r0, n, dist_col, kNN,
+                                             L.i, L.j, L.d, c->stream, L.heap);
+      if (e == hipSuccess) {
+        e = copy_knn(c, L, (size_t)(r1 - r0) * kNN, i_vec + r0 * kNN, j_vec + r0 * kNN,
+                     dists + r0 * kNN);
+      }
       if (e != hipSuccess) rc = fail(PPSK_ERR_HIP, std::string("kNN select: ") + hipGetErrorString(e));
     }
     hipStreamSynchronize(c->stream);  // nothing queued may outlive its buffers
-    if (dtab) hipFree(dtab);
-    if (d_i) hipFree(d_i);
-    if (d_j) hipFree(d_j);
-    if (d_d) hipFree(d_d);
-    if (heap_ws) hipFree(heap_ws);
+    trim(&c->table, &c->table_bytes);
+    trim(&c->sel, &c->sel_bytes);
     if (rc == PPSK_OK) rc = read_fail(c, &nf, &ff);
   }
   set_timing(tm);
@@ -1468,7 +1614,7 @@ int ppsk_threshold(ppsk_set* ref, int32_t random_mode, int32_t n_clusters, const
   const int64_t n = ref->n;
   CallScope scope(c, dense_items(ref, ref, true, 0, n, false));
   const size_t tri_bytes = std::max<size_t>((size_t)n * (n - 1) / 2 * sizeof(float2), 8);
-  if (int rc = grow(&c->out, &c->out_bytes, tri_bytes)) return rc;
+  if (int rc = grow_out(c, tri_bytes)) return rc;
   Timing tm;
   unsigned long long nf = 0, ff = 0;
   int rc = PPSK_OK;
@@ -1515,7 +1661,7 @@ int ppsk_self_pass(ppsk_set* ref, int32_t random_mode, int32_t n_clusters, const
   const int64_t n = ref->n;
   CallScope scope(c, dense_items(ref, ref, true, 0, n, dense_out != nullptr));
   const size_t tri_bytes = std::max<size_t>((size_t)n * (n - 1) / 2 * sizeof(float2), 8);
-  if (int rc = grow(&c->out, &c->out_bytes, tri_bytes)) return rc;
+  if (int rc = grow_out(c, tri_bytes)) return rc;
   Timing tm;
   unsigned long long nf = 0, ff = 0;
   int rc = PPSK_OK;
@@ -1582,7 +1728,7 @@ int ppsk_host_free(void* ptr) {
 int ppsk_device_alloc(int device_id, size_t bytes, void** ptr) {
   DeviceCtx* c = nullptr;
   if (int rc = get_ctx(device_id, &c)) return rc;
-  HIP_TRY(hipMalloc(ptr, bytes));
+  HIP_TRY(device_malloc_all(c, ptr, bytes, false));
   return PPSK_OK;
 }
 

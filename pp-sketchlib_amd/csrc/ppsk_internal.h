@@ -230,6 +230,9 @@ hipError_t launch_batch(const BatchArgs& a, int variant, int grid, hipStream_t s
 // when step is 0.
 hipError_t launch_band_setup(ItemTile* tiles, int64_t rows, int64_t n_ct, int64_t step,
                              unsigned long long* fail, uint32_t* fail_rows, hipStream_t stream);
+// Start of a call: fit failures {0, none} and a progress count of 0.
+hipError_t launch_call_reset(unsigned long long* fail, unsigned long long* progress,
+                             hipStream_t stream);
 hipError_t launch_batch_reset(uint32_t* queue_next, unsigned long long* fail, int n_jobs,
                               hipStream_t stream, unsigned long long* progress = nullptr);
 // Zeroes n tile completion counters and sets fail ([2]: count, first row; may

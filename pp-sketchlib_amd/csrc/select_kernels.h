@@ -62,10 +62,4 @@ hipError_t launch_threshold_write(const float2* dd, int64_t rows, int64_t n, boo
 // (device memory of rows + 1 entries; one workgroup).
 hipError_t launch_offsets_scan(int64_t* counts, int64_t rows, hipStream_t stream);
 
-// dd: condensed float2 (core, acc) of the self upper triangle of n samples.
-// Allocates the device outputs (*d_i, *d_j, *d_d; caller frees with hipFree).
-hipError_t threshold_compact(const float2* dd, int64_t n, int dist_col, float cutoff,
-                             int64_t* total, int64_t** d_i, int64_t** d_j, float** d_d,
-                             hipStream_t stream);
-
 }  // namespace ppsk

@@ -22,7 +22,6 @@
 
 #include <cmath>
 #include <cstdint>
-#include <vector>
 
 #include "select_kernels.h"
 
@@ -521,48 +520,6 @@ hipError_t launch_offsets_scan(int64_t* counts, int64_t rows, hipStream_t stream
   if (rows < 0) return hipErrorInvalidValue;
   offsets_scan_kernel<<<1, TB, 0, stream>>>(counts, rows);
   return hipGetLastError();
-}
-
-hipError_t threshold_compact(const float2* dd, int64_t n, int dist_col, float cutoff,
-                             int64_t* total, int64_t** d_i, int64_t** d_j, float** d_d,
-                             hipStream_t stream) {
-  *total = 0;
-  *d_i = nullptr;
-  *d_j = nullptr;
-  *d_d = nullptr;
-  const int64_t rows = n > 1 ? n - 1 : 0;
-  if (rows == 0) return hipSuccess;
-  int64_t* counts = nullptr;
-  hipError_t e = hipMalloc(&counts, rows * sizeof(int64_t));
-  if (e != hipSuccess) return e;
-  e = launch_threshold_count(dd, rows, n, false, dist_col, cutoff, counts, stream);
-  std::vector<int64_t> h(rows);
-  if (e == hipSuccess) e = hipMemcpyAsync(h.data(), counts, rows * sizeof(int64_t),
-                                          hipMemcpyDeviceToHost, stream);
-  if (e == hipSuccess) e = hipStreamSynchronize(stream);
-  if (e != hipSuccess) {
-    hipFree(counts);
-    return e;
-  }
-  int64_t run = 0;
-  for (int64_t r = 0; r < rows; ++r) {
-    const int64_t c = h[r];
-    h[r] = run;
-    run += c;
-  }
-  *total = run;
-  e = hipMemcpyAsync(counts, h.data(), rows * sizeof(int64_t), hipMemcpyHostToDevice, stream);
-  const size_t m = (size_t)(run > 0 ? run : 1);
-  if (e == hipSuccess) e = hipMalloc(d_i, m * sizeof(int64_t));
-  if (e == hipSuccess) e = hipMalloc(d_j, m * sizeof(int64_t));
-  if (e == hipSuccess) e = hipMalloc(d_d, m * sizeof(float));
-  if (e == hipSuccess && run > 0) {
-    e = launch_threshold_write(dd, rows, n, false, dist_col, cutoff, counts, *d_i, *d_j, *d_d,
-                               stream);
-  }
-  if (e == hipSuccess) e = hipStreamSynchronize(stream);
-  hipFree(counts);
-  return e;
 }
 
 }  // namespace ppsk

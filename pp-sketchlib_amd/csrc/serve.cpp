@@ -118,7 +118,10 @@ struct ThrPart {
 struct ppsk_request {
   int64_t ticket = 0;
   int64_t n_q = 0;
-  std::vector<uint64_t> raw;  // [n_q][n_k][s64 * 14]
+  // the queries' sketches [n_q][n_k][s64 * 14], equal-base terms [n_q][n_k] and
+  // cluster ids [n_q] in the server's query memory (bytes > 0), or in raw, jv, cl
+  size_t at = 0, bytes = 0, at_jv = 0, at_cl = 0;
+  std::vector<uint64_t> raw;
   std::vector<double> jv;     // [n_q][n_k] equal-base terms
   std::vector<uint16_t> cl;   // [n_q] Monte Carlo cluster ids
   ppsk_result res;            // public view of the vectors below
@@ -152,6 +155,15 @@ struct ppsk_server {
   bool split = true;      // no tile shape or kernel forced
   Arena arena;
   void* arena_mem = nullptr;
+  // Memory of submitted queries, filled by ppsk_server_submit from the caller's
+  // arrays, so that a step reads them where they are: kept on the host until
+  // their step, 237 queries (41 MB) in four requests cost 6 ms of page faults,
+  // copies and stopped queues (freeing memory that a pageable copy locked) of
+  // a 10 ms burst.  4 x max_rows queries, at most 256 MiB; a request that finds
+  // no room there waits on the host.
+  Arena queries;
+  void* queries_mem = nullptr;
+  hipStream_t upload = nullptr;
   std::mutex mu;
   std::condition_variable cv_work, cv_done;
   std::deque<ppsk_request*> pending;
@@ -346,19 +358,27 @@ int run_step(ppsk_server* s, Worker& w, std::vector<Piece>& batch, int64_t rows,
   int64_t o = 0;
   for (const Piece& pc : batch) {
     const ppsk_request* r = pc.r;
-    STEP_TRY(hipMemcpyAsync(staging + (size_t)o * words, r->raw.data() + (size_t)pc.q0 * words,
-                            (size_t)pc.n * s->per_sample, hipMemcpyHostToDevice, w.st));
-    if (!r->jv.empty()) {
-      STEP_TRY(hipMemcpyAsync(jv + (size_t)o * n_k, r->jv.data() + (size_t)pc.q0 * n_k,
-                              (size_t)pc.n * n_k * sizeof(double), hipMemcpyHostToDevice, w.st));
+    const bool resident = r->bytes > 0;
+    const hipMemcpyKind kind = resident ? hipMemcpyDeviceToDevice : hipMemcpyHostToDevice;
+    const char* base = (const char*)s->queries_mem + r->at;
+    const uint64_t* raw = (const uint64_t*)base + (size_t)pc.q0 * words;
+    if (!resident) {
+      STEP_TRY(hipMemcpyAsync(staging + (size_t)o * words, r->raw.data() + (size_t)pc.q0 * words,
+                              (size_t)pc.n * s->per_sample, kind, w.st));
+      raw = staging + (size_t)o * words;
     }
-    if (!r->cl.empty()) {
-      STEP_TRY(hipMemcpyAsync(qcl + o, r->cl.data() + pc.q0, (size_t)pc.n * sizeof(uint16_t),
-                              hipMemcpyHostToDevice, w.st));
+    if (s->random_mode == PPSK_RANDOM_EQUAL_BASE) {
+      const double* from = resident ? (const double*)(base + r->at_jv) : r->jv.data();
+      STEP_TRY(hipMemcpyAsync(jv + (size_t)o * n_k, from + (size_t)pc.q0 * n_k,
+                              (size_t)pc.n * n_k * sizeof(double), kind, w.st));
     }
+    if (s->random_mode == PPSK_RANDOM_MC) {
+      const uint16_t* from = resident ? (const uint16_t*)(base + r->at_cl) : r->cl.data();
+      STEP_TRY(hipMemcpyAsync(qcl + o, from + pc.q0, (size_t)pc.n * sizeof(uint16_t), kind, w.st));
+    }
+    STEP_TRY(ppsk::launch_stripe(raw, pc.n, o, n_k, ref->s64, (int32_t)L.nbq, stripes, w.st));
     o += pc.n;
   }
-  STEP_TRY(ppsk::launch_stripe(staging, rows, 0, n_k, ref->s64, (int32_t)L.nbq, stripes, w.st));
   // per-tile completion counters of the per-(tile, k) kernel (the queue
   // counters of a persistent step are reset by launch_batch_reset)
   if (!L.persistent && !L.items) {
@@ -571,6 +591,44 @@ int run_step(ppsk_server* s, Worker& w, std::vector<Piece>& batch, int64_t rows,
   return PPSK_OK;
 }
 
+// The queries of a new request into the server's query memory; without room
+// there, into the request.
+int take_queries(ppsk_server* s, ppsk_request* r, const uint64_t* raw) {
+  const size_t raw_bytes = (size_t)r->n_q * s->per_sample;
+  const size_t jv_bytes = r->jv.size() * sizeof(double), cl_bytes = r->cl.size() * sizeof(uint16_t);
+  DeviceCtx* c = nullptr;
+  if (s->queries_mem && s->upload) {
+    const size_t at_jv = align_up(raw_bytes), at_cl = at_jv + align_up(jv_bytes);
+    const size_t bytes = at_cl + align_up(cl_bytes);
+    std::lock_guard<std::mutex> lk(s->mu);
+    if (s->queries.alloc(bytes, &r->at)) {
+      r->bytes = bytes;
+      r->at_jv = at_jv;
+      r->at_cl = at_cl;
+    }
+  }
+  if (!r->bytes) {
+    r->raw.assign(raw, raw + raw_bytes / sizeof(uint64_t));
+    return PPSK_OK;
+  }
+  char* to = (char*)s->queries_mem + r->at;
+  int rc = get_ctx(s->device, &c);
+  if (rc == PPSK_OK) {
+    hipError_t e = copy_to_device(c, to, raw, raw_bytes, s->upload);
+    if (e == hipSuccess) e = copy_to_device(c, to + r->at_jv, r->jv.data(), jv_bytes, s->upload);
+    if (e == hipSuccess) e = copy_to_device(c, to + r->at_cl, r->cl.data(), cl_bytes, s->upload);
+    const hipError_t es = hipStreamSynchronize(s->upload);
+    if (e == hipSuccess) e = es;
+    if (e != hipSuccess) rc = fail(PPSK_ERR_HIP, std::string("query upload: ") + hipGetErrorString(e));
+  }
+  if (rc != PPSK_OK) {
+    std::lock_guard<std::mutex> lk(s->mu);
+    s->queries.release(r->at, r->bytes);
+    r->bytes = 0;
+  }
+  return rc;
+}
+
 // Rows of the next piece of the oldest request in a step of its own.
 int64_t head_piece_rows(const ppsk_server* s) {
   const ppsk_request* r = s->pending.front();
@@ -740,6 +798,7 @@ void worker_main(ppsk_server* s, Worker* w) {
         }
         r->rows_done += pc.n;
         if (r->rows_done == r->n_q) {
+          if (r->bytes) s->queries.release(r->at, r->bytes);
           finish_request(r, t);
           s->requests_done += 1;
         }
@@ -835,7 +894,7 @@ int ppsk_server_create(ppsk_set* ref, int32_t random_mode, int32_t n_clusters,
       return fail(PPSK_ERR_MEMORY, std::string("serving Monte Carlo table: ") + hipGetErrorString(et));
     }
   }
-  hipError_t e = hipMalloc(&s->arena_mem, arena_bytes);
+  hipError_t e = device_malloc_all(c, &s->arena_mem, arena_bytes, false);
   if (e != hipSuccess) {
     if (s->d_table) hipFree(s->d_table);
     delete s;
@@ -843,11 +902,23 @@ int ppsk_server_create(ppsk_set* ref, int32_t random_mode, int32_t n_clusters,
   }
   s->arena.init((char*)s->arena_mem, arena_bytes);
   s->t0 = std::chrono::steady_clock::now();
+  const size_t query_bytes =
+      align_up(std::min<size_t>((size_t)256 << 20, 4 * (size_t)max_rows * (s->per_sample + 16 * ref->n_k)));
+  if (hipMalloc(&s->queries_mem, query_bytes) == hipSuccess) {
+    s->queries.init((char*)s->queries_mem, query_bytes);
+  } else {
+    (void)hipGetLastError();  // every request waits on the host
+    s->queries_mem = nullptr;
+  }
   std::vector<hipStream_t> streams;
   if (create_slot_streams(n_slots, &streams) != PPSK_OK) {
     for (hipStream_t st : streams) hipStreamDestroy(st);
     ppsk_server_free(s);
     return fail(PPSK_ERR_HIP, "serving stream creation");
+  }
+  if (hipStreamCreateWithFlags(&s->upload, hipStreamNonBlocking) != hipSuccess) {
+    (void)hipGetLastError();
+    s->upload = nullptr;
   }
   for (int i = 0; i < n_slots; ++i) {
     auto* w = new Worker();
@@ -883,7 +954,6 @@ int ppsk_server_submit(ppsk_server* s, int64_t n_queries, const uint64_t* raw,
   const ppsk_set* ref = s->ref;
   auto* r = new ppsk_request();
   r->n_q = n_queries;
-  r->raw.assign(raw, raw + (size_t)n_queries * (s->per_sample / sizeof(uint64_t)));
   if (s->random_mode == PPSK_RANDOM_EQUAL_BASE) {
     if (!lengths) {
       delete r;
@@ -919,9 +989,14 @@ int ppsk_server_submit(ppsk_server* s, int64_t n_queries, const uint64_t* raw,
     r->kd.resize(nk);
   }
   std::memset(&r->res, 0, sizeof(r->res));
+  if (int rc = take_queries(s, r, raw)) {
+    delete r;
+    return rc;
+  }
   {
     std::lock_guard<std::mutex> lk(s->mu);
     if (s->stop) {
+      if (r->bytes) s->queries.release(r->at, r->bytes);
       delete r;
       return fail(PPSK_ERR_STATE, "server stopped");
     }
@@ -1016,6 +1091,8 @@ int ppsk_server_free(ppsk_server* s) {
   }
   hipSetDevice(s->device);
   if (s->arena_mem) hipFree(s->arena_mem);
+  if (s->queries_mem) hipFree(s->queries_mem);
+  if (s->upload) hipStreamDestroy(s->upload);
   if (s->d_table) hipFree(s->d_table);
   delete s;
   return PPSK_OK;

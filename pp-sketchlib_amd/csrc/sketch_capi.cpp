@@ -17,10 +17,13 @@ namespace {
 constexpr int64_t UNIT = 1024;          // most k-mer start positions per lane
 constexpr int64_t GROUP_UNITS = 1024;   // most units per workgroup task
 
-struct DevBuf {
-  void* p = nullptr;
-  ~DevBuf() {
-    if (p) hipFree(p);
+// Consecutive parts of the call's buffer, each at a multiple of 256 bytes.
+struct Parts {
+  size_t used = 0;
+  size_t take(size_t bytes) {
+    const size_t at = used;
+    used += (std::max<size_t>(bytes, 1) + 255) / 256 * 256;
+    return at;
   }
 };
 
@@ -78,15 +81,17 @@ int64_t unit_windows(const int64_t* contig_off, const int64_t* sample_contig, in
   return hi;
 }
 
+// contigs: the contigs of contig_off wherever they lie, or null: one after the
+// other in seq.
 int sketch_impl(int device_id, int64_t n_samples, const char* seq, int64_t seq_bytes,
-                const int64_t* contig_off, int64_t n_contigs, const int64_t* sample_contig,
+                const char* const* contigs, const int64_t* contig_off, int64_t n_contigs, const int64_t* sample_contig,
                 int32_t n_k, const int32_t* klist, int32_t sketchsize64, int32_t use_rc,
                 int32_t codon, int32_t min_count, int32_t exact, uint64_t* raw_out,
                 double* inv_minhash, int32_t* densified) {
   if (n_samples < 1 || !sample_contig || !raw_out) {
     return fail(PPSK_ERR_ARG, "sketching needs at least one sample and an output buffer");
   }
-  if (n_contigs < 0 || (n_contigs > 0 && (!contig_off || !seq))) {
+  if (n_contigs < 0 || (n_contigs > 0 && (!contig_off || (!seq && !contigs)))) {
     return fail(PPSK_ERR_ARG, "contig offsets / sequence missing");
   }
   if (n_k < 1 || n_k > ppsk::MAXK || !klist) {
@@ -156,9 +161,9 @@ int sketch_impl(int device_id, int64_t n_samples, const char* seq, int64_t seq_b
   std::vector<ppsk::SketchGroup> groups;
   bool lds_bins = false;
   if (!filtered) {
-    hipDeviceProp_t prop;
-    HIP_TRY(hipGetDeviceProperties(&prop, device_id));
-    lds_bins = (size_t)nbins * sizeof(uint64_t) + 512 <= prop.sharedMemPerBlock;
+    int lds = 0;
+    HIP_TRY(hipDeviceGetAttribute(&lds, hipDeviceAttributeMaxSharedMemoryPerBlock, device_id));
+    lds_bins = (size_t)nbins * sizeof(uint64_t) + 512 <= (size_t)lds;
     int slots = 0;
     HIP_TRY(ppsk::sketch_hash_slots(a, lds_bins, &slots));
     std::vector<int64_t> spans;
@@ -178,41 +183,77 @@ int sketch_impl(int device_id, int64_t n_samples, const char* seq, int64_t seq_b
     }
   }
 
-  DevBuf d_seq, d_units, d_groups, d_k, d_signs, d_raw, d_mh, d_dens, d_next;
+  // a read set's unit lists of several jobs (one sample, one k) are uploaded at
+  // once: as many jobs as keep the lists within 64 MiB
+  int64_t max_w = 0, max_u = 0;
+  const size_t unit_bytes = sizeof(ppsk::SketchUnit) + sizeof(int64_t);
+  size_t list_units = 0, ws_bytes = 0;
+  if (filtered) {
+    for (int64_t s = 0; s < n_samples; ++s) {
+      // the smallest k has the most windows: every later job fits max_w / max_u
+      int64_t w = 0, u = 0;
+      for (int64_t ci = sample_contig[s]; ci < sample_contig[s + 1]; ++ci) {
+        const int64_t n = contig_off[ci + 1] - contig_off[ci] - span(klist[0]) + 1;
+        if (n <= 0) continue;
+        w += n;
+        u += (n + UNIT - 1) / UNIT;
+      }
+      max_w = std::max(max_w, w);
+      max_u = std::max(max_u, u);
+    }
+    list_units = std::max<size_t>((size_t)max_u, ((size_t)64 << 20) / unit_bytes);
+    list_units = std::min<size_t>(list_units, (size_t)max_u * n_k * n_samples);
+    ws_bytes = ppsk::reads_workspace_bytes(max_w);
+  }
+
+  // one buffer for the call, kept with the context up to 1 GiB
   const size_t raw_words = (size_t)n_samples * n_k * sketchsize64 * ppsk::BBITS_SK;
+  Parts parts;
+  const size_t stats = (size_t)n_samples * n_k;
   // base codes, padded both sides for the kernel's stream loads
-  hipError_t e =
-      hipMalloc(&d_seq.p, (size_t)(ppsk::CODE_PAD_FRONT + seq_bytes + ppsk::CODE_PAD_BACK));
-  if (e == hipSuccess) e = hipMalloc(&d_units.p, std::max<size_t>(units.size(), 1) * sizeof(ppsk::SketchUnit));
-  if (e == hipSuccess) e = hipMalloc(&d_groups.p, std::max<size_t>(groups.size(), 1) * sizeof(ppsk::SketchGroup));
-  if (e == hipSuccess) e = hipMalloc(&d_k.p, n_k * sizeof(int32_t));
-  if (e == hipSuccess) e = hipMalloc(&d_signs.p, (size_t)n_samples * n_k * nbins * sizeof(uint64_t));
-  if (e == hipSuccess) e = hipMalloc(&d_raw.p, raw_words * sizeof(uint64_t));
-  if (e == hipSuccess) e = hipMalloc(&d_mh.p, (size_t)n_samples * n_k * sizeof(double));
-  if (e == hipSuccess) e = hipMalloc(&d_dens.p, (size_t)n_samples * n_k * sizeof(int32_t));
-  if (e == hipSuccess) e = hipMalloc(&d_next.p, sizeof(int));
-  if (e != hipSuccess) {
-    return fail(PPSK_ERR_MEMORY, std::string("sketch buffers: ") + hipGetErrorString(e));
+  const size_t at_seq = parts.take((size_t)(ppsk::CODE_PAD_FRONT + seq_bytes + ppsk::CODE_PAD_BACK));
+  const size_t at_units = parts.take(units.size() * sizeof(ppsk::SketchUnit));
+  const size_t at_groups = parts.take(groups.size() * sizeof(ppsk::SketchGroup));
+  const size_t at_k = parts.take(n_k * sizeof(int32_t));
+  const size_t at_signs = parts.take(stats * nbins * sizeof(uint64_t));
+  const size_t at_raw = parts.take(raw_words * sizeof(uint64_t));
+  const size_t at_stats = parts.take(stats * (sizeof(double) + sizeof(int32_t)));
+  const size_t at_next = parts.take(sizeof(int));
+  const size_t at_lists = parts.take(list_units * unit_bytes);
+  const size_t at_ws = parts.take(ws_bytes);
+  if (int rc = grow(&c->sketch, &c->sketch_bytes, parts.used)) return rc;
+  struct Trim {
+    DeviceCtx* c;
+    ~Trim() { trim(&c->sketch, &c->sketch_bytes); }
+  } trimmed{c};
+  char* mem = (char*)c->sketch;
+  uint8_t* codes = (uint8_t*)(mem + at_seq) + ppsk::CODE_PAD_FRONT;
+  if (contigs) {
+    HIP_TRY(fill_device(c, codes, (size_t)seq_bytes, c->stream, [&](char* to, size_t at, size_t n) {
+      int64_t ci = std::upper_bound(contig_off, contig_off + n_contigs + 1, (int64_t)at) - contig_off - 1;
+      for (size_t done = 0; done < n; ++ci) {
+        const size_t from = at + done - (size_t)contig_off[ci];
+        const size_t m = std::min(n - done, (size_t)(contig_off[ci + 1] - contig_off[ci]) - from);
+        std::memcpy(to + done, contigs[ci] + from, m);
+        done += m;
+      }
+    }));
+  } else {
+    HIP_TRY(copy_to_device(c, codes, seq, (size_t)seq_bytes, c->stream));
   }
-  uint8_t* codes = (uint8_t*)d_seq.p + ppsk::CODE_PAD_FRONT;
-  if (seq_bytes > 0) {
-    HIP_TRY(hipMemcpyAsync(codes, seq, seq_bytes, hipMemcpyHostToDevice, c->stream));
-  }
-  if (!units.empty()) {
-    HIP_TRY(hipMemcpyAsync(d_units.p, units.data(), units.size() * sizeof(ppsk::SketchUnit),
-                           hipMemcpyHostToDevice, c->stream));
-    HIP_TRY(hipMemcpyAsync(d_groups.p, groups.data(), groups.size() * sizeof(ppsk::SketchGroup),
-                           hipMemcpyHostToDevice, c->stream));
-  }
-  HIP_TRY(hipMemcpyAsync(d_k.p, klist, n_k * sizeof(int32_t), hipMemcpyHostToDevice, c->stream));
+  HIP_TRY(copy_to_device(c, mem + at_units, units.data(), units.size() * sizeof(ppsk::SketchUnit),
+                         c->stream));
+  HIP_TRY(copy_to_device(c, mem + at_groups, groups.data(),
+                         groups.size() * sizeof(ppsk::SketchGroup), c->stream));
+  HIP_TRY(copy_to_device(c, mem + at_k, klist, n_k * sizeof(int32_t), c->stream));
   a.codes = codes;
-  a.units = (const ppsk::SketchUnit*)d_units.p;
-  a.groups = (const ppsk::SketchGroup*)d_groups.p;
-  a.klist = (const int32_t*)d_k.p;
-  a.signs = (uint64_t*)d_signs.p;
-  a.raw = (uint64_t*)d_raw.p;
-  a.inv_minhash = (double*)d_mh.p;
-  a.densified = (int32_t*)d_dens.p;
+  a.units = (const ppsk::SketchUnit*)(mem + at_units);
+  a.groups = (const ppsk::SketchGroup*)(mem + at_groups);
+  a.klist = (const int32_t*)(mem + at_k);
+  a.signs = (uint64_t*)(mem + at_signs);
+  a.raw = (uint64_t*)(mem + at_raw);
+  a.inv_minhash = (double*)(mem + at_stats);
+  a.densified = (int32_t*)(a.inv_minhash + stats);
 
   hipEvent_t e0 = pool_event(c, 0), e1 = pool_event(c, 1);
   if (!e0 || !e1) return fail(PPSK_ERR_HIP, "event creation failed");
@@ -220,44 +261,32 @@ int sketch_impl(int device_id, int64_t n_samples, const char* seq, int64_t seq_b
   HIP_TRY(ppsk::launch_sketch_decode(codes, seq_bytes, c->stream));
   int64_t items = (int64_t)units.size();
   if (!filtered) {
-    HIP_TRY(ppsk::launch_sketch(a, (int64_t)groups.size(), lds_bins, (int*)d_next.p, c->stream));
+    HIP_TRY(ppsk::launch_sketch(a, (int64_t)groups.size(), lds_bins, (int*)(mem + at_next), c->stream));
   } else {
     // one (sample, k) at a time through the counting pipeline
     HIP_TRY(ppsk::launch_sketch_reset(a, c->stream));
-    int64_t max_w = 0, max_u = 0;
-    for (int64_t s = 0; s < n_samples; ++s) {
-      std::vector<ppsk::SketchUnit> u;
-      const int64_t w = sample_units(contig_off, sample_contig[s], sample_contig[s + 1],
-                                     span(klist[0]), UNIT, u, nullptr);
-      max_w = std::max(max_w, w);
-      max_u = std::max<int64_t>(max_u, (int64_t)u.size());
-    }
-    DevBuf d_ws, d_ju, d_jw;
-    const size_t ws_bytes = ppsk::reads_workspace_bytes(max_w);
-    e = hipMalloc(&d_ws.p, ws_bytes);
-    if (e == hipSuccess) e = hipMalloc(&d_ju.p, (size_t)std::max<int64_t>(max_u, 1) * sizeof(ppsk::SketchUnit));
-    if (e == hipSuccess) e = hipMalloc(&d_jw.p, (size_t)std::max<int64_t>(max_u, 1) * sizeof(int64_t));
-    if (e != hipSuccess) {
-      return fail(PPSK_ERR_MEMORY, std::string("read filter workspace: ") + hipGetErrorString(e));
-    }
+    ppsk::SketchUnit* d_ju = (ppsk::SketchUnit*)(mem + at_lists);
+    int64_t* d_jw = (int64_t*)(d_ju + list_units);
     std::vector<ppsk::SketchUnit> ju;
     std::vector<int64_t> jw;
+    size_t listed = 0;  // units of the lists in use
     for (int64_t s = 0; s < n_samples; ++s) {
       for (int kk = 0; kk < n_k; ++kk) {
         ju.clear();
         jw.clear();
-        // the smallest k has the most windows: every later job fits max_w / max_u
         const int64_t nw = sample_units(contig_off, sample_contig[s], sample_contig[s + 1],
                                         span(klist[kk]), UNIT, ju, &jw);
         if (nw == 0) continue;
-        HIP_TRY(hipMemcpyAsync(d_ju.p, ju.data(), ju.size() * sizeof(ppsk::SketchUnit),
-                               hipMemcpyHostToDevice, c->stream));
-        HIP_TRY(hipMemcpyAsync(d_jw.p, jw.data(), jw.size() * sizeof(int64_t),
-                               hipMemcpyHostToDevice, c->stream));
+        // the stream runs the jobs in order, so lists that start again behind
+        // the last ones are written after their jobs
+        if (listed + ju.size() > list_units) listed = 0;
+        HIP_TRY(copy_to_device(c, d_ju + listed, ju.data(), ju.size() * sizeof(ppsk::SketchUnit),
+                               c->stream));
+        HIP_TRY(copy_to_device(c, d_jw + listed, jw.data(), jw.size() * sizeof(int64_t), c->stream));
         ppsk::ReadsJob rj;
         rj.codes = codes;
-        rj.units = (const ppsk::SketchUnit*)d_ju.p;
-        rj.wbase = (const int64_t*)d_jw.p;
+        rj.units = d_ju + listed;
+        rj.wbase = d_jw + listed;
         rj.n_units = (int64_t)ju.size();
         rj.n_windows = nw;
         rj.k = klist[kk];
@@ -268,24 +297,20 @@ int sketch_impl(int device_id, int64_t n_samples, const char* seq, int64_t seq_b
         rj.binsize = a.binsize;
         rj.recip = (uint32_t)a.bin_recip;
         rj.bins = a.signs + (s * n_k + kk) * nbins;
-        HIP_TRY(ppsk::run_reads_job(rj, d_ws.p, ws_bytes, c->stream));
-        // the unit lists are rewritten by the next job
-        HIP_TRY(hipStreamSynchronize(c->stream));
+        rj.words = c->words;
+        HIP_TRY(ppsk::run_reads_job(rj, mem + at_ws, ws_bytes, c->stream));
+        listed += ju.size();
         items += (int64_t)ju.size();
       }
     }
     HIP_TRY(ppsk::launch_sketch_finish(a, c->stream));
   }
   HIP_TRY(hipEventRecord(e1, c->stream));
-  HIP_TRY(hipMemcpyAsync(raw_out, d_raw.p, raw_words * sizeof(uint64_t), hipMemcpyDeviceToHost,
-                         c->stream));
-  std::vector<double> mh((size_t)n_samples * n_k);
-  std::vector<int32_t> dn((size_t)n_samples * n_k);
-  HIP_TRY(hipMemcpyAsync(mh.data(), d_mh.p, mh.size() * sizeof(double), hipMemcpyDeviceToHost,
-                         c->stream));
-  HIP_TRY(hipMemcpyAsync(dn.data(), d_dens.p, dn.size() * sizeof(int32_t),
-                         hipMemcpyDeviceToHost, c->stream));
-  HIP_TRY(hipStreamSynchronize(c->stream));
+  HIP_TRY(copy_to_host(c, raw_out, a.raw, raw_words * sizeof(uint64_t), c->stream));
+  std::vector<char> st(stats * (sizeof(double) + sizeof(int32_t)));
+  HIP_TRY(copy_to_host(c, st.data(), a.inv_minhash, st.size(), c->stream));
+  const double* mh = (const double*)st.data();
+  const int32_t* dn = (const int32_t*)(mh + stats);
   float ms = 0.f;
   HIP_TRY(hipEventElapsedTime(&ms, e0, e1));
   g_last_ms = ms;
@@ -312,8 +337,9 @@ int ppsk_sketch(int device_id, int64_t n_samples, const char* seq, int64_t seq_b
                 const int64_t* contig_off, int64_t n_contigs, const int64_t* sample_contig,
                 int32_t n_k, const int32_t* klist, int32_t sketchsize64, int32_t use_rc,
                 uint64_t* raw_out, double* inv_minhash, int32_t* densified) {
-  return sketch_impl(device_id, n_samples, seq, seq_bytes, contig_off, n_contigs, sample_contig,
-                     n_k, klist, sketchsize64, use_rc, 0, 0, 0, raw_out, inv_minhash, densified);
+  return sketch_impl(device_id, n_samples, seq, seq_bytes, nullptr, contig_off, n_contigs,
+                     sample_contig, n_k, klist, sketchsize64, use_rc, 0, 0, 0, raw_out, inv_minhash,
+                     densified);
 }
 
 int ppsk_sketch_ex(int device_id, int64_t n_samples, const char* seq, int64_t seq_bytes,
@@ -321,9 +347,23 @@ int ppsk_sketch_ex(int device_id, int64_t n_samples, const char* seq, int64_t se
                    int32_t n_k, const int32_t* klist, int32_t sketchsize64, int32_t use_rc,
                    int32_t codon_phased, int32_t min_count, int32_t exact, uint64_t* raw_out,
                    double* inv_minhash, int32_t* densified) {
-  return sketch_impl(device_id, n_samples, seq, seq_bytes, contig_off, n_contigs, sample_contig,
-                     n_k, klist, sketchsize64, use_rc, codon_phased, min_count, exact, raw_out,
-                     inv_minhash, densified);
+  return sketch_impl(device_id, n_samples, seq, seq_bytes, nullptr, contig_off, n_contigs,
+                     sample_contig, n_k, klist, sketchsize64, use_rc, codon_phased, min_count, exact,
+                     raw_out, inv_minhash, densified);
+}
+
+int ppsk_sketch_contigs(int device_id, int64_t n_samples, const char* const* contigs,
+                        const int64_t* contig_off, int64_t n_contigs, const int64_t* sample_contig,
+                        int32_t n_k, const int32_t* klist, int32_t sketchsize64, int32_t use_rc,
+                        int32_t codon_phased, int32_t min_count, int32_t exact, uint64_t* raw_out,
+                        double* inv_minhash, int32_t* densified) {
+  if (n_contigs > 0 && (!contigs || !contig_off)) {
+    return fail(PPSK_ERR_ARG, "contig offsets / sequence missing");
+  }
+  if (n_contigs > 0 && contig_off[0] != 0) return fail(PPSK_ERR_ARG, "contig offsets must start at 0");
+  return sketch_impl(device_id, n_samples, nullptr, n_contigs > 0 ? contig_off[n_contigs] : 0, contigs,
+                     contig_off, n_contigs, sample_contig, n_k, klist, sketchsize64, use_rc,
+                     codon_phased, min_count, exact, raw_out, inv_minhash, densified);
 }
 
 }  // extern "C"

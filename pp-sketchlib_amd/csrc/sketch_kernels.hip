@@ -523,16 +523,15 @@ hipError_t run_reads_job(const ReadsJob& j, void* ws, size_t ws_bytes, hipStream
                                                         H1);
   if ((e = hipGetLastError()) != hipSuccess) return e;
   // occurrence count
-  int64_t last_t = 0;
-  uint8_t last_st = 0;
-  if ((e = hipMemcpyAsync(&last_t, tix + (W - 1), sizeof(int64_t), hipMemcpyDeviceToHost,
+  j.words[1] = 0;
+  if ((e = hipMemcpyAsync(j.words, tix + (W - 1), sizeof(int64_t), hipMemcpyDeviceToHost,
                           stream)) != hipSuccess ||
-      (e = hipMemcpyAsync(&last_st, st + (W - 1), 1, hipMemcpyDeviceToHost, stream)) !=
+      (e = hipMemcpyAsync(j.words + 1, st + (W - 1), 1, hipMemcpyDeviceToHost, stream)) !=
           hipSuccess ||
       (e = hipStreamSynchronize(stream)) != hipSuccess) {
     return e;
   }
-  const int64_t N = last_t + (last_st != 0 ? 1 : 0);
+  const int64_t N = (int64_t)j.words[0] + (j.words[1] != 0 ? 1 : 0);
   if (N == 0) return hipSuccess;
   int events;
   if (j.exact) {
