@@ -27,58 +27,19 @@ struct Parts {
   }
 };
 
-// Units of one sample's contigs for one k: runs of up to `unit` window starts,
-// pad = 1 on the first unit of a contig; wbase = index of the unit's first
-// window among the sample's windows (sequence order).  Returns the window
-// count.
-int64_t sample_units(const int64_t* contig_off, int64_t c0, int64_t c1, int64_t k, int64_t unit,
-                     std::vector<ppsk::SketchUnit>& units, std::vector<int64_t>* wbase) {
-  int64_t nw = 0;
-  for (int64_t ci = c0; ci < c1; ++ci) {
-    const int64_t windows = contig_off[ci + 1] - contig_off[ci] - k + 1;
-    for (int64_t w = 0; w < windows; w += unit) {
-      units.push_back({contig_off[ci] + w, (int32_t)std::min(unit, windows - w), w == 0 ? 1 : 0});
-      if (wbase) wbase->push_back(nw + w);
-    }
-    if (windows > 0) nw += windows;
-  }
-  return nw;
-}
-
 // Window starts per lane of a hashing launch over `slots` workgroups resident
-// at once.  Units of UNIT windows give the least rolling-in (k - 1 steps per
-// unit), but a launch that fits the slots in one round must spread over all of
-// them: the smallest unit of at least 64 windows whose groups (one unit per
-// lane) need no second round.  6 genomes of 2 Mb at 8 k-mer lengths: 96 groups
-// of 1,024-window units on 512 slots took 494 us, 480 groups of 416 take 248.
-int64_t unit_windows(const int64_t* contig_off, const int64_t* sample_contig, int64_t n_samples,
-                     const std::vector<int64_t>& spans, int64_t slots) {
-  auto groups = [&](int64_t unit) {
-    int64_t g = 0;
-    for (int64_t s = 0; s < n_samples; ++s) {
-      for (int64_t span : spans) {
-        int64_t u = 0;
-        for (int64_t c = sample_contig[s]; c < sample_contig[s + 1]; ++c) {
-          const int64_t w = contig_off[c + 1] - contig_off[c] - span + 1;
-          if (w > 0) u += (w + unit - 1) / unit;
-        }
-        g += (u + ppsk::SKETCH_TB - 1) / ppsk::SKETCH_TB;
-      }
-    }
-    return g;
-  };
-  if (groups(UNIT) > slots) return UNIT;
-  int64_t lo = 64, hi = UNIT;  // groups(hi) <= slots
-  while (lo < hi) {
-    const int64_t mid = (lo + hi) / 2 / 16 * 16;
-    if (mid < lo) break;
-    if (groups(mid) <= slots) {
-      hi = mid;
-    } else {
-      lo = mid + 16;
-    }
-  }
-  return hi;
+// at once, for `windows` windows of `pieces` (contig, k) pairs in `jobs`
+// (sample, k) pairs.  Units of UNIT windows give the least rolling-in (k - 1
+// steps per unit), but a launch that fits the slots in one round must spread
+// over all of them: the smallest unit of at least 64 windows whose groups (one
+// unit per lane; at most windows / unit + pieces units, the last group of a job
+// partly filled) need no second round.  6 genomes of 2 Mb at 8 k-mer lengths: 96
+// groups of 1,024-window units on 512 slots took 494 us, 480 groups of 416 take
+// 207.
+int64_t unit_windows(int64_t windows, int64_t pieces, int64_t jobs, int64_t slots) {
+  const int64_t lanes = (slots - jobs) * ppsk::SKETCH_TB - pieces;
+  if (lanes <= 0 || windows > lanes * UNIT) return UNIT;
+  return std::min(UNIT, std::max<int64_t>(64, ((windows + lanes - 1) / lanes + 15) / 16 * 16));
 }
 
 // contigs: the contigs of contig_off wherever they lie, or null: one after the
@@ -153,58 +114,66 @@ int sketch_impl(int device_id, int64_t n_samples, const char* seq, int64_t seq_b
   a.bin_recip = ~0ULL / a.binsize;
   if (a.bin_recip >> 32) return fail(PPSK_ERR_ARG, "bin reciprocal out of range");
 
-  // unfiltered: units (per k, every contig cut into runs of windows) and groups
-  // (runs of units of one sample and one k) for one hashing launch; bin minima
-  // in LDS when one sample's bins fit a workgroup's LDS (the step table takes
-  // another 400 bytes)
-  std::vector<ppsk::SketchUnit> units;
-  std::vector<ppsk::SketchGroup> groups;
+  // Work units: every contig of every k cut into runs of windows; before_u and
+  // before_w count the units and windows of the (k, contig) pairs before each,
+  // k by k (index kk * n_contigs + contig).  The unit lists are written from
+  // them on the device (launch_sketch_units).
+  int64_t unit = UNIT;
   bool lds_bins = false;
+  std::vector<int64_t> spans;
+  for (int kk = 0; kk < n_k; ++kk) spans.push_back(span(klist[kk]));
   if (!filtered) {
+    // bin minima in LDS when one sample's bins fit a workgroup's LDS (the step
+    // table takes another 400 bytes)
     int lds = 0;
     HIP_TRY(hipDeviceGetAttribute(&lds, hipDeviceAttributeMaxSharedMemoryPerBlock, device_id));
     lds_bins = (size_t)nbins * sizeof(uint64_t) + 512 <= (size_t)lds;
     int slots = 0;
     HIP_TRY(ppsk::sketch_hash_slots(a, lds_bins, &slots));
-    std::vector<int64_t> spans;
-    for (int kk = 0; kk < n_k; ++kk) spans.push_back(span(klist[kk]));
-    const int64_t unit = unit_windows(contig_off, sample_contig, n_samples, spans, slots);
-    const int64_t per_group = unit < UNIT ? ppsk::SKETCH_TB : GROUP_UNITS;
+    const int64_t bases = n_contigs > 0 ? contig_off[n_contigs] - contig_off[0] : 0;
+    unit = unit_windows(bases * n_k, n_contigs * n_k, n_samples * n_k, slots);
+  }
+  const size_t pieces = (size_t)n_contigs * n_k;
+  std::vector<int64_t> before_u(pieces + 1), before_w(pieces + 1);
+  {
+    int64_t nu = 0, nw = 0;
+    size_t f = 0;
     for (int kk = 0; kk < n_k; ++kk) {
-      for (int64_t s = 0; s < n_samples; ++s) {
-        const int64_t u0 = (int64_t)units.size();
-        sample_units(contig_off, sample_contig[s], sample_contig[s + 1], spans[kk], unit, units,
-                     nullptr);
-        const int64_t u1 = (int64_t)units.size();
-        for (int64_t g = u0; g < u1; g += per_group) {
-          groups.push_back({g, std::min(u1, g + per_group), (int32_t)s, kk});
-        }
+      for (int64_t c0 = 0; c0 < n_contigs; ++c0, ++f) {
+        before_u[f] = nu;
+        before_w[f] = nw;
+        const int64_t w = contig_off[c0 + 1] - contig_off[c0] - spans[kk] + 1;
+        if (w <= 0) continue;
+        nw += w;
+        nu += w <= unit ? 1 : (w + unit - 1) / unit;
       }
     }
+    before_u[f] = nu;
+    before_w[f] = nw;
   }
-
-  // a read set's unit lists of several jobs (one sample, one k) are uploaded at
-  // once: as many jobs as keep the lists within 64 MiB
-  int64_t max_w = 0, max_u = 0;
-  const size_t unit_bytes = sizeof(ppsk::SketchUnit) + sizeof(int64_t);
-  size_t list_units = 0, ws_bytes = 0;
-  if (filtered) {
+  // unfiltered: groups (runs of units of one sample and one k) of one hashing
+  // launch; filtered: the units and windows of the largest (sample, k)
+  std::vector<ppsk::SketchGroup> groups;
+  int64_t list_units = 0, max_w = 0;
+  const int64_t per_group = unit < UNIT ? ppsk::SKETCH_TB : GROUP_UNITS;
+  for (int kk = 0; kk < n_k; ++kk) {
     for (int64_t s = 0; s < n_samples; ++s) {
-      // the smallest k has the most windows: every later job fits max_w / max_u
-      int64_t w = 0, u = 0;
-      for (int64_t ci = sample_contig[s]; ci < sample_contig[s + 1]; ++ci) {
-        const int64_t n = contig_off[ci + 1] - contig_off[ci] - span(klist[0]) + 1;
-        if (n <= 0) continue;
-        w += n;
-        u += (n + UNIT - 1) / UNIT;
+      const size_t lo = (size_t)kk * n_contigs + sample_contig[s];
+      const size_t hi = (size_t)kk * n_contigs + sample_contig[s + 1];
+      const int64_t u0 = before_u[lo], u1 = before_u[hi];
+      if (filtered) {
+        list_units = std::max(list_units, u1 - u0);
+        max_w = std::max(max_w, before_w[hi] - before_w[lo]);
+        continue;
       }
-      max_w = std::max(max_w, w);
-      max_u = std::max(max_u, u);
+      for (int64_t g = u0; g < u1; g += per_group) {
+        groups.push_back({g, std::min(u1, g + per_group), (int32_t)s, kk});
+      }
     }
-    list_units = std::max<size_t>((size_t)max_u, ((size_t)64 << 20) / unit_bytes);
-    list_units = std::min<size_t>(list_units, (size_t)max_u * n_k * n_samples);
-    ws_bytes = ppsk::reads_workspace_bytes(max_w);
   }
+  const int64_t total_units = before_u[pieces];
+  if (!filtered) list_units = total_units;
+  const size_t ws_bytes = filtered ? ppsk::reads_workspace_bytes(max_w) : 0;
 
   // one buffer for the call, kept with the context up to 1 GiB
   const size_t raw_words = (size_t)n_samples * n_k * sketchsize64 * ppsk::BBITS_SK;
@@ -212,14 +181,17 @@ int sketch_impl(int device_id, int64_t n_samples, const char* seq, int64_t seq_b
   const size_t stats = (size_t)n_samples * n_k;
   // base codes, padded both sides for the kernel's stream loads
   const size_t at_seq = parts.take((size_t)(ppsk::CODE_PAD_FRONT + seq_bytes + ppsk::CODE_PAD_BACK));
-  const size_t at_units = parts.take(units.size() * sizeof(ppsk::SketchUnit));
+  const size_t at_units = parts.take((size_t)list_units * sizeof(ppsk::SketchUnit));
+  const size_t at_wbase = parts.take(filtered ? (size_t)list_units * sizeof(int64_t) : 0);
+  // contig offsets, spans, before_u, before_w
+  const size_t index_words = (size_t)n_contigs + 1 + n_k + (pieces + 1) * (filtered ? 2 : 1);
+  const size_t at_index = parts.take(index_words * sizeof(int64_t));
   const size_t at_groups = parts.take(groups.size() * sizeof(ppsk::SketchGroup));
   const size_t at_k = parts.take(n_k * sizeof(int32_t));
   const size_t at_signs = parts.take(stats * nbins * sizeof(uint64_t));
   const size_t at_raw = parts.take(raw_words * sizeof(uint64_t));
   const size_t at_stats = parts.take(stats * (sizeof(double) + sizeof(int32_t)));
   const size_t at_next = parts.take(sizeof(int));
-  const size_t at_lists = parts.take(list_units * unit_bytes);
   const size_t at_ws = parts.take(ws_bytes);
   if (int rc = grow(&c->sketch, &c->sketch_bytes, parts.used)) return rc;
   struct Trim {
@@ -241,8 +213,21 @@ int sketch_impl(int device_id, int64_t n_samples, const char* seq, int64_t seq_b
   } else {
     HIP_TRY(copy_to_device(c, codes, seq, (size_t)seq_bytes, c->stream));
   }
-  HIP_TRY(copy_to_device(c, mem + at_units, units.data(), units.size() * sizeof(ppsk::SketchUnit),
-                         c->stream));
+  ppsk::UnitIndex ix;
+  ix.contig_off = (const int64_t*)(mem + at_index);
+  ix.spans = ix.contig_off + n_contigs + 1;
+  ix.before_u = ix.spans + n_k;
+  ix.before_w = filtered ? ix.before_u + pieces + 1 : nullptr;
+  ix.n_contigs = n_contigs;
+  ix.unit = unit;
+  if (n_contigs > 0) {
+    HIP_TRY(copy_to_device(c, (void*)ix.contig_off, contig_off, (n_contigs + 1) * sizeof(int64_t), c->stream));
+  }
+  HIP_TRY(copy_to_device(c, (void*)ix.spans, spans.data(), n_k * sizeof(int64_t), c->stream));
+  HIP_TRY(copy_to_device(c, (void*)ix.before_u, before_u.data(), (pieces + 1) * sizeof(int64_t), c->stream));
+  if (filtered) {
+    HIP_TRY(copy_to_device(c, (void*)ix.before_w, before_w.data(), (pieces + 1) * sizeof(int64_t), c->stream));
+  }
   HIP_TRY(copy_to_device(c, mem + at_groups, groups.data(),
                          groups.size() * sizeof(ppsk::SketchGroup), c->stream));
   HIP_TRY(copy_to_device(c, mem + at_k, klist, n_k * sizeof(int32_t), c->stream));
@@ -259,35 +244,27 @@ int sketch_impl(int device_id, int64_t n_samples, const char* seq, int64_t seq_b
   if (!e0 || !e1) return fail(PPSK_ERR_HIP, "event creation failed");
   HIP_TRY(hipEventRecord(e0, c->stream));
   HIP_TRY(ppsk::launch_sketch_decode(codes, seq_bytes, c->stream));
-  int64_t items = (int64_t)units.size();
+  int64_t items = 0;
+  ppsk::SketchUnit* d_units = (ppsk::SketchUnit*)(mem + at_units);
+  int64_t* d_wbase = (int64_t*)(mem + at_wbase);
   if (!filtered) {
+    items = total_units;
+    HIP_TRY(ppsk::launch_sketch_units(ix, 0, (int64_t)pieces, total_units, d_units, nullptr, c->stream));
     HIP_TRY(ppsk::launch_sketch(a, (int64_t)groups.size(), lds_bins, (int*)(mem + at_next), c->stream));
   } else {
     // one (sample, k) at a time through the counting pipeline
     HIP_TRY(ppsk::launch_sketch_reset(a, c->stream));
-    ppsk::SketchUnit* d_ju = (ppsk::SketchUnit*)(mem + at_lists);
-    int64_t* d_jw = (int64_t*)(d_ju + list_units);
-    std::vector<ppsk::SketchUnit> ju;
-    std::vector<int64_t> jw;
-    size_t listed = 0;  // units of the lists in use
     for (int64_t s = 0; s < n_samples; ++s) {
       for (int kk = 0; kk < n_k; ++kk) {
-        ju.clear();
-        jw.clear();
-        const int64_t nw = sample_units(contig_off, sample_contig[s], sample_contig[s + 1],
-                                        span(klist[kk]), UNIT, ju, &jw);
+        const int64_t lo = kk * n_contigs + sample_contig[s], hi = kk * n_contigs + sample_contig[s + 1];
+        const int64_t nu = before_u[hi] - before_u[lo], nw = before_w[hi] - before_w[lo];
         if (nw == 0) continue;
-        // the stream runs the jobs in order, so lists that start again behind
-        // the last ones are written after their jobs
-        if (listed + ju.size() > list_units) listed = 0;
-        HIP_TRY(copy_to_device(c, d_ju + listed, ju.data(), ju.size() * sizeof(ppsk::SketchUnit),
-                               c->stream));
-        HIP_TRY(copy_to_device(c, d_jw + listed, jw.data(), jw.size() * sizeof(int64_t), c->stream));
+        HIP_TRY(ppsk::launch_sketch_units(ix, lo, hi, nu, d_units, d_wbase, c->stream));
         ppsk::ReadsJob rj;
         rj.codes = codes;
-        rj.units = d_ju + listed;
-        rj.wbase = d_jw + listed;
-        rj.n_units = (int64_t)ju.size();
+        rj.units = d_units;
+        rj.wbase = d_wbase;
+        rj.n_units = nu;
         rj.n_windows = nw;
         rj.k = klist[kk];
         rj.use_rc = use_rc ? 1 : 0;
@@ -299,8 +276,7 @@ int sketch_impl(int device_id, int64_t n_samples, const char* seq, int64_t seq_b
         rj.bins = a.signs + (s * n_k + kk) * nbins;
         rj.words = c->words;
         HIP_TRY(ppsk::run_reads_job(rj, mem + at_ws, ws_bytes, c->stream));
-        listed += ju.size();
-        items += (int64_t)ju.size();
+        items += nu;
       }
     }
     HIP_TRY(ppsk::launch_sketch_finish(a, c->stream));

@@ -31,6 +31,17 @@ struct SketchGroup {
   int32_t kk;
 };
 
+// Where the units of the (k, contig) pairs lie, pair f = kk * n_contigs + contig:
+// before_u[f] units and before_w[f] windows come before it, k by k.
+struct UnitIndex {
+  const int64_t* contig_off;  // [n_contigs + 1]
+  const int64_t* spans;       // [n_k] bases of a window
+  const int64_t* before_u;    // [n_k * n_contigs + 1]
+  const int64_t* before_w;    // the same, or null
+  int64_t n_contigs;
+  int64_t unit;               // window starts per unit
+};
+
 struct SketchArgs {
   const uint8_t* codes;      // base codes; codes[0] is the first base, padded both sides
   const SketchUnit* units;   // per k-mer length index: its own unit list
@@ -53,6 +64,11 @@ struct SketchArgs {
 // CODE_PAD_FRONT bytes before and CODE_PAD_BACK bytes after become code 4.
 // codes must be 16-byte aligned.
 hipError_t launch_sketch_decode(uint8_t* codes, int64_t n, hipStream_t stream);
+
+// Writes the n units of pairs [lo, hi) to units, in order, and with before_w each
+// unit's first window among those pairs' windows to wbase.
+hipError_t launch_sketch_units(const UnitIndex& ix, int64_t lo, int64_t hi, int64_t n,
+                               SketchUnit* units, int64_t* wbase, hipStream_t stream);
 
 // Clears the bin minima, hashes every group, densifies and bit-slices.
 // lds_bins: keep each workgroup's bin minima in LDS (64 s64 * 8 bytes of
