@@ -113,6 +113,22 @@ int sketch_impl(int device_id, int64_t n_samples, const char* seq, int64_t seq_b
   a.binsize = (sign_mod + (uint64_t)nbins - 1ULL) / (uint64_t)nbins;
   a.bin_recip = ~0ULL / a.binsize;
   if (a.bin_recip >> 32) return fail(PPSK_ERR_ARG, "bin reciprocal out of range");
+  {
+    // 2^t = q binsize + r, t from 0 until q has 32 bits (q < 2^16 at t = 61)
+    uint64_t q = 0, r = 1;
+    int t = 0;
+    while ((q >> 31) == 0) {
+      q <<= 1;
+      r <<= 1;
+      if (r >= a.binsize) {
+        r -= a.binsize;
+        ++q;
+      }
+      ++t;
+    }
+    a.bin_g = (uint32_t)q;
+    a.bin_s = t - 61;
+  }
 
   // Work units: every contig of every k cut into runs of windows; before_u and
   // before_w count the units and windows of the (k, contig) pairs before each,

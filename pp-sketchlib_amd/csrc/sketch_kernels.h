@@ -54,6 +54,8 @@ struct SketchArgs {
   int64_t n_samples;
   uint64_t binsize;          // ceil((2^61 - 1) / (64 s64))
   uint64_t bin_recip;        // floor((2^64 - 1) / binsize), < 2^32
+  uint32_t bin_g;            // floor(2^(61 + bin_s) / binsize), in [2^31, 2^32)
+  int32_t bin_s;
   uint64_t* signs;           // [n_samples][n_k][64 s64] bin minima (work)
   uint64_t* raw;             // [n_samples][n_k][s64 * 14] output words
   double* inv_minhash;       // [n_samples][n_k] bin 0 / (2^61 - 1), before densifying

@@ -85,6 +85,26 @@ __device__ __forceinline__ uint64_t rot_inv_by(uint64_t x) {
          (((lo >> S) | (lo << (33 - S))) & 0x1FFFFFFFFULL);
 }
 
+// rot and rot^-1 on the two words: 5 and 4 instructions (the shifts of the
+// 31-bit and 33-bit parts as they stand take 12 to 14).
+template <>
+__device__ __forceinline__ uint64_t rot_by<1>(uint64_t x) {
+  const uint32_t w0 = (uint32_t)x, w1 = (uint32_t)(x >> 32);
+  // bits 1 .. 32 from bits 0 .. 31, bit 0 from bit 32; bits 34 .. 63 from 33 ..
+  // 62, bit 33 from bit 63
+  const uint32_t lo = (w0 << 1) | (w1 & 1u);
+  const uint32_t hi = __builtin_amdgcn_alignbit(w1, w0, 31);
+  return ((uint64_t)((hi & ~2u) | ((w1 >> 30) & 2u)) << 32) | lo;
+}
+
+template <>
+__device__ __forceinline__ uint64_t rot_inv_by<1>(uint64_t x) {
+  const uint32_t w0 = (uint32_t)x, w1 = (uint32_t)(x >> 32);
+  const uint32_t lo = __builtin_amdgcn_alignbit(w1, w0, 1);
+  const uint32_t hi = __builtin_amdgcn_alignbit(w1 >> 1, w1, 1);
+  return ((uint64_t)((hi & ~1u) | (w0 & 1u)) << 32) | lo;
+}
+
 __device__ __forceinline__ uint64_t rotj(uint64_t x, unsigned j) {
   uint64_t hi = x >> 33, lo = x & 0x1FFFFFFFFULL;
   const unsigned a = j % 31, b = j % 33;
@@ -200,28 +220,56 @@ __device__ __forceinline__ void roll_unit(const uint8_t* codes, const SketchUnit
       wi[q] = __builtin_amdgcn_alignbyte(q < 3 ? ic[q + 1] : in_[0], ic[q], ish);
       wo[q] = __builtin_amdgcn_alignbyte(q < 3 ? oc[q + 1] : on_[0], oc[q], osh);
     }
+    // A block in the middle of a unit with every base known, as nearly all are:
+    // each step ends a valid window and rolls a base out.  (Codon-phased seeds
+    // keep the general steps: with both ways their three states do not fit the
+    // 128 registers that two workgroups per CU leave.)
+    const bool plain = i0 >= lag && i0 + 16 <= steps && i0 - span >= last_bad &&
+                       ((wi[0] | wi[1] | wi[2] | wi[3]) & 0x04040404u) == 0u;
+    if (STRIDE == 1 && __all(plain)) {
+      uint32_t pair[4];
 #pragma unroll
-    for (int half = 0; half < 2; ++half) {
-      StepTerms t[8];
-      uint32_t bad = 0;
+      for (int q = 0; q < 4; ++q) pair[q] = wi[q] * 5u + wo[q];  // bytes stay below 25
 #pragma unroll
-      for (int jj = 0; jj < 8; ++jj) {
-        const int j = half * 8 + jj;
-        const uint32_t cin = (wi[j >> 2] >> (8 * (j & 3))) & 0xFFu;
-        uint32_t cout = (wo[j >> 2] >> (8 * (j & 3))) & 0xFFu;
-        cout = i0 + j >= lag ? cout : 4u;
-        t[jj] = terms[cin * 5 + cout];
-        bad |= (cin == 4u ? 1u : 0u) << jj;
+      for (int half = 0; half < 2; ++half) {
+        StepTerms t[8];
+#pragma unroll
+        for (int jj = 0; jj < 8; ++jj) {
+          const int j = half * 8 + jj;
+          t[jj] = terms[(pair[j >> 2] >> (8 * (j & 3))) & 0xFFu];
+        }
+#pragma unroll
+        for (int jj = 0; jj < 8; ++jj) {
+          const int j = half * 8 + jj, q = j % STRIDE;
+          fh[q] = rot_by<STRIDE>(fh[q]) ^ t[jj].f;
+          rh[q] = rot_inv_by<STRIDE>(rh[q] ^ t[jj].r);
+          emit(i0 + j - span + 1, (use_rc & (rh[q] < fh[q])) ? rh[q] : fh[q]);
+        }
       }
+    } else {
 #pragma unroll
-      for (int jj = 0; jj < 8; ++jj) {
-        const int j = half * 8 + jj, q = j % STRIDE;
-        const int i = i0 + j;
-        fh[q] = rot_by<STRIDE>(fh[q]) ^ t[jj].f;
-        rh[q] = rot_inv_by<STRIDE>(rh[q] ^ t[jj].r);
-        last_bad = (bad >> jj) & 1u ? i : last_bad;
-        if (i - span >= last_bad && i < steps) {
-          emit(i - span + 1, (use_rc && rh[q] < fh[q]) ? rh[q] : fh[q]);
+      for (int half = 0; half < 2; ++half) {
+        StepTerms t[8];
+        uint32_t bad = 0;
+#pragma unroll
+        for (int jj = 0; jj < 8; ++jj) {
+          const int j = half * 8 + jj;
+          const uint32_t cin = (wi[j >> 2] >> (8 * (j & 3))) & 0xFFu;
+          uint32_t cout = (wo[j >> 2] >> (8 * (j & 3))) & 0xFFu;
+          cout = i0 + j >= lag ? cout : 4u;
+          t[jj] = terms[cin * 5 + cout];
+          bad |= (cin == 4u ? 1u : 0u) << jj;
+        }
+#pragma unroll
+        for (int jj = 0; jj < 8; ++jj) {
+          const int j = half * 8 + jj, q = j % STRIDE;
+          const int i = i0 + j;
+          fh[q] = rot_by<STRIDE>(fh[q]) ^ t[jj].f;
+          rh[q] = rot_inv_by<STRIDE>(rh[q] ^ t[jj].r);
+          last_bad = (bad >> jj) & 1u ? i : last_bad;
+          if (i - span >= last_bad && i < steps) {
+            emit(i - span + 1, (use_rc & (rh[q] < fh[q])) ? rh[q] : fh[q]);
+          }
         }
       }
     }
@@ -289,16 +337,45 @@ __device__ __forceinline__ uint64_t bin_of(uint64_t h, uint64_t binsize, uint32_
   return bin;
 }
 
+// h mod (2^61 - 1) and its bin from 32-bit arithmetic.  With g = floor(2^(61 + s) /
+// binsize) in [2^31, 2^32), floor(h / 2^29) g is below h 2^(32 + s) / binsize by less
+// than 2^33, so its upper word, which counts bins in steps of 2^-s, is at most 2 too
+// low: only a value that those 2 could carry into the next bin (and h within 7 of
+// the modulus, whose end around is left out) takes the 64-bit way.  s is 17 at
+// 9,984 bins: 1 window in 2^16.  With the plain blocks of roll_unit this is 35
+// VALU instructions a window instead of 58; 6 genomes of 2 Mb at 8 k-mer lengths
+// (96 million windows) hash in 141 us instead of 200.
+struct BinScale {
+  uint64_t binsize;
+  uint32_t recip;  // bin_of
+  uint32_t g;
+  int s;
+};
+
+__device__ __forceinline__ uint64_t mod_bin(uint64_t h0, const BinScale& b, uint32_t& bin) {
+  uint64_t h = (h0 & SIGN_MOD) + (h0 >> 61);
+  const uint32_t top = (uint32_t)(h >> 32);
+  const uint32_t x = __umulhi(__builtin_amdgcn_alignbit(top, (uint32_t)h, 29), b.g);
+  bin = x >> b.s;
+  const bool rare = top >= 0x1FFFFFFFu || ((x + 2u) >> b.s) != bin;
+  if (__builtin_expect(__ballot(rare) != 0ULL, 0)) {  // a scalar branch around the 64-bit way
+    if (rare) {
+      h = mod_sign(h0);
+      bin = (uint32_t)bin_of(h, b.binsize, b.recip);
+    }
+  }
+  return h;
+}
+
 template <bool LDS_BINS, int STRIDE>
-__global__ __launch_bounds__(SKETCH_TB) void sketch_hash_kernel(SketchArgs a, int64_t n_groups,
+__global__ __launch_bounds__(SKETCH_TB, 4) void sketch_hash_kernel(SketchArgs a, int64_t n_groups,
                                                                 int* next_group) {
   extern __shared__ uint64_t lbins[];
   __shared__ StepTerms terms[25];
   __shared__ int64_t cur_group;
   __shared__ int cur_k;
   const int64_t nbins = (int64_t)a.s64 * 64;
-  const uint64_t binsize = a.binsize;
-  const uint32_t recip = (uint32_t)a.bin_recip;
+  const BinScale bs{a.binsize, (uint32_t)a.bin_recip, a.bin_g, a.bin_s};
   const bool use_rc = a.use_rc != 0;
   if (threadIdx.x == 0) cur_k = -1;
   // groups are taken from a counter until none is left: every workgroup
@@ -321,8 +398,8 @@ __global__ __launch_bounds__(SKETCH_TB) void sketch_hash_kernel(SketchArgs a, in
     if (threadIdx.x == 0) cur_k = k;
     for (int64_t u = g.unit0 + threadIdx.x; u < g.unit1; u += SKETCH_TB) {
       roll_unit<STRIDE>(a.codes, a.units[u], k, use_rc, terms, [&](int, uint64_t h0) {
-        const uint64_t h = mod_sign(h0);
-        const uint64_t bin = bin_of(h, binsize, recip);
+        uint32_t bin;
+        const uint64_t h = mod_bin(h0, bs, bin);
         if (LDS_BINS) {
           atomicMin((unsigned long long*)&lbins[bin], (unsigned long long)h);
         } else if (h < gbins[bin]) {

@@ -46,3 +46,35 @@ def test_units_against_oracle(min_count, exact):
             want_dn |= int(d != 0)
         assert mh[s] == pytest.approx(want_mh, rel=0, abs=1e-15), s
         assert dn[s] == want_dn, s
+
+
+def test_unknown_base_at_every_step():
+    # a base that is not A, C, G or T at every position of three blocks of 16
+    # steps, and none: blocks with and without unknown bases, before and after
+    # the first k, in the same workgroup
+    rng = np.random.default_rng(11)
+    base = rng.choice(np.frombuffer(b"ACGT", np.uint8), 400)
+    samples = [[base.tobytes()]]
+    for p in list(range(48)) + [383, 384, 398, 399]:
+        seq = base.copy()
+        seq[p] = ord("N")
+        seq[(p + 200) % 400] = ord("-")
+        samples.append([seq.tobytes()])
+    raw, _, _ = H.sketch(samples, [3, 13, 31], 1)
+    for s, contigs in enumerate(samples):
+        for x, k in enumerate([3, 13, 31]):
+            assert np.array_equal(raw[s, x], O.sketch(contigs, k, 1, True)[0]), (s, k)
+
+
+@pytest.mark.parametrize("s64", [1, 16, 156, 1023])
+def test_bins_against_oracle(s64):
+    # 32-bit bins with the 64-bit way for values next to a bin's end: 120,000
+    # windows per k-mer length at the smallest and largest bin counts
+    rng = np.random.default_rng(s64)
+    seq = rng.choice(np.frombuffer(b"ACGT", np.uint8), 120000).tobytes()
+    for use_rc in (True, False):
+        raw, mh, _ = H.sketch([[seq]], [15, 27], s64, use_rc=use_rc)
+        want = [O.sketch([seq], k, s64, use_rc) for k in (15, 27)]
+        for x in range(2):
+            assert np.array_equal(raw[0, x], want[x][0]), (s64, use_rc, x)
+        assert mh[0] == pytest.approx(want[0][1] + want[1][1], rel=0, abs=1e-15)
