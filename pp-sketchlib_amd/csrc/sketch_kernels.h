@@ -107,7 +107,7 @@ struct ReadsJob {
   uint64_t binsize;
   uint32_t recip;
   uint64_t* bins;  // this (sample, k)'s bin minima
-  unsigned long long* words;  // two page-locked words for the occurrence count
+  unsigned long long* words;  // three page-locked words for the job's totals
 };
 // Device workspace a job of up to max_windows windows needs.
 size_t reads_workspace_bytes(int64_t max_windows);

@@ -28,6 +28,7 @@
 
 #include <algorithm>
 #include <cstdint>
+#include <cstring>
 
 #include <hipcub/hipcub.hpp>
 
@@ -446,8 +447,12 @@ __device__ __forceinline__ uint64_t multi_hash1(uint64_t h0, int k) {
   return t ^ (t >> 27);
 }
 
+// One wave per workgroup: a read is one unit, so 20,000 of them are 80 workgroups
+// of 256 lanes and 316 of 64 (50 and 36 us).
+constexpr int READS_TB = 64;
+
 template <int STRIDE>
-__global__ __launch_bounds__(256) void reads_hash_kernel(ReadsJob j, uint64_t* h0, uint8_t* st) {
+__global__ __launch_bounds__(READS_TB) void reads_hash_kernel(ReadsJob j, uint64_t* h0, uint8_t* st) {
   __shared__ StepTerms terms[25];
   if (threadIdx.x < 25) terms[threadIdx.x] = step_terms(threadIdx.x, STRIDE * j.k);
   __syncthreads();
@@ -463,40 +468,85 @@ __global__ __launch_bounds__(256) void reads_hash_kernel(ReadsJob j, uint64_t* h
   }
 }
 
-// rs[w] = w if a run of valid windows starts at w, else -1
-__global__ void reads_run_kernel(const uint8_t* st, int64_t n, int64_t* rs) {
-  for (int64_t w = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; w < n;
-       w += (int64_t)gridDim.x * blockDim.x) {
+// 1 for a valid window, and 2^32 for the first window of a run of them: one
+// prefix sum numbers both the occurrences and the runs (fewer than 2^29 each).
+struct Numbering {
+  const uint8_t* st;
+  __device__ __forceinline__ uint64_t operator()(int64_t w) const {
     const uint8_t s = st[w];
-    rs[w] = (s != 0 && (s == 3 || w == 0 || st[w - 1] == 0)) ? w : -1;
+    if (s == 0) return 0;
+    return (s == 3 || w == 0 || st[w - 1] == 0) ? (1ULL << 32) + 1 : 1;
   }
+};
+
+// Counts of a job and what its cells share (Totals::shared): the cell between
+// rows 1 and 2 belongs to an occurrence (1) and to a run (2), or both rows of a
+// run lie on the cell between rows 2 and 3 (4).
+struct Totals {
+  unsigned long long occurrences, runs;
+  unsigned int shared, pad;
+};
+
+__device__ __forceinline__ uint32_t cm_cell(uint64_t h, uint32_t r) {
+  return (uint32_t)(r * CM_MASK + ((h >> (27 * (r & 1))) & CM_MASK));
 }
 
-// occurrence t = tix[w] of every valid window: H0[t], H1[t].  Hash 1 mixes
-// hash 0 of the run's first window (dense seeds) or of the window itself
-// (codon-phased seeds: the spaced-seed iterator recomputes it every step);
-// span is the iterator's k, the seed's span.
-__global__ void reads_compact_kernel(const uint8_t* st, const uint64_t* h0, const int64_t* run,
-                                     const int64_t* tix, int64_t n, int span, int own_hash,
-                                     uint64_t* H0, uint64_t* H1) {
+// Occurrence t of every valid window w: its hash H0[t]; with by_run also its run
+// U[t], each run's first occurrence RT[u] and hash 1 RH[u], and the events of
+// rows 0 and 1.
+__global__ void reads_compact_kernel(const uint8_t* st, const uint64_t* h0, const uint64_t* number,
+                                     int64_t n, int span, bool by_run, uint64_t* H0, uint32_t* U,
+                                     uint32_t* RT, uint64_t* RH, uint2* key, uint2* val,
+                                     Totals* totals) {
   for (int64_t w = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; w < n;
        w += (int64_t)gridDim.x * blockDim.x) {
-    if (st[w] != 0) {
-      const int64_t t = tix[w];
-      H0[t] = h0[w];
-      H1[t] = multi_hash1(h0[own_hash ? w : run[w]], span);
+    const uint64_t before = number[w], own = Numbering{st}(w);
+    if (w == n - 1) {
+      totals->occurrences = (uint32_t)(before + own);
+      totals->runs = (before + own) >> 32;
     }
+    if (own == 0) continue;
+    const uint32_t t = (uint32_t)before;
+    const uint64_t h = h0[w];
+    H0[t] = h;
+    if (!by_run) continue;
+    const uint32_t u = (uint32_t)((before + own) >> 32) - 1u;
+    U[t] = u;
+    key[t] = make_uint2(cm_cell(h, 0), cm_cell(h, 1));
+    val[t] = make_uint2(2u * t, 2u * t + 1u);
+    unsigned int shared = cm_cell(h, 1) == 2u * CM_MASK ? 1u : 0u;
+    if (own >> 32) {
+      const uint64_t g = multi_hash1(h, span);
+      RT[u] = t;
+      RH[u] = g;
+      if (cm_cell(g, 2) == 2u * CM_MASK) shared |= 2u;
+      if (cm_cell(g, 2) == cm_cell(g, 3)) shared |= 4u;
+    }
+    if (shared) atomicOr(&totals->shared, shared);
   }
 }
 
-__global__ void reads_cm_keys_kernel(const uint64_t* H0, const uint64_t* H1, int64_t n,
-                                     uint32_t* key, uint32_t* val) {
+// Events of rows 2 and 3, one per run, behind the 2 n_occ of rows 0 and 1.
+__global__ void reads_run_keys_kernel(const uint64_t* RH, int64_t n_runs, int64_t n_occ,
+                                      uint2* key, uint2* val) {
+  for (int64_t u = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; u < n_runs;
+       u += (int64_t)gridDim.x * blockDim.x) {
+    const uint64_t g = RH[u];
+    const uint32_t v = (uint32_t)(2 * (n_occ + u));
+    key[n_occ + u] = make_uint2(cm_cell(g, 2), cm_cell(g, 3));
+    val[n_occ + u] = make_uint2(v, v + 1u);
+  }
+}
+
+// All four events of every occurrence: hash 1 is that of its run, or its own
+// (codon-phased seeds: the spaced-seed iterator recomputes it every step).
+__global__ void reads_cm_keys_kernel(const uint64_t* H0, const uint64_t* RH, const uint32_t* U,
+                                     int span, int64_t n, uint32_t* key, uint32_t* val) {
   for (int64_t e = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; e < 4 * n;
        e += (int64_t)gridDim.x * blockDim.x) {
     const int64_t t = e >> 2;
     const uint32_t r = (uint32_t)(e & 3);
-    const uint64_t hv = r < 2 ? H0[t] : H1[t];
-    key[e] = (uint32_t)(r * CM_MASK + ((hv >> (27 * (r & 1))) & CM_MASK));
+    key[e] = cm_cell(r < 2 ? H0[t] : RH ? RH[U[t]] : multi_hash1(H0[t], span), r);
     val[e] = (uint32_t)e;
   }
 }
@@ -521,27 +571,54 @@ __global__ void reads_pass_kernel(const Key* key, const uint32_t* val, int64_t n
   }
 }
 
-__global__ void reads_bin_kernel(const uint64_t* H0, const uint8_t* pass, int64_t n, int events,
+// The same with rows 2 and 3 counted by run (val >= events): a run's events of a
+// row lie on one cell, its occurrences one after the other, so the count at
+// occurrence o of the run is o + 1 plus the lengths of the earlier runs of that
+// cell, which lie just before it in sorted order.  wait[u]: the first occurrence of
+// run u at which both rows' counts reach m.
+__global__ void reads_pass_runs_kernel(const uint32_t* key, const uint32_t* val, int64_t n, int m,
+                                       int64_t events, const uint32_t* RT, int64_t n_runs,
+                                       uint8_t* pass, uint32_t* wait) {
+  for (int64_t s = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; s < n;
+       s += (int64_t)gridDim.x * blockDim.x) {
+    const uint32_t v = val[s], own = key[s];
+    if (v < events) {
+      if (!(s >= m - 1 && key[s - (m - 1)] == own)) pass[v] = 0;
+      continue;
+    }
+    int64_t before = 0;
+    for (int64_t p = s - 1; p >= 0 && before < m - 1 && key[p] == own; --p) {
+      const uint32_t u = (uint32_t)((val[p] - events) >> 1);
+      before += (u + 1 < n_runs ? RT[u + 1] : (uint32_t)(events >> 1)) - RT[u];
+    }
+    if (before < m - 1) atomicMax(&wait[(v - events) >> 1], (uint32_t)(m - 1 - before));
+  }
+}
+
+// EVENTS: pass flags per occurrence (1 exact, 2 with runs, 4).
+template <int EVENTS>
+__global__ void reads_bin_kernel(const uint64_t* H0, const uint8_t* pass, int64_t n,
+                                 const uint32_t* U, const uint32_t* RT, const uint32_t* wait,
                                  uint64_t binsize, uint32_t recip, uint64_t* bins) {
   for (int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; t < n;
        t += (int64_t)gridDim.x * blockDim.x) {
-    bool ok = true;
-    for (int r = 0; r < events; ++r) ok = ok && pass[t * events + r];
+    const uint64_t h0 = H0[t];
+    bool ok;
+    if (EVENTS == 1) {
+      ok = pass[t] != 0;
+    } else if (EVENTS == 2) {
+      const uint32_t u = U[t];
+      ok = reinterpret_cast<const uint16_t*>(pass)[t] == 0x0101u && (uint32_t)t - RT[u] >= wait[u];
+    } else {
+      ok = reinterpret_cast<const uint32_t*>(pass)[t] == 0x01010101u;
+    }
     if (ok) {
-      const uint64_t h = mod_sign(H0[t]);
+      const uint64_t h = mod_sign(h0);
       const uint64_t bin = bin_of(h, binsize, recip);
       if (h < bins[bin]) atomicMin((unsigned long long*)&bins[bin], (unsigned long long)h);
     }
   }
 }
-
-struct Max64 {
-  __device__ __forceinline__ int64_t operator()(int64_t a, int64_t b) const { return a > b ? a : b; }
-};
-
-struct ValidOne {
-  __device__ __forceinline__ int64_t operator()(uint8_t s) const { return s != 0 ? 1 : 0; }
-};
 
 inline unsigned grid_for(int64_t n) {
   return (unsigned)std::max<int64_t>(1, std::min<int64_t>((n + 255) / 256, 65536));
@@ -559,19 +636,21 @@ struct Carve {
   }
 };
 
+hipcub::TransformInputIterator<uint64_t, Numbering, hipcub::CountingInputIterator<int64_t>> numbers(
+    const uint8_t* st) {
+  return {hipcub::CountingInputIterator<int64_t>(0), Numbering{st}};
+}
+
 size_t cub_temp_bytes(int64_t max_windows) {
-  size_t a = 0, b = 0, c = 0, d = 0;
   const int64_t W = std::max<int64_t>(max_windows, 1);
-  hipcub::TransformInputIterator<int64_t, ValidOne, const uint8_t*> it(nullptr, ValidOne());
-  (void)hipcub::DeviceScan::InclusiveScan(nullptr, a, (const int64_t*)nullptr, (int64_t*)nullptr,
-                                    Max64(), (int)W);
-  (void)hipcub::DeviceScan::ExclusiveSum(nullptr, b, it, (int64_t*)nullptr, (int)W);
-  (void)hipcub::DeviceRadixSort::SortPairs(nullptr, c, (const uint32_t*)nullptr, (uint32_t*)nullptr,
+  size_t a = 0, b = 0, c = 0;
+  (void)hipcub::DeviceScan::ExclusiveSum(nullptr, a, numbers(nullptr), (uint64_t*)nullptr, (int)W);
+  (void)hipcub::DeviceRadixSort::SortPairs(nullptr, b, (const uint32_t*)nullptr, (uint32_t*)nullptr,
                                      (const uint32_t*)nullptr, (uint32_t*)nullptr, (int)(4 * W),
                                      0, 29);
-  (void)hipcub::DeviceRadixSort::SortPairs(nullptr, d, (const uint64_t*)nullptr, (uint64_t*)nullptr,
+  (void)hipcub::DeviceRadixSort::SortPairs(nullptr, c, (const uint64_t*)nullptr, (uint64_t*)nullptr,
                                      (const uint32_t*)nullptr, (uint32_t*)nullptr, (int)W, 0, 64);
-  return std::max(std::max(a, b), std::max(c, d));
+  return std::max(std::max(a, b), c);
 }
 
 }  // namespace
@@ -581,11 +660,13 @@ size_t reads_workspace_bytes(int64_t max_windows) {
   const int64_t W = std::max<int64_t>(max_windows, 1);
   c.take<uint64_t>(W);      // h0
   c.take<uint8_t>(W);       // st
-  c.take<int64_t>(W);       // rs
-  c.take<int64_t>(W);       // run
-  c.take<int64_t>(W);       // tix
+  c.take<uint64_t>(W);      // number
   c.take<uint64_t>(W);      // H0
-  c.take<uint64_t>(W);      // H1
+  c.take<uint32_t>(W);      // U
+  c.take<uint32_t>(W);      // RT
+  c.take<uint64_t>(W);      // RH
+  c.take<uint32_t>(W);      // wait
+  c.take<Totals>(1);
   c.take<uint32_t>(4 * W);  // keys in (count-min) / 2 W for exact
   c.take<uint32_t>(4 * W);  // keys out
   c.take<uint32_t>(4 * W);  // vals in
@@ -595,6 +676,13 @@ size_t reads_workspace_bytes(int64_t max_windows) {
   return c.used;
 }
 
+// With dense seeds every occurrence of a run has the run's hash 1, so rows 2 and 3
+// are sorted and counted by run: 2 events per occurrence and 2 per run instead of
+// 4 per occurrence.  680,000 occurrences in 20,000 runs: sorting 410 -> 262 us, a call
+// of five such jobs 4.57 -> 3.36 ms.  That needs
+// each cell's events to be all of occurrences or all of runs; the flat cells of
+// rows 1 and 2 (and of rows 2 and 3 for one run) meet in one cell, which takes the
+// general way in the rare job where both sides use it.
 hipError_t run_reads_job(const ReadsJob& j, void* ws, size_t ws_bytes, hipStream_t stream) {
   const int64_t W = j.n_windows;
   if (W <= 0) return hipSuccess;
@@ -602,11 +690,13 @@ hipError_t run_reads_job(const ReadsJob& j, void* ws, size_t ws_bytes, hipStream
   Carve c{static_cast<char*>(ws)};
   uint64_t* h0 = c.take<uint64_t>(W);
   uint8_t* st = c.take<uint8_t>(W);
-  int64_t* rs = c.take<int64_t>(W);
-  int64_t* run = c.take<int64_t>(W);
-  int64_t* tix = c.take<int64_t>(W);
+  uint64_t* number = c.take<uint64_t>(W);
   uint64_t* H0 = c.take<uint64_t>(W);
-  uint64_t* H1 = c.take<uint64_t>(W);
+  uint32_t* U = c.take<uint32_t>(W);
+  uint32_t* RT = c.take<uint32_t>(W);
+  uint64_t* RH = c.take<uint64_t>(W);
+  uint32_t* wait = c.take<uint32_t>(W);
+  Totals* totals = c.take<Totals>(1);
   uint32_t* kin = c.take<uint32_t>(4 * W);
   uint32_t* kout = c.take<uint32_t>(4 * W);
   uint32_t* vin = c.take<uint32_t>(4 * W);
@@ -616,56 +706,60 @@ hipError_t run_reads_job(const ReadsJob& j, void* ws, size_t ws_bytes, hipStream
   void* temp = c.take<char>((int64_t)temp_bytes);
 
   hipError_t e = hipMemsetAsync(st, 0, (size_t)W, stream);
+  if (e == hipSuccess) e = hipMemsetAsync(totals, 0, sizeof(Totals), stream);
   if (e != hipSuccess) return e;
+  const unsigned units = (unsigned)std::min<int64_t>((j.n_units + READS_TB - 1) / READS_TB, 65536);
   if (j.codon) {
-    reads_hash_kernel<3><<<grid_for(j.n_units), 256, 0, stream>>>(j, h0, st);
+    reads_hash_kernel<3><<<units, READS_TB, 0, stream>>>(j, h0, st);
   } else {
-    reads_hash_kernel<1><<<grid_for(j.n_units), 256, 0, stream>>>(j, h0, st);
+    reads_hash_kernel<1><<<units, READS_TB, 0, stream>>>(j, h0, st);
   }
-  reads_run_kernel<<<grid_for(W), 256, 0, stream>>>(st, W, rs);
   if ((e = hipGetLastError()) != hipSuccess) return e;
   size_t tb = temp_bytes;
-  e = hipcub::DeviceScan::InclusiveScan(temp, tb, rs, run, Max64(), (int)W, stream);
-  if (e != hipSuccess) return e;
-  hipcub::TransformInputIterator<int64_t, ValidOne, const uint8_t*> valid(st, ValidOne());
-  tb = temp_bytes;
-  e = hipcub::DeviceScan::ExclusiveSum(temp, tb, valid, tix, (int)W, stream);
+  e = hipcub::DeviceScan::ExclusiveSum(temp, tb, numbers(st), number, (int)W, stream);
   if (e != hipSuccess) return e;
   const int span = j.codon ? 3 * j.k - 2 : j.k;
-  reads_compact_kernel<<<grid_for(W), 256, 0, stream>>>(st, h0, run, tix, W, span, j.codon, H0,
-                                                        H1);
+  const bool by_run = !j.codon && !j.exact;
+  reads_compact_kernel<<<grid_for(W), 256, 0, stream>>>(st, h0, number, W, span, by_run, H0, U, RT, RH,
+                                                        (uint2*)kin, (uint2*)vin, totals);
   if ((e = hipGetLastError()) != hipSuccess) return e;
-  // occurrence count
-  j.words[1] = 0;
-  if ((e = hipMemcpyAsync(j.words, tix + (W - 1), sizeof(int64_t), hipMemcpyDeviceToHost,
-                          stream)) != hipSuccess ||
-      (e = hipMemcpyAsync(j.words + 1, st + (W - 1), 1, hipMemcpyDeviceToHost, stream)) !=
+  static_assert(sizeof(Totals) == 3 * sizeof(unsigned long long), "words");
+  if ((e = hipMemcpyAsync(j.words, totals, sizeof(Totals), hipMemcpyDeviceToHost, stream)) !=
           hipSuccess ||
       (e = hipStreamSynchronize(stream)) != hipSuccess) {
     return e;
   }
-  const int64_t N = (int64_t)j.words[0] + (j.words[1] != 0 ? 1 : 0);
+  Totals got;
+  std::memcpy(&got, j.words, sizeof(got));
+  const int64_t N = (int64_t)got.occurrences, R = (int64_t)got.runs;
   if (N == 0) return hipSuccess;
-  int events;
+  tb = temp_bytes;
   if (j.exact) {
-    events = 1;
-    uint64_t* k64in = reinterpret_cast<uint64_t*>(kin);
     uint64_t* k64out = reinterpret_cast<uint64_t*>(kout);
-    e = hipMemcpyAsync(k64in, H0, (size_t)N * sizeof(uint64_t), hipMemcpyDeviceToDevice, stream);
-    if (e != hipSuccess) return e;
     reads_iota_kernel<<<grid_for(N), 256, 0, stream>>>(vin, N);
-    tb = temp_bytes;
-    e = hipcub::DeviceRadixSort::SortPairs(temp, tb, k64in, k64out, vin, vout, (int)N, 0, 64,
-                                           stream);
+    e = hipcub::DeviceRadixSort::SortPairs(temp, tb, H0, k64out, vin, vout, (int)N, 0, 64, stream);
     if (e != hipSuccess) return e;
     e = hipMemsetAsync(pass, 1, (size_t)N, stream);
     if (e != hipSuccess) return e;
     reads_pass_kernel<uint64_t><<<grid_for(N), 256, 0, stream>>>(k64out, vout, N, j.min_count,
                                                                   pass);
+    reads_bin_kernel<1><<<grid_for(N), 256, 0, stream>>>(H0, pass, N, nullptr, nullptr, nullptr,
+                                                         j.binsize, j.recip, j.bins);
+  } else if (by_run && (got.shared & 3u) != 3u && (got.shared & 4u) == 0u) {
+    const int64_t n = 2 * (N + R);
+    reads_run_keys_kernel<<<grid_for(R), 256, 0, stream>>>(RH, R, N, (uint2*)kin, (uint2*)vin);
+    e = hipcub::DeviceRadixSort::SortPairs(temp, tb, kin, kout, vin, vout, (int)n, 0, 29, stream);
+    if (e != hipSuccess) return e;
+    e = hipMemsetAsync(pass, 1, (size_t)(2 * N), stream);
+    if (e == hipSuccess) e = hipMemsetAsync(wait, 0, (size_t)R * sizeof(uint32_t), stream);
+    if (e != hipSuccess) return e;
+    reads_pass_runs_kernel<<<grid_for(n), 256, 0, stream>>>(kout, vout, n, j.min_count, 2 * N, RT, R,
+                                                            pass, wait);
+    reads_bin_kernel<2><<<grid_for(N), 256, 0, stream>>>(H0, pass, N, U, RT, wait, j.binsize,
+                                                         j.recip, j.bins);
   } else {
-    events = 4;
-    reads_cm_keys_kernel<<<grid_for(4 * N), 256, 0, stream>>>(H0, H1, N, kin, vin);
-    tb = temp_bytes;
+    reads_cm_keys_kernel<<<grid_for(4 * N), 256, 0, stream>>>(H0, by_run ? RH : nullptr, U, span, N,
+                                                              kin, vin);
     e = hipcub::DeviceRadixSort::SortPairs(temp, tb, kin, kout, vin, vout, (int)(4 * N), 0, 29,
                                            stream);
     if (e != hipSuccess) return e;
@@ -673,9 +767,9 @@ hipError_t run_reads_job(const ReadsJob& j, void* ws, size_t ws_bytes, hipStream
     if (e != hipSuccess) return e;
     reads_pass_kernel<uint32_t><<<grid_for(4 * N), 256, 0, stream>>>(kout, vout, 4 * N,
                                                                       j.min_count, pass);
+    reads_bin_kernel<4><<<grid_for(N), 256, 0, stream>>>(H0, pass, N, nullptr, nullptr, nullptr,
+                                                         j.binsize, j.recip, j.bins);
   }
-  reads_bin_kernel<<<grid_for(N), 256, 0, stream>>>(H0, pass, N, events, j.binsize, j.recip,
-                                                    j.bins);
   return hipGetLastError();
 }
 
