@@ -9,9 +9,13 @@ tree-evolution model and resident in HBM before timing starts.
 
 Prints one JSON line:
   value      distances (pairs) per second over the timed steps
-  roofline   int32 VALU issue bound of the distance-tile kernel: algorithmic
-             ops per pair = sum_k s64 * (2 * bbits + 2) = 37,440, divided by
-             the kernel's HIP-event duration on its launch stream
+  roofline   int32 VALU issue bound of a distance pass: the lane operations its
+             kernels issue (SQ_INSTS_VALU x 64 of the committed profile of the
+             same pass) divided by the pass's HIP-event duration on its launch
+             stream.  plane_ops_per_pair = sum_k s64 * (2 * bbits + 2) = 37,440
+             is what matching the sketches' 14 bit planes as they are takes; the
+             pass matches ranks of the values instead (7 to 9 planes), so
+             plane_rate, that work over the same time, is above the peak
   cpu_baseline  the CPU oracle (C++/OpenMP restatement of the reference CPU
              path), compiled on this host with -march=native, on a bounded
              sample of the same workload: median of 3 runs at 16 threads and
@@ -110,14 +114,14 @@ def measured_valu_peak():
     return ops.value / 1e12
 
 
-def traffic_from_profile():
-    """HBM bytes per distance pass from the committed rocprofv3 counter summary."""
-    path = os.path.join(ROOT, "profiles", "dist_batch_allvsall_8192_traffic.json")
-    if not os.path.exists(path):
-        return None
+def pass_profile(n):
+    """Counter summary of the committed rocprofv3 profile of the 8,192-sample pass
+    (HBM bytes and VALU lane operations per pass); empty for another size."""
+    path = os.path.join(ROOT, "profiles", "dist_coded_allvsall_8192.json")
+    if n != N_SAMPLES or not os.path.exists(path):
+        return {}
     with open(path) as f:
-        d = json.load(f)
-    return d.get("hbm_bytes_per_pass")
+        return json.load(f)
 
 
 def _host_cpu():
@@ -242,23 +246,26 @@ def main():
     print(f"# {a.steps} steps in {wall:.3f}s", file=sys.stderr, flush=True)
 
     value = pairs * a.steps / wall
-    # one step is one pass over every pair: the persistent tile kernel
-    # (dist_batch) plus, when its last round of whole tiles would be mostly
-    # idle, one launch of the per-(tile, k) kernel for those tiles; the HIP
-    # events bracket both launches of the pass on their stream
+    # one step is one pass over every pair: coding, matching and output kernels
+    # (one launch each while the codes fit their scratch); the HIP events bracket
+    # them on their stream
     pass_ms = sum(kernel_ms) / a.steps
-    achieved = OPS_PER_PAIR * pairs / (pass_ms * 1e-3) / 1e12
+    profile = pass_profile(a.n)
+    ops = profile.get("valu_lane_ops_per_pass")
+    achieved = ops / (pass_ms * 1e-3) / 1e12 if ops else None
     roofline = {
         "bound": "valu",
-        "achieved": round(achieved, 3),
+        "achieved": round(achieved, 3) if ops else None,
         "peak": round(PEAK_TOPS, 3),
         "unit": "TOP/s",
-        "frac": round(achieved / PEAK_TOPS, 4),
-        "traffic": traffic_from_profile(),
-        "kernel": "dist_batch + dist_tiles_diagonal (last partial round: the diagonal tiles)",
+        "frac": round(achieved / PEAK_TOPS, 4) if ops else None,
+        "traffic": profile.get("hbm_bytes_per_pass"),
+        "kernel": "code_kernel + dist_coded + dist_items_out",
         "kernel_ms": round(pass_ms, 3),
         "launches_per_step": round(launches / a.steps, 2),
-        "ops_per_pair": OPS_PER_PAIR,
+        "ops_per_pair": round(ops / pairs) if ops else None,
+        "plane_ops_per_pair": OPS_PER_PAIR,
+        "plane_rate": round(OPS_PER_PAIR * pairs / (pass_ms * 1e-3) / 1e12, 3),
         "peak_measured": None,
     }
     peak_meas = measured_valu_peak()

@@ -71,7 +71,7 @@ def large(a):
         "metric": "distances/sec, 32,768-sample all-vs-all streamed to host + kNN=10",
         "value": round(pairs / wall, 1), "unit": "distances/s", "n_gpus": 1,
         "wall_s": round(wall, 4), "dist_kernel_ms": round(ms, 2),
-        "valu_frac": round(pairs * _ops_per_pair(8, S64) / (ms * 1e-3) / 39.3216e12, 4),
+        "plane_valu_frac": round(pairs * _ops_per_pair(8, S64) / (ms * 1e-3) / 39.3216e12, 4),
         "dense_bytes_to_host": pairs * 8,
         "host_rate_GBps": round(pairs * 8 / wall / 1e9, 2),
         "config": {"workload": "large all-vs-all, dense FP32 to pinned host + kNN=10",
