@@ -1361,8 +1361,11 @@ int ppsk_set_upload(ppsk_set* s, int64_t first, int64_t count, const uint64_t* r
     }
     if (e == hipSuccess) e = hipEventRecord(c->raw_striped[turn], c->stream);
   }
-  if (e == hipSuccess) e = hipStreamSynchronize(c->copy_stream);  // raw may be changed from here
-  if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
+  // also after an error: raw may be changed, and the buffer filled anew, from here
+  for (hipStream_t st : {c->copy_stream, c->stream}) {
+    const hipError_t es = hipStreamSynchronize(st);
+    if (e == hipSuccess) e = es;
+  }
   if (e != hipSuccess) return fail(PPSK_ERR_HIP, std::string("upload: ") + hipGetErrorString(e));
   return PPSK_OK;
 }

@@ -212,7 +212,10 @@ int sketch_impl(int device_id, int64_t n_samples, const char* seq, int64_t seq_b
   if (int rc = grow(&c->sketch, &c->sketch_bytes, parts.used)) return rc;
   struct Trim {
     DeviceCtx* c;
-    ~Trim() { trim(&c->sketch, &c->sketch_bytes); }
+    ~Trim() {
+      hipStreamSynchronize(c->stream);  // after an error: nothing may still read the inputs
+      trim(&c->sketch, &c->sketch_bytes);
+    }
   } trimmed{c};
   char* mem = (char*)c->sketch;
   uint8_t* codes = (uint8_t*)(mem + at_seq) + ppsk::CODE_PAD_FRONT;
