@@ -69,7 +69,6 @@ struct ppsk_batch {
   unsigned long long* d_fail = nullptr; // [n_jobs][2]
   uint32_t* d_queue = nullptr;          // [BATCH_QUEUES]
   uint16_t* scratch = nullptr;
-  size_t scratch_bytes = 0;
   Plan plans[ppsk::BATCH_MIXED + 1];
   int variant = 0;                      // chosen plan (0: not chosen yet)
   double tune_ms[ppsk::BATCH_MIXED + 1] = {};
@@ -390,7 +389,7 @@ int build_plan(ppsk_batch* b, int plan) {
       need = std::max(need, (size_t)g * b->max_k * ppsk::variant_tile_rows(v) *
                                 ppsk::variant_tile_cols(v) * sizeof(uint16_t));
     }
-    if (int rc = grow((void**)&b->scratch, &b->scratch_bytes, need)) return rc;
+    HIP_TRY(device_malloc(c, (void**)&b->scratch, need, WS_ALL));
   }
   HIP_TRY(hipMalloc(&pl.items, std::max<size_t>(all.size(), 1) * sizeof(ppsk::BatchItem)));
   HIP_TRY(hipMemcpy(pl.items, all.data(), all.size() * sizeof(ppsk::BatchItem),

@@ -155,8 +155,17 @@ DeviceCtx* find_ctx(int device);
 // current device (hipGetSymbolAddress), called once per device at context
 // creation.
 int noalloc_init(void** scratch);
-// Device buffer of at least `need` bytes (reallocated, contents lost).
-int grow(void** ptr, size_t* have, size_t need);
+// Workspaces of a context that a call may free for another one's sake while it
+// holds c->mu and does not use them itself.
+enum Workspace : unsigned {
+  WS_COUNTS = 1, WS_CODES = 2, WS_SEL = 4, WS_HITS = 8, WS_TABLE = 16, WS_SKETCH = 32,
+  WS_PSCRATCH = 64, WS_ALL = 127
+};
+// Workspace of at least `need` bytes (reallocated, contents lost).  Where the
+// device has no room for it, or the context's workspaces would pass
+// PPSK_SCRATCH_BYTES together, the spare blocks of freed sets and then the
+// workspaces in `idle` are given up for it.
+int grow(DeviceCtx* c, void** ptr, size_t* have, size_t need, unsigned idle);
 // Frees a buffer that a call left larger than a context keeps (1 GiB).
 void trim(void** ptr, size_t* have);
 // hipMalloc of a sketch set's stripes, and its release.  A context keeps up to
@@ -165,11 +174,12 @@ void trim(void** ptr, size_t* have);
 // of a call of 2.5 ms), and gives them back when an allocation fails.
 hipError_t set_memory(DeviceCtx* c, size_t bytes, void** out, size_t* got);
 void release_set_memory(DeviceCtx* c, void* p, size_t bytes);
-// hipMalloc that gives the spare blocks back and tries again when it fails.
-hipError_t device_malloc(DeviceCtx* c, void** p, size_t bytes);
-// The same, which before a last try frees the workspaces that no call is using
-// (codes, lists, tables, sketching); locked: the caller holds c->mu.
-hipError_t device_malloc_all(DeviceCtx* c, void** p, size_t bytes, bool locked);
+// hipMalloc that gives the spare blocks back and tries again when it fails, and
+// before a last try frees the workspaces in `idle` (the caller holds c->mu).
+hipError_t device_malloc(DeviceCtx* c, void** p, size_t bytes, unsigned idle = 0);
+// The same with every workspace, once no call is using them; the caller does not
+// hold c->mu.
+hipError_t device_malloc_wait(DeviceCtx* c, void** p, size_t bytes);
 // c->out of at least `need` bytes, at the start of a call.
 int grow_out(DeviceCtx* c, size_t need);
 

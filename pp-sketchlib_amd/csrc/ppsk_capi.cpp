@@ -160,18 +160,40 @@ DeviceCtx* find_ctx(int device) {
   return g_ctx[device];
 }
 
-int grow(void** ptr, size_t* have, size_t need) {
-  if (*have >= need && *ptr) return PPSK_OK;
+// Most bytes of a context's workspaces (PPSK_SCRATCH_BYTES; none: what the device has).
+size_t scratch_limit() {
+  const char* e = std::getenv("PPSK_SCRATCH_BYTES");
+  const long long v = e ? std::atoll(e) : 0;
+  return v > 0 ? (size_t)v : ~(size_t)0;
+}
+
+size_t scratch_held(const DeviceCtx* c) {
+  return c->counts_bytes + c->pscratch_bytes + c->pitems_bytes + c->codes_bytes + c->sel_bytes +
+         c->hits_bytes + c->table_bytes + c->sketch_bytes;
+}
+
+void free_idle(DeviceCtx* c, unsigned idle) {
+  const std::pair<void**, size_t*> ws[] = {{&c->counts, &c->counts_bytes}, {&c->codes, &c->codes_bytes},
+                                           {&c->sel, &c->sel_bytes}, {&c->hits, &c->hits_bytes},
+                                           {&c->table, &c->table_bytes}, {&c->sketch, &c->sketch_bytes},
+                                           {&c->pscratch, &c->pscratch_bytes}};
+  for (int x = 0; x < 7; ++x) {
+    if (!(idle >> x & 1) || !*ws[x].first) continue;
+    hipFree(*ws[x].first);
+    *ws[x].first = nullptr;
+    *ws[x].second = 0;
+  }
+}
+
+int grow(DeviceCtx* c, void** ptr, size_t* have, size_t need, unsigned idle) {
+  const size_t limit = scratch_limit();
+  if (*have >= need && *ptr && scratch_held(c) <= limit) return PPSK_OK;
   if (*ptr) HIP_TRY(hipFree(*ptr));
   *ptr = nullptr;
   *have = 0;
-  hipError_t e = hipMalloc(ptr, need);
-  if (e == hipErrorOutOfMemory) {
-    int device = 0;
-    DeviceCtx* c = hipGetDevice(&device) == hipSuccess ? find_ctx(device) : nullptr;
-    if (c) e = device_malloc(c, ptr, need);
-  }
-  HIP_TRY(e);
+  if (need > limit || scratch_held(c) > limit - need) free_idle(c, idle);
+  const bool room = need <= limit && scratch_held(c) <= limit - need;
+  HIP_TRY(room ? device_malloc(c, ptr, need, idle) : hipErrorOutOfMemory);
   *have = need;
   return PPSK_OK;
 }
@@ -183,7 +205,7 @@ void trim(void** ptr, size_t* have) {
   *have = 0;
 }
 
-hipError_t device_malloc(DeviceCtx* c, void** p, size_t bytes) {
+hipError_t device_malloc(DeviceCtx* c, void** p, size_t bytes, unsigned idle) {
   hipError_t e = hipMalloc(p, bytes);
   if (e != hipErrorOutOfMemory) return e;
   std::vector<std::pair<void*, size_t>> spare;
@@ -191,27 +213,25 @@ hipError_t device_malloc(DeviceCtx* c, void** p, size_t bytes) {
     std::lock_guard<std::mutex> lk(c->spare_mu);
     spare.swap(c->spare);
   }
-  if (spare.empty()) return e;
-  (void)hipGetLastError();
-  for (auto& s : spare) hipFree(s.first);
-  return hipMalloc(p, bytes);
+  if (!spare.empty()) {
+    (void)hipGetLastError();
+    for (auto& s : spare) hipFree(s.first);
+    e = hipMalloc(p, bytes);
+  }
+  if (e == hipErrorOutOfMemory && idle) {
+    (void)hipGetLastError();
+    free_idle(c, idle);
+    e = hipMalloc(p, bytes);
+  }
+  return e;
 }
 
-hipError_t device_malloc_all(DeviceCtx* c, void** p, size_t bytes, bool locked) {
-  hipError_t e = device_malloc(c, p, bytes);
+hipError_t device_malloc_wait(DeviceCtx* c, void** p, size_t bytes) {
+  const hipError_t e = device_malloc(c, p, bytes);
   if (e != hipErrorOutOfMemory) return e;
   (void)hipGetLastError();
-  std::unique_lock<std::mutex> lk(c->mu, std::defer_lock);
-  if (!locked) lk.lock();
-  const std::pair<void**, size_t*> idle[] = {{&c->codes, &c->codes_bytes}, {&c->sel, &c->sel_bytes},
-                                             {&c->hits, &c->hits_bytes}, {&c->table, &c->table_bytes},
-                                             {&c->sketch, &c->sketch_bytes}};
-  for (auto& w : idle) {
-    if (*w.first) hipFree(*w.first);
-    *w.first = nullptr;
-    *w.second = 0;
-  }
-  return hipMalloc(p, bytes);
+  std::lock_guard<std::mutex> lk(c->mu);
+  return device_malloc(c, p, bytes, WS_ALL);
 }
 
 int grow_out(DeviceCtx* c, size_t need) {
@@ -219,10 +239,14 @@ int grow_out(DeviceCtx* c, size_t need) {
   if (c->out) HIP_TRY(hipFree(c->out));
   c->out = nullptr;
   c->out_bytes = 0;
-  HIP_TRY(device_malloc_all(c, &c->out, need, true));
+  HIP_TRY(device_malloc(c, &c->out, need, WS_ALL));
   c->out_bytes = need;
   return PPSK_OK;
 }
+
+// Workspaces free to be given up while a dense pass makes its own (a call's lists
+// and its table may be in use).
+constexpr unsigned PASS_IDLE = WS_CODES | WS_HITS | WS_SKETCH;
 
 constexpr size_t SPARE_BLOCKS = 4, SPARE_BYTES = (size_t)512 << 20;
 
@@ -244,7 +268,7 @@ hipError_t set_memory(DeviceCtx* c, size_t bytes, void** out, size_t* got) {
     }
   }
   *got = bytes;
-  return device_malloc_all(c, out, bytes, false);
+  return device_malloc_wait(c, out, bytes);
 }
 
 void release_set_memory(DeviceCtx* c, void* p, size_t bytes) {
@@ -273,7 +297,7 @@ int grow_tile_done(DeviceCtx* c, size_t n) {
   if (c->tile_done) HIP_TRY(hipFree(c->tile_done));
   c->tile_done = nullptr;
   c->tile_done_n = 0;
-  HIP_TRY(hipMalloc(&c->tile_done, n * sizeof(uint32_t)));
+  HIP_TRY(device_malloc(c, (void**)&c->tile_done, n * sizeof(uint32_t), PASS_IDLE));
   // counters are left at zero by every tile's last workgroup afterwards
   HIP_TRY(hipMemset(c->tile_done, 0, n * sizeof(uint32_t)));
   c->tile_done_n = n;
@@ -455,11 +479,11 @@ int run_dense_tiles(DeviceCtx* c, ppsk::DistParams p, int variant, bool upper, i
   }
   size_t most = 0;
   for (auto& ch : chunks) most = std::max(most, ch.second - ch.first);
-  if (int rc = grow(&c->counts, &c->counts_bytes, most * per_tile)) return rc;
+  if (int rc = grow(c, &c->counts, &c->counts_bytes, most * per_tile, PASS_IDLE | WS_PSCRATCH)) return rc;
   if (int rc = grow_tile_done(c, most)) return rc;
   void* tptr = c->tiles;
   size_t tbytes = c->tiles_n * sizeof(ppsk::Tile);
-  if (int rc = grow(&tptr, &tbytes, tiles.size() * sizeof(ppsk::Tile))) return rc;
+  if (int rc = grow(c, &tptr, &tbytes, tiles.size() * sizeof(ppsk::Tile), PASS_IDLE)) return rc;
   c->tiles = (ppsk::Tile*)tptr;
   c->tiles_n = tbytes / sizeof(ppsk::Tile);
   HIP_TRY(copy_to_device(c, c->tiles, tiles.data(), tiles.size() * sizeof(ppsk::Tile), c->stream));
@@ -583,18 +607,20 @@ int run_dense_persistent(DeviceCtx* c, ppsk::DistParams p, int variant, bool upp
   // per-workgroup count blocks (the mixed-shape kernel's hold 64 x 256 counts)
   const size_t scratch = (size_t)grid * p.n_k * (kernel == ppsk::BATCH_MIXED ? 64 * 256 : tr * tc) *
                          sizeof(uint16_t);
-  if (int rc = grow(&c->pscratch, &c->pscratch_bytes, scratch)) return rc;
-  if (int rc = grow(&c->pitems, &c->pitems_bytes, items.size() * sizeof(ppsk::BatchItem))) return rc;
+  if (int rc = grow(c, &c->pscratch, &c->pscratch_bytes, scratch, PASS_IDLE)) return rc;
+  if (int rc = grow(c, &c->pitems, &c->pitems_bytes, items.size() * sizeof(ppsk::BatchItem), PASS_IDLE)) {
+    return rc;
+  }
   if (!c->pparams) HIP_TRY(hipMalloc(&c->pparams, sizeof(ppsk::DistParams)));
   if (!c->pqueue) HIP_TRY(hipMalloc(&c->pqueue, ppsk::BATCH_QUEUES * sizeof(uint32_t)));
   p.out_row_offset = 0;
   if (most_tail > 0) {
     const size_t per_tile = (size_t)p.n_k * tr * tc * sizeof(uint16_t);
-    if (int rc = grow(&c->counts, &c->counts_bytes, most_tail * per_tile)) return rc;
+    if (int rc = grow(c, &c->counts, &c->counts_bytes, most_tail * per_tile, PASS_IDLE)) return rc;
     if (int rc = grow_tile_done(c, most_tail)) return rc;
     void* tptr = c->tiles;
     size_t tbytes = c->tiles_n * sizeof(ppsk::Tile);
-    if (int rc = grow(&tptr, &tbytes, tail_tiles.size() * sizeof(ppsk::Tile))) return rc;
+    if (int rc = grow(c, &tptr, &tbytes, tail_tiles.size() * sizeof(ppsk::Tile), PASS_IDLE)) return rc;
     c->tiles = (ppsk::Tile*)tptr;
     c->tiles_n = tbytes / sizeof(ppsk::Tile);
     HIP_TRY(copy_to_device(c, c->tiles, tail_tiles.data(), tail_tiles.size() * sizeof(ppsk::Tile),
@@ -883,11 +909,31 @@ ItemPlan plan_items(int64_t n_cols, int n_k, int s64, bool upper, bool same_set,
 // themselves are 6.8 GiB, so that such a pass is one launch.
 constexpr size_t CODE_BUDGET = (size_t)8 << 30;
 
+// Scratch of a plan, in place for one launch after the other: counts, the slab
+// and tile lists, codes.  false: the device has no room for it (counts and codes are
+// given back then).
+bool item_scratch(DeviceCtx* c, const ItemPlan& pl) {
+  if (pl.tiles.empty()) return true;
+  const unsigned idle = PASS_IDLE | WS_PSCRATCH;
+  const size_t counts = pl.count_blocks * ppsk::ITEM_COUNTS * sizeof(uint16_t);
+  const size_t lists = pl.slabs.size() * sizeof(ppsk::CodeGroup) + pl.tiles.size() * sizeof(ppsk::ItemTile);
+  if (grow(c, &c->counts, &c->counts_bytes, counts, idle) == PPSK_OK &&
+      grow(c, &c->pitems, &c->pitems_bytes, lists, idle) == PPSK_OK &&
+      (pl.code_bytes == 0 ||
+       grow(c, &c->codes, &c->codes_bytes, pl.code_bytes, idle & ~WS_CODES) == PPSK_OK)) {
+    return true;
+  }
+  (void)hipGetLastError();
+  free_idle(c, WS_CODES | WS_COUNTS);
+  return false;
+}
+
 // The plan a pass runs: coded when that pays, its scratch in place.  Where the
-// device has no room for the budget the slabs shrink, down to 256 MiB; below
-// that the pass runs on the planes as they are.
-int make_item_plan(DeviceCtx* c, const ppsk::DistParams& p, bool upper, int64_t row_begin,
-                   int64_t row_end, bool host_out, ItemPlan* out) {
+// device has no room for the scratch of a plan the slabs shrink, down to 256 MiB
+// of codes; below that the pass runs on the planes as they are.  false: no room
+// for that either.
+bool make_item_plan(DeviceCtx* c, const ppsk::DistParams& p, bool upper, int64_t row_begin,
+                    int64_t row_end, bool host_out, ItemPlan* out) {
   const bool same = upper;  // the upper triangle of one set
   uint64_t planned = 0;     // what dense_items reported
   if (use_coded(row_end - row_begin, p.n_cols, upper)) {
@@ -896,34 +942,29 @@ int make_item_plan(DeviceCtx* c, const ppsk::DistParams& p, bool upper, int64_t 
       if (planned == 0) planned = out->items;
       call_state(c->device).total += out->items - planned;
       planned = out->items;
-      if (out->code_bytes <= c->codes_bytes) return PPSK_OK;
       if (out->code_bytes > budget) break;  // one block of columns exceeds it
-      if (c->codes) HIP_TRY(hipFree(c->codes));
-      c->codes = nullptr;
-      c->codes_bytes = 0;
-      if (device_malloc(c, &c->codes, out->code_bytes) == hipSuccess) {
-        c->codes_bytes = out->code_bytes;
-        return PPSK_OK;
-      }
-      (void)hipGetLastError();  // no room: the next smaller budget
+      if (item_scratch(c, *out)) return true;
     }
   }
   *out = plan_items(p.n_cols, p.n_k, p.s64, upper, same, row_begin, row_end, host_out, false, 0);
   if (planned) call_state(c->device).total += out->items - planned;
-  return PPSK_OK;
+  return item_scratch(c, *out);
 }
 
 // The split pass: every tile's words cut into runs when there are too few
 // (tile, k-mer length) items to fill the CUs, then one lane per pair for the
 // output.  With host_out, each launch's finished rows are copied out while the
-// next ones compute.
+// next ones compute.  *made: false when the device has no room for its scratch;
+// nothing has been launched then.
 int run_dense_items(DeviceCtx* c, ppsk::DistParams p, bool upper, int64_t row_begin,
-                    int64_t row_end, bool self, size_t elem, void* host_out, Timing* tm) {
+                    int64_t row_end, bool self, size_t elem, void* host_out, Timing* tm, bool* made) {
   ItemPlan pl;
-  if (int rc = make_item_plan(c, p, upper, row_begin, row_end, host_out != nullptr, &pl)) return rc;
+  *made = make_item_plan(c, p, upper, row_begin, row_end, host_out != nullptr, &pl);
+  if (!*made) {
+    call_state(c->device).total -= pl.items;
+    return PPSK_OK;
+  }
   if (pl.tiles.empty()) return PPSK_OK;
-  const size_t item_bytes = ppsk::ITEM_COUNTS * sizeof(uint16_t);
-  if (int rc = grow(&c->counts, &c->counts_bytes, pl.count_blocks * item_bytes)) return rc;
   // one upload: the slab table, then the tiles
   const size_t slab_bytes = pl.coded ? pl.slabs.size() * sizeof(ppsk::CodeGroup) : 0;
   std::vector<char> lists(slab_bytes + pl.tiles.size() * sizeof(ppsk::ItemTile));
@@ -947,7 +988,6 @@ int run_dense_items(DeviceCtx* c, ppsk::DistParams p, bool upper, int64_t row_be
     std::memcpy(lists.data(), pl.slabs.data(), slab_bytes);
   }
   std::memcpy(lists.data() + slab_bytes, pl.tiles.data(), pl.tiles.size() * sizeof(ppsk::ItemTile));
-  if (int rc = grow(&c->pitems, &c->pitems_bytes, lists.size())) return rc;
   HIP_TRY(copy_to_device(c, c->pitems, lists.data(), lists.size(), c->stream));
   const ppsk::CodeGroup* d_slabs = (const ppsk::CodeGroup*)c->pitems;
   const ppsk::ItemTile* d_tiles = (const ppsk::ItemTile*)((char*)c->pitems + slab_bytes);
@@ -1002,21 +1042,27 @@ int run_dense_items(DeviceCtx* c, ppsk::DistParams p, bool upper, int64_t row_be
 // per-(tile, k-mer length) or the persistent kernel of that shape.
 enum class Route { persistent, tiles, items };
 
+// Whole tiles: the persistent kernel, or with fewer than two tiles per resident
+// workgroup one workgroup per (tile, k-mer length).
+Route tile_route(int variant, bool upper, int64_t rows, int64_t n_cols) {
+  if (variant != 2 && variant != 4 && variant != 5) return Route::tiles;
+  const int tr = ppsk::variant_tile_rows(variant), tc = ppsk::variant_tile_cols(variant);
+  const int64_t rt = (rows + tr - 1) / tr, ct = (n_cols + tc - 1) / tc;
+  const int64_t tiles = upper ? rt * ct / 2 : rt * ct;
+  int grid = 0;
+  if (ppsk::batch_grid(variant == 5 ? ppsk::BATCH_MIXED : variant, &grid) != hipSuccess) grid = 0;
+  return grid > 0 && tiles >= 2 * (int64_t)grid ? Route::persistent : Route::tiles;
+}
+
 Route dense_route(int variant, bool upper, int64_t rows, int64_t n_cols) {
-  const char* e = std::getenv("PPSK_PERSISTENT");
-  const bool can = variant == 2 || variant == 4 || variant == 5;
-  if (e) return can && std::atoi(e) != 0 ? Route::persistent : Route::tiles;
+  if (const char* e = std::getenv("PPSK_PERSISTENT")) {
+    const bool can = variant == 2 || variant == 4 || variant == 5;
+    return can && std::atoi(e) != 0 ? Route::persistent : Route::tiles;
+  }
   const bool shape = std::getenv("PPSK_TILE_VARIANT") != nullptr;
   if (!shape && use_coded(rows, n_cols, upper)) return Route::items;
-  if (can) {
-    const int tr = ppsk::variant_tile_rows(variant), tc = ppsk::variant_tile_cols(variant);
-    const int64_t rt = (rows + tr - 1) / tr, ct = (n_cols + tc - 1) / tc;
-    const int64_t tiles = upper ? rt * ct / 2 : rt * ct;
-    int grid = 0;
-    if (ppsk::batch_grid(variant == 5 ? ppsk::BATCH_MIXED : variant, &grid) != hipSuccess) grid = 0;
-    if (grid > 0 && tiles >= 2 * (int64_t)grid) return Route::persistent;
-  }
-  return shape ? Route::tiles : Route::items;
+  const Route r = tile_route(variant, upper, rows, n_cols);
+  return r == Route::tiles && !shape ? Route::items : r;
 }
 
 // Work items a dense pass reports as progress.
@@ -1035,15 +1081,20 @@ uint64_t dense_items(const ppsk_set* rows, const ppsk_set* cols, bool upper, int
 int run_dense(DeviceCtx* c, ppsk::DistParams p, int variant, bool upper, int64_t row_begin,
               int64_t row_end, bool self, size_t elem, void* host_out, Timing* tm) {
   c->words_read = false;
-  switch (dense_route(variant, upper, row_end - row_begin, p.n_cols)) {
-    case Route::persistent:
-      return run_dense_persistent(c, p, variant, upper, row_begin, row_end, self, elem, host_out,
-                                  tm);
-    case Route::items:
-      return run_dense_items(c, p, upper, row_begin, row_end, self, elem, host_out, tm);
-    default:
-      return run_dense_tiles(c, p, variant, upper, row_begin, row_end, self, elem, host_out, tm);
+  Route r = dense_route(variant, upper, row_end - row_begin, p.n_cols);
+  if (r == Route::items) {
+    bool made = false;
+    const int rc = run_dense_items(c, p, upper, row_begin, row_end, self, elem, host_out, tm, &made);
+    if (rc || made) return rc;
+    // no room for a split pass's counts: whole tiles need less (8,192 samples at
+    // 8 k-mer lengths 0.2 GiB against 0.5, 48 samples 256 KiB against 9 MiB)
+    r = tile_route(variant, upper, row_end - row_begin, p.n_cols);
+    call_state(c->device).total += pass_items(row_end - row_begin, p.n_cols, p.n_k, variant, upper);
   }
+  if (r == Route::persistent) {
+    return run_dense_persistent(c, p, variant, upper, row_begin, row_end, self, elem, host_out, tm);
+  }
+  return run_dense_tiles(c, p, variant, upper, row_begin, row_end, self, elem, host_out, tm);
 }
 
 void fill_common(ppsk::DistParams& p, const ppsk_set* rows, const ppsk_set* cols,
@@ -1096,7 +1147,7 @@ int call_table(DeviceCtx* c, const ppsk_set* s, const RandomIn& rnd, float** dta
   *dtab = nullptr;
   if (rnd.mode != PPSK_RANDOM_MC) return PPSK_OK;
   const size_t bytes = (size_t)s->n_k * rnd.n_clusters * rnd.n_clusters * sizeof(float);
-  if (int rc = grow(&c->table, &c->table_bytes, bytes)) return rc;
+  if (int rc = grow(c, &c->table, &c->table_bytes, bytes, WS_ALL & ~WS_TABLE)) return rc;
   *dtab = (float*)c->table;
   HIP_TRY(copy_to_device(c, *dtab, rnd.table, bytes, c->stream));
   return PPSK_OK;
@@ -1162,7 +1213,8 @@ struct KnnLists {
 int knn_lists(DeviceCtx* c, int64_t rows, int kNN, KnnLists* L) {
   const size_t m = ((size_t)rows * kNN + 31) / 32 * 32;
   const size_t hw = ppsk::knn_heap_workspace(rows, kNN);
-  if (int rc = grow(&c->sel, &c->sel_bytes, m * (2 * sizeof(int64_t) + sizeof(float)) + hw)) return rc;
+  const size_t bytes = m * (2 * sizeof(int64_t) + sizeof(float)) + hw;
+  if (int rc = grow(c, &c->sel, &c->sel_bytes, bytes, WS_ALL & ~(WS_SEL | WS_TABLE))) return rc;
   L->i = (int64_t*)c->sel;
   L->j = L->i + m;
   L->d = (float*)(L->j + m);
@@ -1201,7 +1253,10 @@ int threshold_from_triangle(DeviceCtx* c, const float2* tri, int64_t n, int col,
   int64_t total = 0;
   hipError_t e = hipSuccess;
   if (rows > 0) {
-    if (int rc = grow(&c->sel, &c->sel_bytes, (size_t)(rows + 1) * sizeof(int64_t))) return rc;
+    if (int rc = grow(c, &c->sel, &c->sel_bytes, (size_t)(rows + 1) * sizeof(int64_t),
+                      WS_ALL & ~WS_SEL)) {
+      return rc;
+    }
     int64_t* counts = (int64_t*)c->sel;
     e = ppsk::launch_threshold_count(tri, rows, n, false, col, cutoff, counts, c->stream);
     if (e == hipSuccess) e = ppsk::launch_offsets_scan(counts, rows, c->stream);
@@ -1213,7 +1268,8 @@ int threshold_from_triangle(DeviceCtx* c, const float2* tri, int64_t n, int col,
   auto* hd = (float*)std::malloc(std::max<int64_t>(total, 1) * sizeof(float));
   if (hi && hj && hd && total > 0) {
     const size_t m = (size_t)total;
-    if (int rc = grow(&c->hits, &c->hits_bytes, m * (2 * sizeof(int64_t) + sizeof(float)))) {
+    if (int rc = grow(c, &c->hits, &c->hits_bytes, m * (2 * sizeof(int64_t) + sizeof(float)),
+                      WS_ALL & ~(WS_SEL | WS_HITS))) {
       std::free(hi);
       std::free(hj);
       std::free(hd);
@@ -1343,7 +1399,13 @@ int ppsk_set_upload(ppsk_set* s, int64_t first, int64_t count, const uint64_t* r
   std::lock_guard<std::mutex> lk(c->upload_mu);
   const int64_t chunk = std::min<int64_t>(count, std::max<int64_t>(1, (int64_t)((32u << 20) / per_sample)));
   const size_t half = ((size_t)chunk * per_sample + 255) / 256 * 256;
-  if (int rc = grow(&c->raw, &c->raw_bytes, 2 * half)) return rc;
+  if (c->raw_bytes < 2 * half) {
+    if (c->raw) HIP_TRY(hipFree(c->raw));
+    c->raw = nullptr;
+    c->raw_bytes = 0;
+    HIP_TRY(device_malloc_wait(c, &c->raw, 2 * half));
+    c->raw_bytes = 2 * half;
+  }
   hipError_t e = hipSuccess;
   int turn = 0;
   for (int64_t c0 = 0; c0 < count && e == hipSuccess; c0 += chunk, turn ^= 1) {
@@ -1391,7 +1453,7 @@ int ppsk_set_meta(ppsk_set* s, const uint64_t* lengths, int32_t use_rc, const ui
         jv[(size_t)i * s->n_k + kk] = 1 - std::pow(base, (double)lengths[i]);
       }
     }
-    if (!s->jv) HIP_TRY(hipMalloc(&s->jv, jv.size() * sizeof(double)));
+    if (!s->jv) HIP_TRY(device_malloc_wait(c, (void**)&s->jv, jv.size() * sizeof(double)));
     HIP_TRY(copy_to_device(c, s->jv, jv.data(), jv.size() * sizeof(double), c->stream));
     HIP_TRY(hipStreamSynchronize(c->stream));
     s->has_lengths = true;
@@ -1400,7 +1462,7 @@ int ppsk_set_meta(ppsk_set* s, const uint64_t* lengths, int32_t use_rc, const ui
   if (clusters) {
     s->max_cluster = 0;
     for (int64_t i = 0; i < s->n; ++i) s->max_cluster = std::max<int32_t>(s->max_cluster, clusters[i]);
-    if (!s->clusters) HIP_TRY(hipMalloc(&s->clusters, (size_t)s->n * sizeof(uint16_t)));
+    if (!s->clusters) HIP_TRY(device_malloc_wait(c, (void**)&s->clusters, (size_t)s->n * sizeof(uint16_t)));
     HIP_TRY(copy_to_device(c, s->clusters, clusters, (size_t)s->n * sizeof(uint16_t), c->stream));
     HIP_TRY(hipStreamSynchronize(c->stream));
   }
@@ -1731,7 +1793,7 @@ int ppsk_host_free(void* ptr) {
 int ppsk_device_alloc(int device_id, size_t bytes, void** ptr) {
   DeviceCtx* c = nullptr;
   if (int rc = get_ctx(device_id, &c)) return rc;
-  HIP_TRY(device_malloc_all(c, ptr, bytes, false));
+  HIP_TRY(device_malloc_wait(c, ptr, bytes));
   return PPSK_OK;
 }
 

@@ -886,7 +886,7 @@ int ppsk_server_create(ppsk_set* ref, int32_t random_mode, int32_t n_clusters,
   }
   if (random_mode == PPSK_RANDOM_MC) {
     const size_t tb = (size_t)ref->n_k * n_clusters * n_clusters * sizeof(float);
-    hipError_t et = hipMalloc(&s->d_table, tb);
+    hipError_t et = device_malloc_wait(c, (void**)&s->d_table, tb);
     if (et == hipSuccess) et = hipMemcpy(s->d_table, mc_table, tb, hipMemcpyHostToDevice);
     if (et != hipSuccess) {
       if (s->d_table) hipFree(s->d_table);
@@ -894,7 +894,7 @@ int ppsk_server_create(ppsk_set* ref, int32_t random_mode, int32_t n_clusters,
       return fail(PPSK_ERR_MEMORY, std::string("serving Monte Carlo table: ") + hipGetErrorString(et));
     }
   }
-  hipError_t e = device_malloc_all(c, &s->arena_mem, arena_bytes, false);
+  hipError_t e = device_malloc_wait(c, &s->arena_mem, arena_bytes);
   if (e != hipSuccess) {
     if (s->d_table) hipFree(s->d_table);
     delete s;

@@ -209,7 +209,7 @@ int sketch_impl(int device_id, int64_t n_samples, const char* seq, int64_t seq_b
   const size_t at_stats = parts.take(stats * (sizeof(double) + sizeof(int32_t)));
   const size_t at_next = parts.take(sizeof(int));
   const size_t at_ws = parts.take(ws_bytes);
-  if (int rc = grow(&c->sketch, &c->sketch_bytes, parts.used)) return rc;
+  if (int rc = grow(c, &c->sketch, &c->sketch_bytes, parts.used, WS_ALL & ~WS_SKETCH)) return rc;
   struct Trim {
     DeviceCtx* c;
     ~Trim() {
