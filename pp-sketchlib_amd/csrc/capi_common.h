@@ -92,8 +92,9 @@ struct DeviceCtx {
   size_t pitems_bytes = 0;
   ppsk::DistParams* pparams = nullptr;  // the call's parameters in device memory
   uint32_t* pqueue = nullptr;         // queue counters
-  void* codes = nullptr;              // codes of a coded pass (at most CODE_BUDGET)
-  size_t codes_bytes = 0;
+  void* codes = nullptr;              // codes of a coded pass (at most CODE_BUDGET); above 1 GiB
+  size_t codes_bytes = 0;             // kept while a sketch set lives (give_back)
+  std::atomic<int> sets{0};           // sketch sets alive
   hipStream_t tail_stream = nullptr;  // the tail's (tile, k) launch beside the persistent one
   void* noalloc_scratch = nullptr;    // this device's copy of the fixed scratch array
   void* table = nullptr;              // Monte Carlo table of a dense pass

@@ -6,6 +6,10 @@ below that it runs with fewer codes at a time, then on the planes, then as
 whole tiles, which took 80 MiB before passes were split.  Every route computes the
 same 64-bit expressions from the same exact counts, so every byte is the same.
 """
+import os
+import subprocess
+import sys
+
 import numpy as np
 import pytest
 
@@ -58,3 +62,25 @@ def test_no_scratch_is_an_error(sets, monkeypatch):
         assert e.value.code == H.ERR_MEMORY
     monkeypatch.delenv("PPSK_SCRATCH_BYTES")
     assert _same(H.dense(s, **kw)[0], dense)
+
+
+def test_codes_go_back_with_the_last_set(sets):
+    # 4,608 samples: about 1.7 GiB of codes.  With the module's sets alive they stay
+    # for the next pass; a program that has freed its sets gets them back.
+    code = """if True:
+        import ppsk_hip as H
+        kl = list(range(15, 30, 2))
+        raw, _, _ = H.synth(4608, kl, 156, seed=2)
+        for _ in range(2):
+            s = H.SketchSet(raw, kl, 156)
+            d, _ = H.dense_device(s)
+            alive = H.device_init(0)[0]
+            H.device_free(d)
+            s.free()
+            print(H.device_init(0)[0] - alive)
+    """
+    out = subprocess.run([sys.executable, "-c", code], check=True, capture_output=True, text=True,
+                         env={**os.environ, "PYTHONPATH": os.pathsep.join(sys.path)}, timeout=100).stdout
+    stripes = 8 * 36 * 156 * 28 * 128 * 4
+    for freed in map(int, out.split()):
+        assert freed > stripes + 4608 * 4607 // 2 * 8 + (1 << 30)
