@@ -266,12 +266,12 @@ constexpr int64_t SPLIT_BLOCKS = 32768;  // counts of a split plan: 1 GiB
 // Plan 6 as a split pass: every unit's (k-mer length, word run, tile) items,
 // cut into 8 runs like the tiles of the other plans, one for each XCD; the
 // workgroups of a launch go to the XCDs in turn.  Words per item: about 2,400
-// items of equal time in all, at least 8 words (item_runs has the measurements
-// of both).  *made: false when the counts would not fit.
+// items of equal time in all, at least 8 words (cut_items has the measurements
+// of both).  *made: false when the counts or the lists would not fit.
 int build_split(ppsk_batch* b, ppsk_batch::Plan& pl, DeviceCtx* c, bool* made) {
   *made = false;
   const std::vector<Unit> units = plan_units(b, ppsk::BATCH_MIXED);
-  // time of one word of a tile, in 64-row tiles (item_runs)
+  // time of one word of a tile, in 64-row tiles (cut_items)
   auto weight = [](int shape) { return shape == 2 ? 1.0 : (shape == 4 ? 0.57 : 0.37); };
   std::vector<std::vector<ppsk::Tile>> ut;
   double total = 0.0;
@@ -301,8 +301,7 @@ int build_split(ppsk_batch* b, ppsk_batch::Plan& pl, DeviceCtx* c, bool* made) {
     for (int qi = 0; qi < ppsk::BATCH_QUEUES; ++qi) {
       for (int64_t i = items * qi / ppsk::BATCH_QUEUES; i < items * (qi + 1) / ppsk::BATCH_QUEUES; ++i) {
         const int t = t0 + (int)(i % n), ky = (int)(i / n), kk = ky / runs, y = ky % runs;
-        const int w0 = y * words;
-        if (w0 >= r->s64) continue;  // (runs * words may pass the last word by a run)
+        const int w0 = y * words;  // < s64: (runs - 1) * words < s64 by the choice of runs
         q[qi].push_back({t, kk, w0, std::min(words, r->s64 - w0), tiles[t].block0 + ky});
         ++n_items;
       }
@@ -314,15 +313,21 @@ int build_split(ppsk_batch* b, ppsk_batch::Plan& pl, DeviceCtx* c, bool* made) {
   for (int qi = 0; qi < ppsk::BATCH_QUEUES; ++qi) {
     for (size_t i = 0; i < q[qi].size(); ++i) all[i * ppsk::BATCH_QUEUES + qi] = q[qi][i];
   }
-  // no room for the counts: the persistent kernel, which needs none
-  if (hipMalloc(&pl.counts, (size_t)std::max<int64_t>(blocks, 1) * ppsk::ITEM_COUNTS *
-                                sizeof(uint16_t)) != hipSuccess) {
+  // no room: the persistent kernel, which keeps no counts of whole tiles
+  const size_t count_bytes = (size_t)std::max<int64_t>(blocks, 1) * ppsk::ITEM_COUNTS * sizeof(uint16_t);
+  hipError_t e = scratch_malloc(c, (void**)&pl.counts, count_bytes, WS_ALL);
+  if (e == hipSuccess) {
+    e = device_malloc(c, (void**)&pl.tiles, std::max<size_t>(tiles.size(), 1) * sizeof(ppsk::BatchTile), WS_ALL);
+  }
+  if (e == hipSuccess) {
+    e = device_malloc(c, (void**)&pl.runs, std::max<size_t>(all.size(), 1) * sizeof(ppsk::BatchRun), WS_ALL);
+  }
+  if (e == hipErrorOutOfMemory) {
     (void)hipGetLastError();
-    pl.counts = nullptr;
+    free_plan(pl);
     return PPSK_OK;
   }
-  HIP_TRY(hipMalloc(&pl.tiles, std::max<size_t>(tiles.size(), 1) * sizeof(ppsk::BatchTile)));
-  HIP_TRY(hipMalloc(&pl.runs, std::max<size_t>(all.size(), 1) * sizeof(ppsk::BatchRun)));
+  HIP_TRY(e);
   HIP_TRY(hipMemcpy(pl.tiles, tiles.data(), tiles.size() * sizeof(ppsk::BatchTile), hipMemcpyHostToDevice));
   HIP_TRY(hipMemcpy(pl.runs, all.data(), all.size() * sizeof(ppsk::BatchRun), hipMemcpyHostToDevice));
   ppsk::BatchItemArgs a;
@@ -345,12 +350,8 @@ int build_split(ppsk_batch* b, ppsk_batch::Plan& pl, DeviceCtx* c, bool* made) {
   return capture_plan(b, pl, c, [&] { return ppsk::launch_batch_items(a, c->stream); });
 }
 
-int build_plan(ppsk_batch* b, int plan) {
-  auto& pl = b->plans[plan];
-  if (pl.exec) return PPSK_OK;
+int make_plan(ppsk_batch* b, ppsk_batch::Plan& pl, int plan, DeviceCtx* c) {
   const int kernel = plan_kernel(plan);
-  DeviceCtx* c = nullptr;
-  if (int rc = get_ctx(b->device, &c)) return rc;
   if (plan == ppsk::BATCH_MIXED) {
     bool made = false;
     if (int rc = build_split(b, pl, c, &made)) return rc;
@@ -391,7 +392,8 @@ int build_plan(ppsk_batch* b, int plan) {
     }
     HIP_TRY(device_malloc(c, (void**)&b->scratch, need, WS_ALL));
   }
-  HIP_TRY(hipMalloc(&pl.items, std::max<size_t>(all.size(), 1) * sizeof(ppsk::BatchItem)));
+  HIP_TRY(device_malloc(c, (void**)&pl.items, std::max<size_t>(all.size(), 1) * sizeof(ppsk::BatchItem),
+                        WS_ALL));
   HIP_TRY(hipMemcpy(pl.items, all.data(), all.size() * sizeof(ppsk::BatchItem),
                     hipMemcpyHostToDevice));
   ppsk::BatchArgs a;
@@ -404,6 +406,16 @@ int build_plan(ppsk_batch* b, int plan) {
   a.max_k = b->max_k;
   a.ctl = c->ctl;
   return capture_plan(b, pl, c, [&] { return ppsk::launch_batch(a, kernel, pl.grid, c->stream); });
+}
+
+int build_plan(ppsk_batch* b, int plan) {
+  auto& pl = b->plans[plan];
+  if (pl.exec) return PPSK_OK;
+  DeviceCtx* c = nullptr;
+  if (int rc = get_ctx(b->device, &c)) return rc;
+  const int rc = make_plan(b, pl, plan, c);
+  if (rc) free_plan(pl);  // made anew by the next try
+  return rc;
 }
 
 int run_plan(ppsk_batch* b, int plan, double* ms) {
@@ -466,9 +478,11 @@ int ppsk_batch_create(int device_id, const ppsk_job* jobs, int32_t n_jobs, ppsk_
   b->params.resize(n_jobs);
   b->tables.assign(n_jobs, nullptr);
   int rc = PPSK_OK;
-  hipError_t e = hipMalloc(&b->d_fail, (size_t)n_jobs * 2 * sizeof(unsigned long long));
-  if (e == hipSuccess) e = hipMalloc(&b->d_queue, ppsk::BATCH_QUEUES * sizeof(uint32_t));
-  if (e == hipSuccess) e = hipMalloc(&b->d_params, (size_t)n_jobs * sizeof(ppsk::DistParams));
+  hipError_t e = device_malloc(c, (void**)&b->d_fail, (size_t)n_jobs * 2 * sizeof(unsigned long long), WS_ALL);
+  if (e == hipSuccess) e = device_malloc(c, (void**)&b->d_queue, ppsk::BATCH_QUEUES * sizeof(uint32_t), WS_ALL);
+  if (e == hipSuccess) {
+    e = device_malloc(c, (void**)&b->d_params, (size_t)n_jobs * sizeof(ppsk::DistParams), WS_ALL);
+  }
   if (e != hipSuccess) rc = fail(PPSK_ERR_MEMORY, "batch buffers");
   for (int j = 0; j < n_jobs && rc == PPSK_OK; ++j) {
     const ppsk_job& jb = jobs[j];

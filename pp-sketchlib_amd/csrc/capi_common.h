@@ -169,6 +169,8 @@ enum Workspace : unsigned {
 int grow(DeviceCtx* c, void** ptr, size_t* have, size_t need, unsigned idle);
 // Frees a buffer that a call left larger than a context keeps (1 GiB).
 void trim(void** ptr, size_t* have);
+// The allocation of grow, for scratch that another object keeps.
+hipError_t scratch_malloc(DeviceCtx* c, void** p, size_t bytes, unsigned idle);
 // hipMalloc of a sketch set's stripes, and its release.  A context keeps up to
 // 4 blocks of freed sets, together at most 512 MiB, for the next sets of about
 // their size (a set of 333 samples, 47 MB: hipMalloc 0.5 ms and hipFree 0.2 ms

@@ -185,15 +185,19 @@ void free_idle(DeviceCtx* c, unsigned idle) {
   }
 }
 
-int grow(DeviceCtx* c, void** ptr, size_t* have, size_t need, unsigned idle) {
+hipError_t scratch_malloc(DeviceCtx* c, void** p, size_t bytes, unsigned idle) {
   const size_t limit = scratch_limit();
-  if (*have >= need && *ptr && scratch_held(c) <= limit) return PPSK_OK;
+  if (bytes > limit || scratch_held(c) > limit - bytes) free_idle(c, idle);
+  const bool room = bytes <= limit && scratch_held(c) <= limit - bytes;
+  return room ? device_malloc(c, p, bytes, idle) : hipErrorOutOfMemory;
+}
+
+int grow(DeviceCtx* c, void** ptr, size_t* have, size_t need, unsigned idle) {
+  if (*have >= need && *ptr && scratch_held(c) <= scratch_limit()) return PPSK_OK;
   if (*ptr) HIP_TRY(hipFree(*ptr));
   *ptr = nullptr;
   *have = 0;
-  if (need > limit || scratch_held(c) > limit - need) free_idle(c, idle);
-  const bool room = need <= limit && scratch_held(c) <= limit - need;
-  HIP_TRY(room ? device_malloc(c, ptr, need, idle) : hipErrorOutOfMemory);
+  HIP_TRY(scratch_malloc(c, ptr, need, idle));
   *have = need;
   return PPSK_OK;
 }
@@ -1148,7 +1152,7 @@ int upload_table(DeviceCtx* c, const ppsk_set* s, const RandomIn& rnd, float** d
   *dtab = nullptr;
   if (rnd.mode != PPSK_RANDOM_MC) return PPSK_OK;
   const size_t bytes = (size_t)s->n_k * rnd.n_clusters * rnd.n_clusters * sizeof(float);
-  HIP_TRY(device_malloc(c, (void**)dtab, bytes));
+  HIP_TRY(device_malloc(c, (void**)dtab, bytes, WS_ALL));
   HIP_TRY(copy_to_device(c, *dtab, rnd.table, bytes, c->stream));
   return PPSK_OK;
 }
