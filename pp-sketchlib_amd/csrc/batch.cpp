@@ -586,6 +586,8 @@ int ppsk_batch_run(ppsk_batch* b, int32_t variant, uint64_t* n_fail, int32_t* us
     if (v == 0) v = b->variant;
     if (int rc = run_plan(b, v, &ms)) return rc;
   }
+  // another plan was chosen: the split one keeps no counts (up to 1 GiB)
+  if (variant == 0 && v != ppsk::BATCH_MIXED) free_plan(b->plans[ppsk::BATCH_MIXED]);
   std::vector<unsigned long long> f((size_t)b->n_jobs * 2);
   HIP_TRY(copy_to_host(c, f.data(), b->d_fail, f.size() * sizeof(unsigned long long), c->stream));
   uint64_t total = 0;

@@ -28,6 +28,24 @@ def _batch(ref, qry, rows):
     return H.Batch([dict(ref=ref, query=qry.prefix(rows), out="counts")])
 
 
+def test_losing_plan_gives_its_counts_back(sets, monkeypatch):
+    # up to 0.7 GiB of counts as plan 6, which whole tiles do without
+    ref, qry = sets
+    with _batch(ref, qry, 4000) as b:
+        b.run(2)  # builds what plan 2 keeps
+        before = _free()
+        b.run(6)
+        assert before - _free() > 300 << 20
+        want = b.result(0)
+        monkeypatch.setenv("PPSK_BATCH_VARIANT", "2")  # as if plan 2 had been the fastest
+        _, used, _ = b.run()
+        assert used == 2
+        assert before - _free() < 100 << 20
+        for plan in (2, 6):
+            b.run(plan)
+            assert np.array_equal(b.result(0), want)
+
+
 def test_split_plan_without_room(sets, monkeypatch):
     ref, qry = sets
     with _batch(ref, qry, 1000) as b:
