@@ -54,8 +54,6 @@ int fail(int code, const std::string& msg);
     }                                                                              \
   } while (0)
 
-// Per-device state: a launch stream, a copy stream, cached workspaces grown on
-// demand.
 // Page-locked blocks that host copies go through (host_io.cpp): two for each of
 // up to LANES copying threads of one copy at a time.
 struct HostStage {
@@ -67,6 +65,8 @@ struct HostStage {
   hipError_t init();
 };
 
+// Per-device state: a launch stream, a copy stream, cached workspaces grown on
+// demand.
 struct DeviceCtx {
   int device = -1;
   hipStream_t stream = nullptr;
@@ -186,9 +186,12 @@ hipError_t device_malloc_wait(DeviceCtx* c, void** p, size_t bytes);
 // c->out of at least `need` bytes, at the start of a call.
 int grow_out(DeviceCtx* c, size_t need);
 
-// Host copies on `stream` (host_io.cpp).  copy_to_device returns when src may be
-// changed, the copy being queued; copy_to_host when dst is complete.  Fill writes
-// bytes [at, at + n) of the source to `to`, from any thread.
+// Host copies on `stream` (host_io.cpp), on which no other call's kernels may be
+// queued.  copy_to_device returns with the copy queued: an ordinary src may be
+// changed then, a page-locked one is read by the copy itself, so that the caller
+// waits for the stream before it returns to its own.  copy_to_host returns when
+// dst is complete.  Fill writes bytes [at, at + n) of the source to `to`, from any
+// thread.
 using Fill = std::function<void(char* to, size_t at, size_t n)>;
 hipError_t fill_device(DeviceCtx* c, void* dst, size_t bytes, hipStream_t stream, const Fill& fill);
 hipError_t copy_to_device(DeviceCtx* c, void* dst, const void* src, size_t bytes,

@@ -12,6 +12,11 @@
 // other is filled or emptied.  48 MB: 1.7 -> 1.0 ms to the device, 3.0 -> 1.0
 // ms back.  Memory that is known to the runtime (page-locked or on a device) is
 // copied directly.
+//
+// The blocks are one lock for every copy of a device, a server's submits among
+// them, so nothing waits for a kernel while it holds them: copy_to_host waits for
+// the stream first, and a copy to the device goes on a stream that no other call's
+// kernels are queued on.
 #include <hip/hip_runtime.h>
 
 #include <atomic>
@@ -110,6 +115,7 @@ hipError_t copy_to_host(DeviceCtx* c, void* dst, const void* src, size_t bytes,
     const hipError_t e = hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, stream);
     return e == hipSuccess ? hipStreamSynchronize(stream) : e;
   }
+  if (const hipError_t e = hipStreamSynchronize(stream)) return e;
   HostStage& h = c->host;
   std::lock_guard<std::mutex> lk(h.mu);
   std::atomic<size_t> next{0};

@@ -1148,6 +1148,16 @@ size_t tail_split_tiles(size_t n, int grid) {
   return (n > g && r > 0 && r <= g / 2) ? r : 0;
 }
 
+// Per-sample inputs to the device, after the work queued so far; on the copy
+// stream, as a copy behind a pass would hold its page-locked block until the pass
+// ends.
+hipError_t copy_meta(DeviceCtx* c, void* dst, const void* src, size_t bytes) {
+  hipError_t e = hipStreamSynchronize(c->stream);
+  if (e == hipSuccess) e = copy_to_device(c, dst, src, bytes, c->copy_stream);
+  const hipError_t es = hipStreamSynchronize(c->copy_stream);
+  return e == hipSuccess ? es : e;
+}
+
 int upload_table(DeviceCtx* c, const ppsk_set* s, const RandomIn& rnd, float** dtab) {
   *dtab = nullptr;
   if (rnd.mode != PPSK_RANDOM_MC) return PPSK_OK;
@@ -1411,7 +1421,9 @@ int ppsk_set_upload(ppsk_set* s, int64_t first, int64_t count, const uint64_t* r
   if (int rc = get_ctx(s->device, &c)) return rc;
   const size_t per_sample = (size_t)s->n_k * s->s64 * s->bbits * sizeof(uint64_t);
   // Through two halves of a kept buffer on the copy stream, each chunk's stripes
-  // written while the next one crosses the link.
+  // written while the next one crosses the link.  A half is waited for here, not
+  // by the stream: its stripes may be queued behind a pass, and a copy queued
+  // behind them would hold the page-locked blocks that long.
   std::lock_guard<std::mutex> lk(c->upload_mu);
   const int64_t chunk = std::min<int64_t>(count, std::max<int64_t>(1, (int64_t)((32u << 20) / per_sample)));
   const size_t half = ((size_t)chunk * per_sample + 255) / 256 * 256;
@@ -1427,7 +1439,7 @@ int ppsk_set_upload(ppsk_set* s, int64_t first, int64_t count, const uint64_t* r
   for (int64_t c0 = 0; c0 < count && e == hipSuccess; c0 += chunk, turn ^= 1) {
     const int64_t m = std::min(chunk, count - c0);
     uint64_t* to = (uint64_t*)((char*)c->raw + turn * half);
-    e = hipStreamWaitEvent(c->copy_stream, c->raw_striped[turn], 0);
+    e = hipEventSynchronize(c->raw_striped[turn]);
     if (e == hipSuccess) {
       e = copy_to_device(c, to, (const char*)raw + (size_t)c0 * per_sample, (size_t)m * per_sample,
                          c->copy_stream);
@@ -1470,8 +1482,7 @@ int ppsk_set_meta(ppsk_set* s, const uint64_t* lengths, int32_t use_rc, const ui
       }
     }
     if (!s->jv) HIP_TRY(device_malloc_wait(c, (void**)&s->jv, jv.size() * sizeof(double)));
-    HIP_TRY(copy_to_device(c, s->jv, jv.data(), jv.size() * sizeof(double), c->stream));
-    HIP_TRY(hipStreamSynchronize(c->stream));
+    HIP_TRY(copy_meta(c, s->jv, jv.data(), jv.size() * sizeof(double)));
     s->has_lengths = true;
     s->use_rc = use_rc;
   }
@@ -1479,8 +1490,7 @@ int ppsk_set_meta(ppsk_set* s, const uint64_t* lengths, int32_t use_rc, const ui
     s->max_cluster = 0;
     for (int64_t i = 0; i < s->n; ++i) s->max_cluster = std::max<int32_t>(s->max_cluster, clusters[i]);
     if (!s->clusters) HIP_TRY(device_malloc_wait(c, (void**)&s->clusters, (size_t)s->n * sizeof(uint16_t)));
-    HIP_TRY(copy_to_device(c, s->clusters, clusters, (size_t)s->n * sizeof(uint16_t), c->stream));
-    HIP_TRY(hipStreamSynchronize(c->stream));
+    HIP_TRY(copy_meta(c, s->clusters, clusters, (size_t)s->n * sizeof(uint16_t)));
   }
   return PPSK_OK;
 }
