@@ -799,6 +799,13 @@ size_t code_bytes(int n_k, int s64, int64_t nb) {
   return ((size_t)n_k * nb * 2 * s64 + 2) * slot;
 }
 
+// Bytes of a slab's width table, with the 16 entries past its end that may be read;
+// whole 256-byte lines, so that the codes of the slab after it are aligned for the
+// 16-byte copies into LDS.
+size_t width_bytes(int n_k, int s64) {
+  return (((size_t)n_k * 2 * s64 + 16) * sizeof(uint32_t) + 255) / 256 * 256;
+}
+
 ItemPlan plan_items(int64_t n_cols, int n_k, int s64, bool upper, bool same_set, int64_t row_begin,
                     int64_t row_end, bool host_out, bool coded, size_t code_budget) {
   ItemPlan pl;
@@ -839,13 +846,12 @@ ItemPlan plan_items(int64_t n_cols, int n_k, int s64, bool upper, bool same_set,
     }
     const int64_t cb_first = upper ? g0 / 256 : 0;
     const int64_t rb0 = g0 / 256, nrb = (g1 + 255) / 256 - rb0;
-    const size_t width_bytes = ((size_t)n_k * 2 * s64 + 64) * sizeof(uint32_t);
     int64_t step = nct;  // column blocks per slab
     size_t row_bytes = 0;
     bool apart = false;
     if (coded) {
       const size_t block = code_bytes(n_k, s64, 1);
-      const size_t fixed = width_bytes + block + code_bytes(n_k, s64, nrb);
+      const size_t fixed = width_bytes(n_k, s64) + block + code_bytes(n_k, s64, nrb);
       step = std::max<int64_t>(1, code_budget > fixed ? (int64_t)((code_budget - fixed) / block) : 1);
       step = std::min<int64_t>(step, std::max<int64_t>(1, (int64_t)(most / segs.size())));
       // the rows of a self pass are coded with the columns they lie among,
@@ -867,7 +873,7 @@ ItemPlan plan_items(int64_t n_cols, int n_k, int s64, bool upper, bool same_set,
       if (sl.tile1 == sl.tile0) continue;
       sl.r0 = g0;
       sl.r1 = c1 == nct ? g1 : g0;
-      sl.bytes = coded ? code_bytes(n_k, s64, c1 - c0) + row_bytes + width_bytes : 0;
+      sl.bytes = coded ? code_bytes(n_k, s64, c1 - c0) + row_bytes + width_bytes(n_k, s64) : 0;
       slabs.push_back(sl);
       ppsk::CodeGroup cg;
       std::memset(&cg, 0, sizeof(cg));
@@ -984,7 +990,6 @@ int run_dense_items(DeviceCtx* c, ppsk::DistParams p, bool upper, int64_t row_be
   const size_t slab_bytes = pl.coded ? pl.slabs.size() * sizeof(ppsk::CodeGroup) : 0;
   std::vector<char> lists(slab_bytes + pl.tiles.size() * sizeof(ppsk::ItemTile));
   if (pl.coded) {
-    const size_t width_bytes = ((size_t)p.n_k * 2 * p.s64 + 64) * sizeof(uint32_t);
     for (const auto& ch : pl.chunks) {
       char* at = (char*)c->codes;
       for (int x = ch.slab0; x < ch.slab1; ++x) {
@@ -997,7 +1002,7 @@ int run_dense_items(DeviceCtx* c, ppsk::DistParams p, bool upper, int64_t row_be
           at += code_bytes(p.n_k, p.s64, g.nrb);
         }
         g.widths = (uint32_t*)at;
-        at += width_bytes;
+        at += width_bytes(p.n_k, p.s64);
       }
     }
     std::memcpy(lists.data(), pl.slabs.data(), slab_bytes);
