@@ -2090,6 +2090,8 @@ hipError_t launch_coded(const DistParams& p, const ItemArgs& a, const CodeGroup*
   while (grid > 1 && std::gcd(grid, n_groups) != 1) --grid;
   code_kernel<<<(unsigned)std::min(grid, n_code), CODE_TB, 0, stream>>>(p, groups + first_group,
                                                                         n_groups, n_code);
+  // never the matching of planes that were not coded: it walks their widths
+  if ((e = hipGetLastError()) != hipSuccess) return e;
   dist_coded<<<item_grid(a), WAVES * 64, 0, stream>>>(p, a, groups);
   dist_items_out<<<(unsigned)(a.n_tiles * (64 / a.out_rows)), 256, 0, stream>>>(p, a);
   return hipGetLastError();
