@@ -69,14 +69,15 @@ int ppsk_device_init(int device_id, size_t *mem_free, size_t *mem_total,
  * at a time; these three may be called from any thread at any time, also
  * while such a call runs, and need no HIP device (device_id in [0, 64)).
  *
- * ppsk_progress: (tile, k-mer length) work items finished and planned by the
- * call running on the device (*running = 1), or by the last one; *pending = 1
- * while a cancellation request stands.  Any output pointer may be NULL.
+ * ppsk_progress: work items (a tile, a k-mer length and all or a run of the
+ * words) finished and planned by the call running on the device (*running = 1),
+ * or by the last one; a running call's count may lag by 63.  *pending = 1 while
+ * a cancellation request stands.  Any output pointer may be NULL.
  * ppsk_cancel: asks the call running on the device to stop, and every call
  * that starts on the device to stop at once, until ppsk_cancel_reset.  The
  * kernels read the request between work items and finish normally (no
- * trap); the call waits for them and returns PPSK_ERR_CANCELLED, its outputs
- * undefined.
+ * trap; a pass of less than about a millisecond ends first); the call waits
+ * for them and returns PPSK_ERR_CANCELLED, its outputs undefined.
  */
 int ppsk_progress(int device_id, uint64_t *done, uint64_t *total,
                   int32_t *running, int32_t *pending);

@@ -340,9 +340,10 @@ int build_split(ppsk_batch* b, ppsk_batch::Plan& pl, DeviceCtx* c, bool* made) {
   a.n_items = (int32_t)all.size();
   a.out_rows = a.n_tiles * 64 <= 2048 ? 1 : 4;
   a.ctl = c->ctl;
-  // flag reads and progress mirrors as in a dense split pass (run_dense_items)
-  a.watch = total * 6.4 / 512.0 >= 10000.0 ? 1 : 0;
-  if (!a.watch) a.ctl.progress_host = nullptr;
+  if (total * 6.4 / ppsk::ITEM_SLOTS < WATCH_US) {
+    a.ctl.stop = nullptr;
+    a.ctl.progress_host = nullptr;
+  }
   pl.split = true;
   pl.n_items = n_items;
   pl.progress = (uint64_t)n_items;

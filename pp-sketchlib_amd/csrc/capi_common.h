@@ -77,7 +77,7 @@ struct DeviceCtx {
   ppsk::Tile* tiles = nullptr;
   size_t tiles_n = 0;
   // [0] fit failures, [1] first failed row, [2] progress (ctl.progress): one
-  // read at the end of a call
+  // read at the end of a call; [3] cancelled (ctl.stop)
   unsigned long long* fail = nullptr;
   unsigned long long* words = nullptr;  // page-locked copy of the three
   bool words_read = false;              // `words` holds the call's final values
@@ -230,6 +230,8 @@ struct ItemCut {
   int64_t items;
   double work_us;
 };
+// Split passes estimated shorter do not look for a cancellation (item_stopped).
+constexpr double WATCH_US = 1000.0;
 ItemCut cut_items(int64_t n64, int64_t n32, int64_t n16, int n_k, int s64, bool coded);
 // The launch's tiles and cut in its arguments.
 void set_items(ppsk::ItemArgs* a, const ppsk::ItemTile* tiles, int64_t n_tiles, const ItemCut& cut);

@@ -163,6 +163,32 @@ __device__ __forceinline__ void add_progress(const Control& c, unsigned long lon
   }
 }
 
+// Whether the call of an item of a split pass was cancelled (one lane of workgroup
+// `block` asks).  The host's flag and the mirrored progress cross one link for all
+// CUs, about 0.1 us each: read and written in every item, 4,400 short items took
+// 863 us instead of 433.  So one item in 64 reads the flag and passes it on in a
+// device word that the others read, and one in 64 mirrors the progress.  The
+// first workgroups of a call, which start together right after the host has
+// looked, read neither; nor does a pass of less than about 1 ms, which ends
+// before a request could stop it (its call reports the request and the final
+// count all the same): looking took 37 of the 223 us of one query against 6,000.
+constexpr uint32_t ITEM_WATCH = 64, ITEM_MIRROR = 64;
+
+__device__ __forceinline__ bool item_stopped(const Control& c, uint32_t block) {
+  if (__hip_atomic_load(c.stop, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0u) return true;
+  if (block % ITEM_WATCH != 0 || !cancel_seen(c.cancel)) return false;
+  __hip_atomic_store(c.stop, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  return true;
+}
+
+__device__ __forceinline__ void add_item(const Control& c) {
+  if (c.progress == nullptr) return;
+  const unsigned long long done = atomicAdd(c.progress, 1ull) + 1ull;
+  if (c.progress_host != nullptr && done % ITEM_MIRROR == 0) {
+    __hip_atomic_store(c.progress_host, done, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+  }
+}
+
 __device__ __forceinline__ double jaccard_d(uint32_t c, double bins, double rbins, double r) {
   const double obs = bin_fraction(c, bins, rbins);
   const double diff = obs > r ? (obs - r) : 0.0;
@@ -1347,10 +1373,10 @@ __global__ __launch_bounds__(WAVES * 64, 4) void dist_items(DistParams p, ItemAr
   CParams* pp = (CParams*)__builtin_amdgcn_kernarg_segment_ptr();
   ItemAt it;
   if (!item_at(a, p.n_k, p.s64, it)) return;
-  if (a.watch) {
+  if (p.ctl.stop != nullptr && blockIdx.x >= (uint32_t)a.unwatched) {
     // a cancelled call skips the matching; one read per workgroup, shared, so
     // that every wave takes the same branch (the matching has barriers)
-    if (threadIdx.x == 0) s_stop = cancel_seen(p.ctl.cancel) ? 1 : 0;
+    if (threadIdx.x == 0) s_stop = item_stopped(p.ctl, blockIdx.x) ? 1 : 0;
     __syncthreads();
     if (__builtin_amdgcn_readfirstlane(s_stop)) return;
   }
@@ -1369,7 +1395,7 @@ __global__ __launch_bounds__(WAVES * 64, 4) void dist_items(DistParams p, ItemAr
   } else {
     match_item<1>(pp, row0, ct, kk, w0, nw, sB0, sB1, sR, counts, wave, lane);
   }
-  if (threadIdx.x == 0) add_progress(p.ctl, 1ull);
+  if (threadIdx.x == 0) add_item(p.ctl);
 }
 
 // Counts of OUT_K k-mer lengths from their runs' blocks, x[i] at the pair's
@@ -1453,8 +1479,8 @@ __global__ __launch_bounds__(WAVES * 64, 4) void dist_batch_items(BatchItemArgs 
   const BatchRun it = a.items[blockIdx.x];
   const int t = __builtin_amdgcn_readfirstlane(it.tile);
   if (t < 0) return;
-  if (a.watch) {
-    if (threadIdx.x == 0) s_stop = cancel_seen(a.ctl.cancel) ? 1 : 0;
+  if (a.ctl.stop != nullptr && blockIdx.x >= ITEM_SLOTS) {
+    if (threadIdx.x == 0) s_stop = item_stopped(a.ctl, blockIdx.x) ? 1 : 0;
     __syncthreads();
     if (__builtin_amdgcn_readfirstlane(s_stop)) return;
   }
@@ -1478,7 +1504,7 @@ __global__ __launch_bounds__(WAVES * 64, 4) void dist_batch_items(BatchItemArgs 
   } else {
     match_item<1>(pp, row0, ct, kk, w0, nw, sB0, sB1, sR, counts, wave, lane);
   }
-  if (threadIdx.x == 0) add_progress(a.ctl, 1ull);
+  if (threadIdx.x == 0) add_item(a.ctl);
 }
 
 __global__ __launch_bounds__(256) void dist_batch_items_out(BatchItemArgs a) {
@@ -2043,8 +2069,8 @@ __global__ __launch_bounds__(WAVES * 64, 4) void dist_coded(DistParams p, ItemAr
   const int all = 2 * p.s64;  // halves of a sketch
   ItemAt it;
   if (!item_at(a, p.n_k, all, it)) return;
-  if (a.watch) {
-    if (threadIdx.x == 0) s_stop = cancel_seen(p.ctl.cancel) ? 1 : 0;
+  if (p.ctl.stop != nullptr && blockIdx.x >= (uint32_t)a.unwatched) {
+    if (threadIdx.x == 0) s_stop = item_stopped(p.ctl, blockIdx.x) ? 1 : 0;
     __syncthreads();
     if (__builtin_amdgcn_readfirstlane(s_stop)) return;
   }
@@ -2076,7 +2102,7 @@ __global__ __launch_bounds__(WAVES * 64, 4) void dist_coded(DistParams p, ItemAr
   } else {
     coded_item<1>(widths, cols, rws, rpf, halves, buf, row_dst, counts, wave, lane);
   }
-  if (threadIdx.x == 0) add_progress(p.ctl, 1ull);
+  if (threadIdx.x == 0) add_item(p.ctl);
 }
 
 hipError_t launch_coded(const DistParams& p, const ItemArgs& a, const CodeGroup* groups,
@@ -2143,15 +2169,15 @@ hipError_t launch_band_setup(ItemTile* tiles, int64_t rows, int64_t n_ct, int64_
   return hipGetLastError();
 }
 
-__global__ void call_reset_kernel(unsigned long long* fail, unsigned long long* progress) {
+__global__ void call_reset_kernel(unsigned long long* fail, Control ctl) {
   fail[0] = 0ull;
   fail[1] = ~0ull;
-  *progress = 0ull;
+  *ctl.progress = 0ull;
+  *ctl.stop = 0u;
 }
 
-hipError_t launch_call_reset(unsigned long long* fail, unsigned long long* progress,
-                             hipStream_t stream) {
-  call_reset_kernel<<<1, 1, 0, stream>>>(fail, progress);
+hipError_t launch_call_reset(unsigned long long* fail, const Control& ctl, hipStream_t stream) {
+  call_reset_kernel<<<1, 1, 0, stream>>>(fail, ctl);
   return hipGetLastError();
 }
 

@@ -51,7 +51,7 @@ int get_ctx(int device, DeviceCtx** out) {
     c->device = device;
     HIP_TRY(hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking));
     HIP_TRY(hipStreamCreateWithFlags(&c->copy_stream, hipStreamNonBlocking));
-    HIP_TRY(hipMalloc(&c->fail, 3 * sizeof(unsigned long long)));
+    HIP_TRY(hipMalloc(&c->fail, 4 * sizeof(unsigned long long)));
     HIP_TRY(hipHostMalloc((void**)&c->words, 3 * sizeof(unsigned long long), hipHostMallocDefault));
     HIP_TRY(c->host.init());
     HIP_TRY(hipEventCreateWithFlags(&c->raw_copied, hipEventDisableTiming));
@@ -61,7 +61,8 @@ int get_ctx(int device, DeviceCtx** out) {
     // progress / cancellation words: a device counter and two host-mapped,
     // coherent words (device_id < MAX_DEVICES here)
     c->ctl.progress = c->fail + 2;
-    HIP_TRY(hipMemset(c->ctl.progress, 0, sizeof(unsigned long long)));
+    c->ctl.stop = (uint32_t*)(c->fail + 3);
+    HIP_TRY(hipMemset(c->ctl.progress, 0, 2 * sizeof(unsigned long long)));
     void* hw = nullptr;
     HIP_TRY(hipHostMalloc(&hw, 64, hipHostMallocMapped | hipHostMallocCoherent));
     std::memset(hw, 0, 64);
@@ -125,7 +126,7 @@ CallScope::CallScope(DeviceCtx* ctx, uint64_t total) : c(ctx), cs(g_calls[ctx->d
   cs.running.store(1);
   // the device counters start from zero in stream order
   c->words_read = false;
-  (void)ppsk::launch_call_reset(c->fail, c->ctl.progress, c->stream);
+  (void)ppsk::launch_call_reset(c->fail, c->ctl, c->stream);
 }
 
 CallScope::~CallScope() {
@@ -749,11 +750,11 @@ ItemCut cut_items(int64_t n64, int64_t n32, int64_t n16, int n_k, int s64, bool 
   const int64_t pairs = (n64 + n32 + n16) * n_k;
   ItemCut cut;
   cut.n_tall = (int)n64;
-  cut.whole = (int)(n64 * n_k / 512 * 512);
+  cut.whole = (int)(n64 * n_k / ppsk::ITEM_SLOTS * ppsk::ITEM_SLOTS);
   cut.runs = 1;
   cut.run_units = units;
   cut.items = pairs;
-  cut.work_us = ((double)n64 + 0.57 * n32 + 0.37 * n16) * n_k * unit_us * units / 512.0;
+  cut.work_us = ((double)n64 + 0.57 * n32 + 0.37 * n16) * n_k * unit_us * units / ppsk::ITEM_SLOTS;
   const int64_t rest = pairs - cut.whole;
   if (rest == 0) return cut;
   const int shortest = coded ? 16 : 8;
@@ -1015,18 +1016,16 @@ int run_dense_items(DeviceCtx* c, ppsk::DistParams p, bool upper, int64_t row_be
   p.out_row_offset = 0;
   ppsk::ItemArgs a;
   std::memset(&a, 0, sizeof(a));
-  // The items of a pass of more than about 10 ms read the host's cancellation
-  // flag and mirror their progress to the host.  Both cross one link for all
-  // CUs (about 0.1 us each: 4,400 short items took 863 us instead of 433), so a
-  // shorter pass is left to finish; its call reports the cancellation and the
-  // final count either way.
-  a.watch = pl.work_us >= 10000.0 ? 1 : 0;
-  if (!a.watch) p.ctl.progress_host = nullptr;
+  if (pl.work_us < WATCH_US) {
+    p.ctl.stop = nullptr;
+    p.ctl.progress_host = nullptr;
+  }
   for (size_t ci = 0; ci < pl.chunks.size(); ++ci) {
     const ItemPlan::Chunk& ch = pl.chunks[ci];
     hipEvent_t e0 = pool_event(c, 2 * ci), e1 = pool_event(c, 2 * ci + 1);
     if (!e0 || !e1) return fail(PPSK_ERR_HIP, "event creation failed");
     set_items(&a, d_tiles + ch.tile0, (int64_t)(ch.tile1 - ch.tile0), ch.cut);
+    a.unwatched = ci == 0 ? ppsk::ITEM_SLOTS : 0;
     HIP_TRY(hipEventRecord(e0, c->stream));
     if (pl.coded) {
       HIP_TRY(ppsk::launch_coded(p, a, d_slabs, ch.slab0, ch.slab1 - ch.slab0, c->stream));

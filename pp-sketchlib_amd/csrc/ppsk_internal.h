@@ -32,14 +32,15 @@ enum RandomMode : int32_t { RANDOM_NONE = 0, RANDOM_EQUAL_BASE = 1, RANDOM_MC = 
 
 // Progress and cancellation of a call.  cancel: host-mapped flag written by
 // ppsk_cancel, read by the kernels between work items with system-scope
-// loads; progress: device counter of finished (tile, k) items, each update
-// mirrored with a plain system-scope store into the host-mapped word
-// progress_host (stores of different workgroups may land out of order: the
-// host keeps the largest value it has read).
+// loads; progress: device counter of finished work items, mirrored (by every
+// update, in split passes by one in 64) with a plain system-scope store into the
+// host-mapped word progress_host (stores of different workgroups may land out of
+// order: the host keeps the largest value it has read).
 struct Control {
   const uint32_t* cancel;
   unsigned long long* progress;
   unsigned long long* progress_host;
+  uint32_t* stop;  // device word: 1 once an item of the call has seen `cancel` set
 };
 
 // Tile: rows [bi * rows, +rows) x cols [ct * cols, +cols) of the variant's
@@ -113,6 +114,7 @@ struct ItemTile {
   int32_t rows;  // 64, 32 or 16
   int32_t group;  // row group of a coded pass
 };
+constexpr int ITEM_SLOTS = 512;        // workgroups resident at once: 2 per CU
 constexpr int ITEM_COUNTS = 64 * 256;  // counts of one item (u16), whatever its height
 
 // The (tile, k-mer length) pairs of a launch, k-mer length first, those of the
@@ -127,7 +129,7 @@ struct ItemArgs {
   int32_t runs;
   int32_t run_units;  // words (coded pass: halves) per run; the last may hold fewer
   int32_t n_items;    // whole + (n_tiles * n_k - whole) * runs
-  int32_t watch;      // read the cancellation flag in every item
+  int32_t unwatched;  // workgroups that do not look for a cancellation: the first ones
   int32_t out_rows;   // tile rows per output workgroup (divides 16)
 };
 
@@ -177,7 +179,6 @@ struct BatchItemArgs {
   const BatchRun* items;   // [n_items], workgroup b takes item b
   uint16_t* counts;        // blocks of ITEM_COUNTS
   int32_t n_tiles, n_items;
-  int32_t watch;     // read the cancellation flag in every item
   int32_t out_rows;  // tile rows per output workgroup (divides 16)
   Control ctl;
 };
@@ -230,9 +231,8 @@ hipError_t launch_batch(const BatchArgs& a, int variant, int grid, hipStream_t s
 // when step is 0.
 hipError_t launch_band_setup(ItemTile* tiles, int64_t rows, int64_t n_ct, int64_t step,
                              unsigned long long* fail, uint32_t* fail_rows, hipStream_t stream);
-// Start of a call: fit failures {0, none} and a progress count of 0.
-hipError_t launch_call_reset(unsigned long long* fail, unsigned long long* progress,
-                             hipStream_t stream);
+// Start of a call: fit failures {0, none}, a progress count of 0 and no stop.
+hipError_t launch_call_reset(unsigned long long* fail, const Control& ctl, hipStream_t stream);
 hipError_t launch_batch_reset(uint32_t* queue_next, unsigned long long* fail, int n_jobs,
                               hipStream_t stream, unsigned long long* progress = nullptr);
 // Zeroes n tile completion counters and sets fail ([2]: count, first row; may
