@@ -79,7 +79,7 @@ struct DeviceCtx {
   // [0] fit failures, [1] first failed row, [2] progress (ctl.progress): one
   // read at the end of a call; [3] cancelled (ctl.stop)
   unsigned long long* fail = nullptr;
-  unsigned long long* words = nullptr;  // page-locked copy of the three
+  unsigned long long* words = nullptr;  // page-locked copy of the first three; [3] threshold hits
   bool words_read = false;              // `words` holds the call's final values
   void* out = nullptr;
   size_t out_bytes = 0;

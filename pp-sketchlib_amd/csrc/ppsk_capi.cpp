@@ -52,7 +52,7 @@ int get_ctx(int device, DeviceCtx** out) {
     HIP_TRY(hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking));
     HIP_TRY(hipStreamCreateWithFlags(&c->copy_stream, hipStreamNonBlocking));
     HIP_TRY(hipMalloc(&c->fail, 4 * sizeof(unsigned long long)));
-    HIP_TRY(hipHostMalloc((void**)&c->words, 3 * sizeof(unsigned long long), hipHostMallocDefault));
+    HIP_TRY(hipHostMalloc((void**)&c->words, 4 * sizeof(unsigned long long), hipHostMallocDefault));
     HIP_TRY(c->host.init());
     HIP_TRY(hipEventCreateWithFlags(&c->raw_copied, hipEventDisableTiming));
     for (auto& ev : c->raw_striped) HIP_TRY(hipEventCreateWithFlags(&ev, hipEventDisableTiming));
@@ -1289,7 +1289,11 @@ int threshold_from_triangle(DeviceCtx* c, const float2* tri, int64_t n, int col,
     int64_t* counts = (int64_t*)c->sel;
     e = ppsk::launch_threshold_count(tri, rows, n, false, col, cutoff, counts, c->stream);
     if (e == hipSuccess) e = ppsk::launch_offsets_scan(counts, rows, c->stream);
-    if (e == hipSuccess) e = copy_to_host(c, &total, counts + rows, sizeof(total), c->stream);
+    if (e == hipSuccess) {
+      e = hipMemcpyAsync(c->words + 3, counts + rows, sizeof(total), hipMemcpyDeviceToHost, c->stream);
+    }
+    if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
+    if (e == hipSuccess) total = (int64_t)c->words[3];
   }
   if (e != hipSuccess) return fail(PPSK_ERR_HIP, std::string("threshold: ") + hipGetErrorString(e));
   auto* hi = (int64_t*)std::malloc(std::max<int64_t>(total, 1) * sizeof(int64_t));
