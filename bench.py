@@ -9,13 +9,18 @@ tree-evolution model and resident in HBM before timing starts.
 
 Prints one JSON line:
   value      distances (pairs) per second over the timed steps
-  roofline   int32 VALU issue bound of a distance pass: the lane operations its
-             kernels issue (SQ_INSTS_VALU x 64 of the committed profile of the
-             same pass) divided by the pass's HIP-event duration on its launch
-             stream.  plane_ops_per_pair = sum_k s64 * (2 * bbits + 2) = 37,440
-             is what matching the sketches' 14 bit planes as they are takes; the
-             pass matches ranks of the values instead (7 to 9 planes), so
-             plane_rate, that work over the same time, is above the peak
+  roofline   int32 VALU issue bound of a distance pass: the operations that
+             matching its pairs cannot do without (per pair, k-mer length and 32
+             bins the planes of the largest rank there and one count; counted
+             from the sketches, match_ops_per_pass of the committed profile)
+             divided by the pass's HIP-event duration on its launch stream,
+             coding and output included: work issued beside the matching lowers
+             it.  issued_rate: all lane operations the pass's kernels issue
+             (SQ_INSTS_VALU x 64 of that profile) over the same time.
+             plane_ops_per_pair = sum_k s64 * (2 * bbits + 2) = 37,440 is what
+             matching the sketches' 14 bit planes as they are takes; the pass
+             matches ranks of the values instead (7 to 9 planes), so plane_rate,
+             that work over the same time, is above the peak
   cpu_baseline  the CPU oracle (C++/OpenMP restatement of the reference CPU
              path), compiled on this host with -march=native, on a bounded
              sample of the same workload: median of 3 runs at 16 threads and
@@ -116,7 +121,8 @@ def measured_valu_peak():
 
 def pass_profile(n):
     """Counter summary of the committed rocprofv3 profile of the 8,192-sample pass
-    (HBM bytes and VALU lane operations per pass); empty for another size."""
+    (HBM bytes, VALU lane operations, necessary matching operations per pass);
+    empty for another size."""
     path = os.path.join(ROOT, "profiles", "dist_coded_allvsall_8192.json")
     if n != N_SAMPLES or not os.path.exists(path):
         return {}
@@ -251,8 +257,9 @@ def main():
     # them on their stream
     pass_ms = sum(kernel_ms) / a.steps
     profile = pass_profile(a.n)
-    ops = profile.get("valu_lane_ops_per_pass")
+    ops = profile.get("match_ops_per_pass")
     achieved = ops / (pass_ms * 1e-3) / 1e12 if ops else None
+    issued = profile.get("valu_lane_ops_per_pass")
     roofline = {
         "bound": "valu",
         "achieved": round(achieved, 3) if ops else None,
@@ -264,6 +271,7 @@ def main():
         "kernel_ms": round(pass_ms, 3),
         "launches_per_step": round(launches / a.steps, 2),
         "ops_per_pair": round(ops / pairs) if ops else None,
+        "issued_rate": round(issued / (pass_ms * 1e-3) / 1e12, 3) if issued else None,
         "plane_ops_per_pair": OPS_PER_PAIR,
         "plane_rate": round(OPS_PER_PAIR * pairs / (pass_ms * 1e-3) / 1e12, 3),
         "peak_measured": None,
