@@ -1281,7 +1281,7 @@ __global__ __launch_bounds__(WAVES * 64, 4) void dist_batch_mixed(BatchArgs a) {
 // its own.  (Tile, k-mer length) pairs that fill whole rounds of the 512
 // resident workgroups are one item each; the others, all of them in a small
 // pass, are cut into the runs of words that make their rounds shortest
-// (item_runs in the host layer), so that a pass of few tiles spreads over
+// (cut_items in the host layer), so that a pass of few tiles spreads over
 // every CU and a large one has no idle last round.  One item over 156 words
 // takes 0.68 ms by itself, however small the pass: calls on 48 genomes went
 // from 774 to 148 us, one query against 6,000 references from 756 to 255 us
@@ -1551,8 +1551,9 @@ hipError_t launch_items(const DistParams& p, const ItemArgs& a, hipStream_t stre
 // Coded passes: fewer bit planes per pair.
 //
 // A group of at most CODE_ROWS rows holds V distinct values at a bin, V far
-// below the 2^14 a 14-bit value could take (at most 512; 110-170 in 8,192 tree
-// samples), so equality with a row is decided by the value's rank among those
+// below the 2^14 a 14-bit value could take (at most CODE_ROWS; 110-170 in 8,192
+// tree samples, about 750 in unrelated ones, whose 10 planes still beat 14: 30.0
+// ms against 33.8), so equality with a row is decided by the value's rank among those
 // V: code 1 .. V for a value some row of the group holds, 0 for any other.
 // Two codes are equal exactly when the values are, as one of them is always a
 // row's; the match counts are the same whole numbers.  A run of 32 bins

@@ -52,6 +52,23 @@ def test_less_scratch_same_bytes(sets, monkeypatch, limit):
     assert all(_same(a, b) for a, b in zip(H.threshold(s, 0.01, **kw)[:3], thr[:3]))
 
 
+@pytest.mark.parametrize("limit", [60, 100])
+def test_whole_tiles_on_the_persistent_kernel(monkeypatch, limit):
+    # 1,046 tiles: two per resident workgroup, so that the last resort is the
+    # persistent kernel (50 MiB) and not one workgroup per (tile, k-mer length)
+    kl = [15, 21]
+    raw, le, _ = H.synth(5800, kl, 20, seed=4)
+    with H.SketchSet(raw, kl, 20, lengths=le) as s:
+        kw = dict(random_mode=H.RANDOM_EQUAL_BASE, out="jaccard")
+        with monkeypatch.context() as m:
+            m.setenv("PPSK_PERSISTENT", "0")
+            want = H.dense(s, **kw)[0]
+        monkeypatch.setenv("PPSK_SCRATCH_BYTES", str(limit * MB))
+        assert _same(H.dense(s, **kw)[0], want)
+        st = H.progress(0)
+        assert st["done"] == st["total"] > 0
+
+
 def test_no_scratch_is_an_error(sets, monkeypatch):
     s, q, (dense, _, _, _) = sets
     kw = dict(random_mode=H.RANDOM_EQUAL_BASE)
