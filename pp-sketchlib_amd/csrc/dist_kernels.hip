@@ -2135,7 +2135,7 @@ __global__ void batch_reset_kernel(uint32_t* queue_next, unsigned long long* fai
   }
 }
 
-__global__ void band_setup_kernel(ItemTile* tiles, int64_t rows, int64_t n_ct, int64_t step,
+__global__ void band_setup_kernel(ItemTile* tiles, int64_t rows, BandTiles b, int64_t n_ct, int64_t step,
                                   unsigned long long* fail, uint32_t* fail_rows) {
   const int64_t x = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (x < rows) fail_rows[x] = 0u;
@@ -2144,7 +2144,6 @@ __global__ void band_setup_kernel(ItemTile* tiles, int64_t rows, int64_t n_ct, i
     fail[1] = ~0ull;
   }
   if (step == 0) return;
-  const BandTiles b = band_tiles(rows);
   const int64_t per = b.tall + b.shorts;  // tiles of a column block
   if (x >= per * n_ct) return;
   const int64_t c0 = x / (per * step) * step;
@@ -2160,12 +2159,11 @@ __global__ void band_setup_kernel(ItemTile* tiles, int64_t rows, int64_t n_ct, i
   }
 }
 
-hipError_t launch_band_setup(ItemTile* tiles, int64_t rows, int64_t n_ct, int64_t step,
+hipError_t launch_band_setup(ItemTile* tiles, int64_t rows, const BandTiles& b, int64_t n_ct, int64_t step,
                              unsigned long long* fail, uint32_t* fail_rows, hipStream_t stream) {
-  const BandTiles b = band_tiles(rows);
   int64_t n = rows > 0 ? rows : 1;
   if (step > 0 && (b.tall + b.shorts) * n_ct > n) n = (b.tall + b.shorts) * n_ct;
-  band_setup_kernel<<<(unsigned)((n + 255) / 256), 256, 0, stream>>>(tiles, rows, n_ct, step, fail,
+  band_setup_kernel<<<(unsigned)((n + 255) / 256), 256, 0, stream>>>(tiles, rows, b, n_ct, step, fail,
                                                                      fail_rows);
   return hipGetLastError();
 }

@@ -831,6 +831,7 @@ ItemPlan plan_items(int64_t n_cols, int n_k, int s64, bool upper, bool same_set,
     const int64_t n = (rows + ppsk::CODE_ROWS - 1) / ppsk::CODE_ROWS;
     group = ((rows + n - 1) / n + 63) / 64 * 64;
   }
+  const int64_t tall = ppsk::tall_from((rows + 63) / 64 * nct * n_k / (upper ? 2 : 1));
   struct Slab {
     size_t tile0, tile1, bytes;
     int64_t r0, r1;  // rows it completes (r0 == r1: none)
@@ -841,7 +842,7 @@ ItemPlan plan_items(int64_t n_cols, int n_k, int s64, bool upper, bool same_set,
     std::vector<std::pair<int64_t, int32_t>> segs;  // first row, height
     for (int64_t r = g0; r < g1;) {
       const int64_t left = g1 - r;
-      const int32_t h = left > 48 ? 64 : (left > 16 ? 32 : 16);
+      const int32_t h = left >= tall ? 64 : (left > 16 ? 32 : 16);
       segs.emplace_back(r, h);
       r += h;
     }
@@ -1055,10 +1056,15 @@ int run_dense_items(DeviceCtx* c, ppsk::DistParams p, bool upper, int64_t row_be
   return PPSK_OK;
 }
 
-// How a dense pass runs: whole tiles on the persistent kernel when there are
-// at least two per resident workgroup, else as a split pass.
-// PPSK_TILE_VARIANT forces a tile shape and PPSK_PERSISTENT=0 / 1 the
-// per-(tile, k-mer length) or the persistent kernel of that shape.
+// How a dense pass runs: as a split pass, coded where that pays.  PPSK_TILE_VARIANT
+// forces a tile shape and PPSK_PERSISTENT=0 / 1 the per-(tile, k-mer length) or
+// the persistent kernel of that shape; where the device has no room for a split
+// pass's counts, whole tiles run as well.  (The persistent kernel used to take
+// every pass of at least two tiles per resident workgroup.  Against 200,000
+// references, whole tiles / items on the planes: 70 queries 27-29.8 / 18.9 ms, 86
+// 26.2-29.8 / 21.3, 128 26.4-30.0 / 25.1, 256 52.4 / 49.9, 512 105 / 99.6: a round
+// of whole tiles is long, and one workgroup that takes a tile more than the others
+// ends 4 ms after them.)
 enum class Route { persistent, tiles, items };
 
 // Whole tiles: the persistent kernel, or with fewer than two tiles per resident
@@ -1078,10 +1084,8 @@ Route dense_route(int variant, bool upper, int64_t rows, int64_t n_cols) {
     const bool can = variant == 2 || variant == 4 || variant == 5;
     return can && std::atoi(e) != 0 ? Route::persistent : Route::tiles;
   }
-  const bool shape = std::getenv("PPSK_TILE_VARIANT") != nullptr;
-  if (!shape && use_coded(rows, n_cols, upper)) return Route::items;
-  const Route r = tile_route(variant, upper, rows, n_cols);
-  return r == Route::tiles && !shape ? Route::items : r;
+  if (!std::getenv("PPSK_TILE_VARIANT")) return Route::items;
+  return tile_route(variant, upper, rows, n_cols);
 }
 
 // Work items a dense pass reports as progress.

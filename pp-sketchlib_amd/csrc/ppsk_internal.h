@@ -149,14 +149,23 @@ struct CodeGroup {
   int32_t rb0, nrb;
 };
 
-// Rows of a band in tiles: as many 64-row ones as fit (one more for more than
-// 48 rows left), the rest in one of 32 and / or one of 16.
+// Rows past a pass's last multiple of 64 that take a 64-row tile instead of one of
+// 32 and / or one of 16: more than 48, and from 64 (64-row tile, k-mer length)
+// pairs on more than 32.  Every tile streams its columns, so 32 + 16 rows take
+// longer than 64 once the pass fills the CUs: 97 queries x 6,000 references 1,073
+// and 859 us, x 200,000 29.0 and 24.6 ms (coded), 40 x 20,000 1,579 and 1,377
+// us; below that the shorter tiles' items end earlier: 33 x 1,000 143 and 149 us,
+// 100 samples 107 and 124.
+__host__ __device__ inline int64_t tall_from(int64_t pairs) { return pairs >= 64 ? 33 : 49; }
+
+// Rows of a band in tiles, pairs as above: as many 64-row ones as fit (one more
+// for tall_from rows left), the rest in one of 32 and / or one of 16.
 struct BandTiles {
   int64_t tall;
   int shorts, first;  // shorter tiles (0 .. 2) and the height of the first
 };
-__host__ __device__ inline BandTiles band_tiles(int64_t rows) {
-  const int64_t tall = (rows + 15) / 64, left = rows - tall * 64;
+__host__ __device__ inline BandTiles band_tiles(int64_t rows, int64_t pairs) {
+  const int64_t tall = (rows + 64 - tall_from(pairs)) / 64, left = rows - tall * 64;
   if (left <= 0) return {tall, 0, 0};
   return {tall, left > 32 ? 2 : 1, left > 16 ? 32 : 16};
 }
@@ -229,7 +238,7 @@ hipError_t launch_batch(const BatchArgs& a, int variant, int grid, hipStream_t s
 // column blocks [0, n_ct), `step` of them per launch, a launch's 64-row tiles
 // before its shorter ones; clears the band's fit failures.  No tiles written
 // when step is 0.
-hipError_t launch_band_setup(ItemTile* tiles, int64_t rows, int64_t n_ct, int64_t step,
+hipError_t launch_band_setup(ItemTile* tiles, int64_t rows, const BandTiles& b, int64_t n_ct, int64_t step,
                              unsigned long long* fail, uint32_t* fail_rows, hipStream_t stream);
 // Start of a call: fit failures {0, none}, a progress count of 0 and no stop.
 hipError_t launch_call_reset(unsigned long long* fail, const Control& ctl, hipStream_t stream);

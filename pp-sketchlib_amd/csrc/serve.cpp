@@ -190,20 +190,20 @@ int step_variant(const ppsk_server* s, int64_t rows) {
   return 2;
 }
 
-// Device memory of one step, carved from the arena.  A step with at least
-// two tiles per resident workgroup runs the persistent tile kernel (whole
-// tiles from work queues, per-workgroup count blocks), its last partial round
-// as (tile, k-mer length) items when that round would leave most workgroup
-// slots idle (tail tiles, per-tile count scratch).  A smaller step is a split
-// pass: items of a tile, a k-mer length and a run of words, its counts in
-// launches of step_ct column blocks (at most 256 MiB of counts).  A step of 61
-// queries x 8,000 references (8 k-mer lengths, 156 words) took 0.96 ms as
-// (64-row tile, k-mer length) workgroups and takes 0.61 ms as items, which all
-// end together; two overlapping steps of 83 and 92 queries 3.1 and 1.9 ms
-// (96 rows computed for each instead of 128).  Where a slot's share of the
-// arena has no room for that (its counts take up to 4 times as much for a few
-// rows), or a tile shape is forced, it is split per (tile, k-mer length) with
-// per-tile count scratch, launched in chunks of chunk_tiles.
+// Device memory of one step, carved from the arena.  A step is a split pass:
+// items of a tile, a k-mer length and a run of words, its counts in launches of
+// step_ct column blocks (at most 256 MiB of counts).  A step of 61 queries x
+// 8,000 references (8 k-mer lengths, 156 words) took 0.96 ms as (64-row tile,
+// k-mer length) workgroups and takes 0.61 ms as items, which all end together; two
+// overlapping steps of 83 and 92 queries 3.1 and 1.9 ms (96 rows computed for
+// each instead of 128).  Where a slot's share of the arena has no room for that
+// (its counts take up to 4 times as much for a few rows), or a tile shape or
+// kernel is forced, a step with at least two tiles per resident workgroup runs the
+// persistent tile kernel (whole tiles from work queues, per-workgroup count
+// blocks), its last partial round as (tile, k-mer length) items when that round
+// would leave most workgroup slots idle (tail tiles, per-tile count scratch), and
+// a smaller one is split per (tile, k-mer length) with per-tile count scratch,
+// launched in chunks of chunk_tiles.
 struct StepLayout {
   size_t staging, stripes, jv, clusters, band, tiles, scratch, tile_done, fail, fail_rows, params;
   size_t tail_tiles, tail_counts, tail_done, counts, knn_lists, total;
@@ -214,6 +214,11 @@ struct StepLayout {
   int grid;
   int64_t step_ct;
 };
+
+// Row tiles of a split step.
+ppsk::BandTiles step_tiles(const ppsk_server* s, int64_t rows) {
+  return ppsk::band_tiles(rows, (rows + 63) / 64 * ((s->ref->n + 255) / 256) * s->ref->n_k);
+}
 
 // Items of a split step's launch over n_ct column blocks.
 ItemCut band_cut(const ppsk_set* ref, const ppsk::BandTiles& b, int64_t n_ct) {
@@ -231,9 +236,9 @@ StepLayout layout_route(const ppsk_server* s, int64_t rows, bool items) {
   L.n_tiles = ((rows + tr - 1) / tr) * ((r->n + tc - 1) / tc);
   const size_t per_tile = (size_t)r->n_k * tr * tc * sizeof(uint16_t);
   L.grid = v == 2 ? s->grid2 : (v == 4 ? s->grid4 : 0);
-  L.persistent = L.grid > 0 && (s->force_persistent || L.n_tiles >= 2 * (int64_t)L.grid);
+  L.persistent = !items && L.grid > 0 && (s->force_persistent || L.n_tiles >= 2 * (int64_t)L.grid);
   L.chunk_tiles = std::max<int64_t>(1, std::min<int64_t>(L.n_tiles, s->scratch_budget / per_tile));
-  L.items = items && !L.persistent;
+  L.items = items;
   size_t off = 0;
   auto take = [&](size_t bytes) {
     const size_t at = off;
@@ -257,7 +262,7 @@ StepLayout layout_route(const ppsk_server* s, int64_t rows, bool items) {
       L.tail_done = take((size_t)L.tail * sizeof(uint32_t));
     }
   } else if (L.items) {
-    const ppsk::BandTiles b = ppsk::band_tiles(rows);
+    const ppsk::BandTiles b = step_tiles(s, rows);
     const int64_t n_ct = (r->n + 255) / 256, per = b.tall + b.shorts;
     const int64_t most = (int64_t)(s->scratch_budget / (ppsk::ITEM_COUNTS * sizeof(uint16_t)));
     L.step_ct = std::max<int64_t>(1, std::min(n_ct, most / (per * r->n_k)));
@@ -287,7 +292,7 @@ StepLayout layout_route(const ppsk_server* s, int64_t rows, bool items) {
 StepLayout layout(const ppsk_server* s, int64_t rows) {
   if (s->split) {
     const StepLayout L = layout_route(s, rows, true);
-    if (L.persistent || L.total <= s->slot_share) return L;
+    if (L.total <= s->slot_share) return L;
   }
   return layout_route(s, rows, false);
 }
@@ -385,7 +390,7 @@ int run_step(ppsk_server* s, Worker& w, std::vector<Piece>& batch, int64_t rows,
     STEP_TRY(hipMemsetAsync(tile_done, 0, (size_t)L.chunk_tiles * sizeof(uint32_t), w.st));
   }
   const int64_t n_ct = (ref->n + 255) / 256;
-  STEP_TRY(ppsk::launch_band_setup((ppsk::ItemTile*)(mem + L.tiles), rows, n_ct, L.items ? L.step_ct : 0,
+  STEP_TRY(ppsk::launch_band_setup((ppsk::ItemTile*)(mem + L.tiles), rows, step_tiles(s, rows), n_ct, L.items ? L.step_ct : 0,
                                    fail, fail_rows, w.st));
 
   // distances: query rows x every reference, dense band in device memory
@@ -471,7 +476,7 @@ int run_step(ppsk_server* s, Worker& w, std::vector<Piece>& batch, int64_t rows,
     }
     STEP_TRY(hipEventRecord(w.e1, w.st));
   } else if (L.items) {
-    const ppsk::BandTiles b = ppsk::band_tiles(rows);
+    const ppsk::BandTiles b = step_tiles(s, rows);
     const int64_t per = b.tall + b.shorts;
     ppsk::ItemArgs a;
     std::memset(&a, 0, sizeof(a));
