@@ -95,6 +95,7 @@ struct DeviceCtx {
   void* codes = nullptr;              // codes of a coded pass (at most CODE_BUDGET); above 1 GiB
   size_t codes_bytes = 0;             // kept while a sketch set lives (give_back)
   std::atomic<int> sets{0};           // sketch sets alive
+  unsigned in_use = 0;                // table and lists that the running call reads (Workspace)
   hipStream_t tail_stream = nullptr;  // the tail's (tile, k) launch beside the persistent one
   void* noalloc_scratch = nullptr;    // this device's copy of the fixed scratch array
   void* table = nullptr;              // Monte Carlo table of a dense pass

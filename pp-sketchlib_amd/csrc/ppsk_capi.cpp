@@ -126,6 +126,7 @@ CallScope::CallScope(DeviceCtx* ctx, uint64_t total) : c(ctx), cs(g_calls[ctx->d
   cs.running.store(1);
   // the device counters start from zero in stream order
   c->words_read = false;
+  c->in_use = 0;
   (void)ppsk::launch_call_reset(c->fail, c->ctl, c->stream);
 }
 
@@ -249,9 +250,10 @@ int grow_out(DeviceCtx* c, size_t need) {
   return PPSK_OK;
 }
 
-// Workspaces free to be given up while a dense pass makes its own (a call's lists
-// and its table may be in use).
-constexpr unsigned PASS_IDLE = WS_CODES | WS_HITS | WS_SKETCH;
+// Workspaces free to be given up while a dense pass makes its own.
+unsigned pass_idle(const DeviceCtx* c) {
+  return (WS_CODES | WS_HITS | WS_SKETCH | WS_SEL | WS_TABLE) & ~c->in_use;
+}
 
 constexpr size_t SPARE_BLOCKS = 4, SPARE_BYTES = (size_t)512 << 20;
 
@@ -313,7 +315,7 @@ int grow_tile_done(DeviceCtx* c, size_t n) {
   if (c->tile_done) HIP_TRY(hipFree(c->tile_done));
   c->tile_done = nullptr;
   c->tile_done_n = 0;
-  HIP_TRY(device_malloc(c, (void**)&c->tile_done, n * sizeof(uint32_t), PASS_IDLE));
+  HIP_TRY(device_malloc(c, (void**)&c->tile_done, n * sizeof(uint32_t), pass_idle(c)));
   // counters are left at zero by every tile's last workgroup afterwards
   HIP_TRY(hipMemset(c->tile_done, 0, n * sizeof(uint32_t)));
   c->tile_done_n = n;
@@ -495,11 +497,11 @@ int run_dense_tiles(DeviceCtx* c, ppsk::DistParams p, int variant, bool upper, i
   }
   size_t most = 0;
   for (auto& ch : chunks) most = std::max(most, ch.second - ch.first);
-  if (int rc = grow(c, &c->counts, &c->counts_bytes, most * per_tile, PASS_IDLE | WS_PSCRATCH)) return rc;
+  if (int rc = grow(c, &c->counts, &c->counts_bytes, most * per_tile, pass_idle(c) | WS_PSCRATCH)) return rc;
   if (int rc = grow_tile_done(c, most)) return rc;
   void* tptr = c->tiles;
   size_t tbytes = c->tiles_n * sizeof(ppsk::Tile);
-  if (int rc = grow(c, &tptr, &tbytes, tiles.size() * sizeof(ppsk::Tile), PASS_IDLE)) return rc;
+  if (int rc = grow(c, &tptr, &tbytes, tiles.size() * sizeof(ppsk::Tile), pass_idle(c))) return rc;
   c->tiles = (ppsk::Tile*)tptr;
   c->tiles_n = tbytes / sizeof(ppsk::Tile);
   HIP_TRY(copy_to_device(c, c->tiles, tiles.data(), tiles.size() * sizeof(ppsk::Tile), c->stream));
@@ -623,8 +625,8 @@ int run_dense_persistent(DeviceCtx* c, ppsk::DistParams p, int variant, bool upp
   // per-workgroup count blocks (the mixed-shape kernel's hold 64 x 256 counts)
   const size_t scratch = (size_t)grid * p.n_k * (kernel == ppsk::BATCH_MIXED ? 64 * 256 : tr * tc) *
                          sizeof(uint16_t);
-  if (int rc = grow(c, &c->pscratch, &c->pscratch_bytes, scratch, PASS_IDLE)) return rc;
-  if (int rc = grow(c, &c->pitems, &c->pitems_bytes, items.size() * sizeof(ppsk::BatchItem), PASS_IDLE)) {
+  if (int rc = grow(c, &c->pscratch, &c->pscratch_bytes, scratch, pass_idle(c))) return rc;
+  if (int rc = grow(c, &c->pitems, &c->pitems_bytes, items.size() * sizeof(ppsk::BatchItem), pass_idle(c))) {
     return rc;
   }
   if (!c->pparams) HIP_TRY(hipMalloc(&c->pparams, sizeof(ppsk::DistParams)));
@@ -632,11 +634,11 @@ int run_dense_persistent(DeviceCtx* c, ppsk::DistParams p, int variant, bool upp
   p.out_row_offset = 0;
   if (most_tail > 0) {
     const size_t per_tile = (size_t)p.n_k * tr * tc * sizeof(uint16_t);
-    if (int rc = grow(c, &c->counts, &c->counts_bytes, most_tail * per_tile, PASS_IDLE)) return rc;
+    if (int rc = grow(c, &c->counts, &c->counts_bytes, most_tail * per_tile, pass_idle(c))) return rc;
     if (int rc = grow_tile_done(c, most_tail)) return rc;
     void* tptr = c->tiles;
     size_t tbytes = c->tiles_n * sizeof(ppsk::Tile);
-    if (int rc = grow(c, &tptr, &tbytes, tail_tiles.size() * sizeof(ppsk::Tile), PASS_IDLE)) return rc;
+    if (int rc = grow(c, &tptr, &tbytes, tail_tiles.size() * sizeof(ppsk::Tile), pass_idle(c))) return rc;
     c->tiles = (ppsk::Tile*)tptr;
     c->tiles_n = tbytes / sizeof(ppsk::Tile);
     HIP_TRY(copy_to_device(c, c->tiles, tail_tiles.data(), tail_tiles.size() * sizeof(ppsk::Tile),
@@ -937,7 +939,7 @@ constexpr size_t CODE_BUDGET = (size_t)8 << 30;
 // given back then).
 bool item_scratch(DeviceCtx* c, const ItemPlan& pl) {
   if (pl.tiles.empty()) return true;
-  const unsigned idle = PASS_IDLE | WS_PSCRATCH;
+  const unsigned idle = pass_idle(c) | WS_PSCRATCH;
   const size_t counts = pl.count_blocks * ppsk::ITEM_COUNTS * sizeof(uint16_t);
   const size_t lists = pl.slabs.size() * sizeof(ppsk::CodeGroup) + pl.tiles.size() * sizeof(ppsk::ItemTile);
   if (grow(c, &c->counts, &c->counts_bytes, counts, idle) == PPSK_OK &&
@@ -1180,6 +1182,7 @@ int call_table(DeviceCtx* c, const ppsk_set* s, const RandomIn& rnd, float** dta
   if (rnd.mode != PPSK_RANDOM_MC) return PPSK_OK;
   const size_t bytes = (size_t)s->n_k * rnd.n_clusters * rnd.n_clusters * sizeof(float);
   if (int rc = grow(c, &c->table, &c->table_bytes, bytes, WS_ALL & ~WS_TABLE)) return rc;
+  c->in_use |= WS_TABLE;
   *dtab = (float*)c->table;
   HIP_TRY(copy_to_device(c, *dtab, rnd.table, bytes, c->stream));
   return PPSK_OK;
@@ -1246,7 +1249,7 @@ int knn_lists(DeviceCtx* c, int64_t rows, int kNN, KnnLists* L) {
   const size_t m = ((size_t)rows * kNN + 31) / 32 * 32;
   const size_t hw = ppsk::knn_heap_workspace(rows, kNN);
   const size_t bytes = m * (2 * sizeof(int64_t) + sizeof(float)) + hw;
-  if (int rc = grow(c, &c->sel, &c->sel_bytes, bytes, WS_ALL & ~(WS_SEL | WS_TABLE))) return rc;
+  if (int rc = grow(c, &c->sel, &c->sel_bytes, bytes, WS_ALL & ~(WS_SEL | c->in_use))) return rc;
   L->i = (int64_t*)c->sel;
   L->j = L->i + m;
   L->d = (float*)(L->j + m);
@@ -1652,6 +1655,7 @@ int ppsk_knn(ppsk_set* ref, int32_t random_mode, int32_t n_clusters, const float
     if ((rc = call_table(c, ref, rnd, &dtab))) return rc;
     KnnLists L;
     if ((rc = knn_lists(c, band, kNN, &L))) return rc;
+    c->in_use |= WS_SEL;
     for (int64_t r0 = 0; r0 < n && rc == PPSK_OK; r0 += band) {
       const int64_t r1 = std::min(n, r0 + band);
       ppsk::DistParams p;
