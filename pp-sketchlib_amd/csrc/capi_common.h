@@ -199,6 +199,9 @@ hipError_t copy_to_device(DeviceCtx* c, void* dst, const void* src, size_t bytes
                           hipStream_t stream);
 hipError_t copy_to_host(DeviceCtx* c, void* dst, const void* src, size_t bytes, hipStream_t stream);
 
+// memcpy by up to 4 threads from 4 MiB on; src null: zeroes.
+void copy_host(void* dst, const void* src, size_t bytes);
+
 // Tile completion counters, zero on return.
 int grow_tile_done(DeviceCtx* c, size_t n);
 

@@ -65,6 +65,17 @@ int lanes_for(size_t bytes) {
 
 }  // namespace
 
+void copy_host(void* dst, const void* src, size_t bytes) {
+  std::atomic<size_t> next{0};
+  on_lanes(lanes_for(bytes), [&](int) {
+    for (size_t at; (at = next.fetch_add(HostStage::BLOCK)) < bytes;) {
+      const size_t n = std::min(HostStage::BLOCK, bytes - at);
+      if (src) std::memcpy((char*)dst + at, (const char*)src + at, n);
+      else std::memset((char*)dst + at, 0, n);
+    }
+  });
+}
+
 hipError_t HostStage::init() {
   hipError_t e = hipSuccess;
   for (int x = 0; x < 2 * LANES && e == hipSuccess; ++x) {

@@ -121,6 +121,7 @@ struct ppsk_request {
   // the queries' sketches [n_q][n_k][s64 * 14], equal-base terms [n_q][n_k] and
   // cluster ids [n_q] in the server's query memory (bytes > 0), or in raw, jv, cl
   size_t at = 0, bytes = 0, at_jv = 0, at_cl = 0;
+  hipEvent_t uploaded = nullptr;  // they are on the device
   std::vector<uint64_t> raw;
   std::vector<double> jv;     // [n_q][n_k] equal-base terms
   std::vector<uint16_t> cl;   // [n_q] Monte Carlo cluster ids
@@ -155,15 +156,23 @@ struct ppsk_server {
   bool split = true;      // no tile shape or kernel forced
   Arena arena;
   void* arena_mem = nullptr;
-  // Memory of submitted queries, filled by ppsk_server_submit from the caller's
-  // arrays, so that a step reads them where they are: kept on the host until
-  // their step, 237 queries (41 MB) in four requests cost 6 ms of page faults,
-  // copies and stopped queues (freeing memory that a pageable copy locked) of
-  // a 10 ms burst.  4 x max_rows queries, at most 256 MiB; a request that finds
-  // no room there waits on the host.
+  // Memory of submitted queries, page-locked and on the device.  ppsk_server_submit
+  // fills the first from the caller's arrays and queues its copy to the second,
+  // which a step waits for on its stream; submit waits for nothing.  (In ordinary
+  // memory 237 queries, 41 MB, in four requests cost 6 ms of page faults, copies and
+  // stopped queues, as freeing memory that a pageable copy locked stops them, of a
+  // 10 ms burst.  Waiting for the copy made a submit of one query take up to 56 ms:
+  // with four slots and more it shares a hardware queue with one of them.  Copied
+  // by the step itself the burst takes 3.5 ms instead of 3.3.)  4 x max_rows
+  // queries, at most 256 MiB; a request that finds no room there waits in ordinary
+  // memory.
   Arena queries;
   void* queries_mem = nullptr;
+  char* queries_host = nullptr;
   hipStream_t upload = nullptr;
+  std::vector<hipEvent_t> uploads;  // events no request is using
+  std::vector<hipEvent_t> upload_events;  // all of them
+  int32_t submits = 0;  // threads inside ppsk_server_submit
   std::mutex mu;
   std::condition_variable cv_work, cv_done;
   std::deque<ppsk_request*> pending;
@@ -367,7 +376,9 @@ int run_step(ppsk_server* s, Worker& w, std::vector<Piece>& batch, int64_t rows,
     const hipMemcpyKind kind = resident ? hipMemcpyDeviceToDevice : hipMemcpyHostToDevice;
     const char* base = (const char*)s->queries_mem + r->at;
     const uint64_t* raw = (const uint64_t*)base + (size_t)pc.q0 * words;
-    if (!resident) {
+    if (resident) {
+      STEP_TRY(hipStreamWaitEvent(w.st, r->uploaded, 0));
+    } else {
       STEP_TRY(hipMemcpyAsync(staging + (size_t)o * words, r->raw.data() + (size_t)pc.q0 * words,
                               (size_t)pc.n * s->per_sample, kind, w.st));
       raw = staging + (size_t)o * words;
@@ -596,17 +607,26 @@ int run_step(ppsk_server* s, Worker& w, std::vector<Piece>& batch, int64_t rows,
   return PPSK_OK;
 }
 
-// The queries of a new request into the server's query memory; without room
-// there, into the request.
+// Gives a request's query memory back (s->mu held; nothing reads it any more).
+void release_queries(ppsk_server* s, ppsk_request* r) {
+  if (!r->bytes) return;
+  s->queries.release(r->at, r->bytes);
+  s->uploads.push_back(r->uploaded);
+  r->bytes = 0;
+}
+
+// The queries of a new request into the server's query memory, their copy to the
+// device queued; without room there, into the request.
 int take_queries(ppsk_server* s, ppsk_request* r, const uint64_t* raw) {
   const size_t raw_bytes = (size_t)r->n_q * s->per_sample;
   const size_t jv_bytes = r->jv.size() * sizeof(double), cl_bytes = r->cl.size() * sizeof(uint16_t);
-  DeviceCtx* c = nullptr;
-  if (s->queries_mem && s->upload) {
+  if (s->upload) {
     const size_t at_jv = align_up(raw_bytes), at_cl = at_jv + align_up(jv_bytes);
     const size_t bytes = at_cl + align_up(cl_bytes);
     std::lock_guard<std::mutex> lk(s->mu);
-    if (s->queries.alloc(bytes, &r->at)) {
+    if (!s->uploads.empty() && s->queries.alloc(bytes, &r->at)) {
+      r->uploaded = s->uploads.back();
+      s->uploads.pop_back();
       r->bytes = bytes;
       r->at_jv = at_jv;
       r->at_cl = at_cl;
@@ -616,22 +636,24 @@ int take_queries(ppsk_server* s, ppsk_request* r, const uint64_t* raw) {
     r->raw.assign(raw, raw + raw_bytes / sizeof(uint64_t));
     return PPSK_OK;
   }
-  char* to = (char*)s->queries_mem + r->at;
-  int rc = get_ctx(s->device, &c);
-  if (rc == PPSK_OK) {
-    hipError_t e = copy_to_device(c, to, raw, raw_bytes, s->upload);
-    if (e == hipSuccess) e = copy_to_device(c, to + r->at_jv, r->jv.data(), jv_bytes, s->upload);
-    if (e == hipSuccess) e = copy_to_device(c, to + r->at_cl, r->cl.data(), cl_bytes, s->upload);
-    const hipError_t es = hipStreamSynchronize(s->upload);
-    if (e == hipSuccess) e = es;
-    if (e != hipSuccess) rc = fail(PPSK_ERR_HIP, std::string("query upload: ") + hipGetErrorString(e));
+  char* host = s->queries_host + r->at;
+  copy_host(host, raw, raw_bytes);
+  if (jv_bytes) std::memcpy(host + r->at_jv, r->jv.data(), jv_bytes);
+  if (cl_bytes) std::memcpy(host + r->at_cl, r->cl.data(), cl_bytes);
+  int device = s->device;  // the caller's current device stays what it was
+  hipError_t e = hipGetDevice(&device);
+  if (e == hipSuccess && device != s->device) e = hipSetDevice(s->device);
+  if (e == hipSuccess) {
+    e = hipMemcpyAsync((char*)s->queries_mem + r->at, host, r->at_cl + cl_bytes, hipMemcpyHostToDevice,
+                       s->upload);
   }
-  if (rc != PPSK_OK) {
-    std::lock_guard<std::mutex> lk(s->mu);
-    s->queries.release(r->at, r->bytes);
-    r->bytes = 0;
-  }
-  return rc;
+  if (e == hipSuccess) e = hipEventRecord(r->uploaded, s->upload);
+  if (device != s->device) (void)hipSetDevice(device);
+  if (e == hipSuccess) return PPSK_OK;
+  (void)hipStreamSynchronize(s->upload);
+  std::lock_guard<std::mutex> lk(s->mu);
+  release_queries(s, r);
+  return fail(PPSK_ERR_HIP, std::string("query upload: ") + hipGetErrorString(e));
 }
 
 // Rows of the next piece of the oldest request in a step of its own.
@@ -803,7 +825,7 @@ void worker_main(ppsk_server* s, Worker* w) {
         }
         r->rows_done += pc.n;
         if (r->rows_done == r->n_q) {
-          if (r->bytes) s->queries.release(r->at, r->bytes);
+          release_queries(s, r);
           finish_request(r, t);
           s->requests_done += 1;
         }
@@ -909,22 +931,33 @@ int ppsk_server_create(ppsk_set* ref, int32_t random_mode, int32_t n_clusters,
   s->t0 = std::chrono::steady_clock::now();
   const size_t query_bytes =
       align_up(std::min<size_t>((size_t)256 << 20, 4 * (size_t)max_rows * (s->per_sample + 16 * ref->n_k)));
-  if (hipMalloc(&s->queries_mem, query_bytes) == hipSuccess) {
+  // one event for each request that waits there; further ones wait in ordinary memory
+  bool queries = hipMalloc(&s->queries_mem, query_bytes) == hipSuccess &&
+                 hipHostMalloc((void**)&s->queries_host, query_bytes, hipHostMallocDefault) == hipSuccess;
+  for (int x = 0; x < 256 && queries; ++x) {
+    hipEvent_t ev = nullptr;
+    if (hipEventCreateWithFlags(&ev, hipEventDisableTiming) != hipSuccess) break;
+    s->uploads.push_back(ev);
+  }
+  if (queries) {
+    copy_host(s->queries_host, nullptr, query_bytes);  // the pages' first touch
     s->queries.init((char*)s->queries_mem, query_bytes);
   } else {
-    (void)hipGetLastError();  // every request waits on the host
-    s->queries_mem = nullptr;
+    (void)hipGetLastError();  // every request waits in ordinary memory
   }
+  s->upload_events = s->uploads;
   std::vector<hipStream_t> streams;
-  if (create_slot_streams(n_slots + 1, &streams) != PPSK_OK) {
+  if (create_slot_streams(n_slots + (queries ? 1 : 0), &streams) != PPSK_OK) {
     for (hipStream_t st : streams) hipStreamDestroy(st);
     ppsk_server_free(s);
     return fail(PPSK_ERR_HIP, "serving stream creation");
   }
-  // the queries' uploads on a queue of their own where there is one: on a slot's
-  // queue they waited for its distance kernels (four requests 3.7 -> 3.2 ms)
-  s->upload = streams.back();
-  streams.pop_back();
+  if (queries) {
+    // on a queue of their own where there is one: on a slot's queue the uploads
+    // waited for its distance kernels (four requests 3.7 -> 3.2 ms)
+    s->upload = streams.back();
+    streams.pop_back();
+  }
   for (int i = 0; i < n_slots; ++i) {
     auto* w = new Worker();
     w->st = streams[i];
@@ -950,6 +983,19 @@ int ppsk_server_create(ppsk_set* ref, int32_t random_mode, int32_t n_clusters,
 int ppsk_server_submit(ppsk_server* s, int64_t n_queries, const uint64_t* raw,
                        const uint64_t* lengths, const uint16_t* clusters, int64_t* ticket) {
   if (!s || !ticket) return fail(PPSK_ERR_ARG, "server / ticket is NULL");
+  // ppsk_server_free waits for the submits that began before it
+  struct Inside {
+    ppsk_server* s;
+    explicit Inside(ppsk_server* sv) : s(sv) {
+      std::lock_guard<std::mutex> lk(s->mu);
+      s->submits += 1;
+    }
+    ~Inside() {
+      std::lock_guard<std::mutex> lk(s->mu);
+      s->submits -= 1;
+      if (s->submits == 0) s->cv_done.notify_all();
+    }
+  } inside(s);
   if (n_queries < 1 || !raw) return fail(PPSK_ERR_ARG, "a request needs at least one query sketch");
   // a request larger than max_rows is served in pieces of at most max_rows
   // rows, so only a piece has to fit the arena
@@ -1001,8 +1047,7 @@ int ppsk_server_submit(ppsk_server* s, int64_t n_queries, const uint64_t* raw,
   {
     std::lock_guard<std::mutex> lk(s->mu);
     if (s->stop) {
-      if (r->bytes) s->queries.release(r->at, r->bytes);
-      delete r;
+      delete r;  // (its query memory goes with the server)
       return fail(PPSK_ERR_STATE, "server stopped");
     }
     r->ticket = s->next_ticket++;
@@ -1078,8 +1123,9 @@ int ppsk_server_free(ppsk_server* s) {
   for (auto& t : s->workers) t.join();
   {
     std::unique_lock<std::mutex> lk(s->mu);
-    // every request not yet served fails; waiters collect their failure and
-    // leave before any request or the server is deleted
+    // every request not yet served fails; submits and waiters collect their failure
+    // and leave before any request or the server is deleted
+    s->cv_done.wait(lk, [&] { return s->submits == 0; });
     for (auto& kv : s->tickets) {
       ppsk_request* r = kv.second;
       if (!r->done) {
@@ -1096,8 +1142,13 @@ int ppsk_server_free(ppsk_server* s) {
   }
   hipSetDevice(s->device);
   if (s->arena_mem) hipFree(s->arena_mem);
+  if (s->upload) {
+    hipStreamSynchronize(s->upload);
+    hipStreamDestroy(s->upload);
+  }
+  for (hipEvent_t ev : s->upload_events) hipEventDestroy(ev);
   if (s->queries_mem) hipFree(s->queries_mem);
-  if (s->upload) hipStreamDestroy(s->upload);
+  if (s->queries_host) hipHostFree(s->queries_host);
   if (s->d_table) hipFree(s->d_table);
   delete s;
   return PPSK_OK;
