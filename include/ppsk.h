@@ -267,12 +267,13 @@ int ppsk_batch_create(int device_id, const ppsk_job *jobs, int32_t n_jobs,
                       ppsk_batch **out);
 
 /*
- * Run every job: one graph launch (queue reset + persistent kernel), replayed
+ * Run every job: one graph launch (queue reset + the plan's kernels), replayed
  * on later runs.  variant: the plan -- every job in one tile shape (2:
  * 64 x 256, 4: 32 x 256, 5: 16 x 256), 6: each job's rows split over the
  * three tile heights (row tiles laid from its first row, each at a multiple
- * of its own height; one persistent launch running every shape), or 0 for
- * the autotuner.  On the first run of a batch with an unseen job-shape
+ * of its own height; as items of a tile, a k-mer length and a run of words
+ * while their counts fit 1 GiB, else one persistent launch running every
+ * shape), or 0 for the autotuner.  On the first run of a batch with an unseen job-shape
  * signature the autotuner times plans 2, 4 and 5 on the batch itself,
  * derives each shape's throughput on padded work, splits every job's rows
  * for the least estimated time, times that plan 6 too and keeps the fastest
@@ -370,8 +371,9 @@ int ppsk_server_free(ppsk_server *server);
 
 /*
  * Timing of the last dense/kNN/threshold call on this thread, measured with
- * HIP events on the launch stream: summed duration of the distance-tile
- * kernel launches and their number.
+ * HIP events on the launch stream: summed duration of the distance launches
+ * (coding, matching and output kernels of a launch together), their number and
+ * their work items.
  */
 int ppsk_last_timing(double *kernel_ms, int64_t *n_launches, int64_t *n_items);
 
