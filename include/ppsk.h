@@ -310,7 +310,9 @@ int ppsk_batch_free(ppsk_batch *batch);
  * step takes its next rows and the rest stays at the head of the queue, so
  * requests of any size are accepted and a large one runs on several steps at
  * once.  Requests arriving while other steps run join the next step that has
- * room, and steps of different workers overlap on the GPU.  max_rows bounds
+ * room, and steps of different workers overlap on the GPU.  Waiting queries lie
+ * in page-locked and device memory of the server, up to 4 * max_rows of them and
+ * 256 MiB of each; the others in ordinary memory.  max_rows bounds
  * a step's duration and with it the latency a step adds to the requests
  * queued behind it.  A request's results do not depend on the steps it
  * joins.
