@@ -81,6 +81,8 @@ struct DeviceCtx {
   unsigned long long* fail = nullptr;
   unsigned long long* words = nullptr;  // page-locked copy of the first three; [3] threshold hits
   bool words_read = false;              // `words` holds the call's final values
+  static constexpr size_t RESULT = (size_t)2 << 20;
+  char* result = nullptr;               // page-locked: lists of a call, up to RESULT bytes
   void* out = nullptr;
   size_t out_bytes = 0;
   hipStream_t copy_stream = nullptr;  // device -> host copies of finished rows

@@ -53,6 +53,8 @@ int get_ctx(int device, DeviceCtx** out) {
     HIP_TRY(hipStreamCreateWithFlags(&c->copy_stream, hipStreamNonBlocking));
     HIP_TRY(hipMalloc(&c->fail, 4 * sizeof(unsigned long long)));
     HIP_TRY(hipHostMalloc((void**)&c->words, 4 * sizeof(unsigned long long), hipHostMallocDefault));
+    HIP_TRY(hipHostMalloc((void**)&c->result, DeviceCtx::RESULT, hipHostMallocDefault));
+    std::memset(c->result, 0, DeviceCtx::RESULT);
     HIP_TRY(c->host.init());
     HIP_TRY(hipEventCreateWithFlags(&c->raw_copied, hipEventDisableTiming));
     for (auto& ev : c->raw_striped) HIP_TRY(hipEventCreateWithFlags(&ev, hipEventDisableTiming));
@@ -1257,11 +1259,26 @@ int knn_lists(DeviceCtx* c, int64_t rows, int kNN, KnnLists* L) {
   return PPSK_OK;
 }
 
-hipError_t copy_knn(DeviceCtx* c, const KnnLists& L, size_t m, int64_t* i_vec, int64_t* j_vec,
-                    float* dists) {
-  hipError_t e = copy_to_host(c, i_vec, L.i, m * sizeof(int64_t), c->stream);
-  if (e == hipSuccess) e = copy_to_host(c, j_vec, L.j, m * sizeof(int64_t), c->stream);
-  if (e == hipSuccess) e = copy_to_host(c, dists, L.d, m * sizeof(float), c->stream);
+// m entries of three lists that lie at d_i, d_j, d_d, in this order in one buffer,
+// to the host.  Up to 2 MiB come in one copy behind the kernels, through the
+// context's own page-locked memory: kNN of 451 samples 337 us a call, 347 with
+// a wait for the kernels before three copies through the shared blocks.
+hipError_t copy_lists(DeviceCtx* c, const int64_t* d_i, const int64_t* d_j, const float* d_d, size_t m,
+                      int64_t* i_vec, int64_t* j_vec, float* dists) {
+  const size_t at_j = (const char*)d_j - (const char*)d_i, at_d = (const char*)d_d - (const char*)d_i;
+  const size_t bytes = at_d + m * sizeof(float);
+  if (bytes <= DeviceCtx::RESULT) {
+    hipError_t e = hipMemcpyAsync(c->result, d_i, bytes, hipMemcpyDeviceToHost, c->stream);
+    if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
+    if (e != hipSuccess) return e;
+    std::memcpy(i_vec, c->result, m * sizeof(int64_t));
+    std::memcpy(j_vec, c->result + at_j, m * sizeof(int64_t));
+    std::memcpy(dists, c->result + at_d, m * sizeof(float));
+    return hipSuccess;
+  }
+  hipError_t e = copy_to_host(c, i_vec, d_i, m * sizeof(int64_t), c->stream);
+  if (e == hipSuccess) e = copy_to_host(c, j_vec, d_j, m * sizeof(int64_t), c->stream);
+  if (e == hipSuccess) e = copy_to_host(c, dists, d_d, m * sizeof(float), c->stream);
   return e;
 }
 
@@ -1272,7 +1289,7 @@ int knn_from_triangle(DeviceCtx* c, const float* tri, int64_t n, int col, int kN
   KnnLists L;
   if (int rc = knn_lists(c, n, kNN, &L)) return rc;
   hipError_t e = ppsk::launch_knn_select_triangle(tri, n, col, kNN, L.i, L.j, L.d, c->stream, L.heap);
-  if (e == hipSuccess) e = copy_knn(c, L, (size_t)n * kNN, i_vec, j_vec, dists);
+  if (e == hipSuccess) e = copy_lists(c, L.i, L.j, L.d, (size_t)n * kNN, i_vec, j_vec, dists);
   if (e != hipSuccess) hipStreamSynchronize(c->stream);  // nothing queued may outlive its buffers
   trim(&c->sel, &c->sel_bytes);
   if (e != hipSuccess) return fail(e == hipErrorOutOfMemory ? PPSK_ERR_MEMORY : PPSK_ERR_HIP,
@@ -1319,9 +1336,7 @@ int threshold_from_triangle(DeviceCtx* c, const float2* tri, int64_t n, int col,
     float* d_d = (float*)(d_j + m);
     e = ppsk::launch_threshold_write(tri, rows, n, false, col, cutoff, (int64_t*)c->sel, d_i, d_j,
                                      d_d, c->stream);
-    if (e == hipSuccess) e = copy_to_host(c, hi, d_i, m * sizeof(int64_t), c->stream);
-    if (e == hipSuccess) e = copy_to_host(c, hj, d_j, m * sizeof(int64_t), c->stream);
-    if (e == hipSuccess) e = copy_to_host(c, hd, d_d, m * sizeof(float), c->stream);
+    if (e == hipSuccess) e = copy_lists(c, d_i, d_j, d_d, m, hi, hj, hd);
     if (e != hipSuccess) hipStreamSynchronize(c->stream);
   }
   trim(&c->sel, &c->sel_bytes);
@@ -1677,8 +1692,8 @@ int ppsk_knn(ppsk_set* ref, int32_t random_mode, int32_t n_clusters, const float
       hipError_t e = ppsk::launch_knn_select((const float*)c->out, r0, r1 - r0, n, dist_col, kNN,
                                              L.i, L.j, L.d, c->stream, L.heap);
       if (e == hipSuccess) {
-        e = copy_knn(c, L, (size_t)(r1 - r0) * kNN, i_vec + r0 * kNN, j_vec + r0 * kNN,
-                     dists + r0 * kNN);
+        e = copy_lists(c, L.i, L.j, L.d, (size_t)(r1 - r0) * kNN, i_vec + r0 * kNN, j_vec + r0 * kNN,
+                       dists + r0 * kNN);
       }
       if (e != hipSuccess) rc = fail(PPSK_ERR_HIP, std::string("kNN select: ") + hipGetErrorString(e));
     }
