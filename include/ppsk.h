@@ -76,7 +76,7 @@ int ppsk_device_init(int device_id, size_t *mem_free, size_t *mem_total,
  * ppsk_cancel: asks the call running on the device to stop, and every call
  * that starts on the device to stop at once, until ppsk_cancel_reset.  The
  * kernels read the request between work items and finish normally (no
- * trap; a pass of less than about a millisecond ends first); the call waits
+ * trap; a pass of less than about two milliseconds ends first); the call waits
  * for them and returns PPSK_ERR_CANCELLED, its outputs undefined.
  */
 int ppsk_progress(int device_id, uint64_t *done, uint64_t *total,

@@ -237,7 +237,7 @@ struct ItemCut {
   double work_us;
 };
 // Split passes estimated shorter do not look for a cancellation (item_stopped).
-constexpr double WATCH_US = 1000.0;
+constexpr double WATCH_US = 2000.0;
 ItemCut cut_items(int64_t n64, int64_t n32, int64_t n16, int n_k, int s64, bool coded);
 // The launch's tiles and cut in its arguments.
 void set_items(ppsk::ItemArgs* a, const ppsk::ItemTile* tiles, int64_t n_tiles, const ItemCut& cut);

@@ -169,7 +169,7 @@ __device__ __forceinline__ void add_progress(const Control& c, unsigned long lon
 // 863 us instead of 433.  So one item in 64 reads the flag and passes it on in a
 // device word that the others read, and one in 64 mirrors the progress.  The
 // first workgroups of a call, which start together right after the host has
-// looked, read neither; nor does a pass of less than about 1 ms, which ends
+// looked, read neither; nor does a pass of less than about 2 ms, which ends
 // before a request could stop it (its call reports the request and the final
 // count all the same): looking took 37 of the 223 us of one query against 6,000.
 constexpr uint32_t ITEM_WATCH = 64, ITEM_MIRROR = 64;
