@@ -1160,12 +1160,13 @@ size_t tail_split_tiles(size_t n, int grid) {
   return (n > g && r > 0 && r <= g / 2) ? r : 0;
 }
 
-// Per-sample inputs to the device, between calls: a copy behind a pass would hold
-// its page-locked block until the pass ends.
+// Per-sample inputs to the device, after the work queued so far; on the copy
+// stream, as a copy behind a pass would hold its page-locked block until the pass
+// ends.
 hipError_t copy_meta(DeviceCtx* c, void* dst, const void* src, size_t bytes) {
-  std::lock_guard<std::mutex> lk(c->mu);
-  const hipError_t e = copy_to_device(c, dst, src, bytes, c->stream);
-  const hipError_t es = hipStreamSynchronize(c->stream);
+  hipError_t e = hipStreamSynchronize(c->stream);
+  if (e == hipSuccess) e = copy_to_device(c, dst, src, bytes, c->copy_stream);
+  const hipError_t es = hipStreamSynchronize(c->copy_stream);
   return e == hipSuccess ? es : e;
 }
 
