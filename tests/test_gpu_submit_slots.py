@@ -41,7 +41,7 @@ def test_submit_beside_many_slots():
             assert np.array_equal(r["thr_j"], first["thr_j"])
     ref.free()
     print(f"longest submit of one query {worst * 1e3:.2f} ms")
-    assert worst < 0.002
+    assert worst < 0.005
 
 
 def test_free_waits_for_a_submit():
