@@ -39,6 +39,7 @@
 #include <map>
 #include <mutex>
 #include <string>
+#include <system_error>
 #include <thread>
 #include <vector>
 
@@ -121,7 +122,6 @@ struct ppsk_request {
   // the queries' sketches [n_q][n_k][s64 * 14], equal-base terms [n_q][n_k] and
   // cluster ids [n_q] in the server's query memory (bytes > 0), or in raw, jv, cl
   size_t at = 0, bytes = 0, at_jv = 0, at_cl = 0;
-  hipEvent_t uploaded = nullptr;  // they are on the device
   std::vector<uint64_t> raw;
   std::vector<double> jv;     // [n_q][n_k] equal-base terms
   std::vector<uint16_t> cl;   // [n_q] Monte Carlo cluster ids
@@ -157,21 +157,24 @@ struct ppsk_server {
   Arena arena;
   void* arena_mem = nullptr;
   // Memory of submitted queries, page-locked and on the device.  ppsk_server_submit
-  // fills the first from the caller's arrays and queues its copy to the second,
-  // which a step waits for on its stream; submit waits for nothing.  (In ordinary
-  // memory 237 queries, 41 MB, in four requests cost 6 ms of page faults, copies and
-  // stopped queues, as freeing memory that a pageable copy locked stops them, of a
-  // 10 ms burst.  Waiting for the copy made a submit of one query take up to 56 ms:
-  // with four slots and more it shares a hardware queue with one of them.  Copied
-  // by the step itself the burst takes 3.5 ms instead of 3.3.)  4 x max_rows
-  // queries, at most 256 MiB; a request that finds no room there waits in ordinary
-  // memory.
+  // fills the first from the caller's arrays; a thread copies it to the second and
+  // passes the request on to `pending`.  So submit waits for nothing: waiting for
+  // the copy made a submit of one query take up to 56 ms (with four slots and more
+  // it shares a hardware queue with one of them), and queueing a copy blocks for 4
+  // to 12 ms now and then.  (In ordinary memory 237 queries, 41 MB, in four requests
+  // cost 6 ms of page faults, copies and stopped queues, as freeing memory that a
+  // pageable copy locked stops them, of a 10 ms burst.  Passed on before its copy
+  // has ended, a request starts its step beside the one before it and not one copy
+  // later, and both end their kNN together: 3.5 ms a burst instead of 3.2.)  4 x
+  // max_rows queries, at most 256 MiB; a request that finds no room there waits in
+  // ordinary memory.
   Arena queries;
   void* queries_mem = nullptr;
   char* queries_host = nullptr;
   hipStream_t upload = nullptr;
-  std::vector<hipEvent_t> uploads;  // events no request is using
-  std::vector<hipEvent_t> upload_events;  // all of them
+  std::thread uploader;
+  std::deque<ppsk_request*> fresh;  // requests the uploader has yet to pass on
+  std::condition_variable cv_upload;
   int32_t submits = 0;  // threads inside ppsk_server_submit
   std::mutex mu;
   std::condition_variable cv_work, cv_done;
@@ -376,9 +379,7 @@ int run_step(ppsk_server* s, Worker& w, std::vector<Piece>& batch, int64_t rows,
     const hipMemcpyKind kind = resident ? hipMemcpyDeviceToDevice : hipMemcpyHostToDevice;
     const char* base = (const char*)s->queries_mem + r->at;
     const uint64_t* raw = (const uint64_t*)base + (size_t)pc.q0 * words;
-    if (resident) {
-      STEP_TRY(hipStreamWaitEvent(w.st, r->uploaded, 0));
-    } else {
+    if (!resident) {
       STEP_TRY(hipMemcpyAsync(staging + (size_t)o * words, r->raw.data() + (size_t)pc.q0 * words,
                               (size_t)pc.n * s->per_sample, kind, w.st));
       raw = staging + (size_t)o * words;
@@ -611,22 +612,19 @@ int run_step(ppsk_server* s, Worker& w, std::vector<Piece>& batch, int64_t rows,
 void release_queries(ppsk_server* s, ppsk_request* r) {
   if (!r->bytes) return;
   s->queries.release(r->at, r->bytes);
-  s->uploads.push_back(r->uploaded);
   r->bytes = 0;
 }
 
-// The queries of a new request into the server's query memory, their copy to the
-// device queued; without room there, into the request.
-int take_queries(ppsk_server* s, ppsk_request* r, const uint64_t* raw) {
+// The queries of a new request into the server's query memory; without room
+// there, into the request.
+void take_queries(ppsk_server* s, ppsk_request* r, const uint64_t* raw) {
   const size_t raw_bytes = (size_t)r->n_q * s->per_sample;
   const size_t jv_bytes = r->jv.size() * sizeof(double), cl_bytes = r->cl.size() * sizeof(uint16_t);
   if (s->upload) {
     const size_t at_jv = align_up(raw_bytes), at_cl = at_jv + align_up(jv_bytes);
     const size_t bytes = at_cl + align_up(cl_bytes);
     std::lock_guard<std::mutex> lk(s->mu);
-    if (!s->uploads.empty() && s->queries.alloc(bytes, &r->at)) {
-      r->uploaded = s->uploads.back();
-      s->uploads.pop_back();
+    if (s->queries.alloc(bytes, &r->at)) {
       r->bytes = bytes;
       r->at_jv = at_jv;
       r->at_cl = at_cl;
@@ -634,26 +632,47 @@ int take_queries(ppsk_server* s, ppsk_request* r, const uint64_t* raw) {
   }
   if (!r->bytes) {
     r->raw.assign(raw, raw + raw_bytes / sizeof(uint64_t));
-    return PPSK_OK;
+    return;
   }
   char* host = s->queries_host + r->at;
   copy_host(host, raw, raw_bytes);
   if (jv_bytes) std::memcpy(host + r->at_jv, r->jv.data(), jv_bytes);
   if (cl_bytes) std::memcpy(host + r->at_cl, r->cl.data(), cl_bytes);
-  int device = s->device;  // the caller's current device stays what it was
-  hipError_t e = hipGetDevice(&device);
-  if (e == hipSuccess && device != s->device) e = hipSetDevice(s->device);
-  if (e == hipSuccess) {
-    e = hipMemcpyAsync((char*)s->queries_mem + r->at, host, r->at_cl + cl_bytes, hipMemcpyHostToDevice,
-                       s->upload);
+}
+
+// Passes requests on in their order, their queries on the device.
+void uploader_main(ppsk_server* s) {
+  const hipError_t ed = hipSetDevice(s->device);
+  for (;;) {
+    ppsk_request* r = nullptr;
+    {
+      std::unique_lock<std::mutex> lk(s->mu);
+      s->cv_upload.wait(lk, [&] { return s->stop || !s->fresh.empty(); });
+      if (s->stop) return;
+      r = s->fresh.front();
+      s->fresh.pop_front();
+    }
+    hipError_t e = ed;
+    if (r->bytes) {
+      if (e == hipSuccess) {
+        e = hipMemcpyAsync((char*)s->queries_mem + r->at, s->queries_host + r->at, r->bytes,
+                           hipMemcpyHostToDevice, s->upload);
+      }
+      const hipError_t es = hipStreamSynchronize(s->upload);
+      if (e == hipSuccess) e = es;
+    }
+    std::lock_guard<std::mutex> lk(s->mu);
+    if (e == hipSuccess) {
+      s->pending.push_back(r);
+      s->cv_work.notify_one();
+    } else {
+      release_queries(s, r);
+      r->status = PPSK_ERR_HIP;
+      r->error = std::string("query upload: ") + hipGetErrorString(e);
+      r->done = true;
+      s->cv_done.notify_all();
+    }
   }
-  if (e == hipSuccess) e = hipEventRecord(r->uploaded, s->upload);
-  if (device != s->device) (void)hipSetDevice(device);
-  if (e == hipSuccess) return PPSK_OK;
-  (void)hipStreamSynchronize(s->upload);
-  std::lock_guard<std::mutex> lk(s->mu);
-  release_queries(s, r);
-  return fail(PPSK_ERR_HIP, std::string("query upload: ") + hipGetErrorString(e));
 }
 
 // Rows of the next piece of the oldest request in a step of its own.
@@ -931,21 +950,14 @@ int ppsk_server_create(ppsk_set* ref, int32_t random_mode, int32_t n_clusters,
   s->t0 = std::chrono::steady_clock::now();
   const size_t query_bytes =
       align_up(std::min<size_t>((size_t)256 << 20, 4 * (size_t)max_rows * (s->per_sample + 16 * ref->n_k)));
-  // one event for each request that waits there; further ones wait in ordinary memory
   bool queries = hipMalloc(&s->queries_mem, query_bytes) == hipSuccess &&
                  hipHostMalloc((void**)&s->queries_host, query_bytes, hipHostMallocDefault) == hipSuccess;
-  for (int x = 0; x < 256 && queries; ++x) {
-    hipEvent_t ev = nullptr;
-    if (hipEventCreateWithFlags(&ev, hipEventDisableTiming) != hipSuccess) break;
-    s->uploads.push_back(ev);
-  }
   if (queries) {
     copy_host(s->queries_host, nullptr, query_bytes);  // the pages' first touch
     s->queries.init((char*)s->queries_mem, query_bytes);
   } else {
     (void)hipGetLastError();  // every request waits in ordinary memory
   }
-  s->upload_events = s->uploads;
   std::vector<hipStream_t> streams;
   if (create_slot_streams(n_slots + (queries ? 1 : 0), &streams) != PPSK_OK) {
     for (hipStream_t st : streams) hipStreamDestroy(st);
@@ -957,6 +969,12 @@ int ppsk_server_create(ppsk_set* ref, int32_t random_mode, int32_t n_clusters,
     // waited for its distance kernels (four requests 3.7 -> 3.2 ms)
     s->upload = streams.back();
     streams.pop_back();
+    try {
+      s->uploader = std::thread(uploader_main, s);
+    } catch (const std::system_error&) {
+      hipStreamDestroy(s->upload);
+      s->upload = nullptr;
+    }
   }
   for (int i = 0; i < n_slots; ++i) {
     auto* w = new Worker();
@@ -1040,10 +1058,7 @@ int ppsk_server_submit(ppsk_server* s, int64_t n_queries, const uint64_t* raw,
     r->kd.resize(nk);
   }
   std::memset(&r->res, 0, sizeof(r->res));
-  if (int rc = take_queries(s, r, raw)) {
-    delete r;
-    return rc;
-  }
+  take_queries(s, r, raw);
   {
     std::lock_guard<std::mutex> lk(s->mu);
     if (s->stop) {
@@ -1054,10 +1069,14 @@ int ppsk_server_submit(ppsk_server* s, int64_t n_queries, const uint64_t* raw,
     r->res.n_queries = n_queries;
     r->res.t_submit = now_s(s->t0);
     s->tickets[r->ticket] = r;
-    s->pending.push_back(r);
     *ticket = r->ticket;
+    if (s->upload) {
+      s->fresh.push_back(r);
+    } else {
+      s->pending.push_back(r);
+    }
   }
-  s->cv_work.notify_one();
+  (s->upload ? s->cv_upload : s->cv_work).notify_one();
   return PPSK_OK;
 }
 
@@ -1120,7 +1139,9 @@ int ppsk_server_free(ppsk_server* s) {
     s->stop = true;
   }
   s->cv_work.notify_all();
+  s->cv_upload.notify_all();
   for (auto& t : s->workers) t.join();
+  if (s->uploader.joinable()) s->uploader.join();
   {
     std::unique_lock<std::mutex> lk(s->mu);
     // every request not yet served fails; submits and waiters collect their failure
@@ -1135,6 +1156,7 @@ int ppsk_server_free(ppsk_server* s) {
       }
     }
     s->pending.clear();
+    s->fresh.clear();
     s->cv_done.notify_all();
     s->cv_done.wait(lk, [&] { return s->waiters == 0; });
     for (auto& kv : s->tickets) delete kv.second;
@@ -1146,7 +1168,6 @@ int ppsk_server_free(ppsk_server* s) {
     hipStreamSynchronize(s->upload);
     hipStreamDestroy(s->upload);
   }
-  for (hipEvent_t ev : s->upload_events) hipEventDestroy(ev);
   if (s->queries_mem) hipFree(s->queries_mem);
   if (s->queries_host) hipHostFree(s->queries_host);
   if (s->d_table) hipFree(s->d_table);
